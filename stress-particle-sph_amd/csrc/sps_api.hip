@@ -52,10 +52,13 @@ static inline unsigned nblk8(long long n) {
     unsigned b = nblk(n);
     return (b + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
 }
-// tiles of TILE receivers, a multiple of the XCD count
-static inline unsigned ntile8(long long n) {
-    unsigned b = (unsigned)((n + TILE - 1) / TILE);
-    return (b + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
+// Tiles held for n receivers, a multiple of the XCD count: n / TILE rounded
+// up, and with `strips` > 0 (tiles that end at strip ends, k_count_tiles) one more
+// per strip of the domain box, at most twice as many in all.
+static inline int ntiles(long long n, double strips) {
+    const long long plain = (n + TILE - 1) / TILE;
+    const long long extra = strips > 0 ? (long long)std::min(strips, (double)plain + 16) : 0;
+    return (int)((plain + extra + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
 }
 
 
@@ -195,6 +198,8 @@ struct sps_handle {
     DBuf<Tile> tiles;
     DBuf<StagePlan> plans;
     int ntile_n = 0, ntile_s = 0;
+    DBuf<int> tile_start;         // k_count_tiles: first tile of each strip (scratch)
+    DBuf<int2> tile_range;        // per tile: its receivers
     double h_uniform = 0.0;   // the smoothing length of every particle, or 0 when they differ
     bool mixed = false;       // SPS_MODE_FAST: the mixed-precision stage kernels
     // pair lists kept over steps (mixed form): built with this skin, reused
@@ -248,7 +253,7 @@ struct sps_handle {
     PairLists lists() {
         return PairLists{list_ia.p,  list_ib.p,  list_wa.p, list_gxa.p,          list_gya.p,
                          list_gxb.p, list_gyb.p, xsph ? list_wb.p : nullptr, deg_a.p, deg_b.p,
-                         tile_ok.p,  ntile_n,    tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
+                         tile_ok.p,  ntile_n,    tile_range.p, tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
     }
 };
 
@@ -525,8 +530,15 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     rc |= dalloc(h->tmp_orig, nt2); rc |= dalloc(h->tmp_src, nt2); rc |= dalloc(h->proc, nt2);
     rc |= dalloc(h->moved, nblk(nt2));
     rc |= dalloc(h->proc_to_slot, nt2); rc |= dalloc(h->cnt, nt2); rc |= dalloc(h->off, nt2);
-    h->ntile_n = (int)ntile8(nn);
-    h->ntile_s = (int)ntile8(nt - nn);
+    // strips of 8 cells 2h wide with h = 0.8 dx, as small as the decks have it
+    // (with smaller h and a body across the whole box k_count_tiles may not find
+    // room for tiles that end at strip ends and falls back)
+    const double strips = h->mixed || !(params->dx > 0) ? 0.0
+        : (params->xmax_domain[0] - params->xmin_domain[0]) / (STRIP * 1.6 * params->dx) + 2;
+    h->ntile_n = ntiles(nn, strips);
+    h->ntile_s = ntiles(nt - nn, strips);
+    rc |= dalloc(h->tile_start, 2 * (size_t)TSTART_MAX);
+    rc |= dalloc(h->tile_range, (size_t)h->ntile_n + h->ntile_s);
     {
         const size_t wa = (size_t)(h->ntile_n + h->ntile_s) * LGROUPS * TILE, wb = (size_t)h->ntile_n * LGROUPS * TILE;
         rc |= dalloc(h->list_ia, wa); rc |= dalloc(h->list_wa, wa); rc |= dalloc(h->list_gxa, wa);
@@ -712,6 +724,8 @@ static int search(sps_handle *h, bool fresh_list) {
     LAUNCH(K_PROC, nblk(nt2), BLOCK, k_proc_slot, h->cell.p, h->kstart.p, h->cstart_rm.p, h->grid.p, h->proc.p,
            nn, nt, nt2);
     LAUNCH(K_PROC, nblk(nt2), BLOCK, k_proc_to_slot, h->proc.p, h->proc_to_slot.p, nt2);
+    LAUNCH(K_PROC, 2, TILES_BLOCK, k_count_tiles, h->kstart.p, h->grid.p, h->tile_start.p, h->tile_range.p, h->ntile_n,
+           h->ntile_s, nn, nt, h->mixed ? 0 : 1);
     // counts, offsets, split
     LAUNCH(K_SPLIT, nblk(nt2), BLOCK, k_surf_zero, h->cnt.p, (long long)nt2);
     LAUNCH(K_SPLIT, 1, 64, k_split_reset, h->split.p, fresh_list ? 1 : 0);
@@ -727,26 +741,26 @@ static int search(sps_handle *h, bool fresh_list) {
             HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
             HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
             if (!h->mixed)
-                k_count_lists<KIND_SP, true><<<ntile8(nt - nn), TILE, lds_count(h), h->stream2>>>(
-                    V, C.x.p, C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, nn, nt - nn, h->skin);
+                k_count_lists<KIND_SP, true><<<h->ntile_s, TILE, lds_count(h), h->stream2>>>(
+                    V, C.x.p, C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
             else
-                k_count_lists<KIND_SP, false><<<ntile8(nt - nn), TILE, lds_count(h), h->stream2>>>(
-                    V, C.x.p, C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, nn, nt - nn, h->skin);
+                k_count_lists<KIND_SP, false><<<h->ntile_s, TILE, lds_count(h), h->stream2>>>(
+                    V, C.x.p, C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
             HIP_TRY(hipEventRecord(h->ev_join, h->stream2));
         }
         // the mixed-precision stage kernels compute the kernel values themselves
         if (nn > 0 && !h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, ntile8(nn), TILE, lds_count(h), (k_count_lists<KIND_NODE, true>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, 0, nn, h->skin);
+            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_n, TILE, lds_count(h), (k_count_lists<KIND_NODE, true>), V, C.x.p,
+                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
         if (nn > 0 && h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, ntile8(nn), TILE, lds_count(h), (k_count_lists<KIND_NODE, false>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, 0, nn, h->skin);
+            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_n, TILE, lds_count(h), (k_count_lists<KIND_NODE, false>), V, C.x.p,
+                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
         if (!fork && nt > nn && !h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, ntile8(nt - nn), TILE, lds_count(h), (k_count_lists<KIND_SP, true>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, nn, nt - nn, h->skin);
+            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_s, TILE, lds_count(h), (k_count_lists<KIND_SP, true>), V, C.x.p,
+                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
         if (!fork && nt > nn && h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, ntile8(nt - nn), TILE, lds_count(h), (k_count_lists<KIND_SP, false>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, nn, nt - nn, h->skin);
+            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_s, TILE, lds_count(h), (k_count_lists<KIND_SP, false>), V, C.x.p,
+                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
         if (nt2 > nt)
             LAUNCH(K_COUNT_DUMMY, nblk8(nt2 - nt), BLOCK, k_count, C.x.p, C.hsml.p, h->cell.p, h->kstart.p, h->proc.p,
                    h->grid.p, h->cnt.p, h->split.p, nn, nt, nt, nt2);
@@ -824,10 +838,10 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
         // the outside approach's stress_point_update + adapt_stress2 on the
         // step's lists (2_...:99-109)
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
                        tanfi, coh, hu, nn);
         if (nt > nn)
-            LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
+            LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
                        h->dp, time_sph, 0.0, 0, adapt, hu, nn, nt, stepv, nullptr);
     }
     LAUNCH(K_RK_INIT, nblk(nt2), BLOCK, k_stage_first, SB, W, adapt, tanfi, coh, nn, nt, nt2);
@@ -842,28 +856,28 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
             HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
             HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
             hipStream_t s2 = h->stream2;
-            k_spu_nodes_mix<<<ntile8(nn), TILE, LAY_SPU_NODES_MIX.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, hu, nn);
+            k_spu_nodes_mix<<<h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, hu, nn);
             if (bcs)
                 k_bcs<<<nblk(nn), BLOCK, 0, s2>>>(SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p,
                                                  h->ifsigman, h->normal.p, nn, nullptr, nullptr);
             // the nodes' artificial viscosity reads only node data, after the
             // node side and the second BC call (k_deriv_nodes_mix takes it)
             if (h->dp.do_av)
-                k_av_nodes_mix<<<ntile8(nn), TILE, LAY_DERIV_NODES_MIX.bytes, s2>>>(SB, V, PL, h->dp, hu,
+                k_av_nodes_mix<<<h->ntile_n, TILE, LAY_DERIV_NODES_MIX.bytes, s2>>>(SB, V, PL, h->dp, hu,
                                                                                      h->av_nodes.p, nn);
             HIP_TRY(hipEventRecord(h->ev_join, s2));
         } else {
             if (nn > 0)
-                LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
+                LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
                            tanfi, coh, hu, nn);
             if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
         }
         if (nt > nn)
-            LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
+            LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
                        h->dp, time_sph, f2rk[st], 1, adapt, hu, nn, nt, stepv, h->sig2.p);
         if (fork) HIP_TRY(hipStreamWaitEvent(h->stream, h->ev_join, 0));
         if (nn > 0)
-            LAUNCH_LDS(K_DERIV_NODES, ntile8(nn), TILE, LAY_DERIV_NODES_MIX.bytes, k_deriv_nodes_mix, SB, W, V, PL,
+            LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, LAY_DERIV_NODES_MIX.bytes, k_deriv_nodes_mix, SB, W, V, PL,
                        h->dp, gxg, gyg, f2rk[st], h->err.p, hu, nn, stepv, nt > nn ? h->sig2.p : SB.stress,
                        fork && h->dp.do_av ? h->av_nodes.p : nullptr);
         if (st == 3 && nt2 > nt)
@@ -879,17 +893,17 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
     }
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
     if (nn > 0)
-        LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt, tanfi,
+        LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt, tanfi,
                    coh, hu, nn);
     if (nt > nn)
-        LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL, h->dp,
+        LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL, h->dp,
                    time_sph, 0.0, 0, adapt, hu, nn, nt, stepv, nullptr);
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
     const bool xsph = h->xsph && h->p.update_x;
     if (xsph && nn > 0)
-        LAUNCH_LDS(K_XSPH, ntile8(nn), TILE, LAY_XSPH_MIX.bytes, (k_xsph_mix<KIND_NODE>), SB, V, PL, hu, h->xsph_v.p);
+        LAUNCH_LDS(K_XSPH, h->ntile_n, TILE, LAY_XSPH_MIX.bytes, (k_xsph_mix<KIND_NODE>), SB, V, PL, hu, h->xsph_v.p);
     if (xsph && nt > nn)
-        LAUNCH_LDS(K_XSPH, ntile8(nt - nn), TILE, LAY_XSPH_MIX.bytes, (k_xsph_mix<KIND_SP>), SB, V, PL, hu, h->xsph_v.p);
+        LAUNCH_LDS(K_XSPH, h->ntile_s, TILE, LAY_XSPH_MIX.bytes, (k_xsph_mix<KIND_SP>), SB, V, PL, hu, h->xsph_v.p);
     LAUNCH(K_POSITION, nblk(nt), BLOCK, k_position, SB, W, dt, h->p.update_x, nn, nt,
            xsph ? (const double2 *)h->xsph_v.p : (const double2 *)nullptr, h->err.p, 0);
     if (shift >= 0 && h->p.update_x && nn > 0) {
@@ -1056,9 +1070,9 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
     if (h->outside && h->p.sph_shift && itimestep > 1 && (itimestep - 1) % h->p.shift_update == 0) {
         // stress_point_update + adapt_stress2 on the new lists (2_...:99-109)
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
         if (nt > nn)
-            LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp,
+            LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp,
                        time_sph, 0.0, 0, adapt, nn, nt, nullptr);
     }
     const bool lf = h->integrator == SPS_INTEGRATOR_LEAPFROG;
@@ -1074,23 +1088,23 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
         const double kdt = h->lf_first ? 0.5 * dt : dt;
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, bci_prev);
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, bci_prev);
         if (nt > nn)
-            LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph,
+            LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph,
                        0.0, 0, adapt, nn, nt, nullptr);
         const bool av = h->dp.do_av && nn > 0;
-        if (av) LAUNCH_LDS(K_AV_NODES, ntile8(nn), TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
+        if (av) LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
         if (nn > 0)
-            LAUNCH_LDS(K_DERIV_NODES, ntile8(nn), TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp,
+            LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp,
                        gxg, gyg, 1.0, h->err.p, nn, SB.stress, av ? h->av_nodes.p : nullptr);
         LAUNCH(K_STAGE_BEGIN, nblk(nn), BLOCK, k_lf_kick, SB, W, kdt, nn);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
         if (nt > nn)
-            LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
+            LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
                        1.0, 1, adapt, nn, nt, nullptr);
         if (nt2 > nt) LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
         LAUNCH(K_RK_FINAL, nblk(nt), BLOCK, k_lf_final, SB, W, dt, adapt, tanfi, coh, nn, nt, h->err.p);
@@ -1115,26 +1129,26 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
             HIP_TRY(hipEventRecord(h->ev_fork, s));
             HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
             hipStream_t s2 = h->stream2;
-            k_spu_nodes<<<ntile8(nn), TILE, LAY_SPU_NODES.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, nn);
+            k_spu_nodes<<<h->ntile_n, TILE, LAY_SPU_NODES.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, nn);
             if (bcs)
                 k_bcs<<<nblk(nn), BLOCK, 0, s2>>>(SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman,
                                                  h->normal.p, nn, st ? bci_cur : nullptr,
                                                  st ? nullptr : bci_prev);
-            if (av) k_av_nodes<<<ntile8(nn), TILE, lds_av_nodes(h), s2>>>(SB, V, PL, h->dp, h->av_nodes.p, nn);
+            if (av) k_av_nodes<<<h->ntile_n, TILE, lds_av_nodes(h), s2>>>(SB, V, PL, h->dp, h->av_nodes.p, nn);
             HIP_TRY(hipEventRecord(h->ev_join, s2));
         } else {
             if (nn > 0)
-                LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh,
+                LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh,
                            nn);
             if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, st ? bci_cur : nullptr, st ? nullptr : bci_prev);
-            if (av) LAUNCH_LDS(K_AV_NODES, ntile8(nn), TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
+            if (av) LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
         }
         if (nt > nn)
-            LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
+            LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
                        f2rk[st], 1, adapt, nn, nt, h->sig2.p);
         if (fork) HIP_TRY(hipStreamWaitEvent(s, h->ev_join, 0));
         if (nn > 0)
-            LAUNCH_LDS(K_DERIV_NODES, ntile8(nn), TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp, gxg,
+            LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp, gxg,
                        gyg, f2rk[st], h->err.p, nn, nt > nn ? h->sig2.p : SB.stress, av ? h->av_nodes.p : nullptr);
         if (st == 3 && nt2 > nt)
             LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
@@ -1145,18 +1159,18 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
                hook ? 1 : 0, h->err.p);
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
     if (nn > 0)
-        LAUNCH_LDS(K_SPU_NODES, ntile8(nn), TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+        LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
     if (nt > nn)
-        LAUNCH_LDS(K_SP_UPDATE, ntile8(nt - nn), TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph, 0.0,
+        LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph, 0.0,
                    0, adapt, nn, nt, nullptr);
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
     if (h->bcint && nn > 0)   // the next step's first BC calls see this step's list
         LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcint_keep, h->nodeinfo.p, SB.orig, h->bcint_prev.p, nn);
     const bool xsph = h->xsph && h->p.update_x;
     if (xsph && nn > 0)
-        LAUNCH_LDS(K_XSPH, ntile8(nn), TILE, LAY_XSPH.bytes, (k_xsph<KIND_NODE>), SB, V, PL, h->xsph_v.p);
+        LAUNCH_LDS(K_XSPH, h->ntile_n, TILE, LAY_XSPH.bytes, (k_xsph<KIND_NODE>), SB, V, PL, h->xsph_v.p);
     if (xsph && nt > nn)
-        LAUNCH_LDS(K_XSPH, ntile8(nt - nn), TILE, LAY_XSPH.bytes, (k_xsph<KIND_SP>), SB, V, PL, h->xsph_v.p);
+        LAUNCH_LDS(K_XSPH, h->ntile_s, TILE, LAY_XSPH.bytes, (k_xsph<KIND_SP>), SB, V, PL, h->xsph_v.p);
     LAUNCH(K_POSITION, nblk(nt), BLOCK, k_position, SB, W, dt, h->p.update_x, nn, nt, xsph ? h->xsph_v.p : nullptr,
            h->err.p, lf ? 1 : 0);
     if (h->p.update_x) {   // 2_...:150-154
@@ -1512,7 +1526,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
     dfree(h->cnt); dfree(h->off); dfree(h->scan_tmp); dfree(h->ctot); dfree(h->cstart_rm); dfree(h->err);
     dfree(h->list_ia); dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya); dfree(h->list_ib);
-    dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tiles); dfree(h->plans);
+    dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->tiles); dfree(h->plans);
     dfree(h->list_wb); dfree(h->xsph_v);
     dfree(h->x_build); dfree(h->dmax); dfree(h->surr_count); dfree(h->surr_slot); dfree(h->surr_sn);
     dfree(h->surr_str); dfree(h->surr_feat); dfree(h->surr_stats); dfree(h->plog); dfree(h->surr_mat);

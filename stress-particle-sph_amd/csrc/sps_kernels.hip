@@ -1003,10 +1003,10 @@ struct Tile {
     bool fits;              // one strip, at most TROWS rows
 };
 
-__device__ __forceinline__ Tile make_tile(int base, int count, int kr, const SearchView &V, const WalkCtx &C) {
+__device__ __forceinline__ Tile make_tile(int2 range, int kr, const SearchView &V, const WalkCtx &C) {
     Tile T;
-    T.first = base + tile_index() * TILE;
-    T.end = min(T.first + TILE, base + count);
+    T.first = range.x;
+    T.end = range.y;
     T.last = min(T.end, V.kstart[kr * C.L + C.g.ndivt]) - 1;
     T.fits = false;
     T.x0 = T.w = T.wy0 = T.nrows = 0;
@@ -1021,6 +1021,86 @@ __device__ __forceinline__ Tile make_tile(int base, int count, int kr, const Sea
     T.nrows = wy1 - T.wy0 + 1;
     T.fits = (cxl / STRIP) * STRIP == T.x0 && T.nrows <= TROWS;
     return T;
+}
+
+// Receivers [x, y) of every tile (empty past the last one): block 0 the node
+// tiles, block 1 the stress points'.  A tile that crosses from one strip into
+// the next has no window and walks the global storage, 86 us against 15 us
+// for a tile in its strip on the 10 k-particle collapse, where one tile in
+// four crossed and every stage kernel took as long as its crossing tiles; so
+// each strip starts a tile of its own (the last tile of a strip is partly
+// idle: half a tile per strip of about 75 at 1 M nodes).  The out-of-domain
+// particles' bucket counts as one more strip.  When the strips would need
+// more tiles than the capacity cap holds (bodies much taller than wide in
+// many strips), or with aligned = 0, the receivers are cut every TILE slots.
+// aligned is 0 for the mixed form: its positions are rounded relative to the
+// tile's first receiver, so its tiles are part of its result.  Launch two
+// blocks of TILES_BLOCK threads; tstart holds TSTART_MAX entries per block.
+constexpr int TILES_BLOCK = 1024;
+constexpr int TSTART_MAX = 1 << 16;
+
+__global__ void __launch_bounds__(TILES_BLOCK) k_count_tiles(const int *__restrict__ kstart, const Grid *__restrict__ g,
+                                                       int *__restrict__ tstart, int2 *__restrict__ range,
+                                                       int cap_n, int cap_s, int nn, int nt, int aligned) {
+    __shared__ int wsum[TILES_BLOCK / 64];
+    __shared__ int carry;
+    const int k = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int base = k ? nn : 0, end = k ? nt : nn, cap = k ? cap_s : cap_n;
+    int2 *__restrict__ out = range + (k ? cap_n : 0);
+    int *__restrict__ ts = tstart + (k ? TSTART_MAX : 0);
+    const int ndivt = g->ndivt, ndivy = g->ndivy, ndivx = ndivt > 0 ? g->ndivx : 0;
+    const int *__restrict__ ks = kstart + k * (ndivt + 1);
+    const int nstrip = (ndivx + STRIP - 1) / STRIP, ngroup = nstrip + 1;
+    // group s: the strip's slots; the last group: the out-of-domain bucket
+    auto slots = [&](int s) {
+        const int lo = s < nstrip ? ks[s * STRIP * ndivy] : ks[ndivt];
+        const int hi = s < nstrip ? ks[(s + 1 < nstrip ? (s + 1) * STRIP : ndivx) * ndivy] : end;
+        return make_int2(lo, hi);
+    };
+    bool strips = aligned && ngroup <= TSTART_MAX;
+    int total = 0;
+    if (strips) {
+        if (t == 0) carry = 0;
+        __syncthreads();
+        for (int s0 = 0; s0 < ngroup; s0 += TILES_BLOCK) {
+            const int s = s0 + t;
+            int n = 0;
+            if (s < ngroup) {
+                const int2 r = slots(s);
+                n = (r.y - r.x + TILE - 1) / TILE;
+            }
+            int incl = n;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += v;
+            }
+            if (lane == 63) wsum[wave] = incl;
+            __syncthreads();
+            int before = carry, sum = 0;
+            for (int w = 0; w < TILES_BLOCK / 64; ++w) {
+                if (w < wave) before += wsum[w];
+                sum += wsum[w];
+            }
+            if (s < ngroup) ts[s] = before + incl - n;
+            __syncthreads();
+            if (t == 0) carry += sum;
+            __syncthreads();
+        }
+        total = carry;
+        strips = total <= cap;
+    }
+    if (strips) {   // one wave per group, its tiles across the lanes
+        for (int s = wave; s < ngroup; s += TILES_BLOCK / 64) {
+            const int2 r = slots(s);
+            const int at = ts[s];
+            for (int q = lane; r.x + q * TILE < r.y; q += 64)
+                out[at + q] = make_int2(r.x + q * TILE, min(r.x + (q + 1) * TILE, r.y));
+        }
+        for (int q = total + t; q < cap; q += TILES_BLOCK) out[q] = make_int2(end, end);
+    } else {
+        for (int q = t; q < cap; q += TILES_BLOCK)
+            out[q] = make_int2(min(base + q * TILE, end), min(base + (q + 1) * TILE, end));
+    }
 }
 
 // Staging plan of one kind's window, in LDS: the strip's main run and the
@@ -1232,6 +1312,7 @@ struct PairLists {
     unsigned short *deg_a, *deg_b;  // per slot: nodes and stress points / nodes
     unsigned char *ok;              // per tile (node tiles, then SP tiles): lists usable
     int ntile_n;                    // node tiles
+    const int2 *range;              // per tile: its receivers (k_count_tiles)
     // each tile's extent and (when it fits) the staging plan of every partner
     // kind, as the search computed them: the stage kernels load them in one
     // round trip instead of deriving them again through dependent loads
@@ -1341,14 +1422,13 @@ template <int KR, bool FILL>
 __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double2 *__restrict__ x,
                                                       const double *__restrict__ hsml,
                                                       unsigned *__restrict__ cnt, Split *__restrict__ split,
-                                                      PairLists PL, double h_uniform, int base, int count,
-                                                      double skin) {
+                                                      PairLists PL, double h_uniform, double skin) {
     __shared__ StagePlan pl[3];
     constexpr const LdsLayout &LY = LAY_COUNT;
     const WalkCtx C = walk_ctx(V);
-    const Tile T = make_tile(base, count, KR, V, C);
     const int tile = tile_index();
     const int ltile = KR == KIND_NODE ? tile : PL.ntile_n + tile;
+    const Tile T = make_tile(PL.range[ltile], KR, V, C);
     if (threadIdx.x == 0) PL.tiles[ltile] = T;
     if (T.first >= T.end) return;
     const int r = T.first + (int)threadIdx.x;

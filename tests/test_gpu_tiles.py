@@ -1,0 +1,79 @@
+"""Tiles of the pair kernels at the sizes where their cutting can go wrong,
+against the oracle, every state field and the pair list bit for bit.
+
+The receivers of a tile come from one strip of the cell grid; a body of fewer
+cells than a strip, a last strip one cell wide, strips that fill their tiles
+exactly or by one particle over, strips of a low body (more strips than the
+tile capacity, which falls back to tiles cut every TILE slots) and particles
+outside the domain box are the edges.
+"""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from conftest import ORACLE_LIB, bits_equal, deck_dir, describe_diff, load_pkg
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("x", "vel", "stress", "internal_vars", "f_drucker", "displ", "grad_u", "ddev_strn", "f_bound", "art_visc",
+          "if_out_domain")
+
+# name: (deck, lattice columns, rows, smoothing factor, other changes)
+BODIES = {
+    "one_particle_row_strip": ("c1_collapse", 21, 2, 1.2, {}),
+    "narrower_than_a_strip": ("c1_collapse", 7, 120, 1.2, {}),
+    "last_strip_one_cell": ("c1_collapse", 21, 90, 1.2, {}),
+    "full_tiles": ("c1_collapse", 64, 64, 1.0, {}),           # 16 columns a strip: 4 tiles exactly
+    "one_over": ("c1_collapse", 65, 65, 1.0, {}),
+    "low_body_many_strips": ("c1_collapse", 400, 4, 0.5, {}),  # falls back: cells one spacing wide
+    "cspm_moving": ("t2_cspm", 50, 37, 1.2, {}),
+    "xsph_two_points": ("t4_xsph", 43, 31, 1.2, {"npoints": 2}),
+    "four_points": ("t5_sp4", 37, 41, 1.2, {}),
+    "four_points_xsph": ("t5_sp4", 30, 30, 1.2, {"xsph": True}),
+}
+
+
+def body(name):
+    sps = load_pkg()
+    deck_name, nx, ny, sml, change = BODIES[name]
+    deck = dataclasses.replace(sps.read_deck(deck_dir(deck_name)), sml=sml, **change)
+    dx = deck.dx
+    # the lattice counts are int(length / dx + 1): half a spacing beyond the last column
+    deck.xs = (0.0, (nx - 0.5) * dx, 0.0, (nx - 0.5) * dx)
+    deck.ys = (0.0, 0.0, (ny - 0.5) * dx, (ny - 0.5) * dx)
+    deck.dy = dx
+    if name == "low_body_many_strips":   # the box close around the body
+        deck.xmin_domain = np.array([-8 * dx, -8 * dx])
+        deck.xmax_domain = np.array([(nx + 4) * dx, (ny + 8) * dx])
+        deck.dummy_nodes, deck.walls = False, []
+    return sps, deck
+
+
+def compare(gpu, ora, what):
+    g, o = gpu.get_state(), ora.get_state()
+    bad = [f"{k}: {describe_diff(o[k], g[k])}" for k in FIELDS if not bits_equal(o[k], g[k])]
+    p, q = gpu.get_pairs(), ora.get_pairs()
+    bad += [f"pairs.{k}" for k in p if not bits_equal(q[k], p[k])]
+    assert not bad, f"{what}: " + "; ".join(bad)
+
+
+@pytest.mark.parametrize("name", sorted(BODIES))
+def test_tiles_against_oracle(name):
+    sps, deck = body(name)
+    gpu = sps.Simulation.from_deck(deck)
+    ora = sps.Simulation.from_deck(deck, lib_path=ORACLE_LIB)
+    print(f"[tiles] {name}: {gpu.n2} particles", flush=True)
+    # a moving start: pair counts rise and fall, so pairs lie on both sides of
+    # the list's high-water mark; a few particles start outside the domain box
+    rng = np.random.default_rng(11)
+    st = sps.initial_state(gpu.parts, gpu.niv)
+    st["vel"][:gpu.n] = 2.0 * rng.standard_normal((gpu.n, 2))
+    for k in (3, gpu.nn + 5):
+        st["x"][k] = deck.xmax_domain + 10.0 * deck.dx
+    for sim in (gpu, ora):
+        sim.set_state(st)
+    for step in range(1, 7):
+        gpu.step(1)
+        ora.step(1)
+        compare(gpu, ora, f"{name} step {step}")
