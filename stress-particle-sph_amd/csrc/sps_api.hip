@@ -158,7 +158,8 @@ struct sps_handle {
     DBuf<unsigned char> moved;    // per block of slots: the permutation moves a particle of it
     DBuf<unsigned> cnt, off, scan_tmp, ctot, cstart_rm;
     // per-step pair lists of the tiled stage kernels
-    DBuf<unsigned long long> list_ia, list_ib;
+    DBuf<unsigned long long> list_ia, list_ib, list_iah, list_ibh;
+    int list_words = 12;          // words of four entries per receiver and list
     DBuf<float4> list_wa, list_gxa, list_gya, list_gxb, list_gyb, list_wb;
     bool xsph = false;            // XSPH position update (list B also for stress points, with w)
     DBuf<double2> xsph_v;
@@ -251,9 +252,9 @@ struct sps_handle {
     long long prof_n[32] = {0};
 
     PairLists lists() {
-        return PairLists{list_ia.p,  list_ib.p,  list_wa.p, list_gxa.p,          list_gya.p,
+        return PairLists{list_ia.p,  list_ib.p,  list_iah.p, list_ibh.p, list_wa.p, list_gxa.p, list_gya.p,
                          list_gxb.p, list_gyb.p, xsph ? list_wb.p : nullptr, deg_a.p, deg_b.p,
-                         tile_ok.p,  ntile_n,    tile_range.p, tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
+                         tile_ok.p,  list_words, ntile_n,    tile_range.p, tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
     }
 };
 
@@ -540,12 +541,20 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     rc |= dalloc(h->tile_start, 2 * (size_t)TSTART_MAX);
     rc |= dalloc(h->tile_range, (size_t)h->ntile_n + h->ntile_s);
     {
-        const size_t wa = (size_t)(h->ntile_n + h->ntile_s) * LGROUPS * TILE, wb = (size_t)h->ntile_n * LGROUPS * TILE;
+        // 48 entries a list, and 24 more per further stress point a node or
+        // cell (about 18 partners within 2h = 2.4 dx each); a receiver with
+        // more leaves its tile without lists.  (The mixed form keeps 48: which
+        // tiles it walks in double precision is part of its result.)
+        if (!h->mixed) h->list_words = 12 + 6 * (std::min(4, (h->ns + nn - 1) / nn) - 1);
+        if (h->list_words < 12) h->list_words = 12;
+        const size_t wt = (size_t)h->list_words * TILE;
+        const size_t wa = (size_t)(h->ntile_n + h->ntile_s) * wt, wb = (size_t)h->ntile_n * wt;
         rc |= dalloc(h->list_ia, wa); rc |= dalloc(h->list_wa, wa); rc |= dalloc(h->list_gxa, wa);
         rc |= dalloc(h->list_gya, wa);
         // list B: node tiles; with XSPH stress-point tiles too, and its w
         rc |= dalloc(h->list_ib, h->xsph ? wa : wb); rc |= dalloc(h->list_gxb, wb); rc |= dalloc(h->list_gyb, wb);
         if (h->xsph) rc |= dalloc(h->list_wb, wa) | dalloc(h->xsph_v, (size_t)nt);
+        if (!h->mixed) rc |= dalloc(h->list_iah, wa) | dalloc(h->list_ibh, h->xsph ? wa : wb);
     }
     rc |= dalloc(h->deg_a, nt); rc |= dalloc(h->deg_b, h->xsph ? nt : nn);
     rc |= dalloc(h->tile_ok, h->ntile_n + h->ntile_s + 1);
@@ -773,6 +782,10 @@ static int search(sps_handle *h, bool fresh_list) {
     LAUNCH(K_SPLIT, nblk(nt2), BLOCK, k_split, h->cnt.p, h->off.p, nt2, h->split.p);
     LAUNCH(K_SPLIT, 1, 64, k_split_partner, C.x.p, C.hsml.p, h->cell.p, h->kstart.p, h->proc.p, h->off.p,
                                      h->proc_to_slot.p, h->grid.p, h->split.p, nn, nt, h->pairs_total.p);
+    if (!h->mixed) {
+        const SearchView V{h->cell.p, h->kstart.p, h->proc.p, h->cnt.p, h->off.p, h->grid.p, h->split.p, h->p.pi};
+        LAUNCH(K_SPLIT, h->ntile_n + h->ntile_s, TILE, k_list_order, V, h->lists());
+    }
     HIP_TRY(hipGetLastError());
     h->search_stale = true;
     return 0;
@@ -1525,7 +1538,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->cellkey); dfree(h->new_cell); dfree(h->cell); dfree(h->kcount); dfree(h->kstart);
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
     dfree(h->cnt); dfree(h->off); dfree(h->scan_tmp); dfree(h->ctot); dfree(h->cstart_rm); dfree(h->err);
-    dfree(h->list_ia); dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya); dfree(h->list_ib);
+    dfree(h->list_ia); dfree(h->list_iah); dfree(h->list_ibh); dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya); dfree(h->list_ib);
     dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->tiles); dfree(h->plans);
     dfree(h->list_wb); dfree(h->xsph_v);
     dfree(h->x_build); dfree(h->dmax); dfree(h->surr_count); dfree(h->surr_slot); dfree(h->surr_sn);

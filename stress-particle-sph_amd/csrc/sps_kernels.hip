@@ -1300,17 +1300,20 @@ __global__ void k_stage_begin(StateBufs S, Work W, double c1, int adapt, double 
 // point's node and dummy partners; list B: a node's node partners.  Entries
 // come four to a word, words of a tile lane-interleaved, so a wave reads its
 // lanes' next four entries with one coalesced load per array.
-constexpr int LMAX = 48;            // entries per receiver and list; more marks the tile unlisted
-constexpr int LGROUPS = LMAX / 4;
-
+// A tile without a window (a narrow strip, more partners than the capacity:
+// every node tile with two or more stress points a cell) has lists too, of
+// 32-bit entries kind << 30 | storage slot whose upper halves are the words
+// of a second array; its walks read the partners' fields from the state.
 struct PairLists {
-    unsigned long long *ia, *ib;    // [tile][LGROUPS][TILE]: four entries per word
+    unsigned long long *ia, *ib;    // [tile][lg][TILE]: four entries per word
+    unsigned long long *iah, *ibh;  // the same, upper halves of the entries by slot
     float4 *wa, *gxa, *gya;         // list A: w, dW/dx_r, dW/dy_r of those entries
     float4 *gxb, *gyb;              // list B (nodes): dW/dx_r, dW/dy_r
     float4 *wb;                     // list B: w (XSPH only; null otherwise, and then stress
                                     // points have no list B)
     unsigned short *deg_a, *deg_b;  // per slot: nodes and stress points / nodes
-    unsigned char *ok;              // per tile (node tiles, then SP tiles): lists usable
+    unsigned char *ok;              // per tile (node tiles, then SP tiles): LIST_*
+    int lg;                         // words per receiver and list; more entries: LIST_NONE
     int ntile_n;                    // node tiles
     const int2 *range;              // per tile: its receivers (k_count_tiles)
     // each tile's extent and (when it fits) the staging plan of every partner
@@ -1324,6 +1327,10 @@ struct PairLists {
     int *nodeinfo;
 };
 
+// What a tile's lists hold: nothing (a receiver has more partners than they
+// take), window indices, or storage slots.
+enum { LIST_NONE = 0, LIST_WINDOW = 1, LIST_SLOTS = 2 };
+
 // Wave `wave` of the block copies the search's plan of kind K for tile
 // ltile into the shared plan (the other waves return at once); the caller
 // puts a barrier after it, as after plan_kind.
@@ -1335,9 +1342,22 @@ __device__ __forceinline__ void load_plan(const PairLists &PL, int ltile, int wa
     for (int i = (int)(threadIdx.x & 63); i < (int)(sizeof(StagePlan) / sizeof(int)); i += 64) dst[i] = src[i];
 }
 
-__device__ __forceinline__ size_t word_at(int tile, int g) {
-    return ((size_t)tile * LGROUPS + g) * TILE + threadIdx.x;
+__device__ __forceinline__ size_t word_at(int lg, int tile, int g) {
+    return ((size_t)tile * lg + g) * TILE + threadIdx.x;
 }
+
+// A list entry of a window and of the storage.
+template <bool SLOTS> struct ListEntry {
+    static __device__ __forceinline__ unsigned make(int kind, int j) {
+        return SLOTS ? ((unsigned)kind << 30) | (unsigned)j : (unsigned)((kind << 14) | j);
+    }
+    static __device__ __forceinline__ unsigned get(unsigned long long lo, unsigned long long hi, int k) {
+        const unsigned e = (unsigned)((lo >> (16 * k)) & 0xffff);
+        return SLOTS ? e | ((unsigned)((hi >> (16 * k)) & 0xffff) << 16) : e;
+    }
+    static __device__ __forceinline__ int kind(unsigned e) { return (int)(SLOTS ? e >> 30 : e >> 14); }
+    static __device__ __forceinline__ int index(unsigned e) { return (int)(SLOTS ? e & 0x3fffffffu : e & 0x3fffu); }
+};
 
 __device__ __forceinline__ void set4(float4 &v, int k, float a) {
     if (k == 0) v.x = a;
@@ -1351,44 +1371,53 @@ __device__ __forceinline__ float get4(const float4 &v, int k) {
 }
 
 // One lane's list being written: entries gathered four to a word in a
-// register, each full word stored.
+// register, each full word stored (hp: the words of the upper halves).
 struct IdxWriter {
-    unsigned long long idx = 0;
+    unsigned long long idx = 0, hi = 0;
     int n = 0;
-    __device__ __forceinline__ void put(int tile, unsigned long long *ip, unsigned e) {
+    template <bool SLOTS>
+    __device__ __forceinline__ void put(int lg, int tile, unsigned long long *ip, unsigned long long *hp, unsigned e) {
         const int k = n & 3;
-        if (k == 0) idx = 0;
-        idx |= (unsigned long long)e << (16 * k);
-        if (k == 3 && n < LMAX) ip[word_at(tile, n >> 2)] = idx;
+        if (k == 0) idx = hi = 0;
+        idx |= (unsigned long long)(e & 0xffff) << (16 * k);
+        if (SLOTS) hi |= (unsigned long long)(e >> 16) << (16 * k);
+        if (k == 3 && n < 4 * lg) {
+            ip[word_at(lg, tile, n >> 2)] = idx;
+            if (SLOTS) hp[word_at(lg, tile, n >> 2)] = hi;
+        }
         ++n;
     }
-    __device__ __forceinline__ void finish(int tile, unsigned long long *ip) {
-        if ((n & 3) != 0 && n < LMAX) ip[word_at(tile, n >> 2)] = idx;
+    __device__ __forceinline__ void finish(int lg, int tile, unsigned long long *ip, unsigned long long *hp) {
+        if ((n & 3) != 0 && n < 4 * lg) {
+            ip[word_at(lg, tile, n >> 2)] = idx;
+            if (hp) hp[word_at(lg, tile, n >> 2)] = hi;
+        }
     }
 };
 
-// Kernel values of a lane's n list entries (n <= LMAX), computed a word at a
+// Kernel values of a lane's n list entries (n <= 4 lg), computed a word at a
 // time with the lanes of a wave in step, so that the stores are whole
 // coalesced words: kernel() of the receiver-side dx, as the stage kernels'
 // global walk computes it.
-template <typename Fields>
-__device__ __forceinline__ void fill_kernel_values(const unsigned long long *ip, float4 *wp, float4 *gxp,
-                                                   float4 *gyp, int tile, int n, const Fields &A, double2 xr,
-                                                   double hr, double h_uniform, double pi, KernelFactor &kf) {
+template <bool SLOTS, typename Fields>
+__device__ __forceinline__ void fill_kernel_values(int lg, const unsigned long long *ip, const unsigned long long *hp,
+                                                   float4 *wp, float4 *gxp, float4 *gyp, int tile, int n,
+                                                   const Fields &A, double2 xr, double hr, double h_uniform,
+                                                   double pi, KernelFactor &kf) {
     const int ng = (n + 3) >> 2;
     // the lane's own words, written by its walk: the next one is loaded
     // while the current one's kernel values are computed
-    unsigned long long next = ng > 0 ? ip[word_at(tile, 0)] : 0ull;
+    unsigned long long next = ng > 0 ? ip[word_at(lg, tile, 0)] : 0ull;
     for (int g = 0; g < ng; ++g) {
-        const size_t o = word_at(tile, g);
-        const unsigned long long word = next;
-        if (g + 1 < ng) next = ip[word_at(tile, g + 1)];
+        const size_t o = word_at(lg, tile, g);
+        const unsigned long long word = next, hi = SLOTS ? hp[o] : 0ull;
+        if (g + 1 < ng) next = ip[word_at(lg, tile, g + 1)];
         float wv[4] = {0.f, 0.f, 0.f, 0.f}, gxv[4] = {0.f, 0.f, 0.f, 0.f}, gyv[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             if (4 * g + k < n) {
-                const int ent = (int)((word >> (16 * k)) & 0xffff);
-                const int kind = ent >> 14, j = ent & 0x3fff;
+                const unsigned ent = ListEntry<SLOTS>::get(word, hi, k);
+                const int kind = ListEntry<SLOTS>::kind(ent), j = ListEntry<SLOTS>::index(ent);
                 const double2 xs = A.xk(kind, j);
                 const double dx0 = xr.x - xs.x, dx1 = xr.y - xs.y;
                 double mh;
@@ -1485,7 +1514,8 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         const int self = lds ? r - self_base : r;
         // h_uniform > 0: every particle has this smoothing length
         const AcceptBounds ub = accept_bounds(h_uniform, h_uniform);
-        auto walk = [&](const auto &Cs, const auto &A, bool lists, auto uni) __attribute__((always_inline)) {
+        auto walk = [&](const auto &Cs, const auto &A, bool lists, auto slots, auto uni) __attribute__((always_inline)) {
+            constexpr bool SLOTS = decltype(slots)::value;
             for (int y = y0; y <= y1; ++y)
                 for (int xx = x0; xx <= x1; ++xx) {
                     const int crm = y * C.g.ndivx + xx;
@@ -1538,11 +1568,11 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
                                 }
                             }
                             if (!lists) continue;
-                            const unsigned e = (unsigned)((ks << 14) | j);
+                            const unsigned e = ListEntry<SLOTS>::make(ks, j);
                             if (in_list_a(KR, ks))
-                                la.put(ltile, PL.ia, e);
+                                la.template put<SLOTS>(PL.lg, ltile, PL.ia, PL.iah, e);
                             else if (ks == KR && list_b)
-                                lb.put(ltile, PL.ib, e);
+                                lb.template put<SLOTS>(PL.lg, ltile, PL.ib, PL.ibh, e);
                         }
                     }
                 }
@@ -1551,15 +1581,16 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         using Gen = std::integral_constant<bool, false>;
         if (lds) {
             if (h_uniform > 0)
-                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, true, Uni{});
+                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, true, Gen{}, Uni{});
             else
-                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, true, Gen{});
+                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, true, Gen{}, Gen{});
         } else {
-            walk(GlobalCells{V.kstart, C.g, C.L}, XHFields{x, hsml}, false, Gen{});
+            // the mixed form's stage kernels walk such a tile's cells themselves
+            walk(GlobalCells{V.kstart, C.g, C.L}, XHFields{x, hsml}, FILL, Uni{}, Gen{});
         }
-        if (lds) {
-            la.finish(ltile, PL.ia);
-            if (list_b) lb.finish(ltile, PL.ib);
+        if (lds || FILL) {
+            la.finish(PL.lg, ltile, PL.ia, lds ? nullptr : PL.iah);
+            if (list_b) lb.finish(PL.lg, ltile, PL.ib, lds ? nullptr : PL.ibh);
         }
         cnt[V.proc[r]] = fk[0] + fk[1] + fk[2];
     }
@@ -1571,36 +1602,121 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
         if ((threadIdx.x & 63) == 0 && v) atomicAdd(&split->n_by_type[pair_type(KR, k)], (unsigned long long)v);
     }
-    const bool over = la.n > LMAX || lb.n > LMAX;
-    const bool any_over = lds ? __syncthreads_or(over) : true;
-    if (threadIdx.x == 0) PL.ok[ltile] = !any_over;
+    const int lmax = 4 * PL.lg;
+    const bool over = la.n > lmax || lb.n > lmax;
+    const bool any_over = lds || FILL ? __syncthreads_or(over) : true;
+    if (threadIdx.x == 0) PL.ok[ltile] = any_over ? LIST_NONE : lds ? LIST_WINDOW : LIST_SLOTS;
     if (FILL && !any_over && active) {
         const double2 xr = x[r];
         const double hr = hsml[r];
         KernelFactor kf;
-        fill_kernel_values(PL.ia, PL.wa, PL.gxa, PL.gya, ltile, la.n, LdsFields<LY>{}, xr, hr, h_uniform, V.pi, kf);
-        if (list_b)
-            fill_kernel_values(PL.ib, PL.wb, KR == KIND_NODE ? PL.gxb : nullptr, KR == KIND_NODE ? PL.gyb : nullptr,
-                               ltile, lb.n, LdsFields<LY>{}, xr, hr, h_uniform, V.pi, kf);
+        float4 *gxb = KR == KIND_NODE ? PL.gxb : nullptr, *gyb = KR == KIND_NODE ? PL.gyb : nullptr;
+        if (lds) {
+            const LdsFields<LY> A{};
+            fill_kernel_values<false>(PL.lg, PL.ia, nullptr, PL.wa, PL.gxa, PL.gya, ltile, la.n, A, xr, hr, h_uniform,
+                                      V.pi, kf);
+            if (list_b)
+                fill_kernel_values<false>(PL.lg, PL.ib, nullptr, PL.wb, gxb, gyb, ltile, lb.n, A, xr, hr, h_uniform,
+                                          V.pi, kf);
+        } else {
+            const XHFields A{x, hsml};
+            fill_kernel_values<true>(PL.lg, PL.ia, PL.iah, PL.wa, PL.gxa, PL.gya, ltile, la.n, A, xr, hr, h_uniform,
+                                     V.pi, kf);
+            if (list_b)
+                fill_kernel_values<true>(PL.lg, PL.ib, PL.ibh, PL.wb, gxb, gyb, ltile, lb.n, A, xr, hr, h_uniform,
+                                         V.pi, kf);
+        }
     }
     if (r < T.end) {
-        PL.deg_a[r] = (unsigned short)(la.n < LMAX ? la.n : LMAX);
-        if (list_b) PL.deg_b[r] = (unsigned short)(lb.n < LMAX ? lb.n : LMAX);
+        PL.deg_a[r] = (unsigned short)(la.n < lmax ? la.n : lmax);
+        if (list_b) PL.deg_b[r] = (unsigned short)(lb.n < lmax ? lb.n : lmax);
         if (KR == KIND_NODE && PL.nodeinfo) PL.nodeinfo[r] = (int)(2u * n_node + (any_dummy ? 1u : 0u));
     }
 }
 
-// The ne entries of one list word, forwards or backwards; every word index
-// is a compile-time constant.
-template <int KMASK, bool NW, bool NG, bool REV, typename Fields, typename F>
-__device__ __forceinline__ void walk_word(unsigned long long word, const float4 &cw, const float4 &cx,
-                                          const float4 &cy, int ne, const Fields &A, F &f) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int kk = REV ? 3 - q : q;
+// The lists into the order in which the reference's linked list holds the
+// pairs.  They are built in ascending discovery index d; the pairs d >= M (a
+// suffix) come first, descending.  A receiver below first_rev has none; with
+// no pair d < M (the first search of a list) every list is reversed.  Runs
+// after the split of the discovery indices is known and ends at once when
+// no pair lies past M, which is most steps; the stage kernels then read every
+// list forwards (with the order decided in their walks instead, a tile with
+// one receiver on both sides of M walked its cells in every stage).
+__device__ __forceinline__ int window_slot(const StagePlan &sc, int i) {
+    if (i < sc.mainn) return sc.mainlo + i;
+    int lo = 0, hi = sc.nh - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (sc.hpos[mid] <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    return sc.hglo[lo] + (i - sc.hpos[lo]);
+}
+
+// One receiver's list: entry k of word g of an array of four-entry words.
+template <typename E, typename W> __device__ __forceinline__ E &list_at(W *p, int lg, int tile, int k) {
+    return reinterpret_cast<E *>(p + word_at(lg, tile, k >> 2))[k & 3];
+}
+template <typename E, typename W>
+__device__ __forceinline__ void reverse_entries(W *p, int lg, int tile, int a, int b) {
+    if (!p) return;
+    for (--b; a < b; ++a, --b) {
+        const E u = list_at<E>(p, lg, tile, a), v = list_at<E>(p, lg, tile, b);
+        list_at<E>(p, lg, tile, a) = v;
+        list_at<E>(p, lg, tile, b) = u;
+    }
+}
+
+__global__ __launch_bounds__(TILE) void k_list_order(SearchView V, PairLists PL) {
+    const WalkCtx C = walk_ctx(V);
+    if (!C.any_rev) return;
+    const int tile = blockIdx.x;
+    const Tile T = PL.tiles[tile];
+    const int r = T.first + (int)threadIdx.x;
+    const int ok = PL.ok[tile];
+    if (r > T.last || ok == LIST_NONE) return;
+    if (C.any_fwd && V.proc[r] < C.sp.first_rev) return;
+    const int pr = C.any_fwd ? V.proc[r] : 0;
+    const bool node = tile < PL.ntile_n;
+    for (int l = 0; l < 2; ++l) {
+        if (l && !node && !PL.wb) continue;
+        const int n = l ? PL.deg_b[r] : PL.deg_a[r];
+        unsigned long long *ip = l ? PL.ib : PL.ia, *hp = ok == LIST_SLOTS ? (l ? PL.ibh : PL.iah) : nullptr;
+        int fwd = C.any_fwd ? n : 0;   // entries with d < M
+        for (int k = 0; k < fwd; ++k) {
+            const unsigned e = list_at<unsigned short>(ip, PL.lg, tile, k);
+            int slot;
+            if (ok == LIST_SLOTS)
+                slot = ListEntry<true>::index(e | ((unsigned)list_at<unsigned short>(hp, PL.lg, tile, k) << 16));
+            else
+                slot = window_slot(PL.plans[(size_t)tile * 3 + ListEntry<false>::kind(e)], ListEntry<false>::index(e));
+            if (pair_reversed(pr, V.proc[slot], V.cnt, V.off, C.sp)) fwd = k;
+        }
+        if (fwd == n) continue;
+        // reversed whole, then its last fwd entries again
+        for (int part = 0; part < 2; ++part) {
+            const int a = part ? n - fwd : 0;
+            reverse_entries<unsigned short>(ip, PL.lg, tile, a, n);
+            reverse_entries<unsigned short>(hp, PL.lg, tile, a, n);
+            reverse_entries<float>(l ? PL.wb : PL.wa, PL.lg, tile, a, n);
+            if (!l || node) {
+                reverse_entries<float>(l ? PL.gxb : PL.gxa, PL.lg, tile, a, n);
+                reverse_entries<float>(l ? PL.gyb : PL.gya, PL.lg, tile, a, n);
+            }
+        }
+    }
+}
+
+// The ne entries of one list word; every word index is a compile-time
+// constant.
+template <int KMASK, bool NW, bool NG, bool SLOTS, typename Fields, typename F>
+__device__ __forceinline__ void walk_word(unsigned long long word, unsigned long long hi, const float4 &cw,
+                                          const float4 &cx, const float4 &cy, int ne, const Fields &A, F &f) {
+#pragma unroll SLOTS ? 1 : 4
+    for (int kk = 0; kk < 4; ++kk) {
         if (kk >= ne) continue;
-        const int ent = (int)((word >> (16 * kk)) & 0xffff);
-        const int kind = ent >> 14, j = ent & 0x3fff;
+        const unsigned ent = ListEntry<SLOTS>::get(word, hi, kk);
+        const int kind = ListEntry<SLOTS>::kind(ent), j = ListEntry<SLOTS>::index(ent);
         if (!((KMASK >> kind) & 1)) continue;
         const float w = NW ? get4(cw, kk) : 0.0f;
         const float gx = NG ? get4(cx, kk) : 0.0f, gy = NG ? get4(cy, kk) : 0.0f;
@@ -1628,17 +1744,16 @@ struct ListWord {
 // are short): start() issues the loads of the first words (callers start
 // before the window staging so that these loads overlap it), run() calls
 // f(kind_tag, fields, j, w, dW/dx_r, dW/dy_r) over the entries of the kinds
-// in KMASK, forwards or backwards (rev is the same for every lane).  NW / NG:
-// the kernel reads w / the gradient.
+// in KMASK.  NW / NG: the kernel reads w / the gradient.  run_slots() is run()
+// for a tile whose lists hold storage slots.
 template <int KMASK, bool NW, bool NG, int DEPTH = 2> struct ListWalk {
     const unsigned long long *ip;
     const float4 *wp, *gxp, *gyp;
-    int tile, deg, ng;
-    bool rev;
+    int lg, tile, deg, ng;
     ListWord a, b;
 
     __device__ __forceinline__ void load(ListWord &d, int g) const {
-        const size_t o = word_at(tile, rev ? ng - 1 - g : g);
+        const size_t o = word_at(lg, tile, g);
         d.idx = ip[o];
         if (NW) d.w = wp[o];
         if (NG) {
@@ -1647,14 +1762,14 @@ template <int KMASK, bool NW, bool NG, int DEPTH = 2> struct ListWalk {
         }
     }
     __device__ __forceinline__ void start(const unsigned long long *ip_, const float4 *wp_, const float4 *gxp_,
-                                          const float4 *gyp_, int tile_, int deg_, bool rev_) {
+                                          const float4 *gyp_, int lg_, int tile_, int deg_) {
         ip = ip_;
         wp = wp_;
         gxp = gxp_;
         gyp = gyp_;
+        lg = lg_;
         tile = tile_;
         deg = deg_;
-        rev = rev_;
         ng = (deg + 3) >> 2;
         const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
         a = b = ListWord{0ull, z, z, z};
@@ -1662,32 +1777,32 @@ template <int KMASK, bool NW, bool NG, int DEPTH = 2> struct ListWalk {
         if (DEPTH > 1 && ng > 1) load(b, 1);
     }
     template <typename Fields, typename F> __device__ __forceinline__ void run(const Fields &A, F &&f) {
-        for (int gi = 0; gi < ng; ++gi) {
+        for (int g = 0; g < ng; ++g) {
             const ListWord c = a;
             if constexpr (DEPTH > 1) {
                 a = b;
-                if (gi + 2 < ng) load(b, gi + 2);
-            } else if (gi + 1 < ng) {
-                load(a, gi + 1);
+                if (g + 2 < ng) load(b, g + 2);
+            } else if (g + 1 < ng) {
+                load(a, g + 1);
             }
-            const int g = rev ? ng - 1 - gi : gi;
-            const int ne = deg - 4 * g < 4 ? deg - 4 * g : 4;
-            if (rev)
-                walk_word<KMASK, NW, NG, true>(c.idx, c.w, c.gx, c.gy, ne, A, f);
-            else
-                walk_word<KMASK, NW, NG, false>(c.idx, c.w, c.gx, c.gy, ne, A, f);
+            walk_word<KMASK, NW, NG, false>(c.idx, 0ull, c.w, c.gx, c.gy, min(deg - 4 * g, 4), A, f);
+        }
+    }
+    template <typename Fields, typename F>
+    __device__ __forceinline__ void run_slots(const unsigned long long *hp, const Fields &A, F &&f) {
+        for (int g = 0; g < ng; ++g) {
+            const ListWord c = a;
+            const unsigned long long hi = hp[word_at(lg, tile, g)];
+            if (g + 1 < ng) load(a, g + 1);
+            walk_word<KMASK, NW, NG, true>(c.idx, hi, c.w, c.gx, c.gy, min(deg - 4 * g, 4), A, f);
         }
     }
 };
 
-// Workgroup-wide tiling decision of a tiled stage kernel: the tile fits the
-// window layout and no receiver of it needs per-pair pass classification.
-// check is this lane's need for that classification (global path).
-__device__ __forceinline__ bool tile_uses_lds(const Tile &T, const SearchView &V, const WalkCtx &C, int r,
-                                              bool &check) {
-    check = C.mixed && r <= T.last && V.proc[r] >= C.sp.first_rev;
-    const bool any = C.mixed ? __syncthreads_or(check) : false;
-    return T.fits && !any;
+// A lane without lists (LIST_NONE) that may hold pairs on both sides of M
+// classifies each pair as it walks its cells.
+__device__ __forceinline__ bool needs_split(const Tile &T, const SearchView &V, const WalkCtx &C, int r) {
+    return C.mixed && r <= T.last && V.proc[r] >= C.sp.first_rev;
 }
 
 // stress_point_update (2_...:403-482) for node receivers: CSPM-normalised
@@ -1703,15 +1818,12 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, P
     const int r = T.first + (int)threadIdx.x;
     const bool inside = r < T.end && V.cell[r] < C.g.ndivt;
     ListWalk<MASK_SP, true, false> lw;
-    lw.start(PL.ia, PL.wa, PL.gxa, PL.gya, tile, inside ? PL.deg_a[r] : 0, !C.any_fwd && C.any_rev);
-    bool check;
-    bool lds = tile_uses_lds(T, V, C, r, check) && PL.ok[tile];
+    lw.start(PL.ia, PL.wa, PL.gxa, PL.gya, PL.lg, tile, inside ? PL.deg_a[r] : 0);
+    const int ok = PL.ok[tile];
+    const bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_SP>(PL, tile, 0, pl);
         __syncthreads();
-        lds = pl.total <= CAP;
-    }
-    if (lds) {
         struct Item {
             double m, rho, iv;
             double4 st;
@@ -1745,9 +1857,12 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, P
     if (inside) {
         if (lds) {
             lw.run(LdsFields<LY>{}, body);
+        } else if (ok == LIST_SLOTS) {
+            lw.run_slots(PL.iah, GlobalFields{S}, body);
         } else {
             int cx, cy;
             cell_xy(V.cell[r], C.g, cx, cy);
+            const bool check = needs_split(T, V, C, r);
             const SplitClass cls{check, check ? V.proc[r] : 0, V.proc, V.cnt, V.off, C.sp};
             walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy, S.x[r],
                                   S.hsml[r], KIND_NODE, r, C.any_fwd ? check : C.any_rev, C.any_fwd, V.pi, cls,
@@ -1841,18 +1956,14 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
     const int r = T.first + (int)threadIdx.x;
     const bool inside = r < T.end && V.cell[r] < C.g.ndivt;
     const int deg = inside ? PL.deg_a[r] : 0;
-    const bool rev_l = !C.any_fwd && C.any_rev;
     ListWalk<MASK_NODE, true, false> lw;
-    lw.start(PL.ia, PL.wa, PL.gxa, PL.gya, ltile, deg, rev_l);
-    bool check;
-    bool lds = tile_uses_lds(T, V, C, r, check) && PL.ok[ltile];
+    lw.start(PL.ia, PL.wa, PL.gxa, PL.gya, PL.lg, ltile, deg);
+    const int ok = PL.ok[ltile];
+    const bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_NODE>(PL, ltile, 0, pl[0]);
         if (deriv) load_plan<KIND_DUMMY>(PL, ltile, 1, pl[1]);
         __syncthreads();
-        lds = pl[0].total <= CAP && (!deriv || pl[1].total <= CAP_D);
-    }
-    if (lds) {
         struct NItem {
             double2 x, v;
             double m, rho;
@@ -1887,10 +1998,11 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
     }
     if (r >= T.end) return;
     int cx = 0, cy = 0;
-    if (inside && !lds) cell_xy(V.cell[r], C.g, cx, cy);
+    if (inside && ok == LIST_NONE) cell_xy(V.cell[r], C.g, cx, cy);
     const double2 xr = S.x[r];
     const double hr = S.hsml[r];
     const LdsFields<LY> LF{};
+    const bool check = ok == LIST_NONE && needs_split(T, V, C, r);
     const SplitClass cls{check, check ? V.proc[r] : 0, V.proc, V.cnt, V.off, C.sp};
     const bool rev_g = C.any_fwd ? check : C.any_rev;
 
@@ -1908,6 +2020,8 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
     if (inside) {
         if (lds)
             lw.run(LF, spu);
+        else if (ok == LIST_SLOTS)
+            lw.run_slots(PL.iah, GlobalFields{S}, spu);
         else
             walk_stencil<MASK_NODE>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy, xr, hr,
                                     KIND_SP, r, rev_g, C.any_fwd, V.pi, cls, spu);
@@ -1973,10 +2087,13 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
         }
     };
     if (inside) {
-        if (lds) {
+        if (ok != LIST_NONE) {
             ListWalk<MASK_NODE | MASK_DUMMY, false, true, SPS_WALK_DEPTH> lg;
-            lg.start(PL.ia, PL.wa, PL.gxa, PL.gya, ltile, deg, rev_l);
-            lg.run(LF, grad);
+            lg.start(PL.ia, PL.wa, PL.gxa, PL.gya, PL.lg, ltile, deg);
+            if (lds)
+                lg.run(LF, grad);
+            else
+                lg.run_slots(PL.iah, GlobalFields{S}, grad);
         } else
             walk_stencil<MASK_NODE | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy,
                                                  xr, hr, KIND_SP, r, rev_g, C.any_fwd, V.pi, cls, grad);
@@ -2101,11 +2218,10 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_deriv_nodes(StateBufs 
     const bool active = r < T.end;
     const int key_r = active ? V.cell[r] : C.g.ndivt;
     const bool inside = key_r < C.g.ndivt;
-    const bool rev_l = !C.any_fwd && C.any_rev;
     ListWalk<MASK_SP | MASK_DUMMY, false, true, SPS_WALK_DEPTH> la;
-    la.start(PL.ia, PL.wa, PL.gxa, PL.gya, tile, inside ? PL.deg_a[r] : 0, rev_l);
-    bool check;
-    const bool tiled = tile_uses_lds(T, V, C, r, check) && PL.ok[tile];
+    la.start(PL.ia, PL.wa, PL.gxa, PL.gya, PL.lg, tile, inside ? PL.deg_a[r] : 0);
+    const int ok = PL.ok[tile];
+    const bool check = ok == LIST_NONE && needs_split(T, V, C, r);
     int cx = 0, cy = 0;
     if (inside) cell_xy(key_r, C.g, cx, cy);
     const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
@@ -2119,14 +2235,11 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_deriv_nodes(StateBufs 
     const LdsFields<LY> LF{};
 
     // phase 1: stress gradient over stress points (type 1) and dummies (type 6)
-    bool lds = tiled;
+    const bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_SP>(PL, tile, 0, pl[0]);
         load_plan<KIND_DUMMY>(PL, tile, 1, pl[1]);
         __syncthreads();
-        lds = pl[0].total <= CAP && pl[1].total <= CAP_D;
-    }
-    if (lds) {
         struct SItem {
             double2 x;
             double m, rho;
@@ -2191,7 +2304,10 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_deriv_nodes(StateBufs 
         {
             StateBufs S2 = S;   // stress points' stresses from sp_stress (the walk reads no node's)
             S2.stress = const_cast<double4 *>(sp_stress);
-            walk_stencil<MASK_SP | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S2}, C.g, cx, cy,
+            if (ok == LIST_SLOTS)
+                la.run_slots(PL.iah, GlobalFields{S2}, grad);
+            else
+                walk_stencil<MASK_SP | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S2}, C.g, cx, cy,
                                                xr, hr, KIND_NODE, r, rev_g, C.any_fwd, V.pi, cls, grad);
         }
     }
@@ -2226,9 +2342,8 @@ __global__ __launch_bounds__(TILE) void k_av_nodes(StateBufs S, SearchView V, Pa
     const bool active = r < T.end;
     const int key_r = active ? V.cell[r] : C.g.ndivt;
     const bool inside = key_r < C.g.ndivt;
-    const bool rev_l = !C.any_fwd && C.any_rev;
-    bool check;
-    const bool tiled = tile_uses_lds(T, V, C, r, check) && PL.ok[tile];
+    const int ok = PL.ok[tile];
+    const bool check = ok == LIST_NONE && needs_split(T, V, C, r);
     int cx = 0, cy = 0;
     if (inside) cell_xy(key_r, C.g, cx, cy);
     const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
@@ -2240,14 +2355,11 @@ __global__ __launch_bounds__(TILE) void k_av_nodes(StateBufs S, SearchView V, Pa
     float ax = 0.0f, ay = 0.0f, visc = 0.0f;
     {
         ListWalk<MASK_NODE, false, true> lb;
-        lb.start(PL.ib, nullptr, PL.gxb, PL.gyb, tile, inside ? PL.deg_b[r] : 0, rev_l);
-        bool lds2 = tiled;
+        lb.start(PL.ib, nullptr, PL.gxb, PL.gyb, PL.lg, tile, inside ? PL.deg_b[r] : 0);
+        const bool lds2 = ok == LIST_WINDOW;
         if (lds2) {
             load_plan<KIND_NODE>(PL, tile, 0, pl[0]);
             __syncthreads();
-            lds2 = pl[0].total <= CAP;
-        }
-        if (lds2) {
             struct NItem {
                 double2 x, v;
                 double h, m, rho;
@@ -2289,6 +2401,8 @@ __global__ __launch_bounds__(TILE) void k_av_nodes(StateBufs S, SearchView V, Pa
         if (inside) {
             if (lds2)
                 lb.run(LF, av);
+            else if (ok == LIST_SLOTS)
+                lb.run_slots(PL.ibh, GlobalFields{S}, av);
             else
                 walk_stencil<MASK_NODE>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy, xr, hr,
                                         KIND_NODE, r, rev_g, C.any_fwd, V.pi, cls, av);
@@ -2325,17 +2439,13 @@ __global__ __launch_bounds__(TILE) void k_xsph(StateBufs S, SearchView V, PairLi
     if (T.first >= T.end) return;
     const int r = T.first + (int)threadIdx.x;
     const bool inside = r < T.end && V.cell[r] < C.g.ndivt;
-    const bool rev_l = !C.any_fwd && C.any_rev;
     ListWalk<(1 << KR), true, false> lw;
-    lw.start(PL.ib, PL.wb, nullptr, nullptr, ltile, inside ? PL.deg_b[r] : 0, rev_l);
-    bool check;
-    bool lds = tile_uses_lds(T, V, C, r, check) && PL.ok[ltile];
+    lw.start(PL.ib, PL.wb, nullptr, nullptr, PL.lg, ltile, inside ? PL.deg_b[r] : 0);
+    const int ok = PL.ok[ltile];
+    const bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KR>(PL, ltile, 0, pl);
         __syncthreads();
-        lds = pl.total <= CAP;
-    }
-    if (lds) {
         struct Item {
             double2 v;
             double m, rho;
@@ -2360,9 +2470,12 @@ __global__ __launch_bounds__(TILE) void k_xsph(StateBufs S, SearchView V, PairLi
     if (inside) {
         if (lds) {
             lw.run(LdsFields<LY>{}, body);
+        } else if (ok == LIST_SLOTS) {
+            lw.run_slots(PL.ibh, GlobalFields{S}, body);
         } else {
             int cx, cy;
             cell_xy(V.cell[r], C.g, cx, cy);
+            const bool check = needs_split(T, V, C, r);
             const SplitClass cls{check, check ? V.proc[r] : 0, V.proc, V.cnt, V.off, C.sp};
             walk_stencil<(1 << KR)>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy, S.x[r],
                                     S.hsml[r], KR, r, C.any_fwd ? check : C.any_rev, C.any_fwd, V.pi, cls, body);

@@ -179,9 +179,9 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
     const int r = T.first + (int)threadIdx.x;
     const bool inside = r < T.end && V.cell[r] < C.g.ndivt;
     ListWalk<MASK_SP, false, false> lw;
-    lw.start(PL.ia, nullptr, nullptr, nullptr, tile, inside ? PL.deg_a[r] : 0, false);
+    lw.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_a[r] : 0);
     const double2 o = S.x[T.first];
-    bool lds = T.fits && PL.ok[tile];
+    bool lds = PL.ok[tile] == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_SP>(PL, tile, 0, pl);
         __syncthreads();
@@ -265,9 +265,9 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
     const bool inside = r < T.end && V.cell[r] < C.g.ndivt;
     const int deg = inside ? PL.deg_a[r] : 0;
     ListWalk<MASK_NODE, false, false> lw;
-    lw.start(PL.ia, nullptr, nullptr, nullptr, ltile, deg, false);
+    lw.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, ltile, deg);
     const double2 o = S.x[T.first];
-    bool lds = T.fits && PL.ok[ltile];
+    bool lds = PL.ok[ltile] == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_NODE>(PL, ltile, 0, pl[0]);
         if (deriv) load_plan<KIND_DUMMY>(PL, ltile, 1, pl[1]);
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
     if (inside) {
         if (lds) {
             ListWalk<MASK_NODE | MASK_DUMMY, false, false> lg;
-            lg.start(PL.ia, nullptr, nullptr, nullptr, ltile, deg, false);
+            lg.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, ltile, deg);
             lg.run(LF, on_the_fly(grad, xrr, (float)hr, hu));
         } else
             walk_stencil<MASK_NODE | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr, KIND_SP,
@@ -419,7 +419,7 @@ __device__ __forceinline__ float2 av_mix(const StateBufs &S, const SearchView &V
     KSum ax, ay;
     if (!P.do_av) return make_float2(0.0f, 0.0f);
     ListWalk<MASK_NODE, false, false> lb;
-    lb.start(PL.ib, nullptr, nullptr, nullptr, tile, inside ? PL.deg_b[r] : 0, false);
+    lb.start(PL.ib, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_b[r] : 0);
     bool lds2 = tiled;
     if (lds2) {
         load_plan<KIND_NODE>(PL, tile, 0, pl);
@@ -491,9 +491,9 @@ __global__ __launch_bounds__(TILE) void k_deriv_nodes_mix(StateBufs S, Work W, S
     const int key_r = active ? V.cell[r] : C.g.ndivt;
     const bool inside = key_r < C.g.ndivt;
     ListWalk<MASK_SP | MASK_DUMMY, false, false> la;
-    la.start(PL.ia, nullptr, nullptr, nullptr, tile, inside ? PL.deg_a[r] : 0, false);
+    la.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_a[r] : 0);
     const double2 o = S.x[T.first];
-    const bool tiled = T.fits && PL.ok[tile];
+    const bool tiled = PL.ok[tile] == LIST_WINDOW;
     int cx = 0, cy = 0;
     if (inside) cell_xy(key_r, C.g, cx, cy);
     const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V
     const int key_r = active ? V.cell[r] : C.g.ndivt;
     const bool inside = key_r < C.g.ndivt;
     const double2 o = S.x[T.first];
-    const bool tiled = T.fits && PL.ok[tile];
+    const bool tiled = PL.ok[tile] == LIST_WINDOW;
     int cx = 0, cy = 0;
     if (inside) cell_xy(key_r, C.g, cx, cy);
     const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
@@ -666,9 +666,9 @@ __global__ __launch_bounds__(TILE) void k_xsph_mix(StateBufs S, SearchView V, Pa
     const int r = T.first + (int)threadIdx.x;
     const bool inside = r < T.end && V.cell[r] < C.g.ndivt;
     ListWalk<(1 << KR), false, false> lw;
-    lw.start(PL.ib, nullptr, nullptr, nullptr, ltile, inside ? PL.deg_b[r] : 0, false);
+    lw.start(PL.ib, nullptr, nullptr, nullptr, PL.lg, ltile, inside ? PL.deg_b[r] : 0);
     const double2 o = S.x[T.first];
-    bool lds = T.fits && PL.ok[ltile];
+    bool lds = PL.ok[ltile] == LIST_WINDOW;
     if (lds) {
         load_plan<KR>(PL, ltile, 0, pl);
         __syncthreads();

@@ -18,5 +18,5 @@
 #define SPS_CAP_D 192  // staged dummies per window
 #endif
 #ifndef SPS_STAGE_WAVES
-#define SPS_STAGE_WAVES 0  // waves per SIMD of the FP64 stage kernels (0: the compiler's choice)
+#define SPS_STAGE_WAVES 4  // waves per SIMD of the FP64 stage kernels (0: the compiler's choice)
 #endif
