@@ -47,11 +47,6 @@ static int fail(int code, const char *fmt, ...) {
     } while (0)
 
 static inline unsigned nblk(long long n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
-// grid of the kernels that place their tiles with xcd_block(): a multiple of 8
-static inline unsigned nblk8(long long n) {
-    unsigned b = nblk(n);
-    return (b + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
-}
 // Tiles held for n receivers, a multiple of the XCD count: n / TILE rounded
 // up, and with `strips` > 0 (tiles that end at strip ends, k_count_tiles) one more
 // per strip of the domain box, at most twice as many in all.
@@ -61,6 +56,9 @@ static inline int ntiles(long long n, double strips) {
     return (int)((plain + extra + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
 }
 
+
+// blocks of k_count for n dummy receivers, sixteen lanes each
+static inline unsigned count_blocks(long long n) { return (unsigned)((n * 16 + BLOCK - 1) / BLOCK); }
 
 template <typename T>
 struct DBuf {
@@ -201,6 +199,7 @@ struct sps_handle {
     int ntile_n = 0, ntile_s = 0;
     DBuf<int> tile_start;         // k_count_tiles: first tile of each strip (scratch)
     DBuf<int2> tile_range;        // per tile: its receivers
+    DBuf<unsigned> type_counts;   // pairs by partner kind: per tile, then per block of dummy receivers
     double h_uniform = 0.0;   // the smoothing length of every particle, or 0 when they differ
     bool mixed = false;       // SPS_MODE_FAST: the mixed-precision stage kernels
     // pair lists kept over steps (mixed form): built with this skin, reused
@@ -254,7 +253,7 @@ struct sps_handle {
     PairLists lists() {
         return PairLists{list_ia.p,  list_ib.p,  list_iah.p, list_ibh.p, list_wa.p, list_gxa.p, list_gya.p,
                          list_gxb.p, list_gyb.p, xsph ? list_wb.p : nullptr, deg_a.p, deg_b.p,
-                         tile_ok.p,  list_words, ntile_n,    tile_range.p, tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
+                         tile_ok.p,  list_words, ntile_n,    tile_range.p, type_counts.p, tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
     }
 };
 
@@ -540,6 +539,7 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     h->ntile_s = ntiles(nt - nn, strips);
     rc |= dalloc(h->tile_start, 2 * (size_t)TSTART_MAX);
     rc |= dalloc(h->tile_range, (size_t)h->ntile_n + h->ntile_s);
+    rc |= dalloc(h->type_counts, 3 * ((size_t)h->ntile_n + h->ntile_s + count_blocks(nt2 - nt)));
     {
         // 48 entries a list, and 24 more per further stress point a node or
         // cell (about 18 partners within 2h = 2.4 dx each); a receiver with
@@ -751,35 +751,36 @@ static int search(sps_handle *h, bool fresh_list) {
             HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
             if (!h->mixed)
                 k_count_lists<KIND_SP, true><<<h->ntile_s, TILE, lds_count(h), h->stream2>>>(
-                    V, C.x.p, C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
+                    V, C.x.p, C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
             else
                 k_count_lists<KIND_SP, false><<<h->ntile_s, TILE, lds_count(h), h->stream2>>>(
-                    V, C.x.p, C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
+                    V, C.x.p, C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
             HIP_TRY(hipEventRecord(h->ev_join, h->stream2));
         }
         // the mixed-precision stage kernels compute the kernel values themselves
         if (nn > 0 && !h->mixed)
             LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_n, TILE, lds_count(h), (k_count_lists<KIND_NODE, true>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
+                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
         if (nn > 0 && h->mixed)
             LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_n, TILE, lds_count(h), (k_count_lists<KIND_NODE, false>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
+                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
         if (!fork && nt > nn && !h->mixed)
             LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_s, TILE, lds_count(h), (k_count_lists<KIND_SP, true>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
+                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
         if (!fork && nt > nn && h->mixed)
             LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_s, TILE, lds_count(h), (k_count_lists<KIND_SP, false>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, h->split.p, PL, h->h_uniform, h->skin);
+                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
         if (nt2 > nt)
-            LAUNCH(K_COUNT_DUMMY, nblk8(nt2 - nt), BLOCK, k_count, C.x.p, C.hsml.p, h->cell.p, h->kstart.p, h->proc.p,
-                   h->grid.p, h->cnt.p, h->split.p, nn, nt, nt, nt2);
+            LAUNCH(K_COUNT_DUMMY, count_blocks(nt2 - nt), BLOCK, k_count, C.x.p, C.hsml.p, h->cell.p, h->kstart.p,
+                   h->proc.p, h->grid.p, h->cnt.p, h->type_counts.p + 3 * ((size_t)h->ntile_n + h->ntile_s), nt, nt2);
         if (fork) HIP_TRY(hipStreamWaitEvent(h->stream, h->ev_join, 0));
     }
     HIP_TRY(hipGetLastError());
     // discovery offsets over all slots (slots past the in-domain count hold 0)
     rc = scan_u32(h, h->cnt.p, h->off.p, nt2, &h->split.p->n);
     if (rc) return rc;
-    LAUNCH(K_SPLIT, nblk(nt2), BLOCK, k_split, h->cnt.p, h->off.p, nt2, h->split.p);
+    LAUNCH(K_SPLIT, nblk(nt2), BLOCK, k_count_split, h->cnt.p, h->off.p, nt2, h->split.p, h->type_counts.p, h->ntile_n,
+           h->ntile_s, h->ntile_n + h->ntile_s + (int)count_blocks(nt2 - nt));
     LAUNCH(K_SPLIT, 1, 64, k_split_partner, C.x.p, C.hsml.p, h->cell.p, h->kstart.p, h->proc.p, h->off.p,
                                      h->proc_to_slot.p, h->grid.p, h->split.p, nn, nt, h->pairs_total.p);
     if (!h->mixed) {
@@ -1539,7 +1540,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
     dfree(h->cnt); dfree(h->off); dfree(h->scan_tmp); dfree(h->ctot); dfree(h->cstart_rm); dfree(h->err);
     dfree(h->list_ia); dfree(h->list_iah); dfree(h->list_ibh); dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya); dfree(h->list_ib);
-    dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->tiles); dfree(h->plans);
+    dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->type_counts); dfree(h->tiles); dfree(h->plans);
     dfree(h->list_wb); dfree(h->xsph_v);
     dfree(h->x_build); dfree(h->dmax); dfree(h->surr_count); dfree(h->surr_slot); dfree(h->surr_sn);
     dfree(h->surr_str); dfree(h->surr_feat); dfree(h->surr_stats); dfree(h->plog); dfree(h->surr_mat);

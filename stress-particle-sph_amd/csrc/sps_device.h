@@ -203,15 +203,7 @@ __device__ __forceinline__ double pair_distance(double dx0, double dx1, double h
     return (r < lim) ? r : -1.0;
 }
 
-// Workgroups are dealt round-robin to the 8 XCDs.  With a grid that is a
-// multiple of 8 this gives XCD k one contiguous eighth of the tiles, so the
-// receivers it handles walk up the same cell strips and share partner data
-// in that XCD's L2.
 constexpr int NUM_XCD = 8;
-__device__ __forceinline__ int xcd_block() {
-    int per = gridDim.x / NUM_XCD;
-    return (blockIdx.x % NUM_XCD) * per + blockIdx.x / NUM_XCD;
-}
 
 // Tile of this workgroup in the tiled pair kernels.  The hardware hands
 // consecutive workgroups to the XCDs in turn; each XCD gets runs of TILE_RUN

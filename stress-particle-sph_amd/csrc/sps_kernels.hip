@@ -470,65 +470,68 @@ __device__ __forceinline__ int pair_type(int ka, int kb) {
 }
 
 // ------------------------------------------------------------------- count
-// For every receiver: pairs it discovers (partners later in processing
-// order; the reference counts n_pairs with these), by pint_type.  The node
-// and stress-point receivers are counted by the tiled k_count_lists below.
-// (Slots [r0, r1), global storage; the dummy receivers.)
-__global__ void k_count(const double2 *__restrict__ x, const double *__restrict__ hsml,
-                        const int *__restrict__ cell, const int *__restrict__ kstart,
-                        const int *__restrict__ proc, const Grid *__restrict__ g,
-                        unsigned *__restrict__ cnt, Split *__restrict__ split, int nn, int nt,
-                        int r0, int r1) {
-    int r = r0 + xcd_block() * blockDim.x + threadIdx.x;
-    unsigned fwd = 0;
-    unsigned t0 = 0, t1 = 0, t2 = 0, t3 = 0, t6 = 0, t9 = 0;   // pairs by pint_type
-    int ndivt = g->ndivt;
-    if (r < r1 && cell[r] < ndivt) {
-        const int L = ndivt + 1;
-        const Grid gg = *g;
-        int kr = kind_of(r, nn, nt);
-        double2 xr = x[r];
-        double hr = hsml[r];
-        Stencil S = make_stencil(cell[r], gg);
-        const int crm_r = S.cy * gg.ndivx + S.cx;
-        for (int y = S.y0; y <= S.y1; ++y) {
-            for (int xx = S.x0; xx <= S.x1; ++xx) {
-                const int key = cell_key(xx, y, gg), crm = y * gg.ndivx + xx;
-                for (int ks = 0; ks < 3; ++ks) {
-                    int lo = kstart[ks * L + key], hi = kstart[ks * L + key + 1];
-                    for (int s = lo; s < hi; ++s) {
-                        if (s == r) continue;
-                        double2 xs = x[s];
-                        double mh;
-                        double rr = pair_distance(xr.x - xs.x, xr.y - xs.y, hr, hsml[s], mh);
-                        if (rr < 0.0) continue;
-                        bool after = crm > crm_r || (crm == crm_r && (ks > kr || (ks == kr && s > r)));
-                        if (after) {
-                            fwd++;
-                            switch (pair_type(kr, ks)) {
-                                case 1: t1++; break;
-                                case 2: t2++; break;
-                                case 3: t3++; break;
-                                case 6: t6++; break;
-                                case 9: t9++; break;
-                                default: t0++; break;
-                            }
-                        }
-                    }
-                }
+// The block's pairs by partner kind, v[k] of every lane, into out[0:3].  One
+// plain store per block: an atomic per wave into the pint_type histogram
+// serialised in memory (94 k atomics on one line at 1 M + 1 M particles) and
+// held the list build at 840 us; k_count_split adds the blocks up.
+__device__ __forceinline__ void block_type_counts(const unsigned (&v)[3], unsigned (*sum)[3],
+                                                  unsigned *__restrict__ out) {
+    const int wave = (int)(threadIdx.x >> 6);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        unsigned a = v[k];
+        for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
+        if ((threadIdx.x & 63) == 0) sum[wave][k] = a;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        unsigned a = 0;
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) a += sum[w][threadIdx.x];
+        out[threadIdx.x] = a;
+    }
+}
+
+// For every dummy receiver (slots [r0, r1)): pairs it discovers (partners
+// later in processing order; the reference counts n_pairs with these), by
+// partner kind.  The node and stress-point receivers are counted by the tiled
+// k_count_lists below.  Sixteen lanes per receiver, lane 3 c + k taking the
+// partners of kind k in the c-th of the five cells that can hold later ones
+// (its own and the four visited after it).
+__global__ __launch_bounds__(BLOCK) void k_count(const double2 *__restrict__ x, const double *__restrict__ hsml,
+                                                 const int *__restrict__ cell, const int *__restrict__ kstart,
+                                                 const int *__restrict__ proc, const Grid *__restrict__ g,
+                                                 unsigned *__restrict__ cnt, unsigned *__restrict__ types, int r0,
+                                                 int r1) {
+    __shared__ unsigned sum[BLOCK / 64][3];
+    const int lane = threadIdx.x & 15;
+    const int r = r0 + (int)(blockIdx.x * (BLOCK / 16) + (threadIdx.x >> 4));
+    const Grid gg = *g;
+    const int key_r = r < r1 ? cell[r] : gg.ndivt;
+    const bool live = key_r < gg.ndivt;
+    unsigned n = 0;
+    if (live && lane < 15) {
+        const int c = lane / 3, ks = lane - 3 * c;
+        int cx, cy;
+        cell_xy(key_r, gg, cx, cy);
+        const int gx = cx + (c == 0 || c == 3 ? 0 : c == 2 ? -1 : 1), gy = cy + (c > 1 ? 1 : 0);
+        if (gx >= 0 && gx < gg.ndivx && gy < gg.ndivy && (c > 0 || ks == KIND_DUMMY)) {
+            const int *__restrict__ k0 = kstart + ks * (gg.ndivt + 1) + cell_key(gx, gy, gg);
+            const int lo = c == 0 ? r + 1 : k0[0], hi = k0[1];
+            const double2 xr = x[r];
+            const double hr = hsml[r];
+            for (int s = lo; s < hi; ++s) {
+                const double2 xs = x[s];
+                double mh;
+                n += pair_distance(xr.x - xs.x, xr.y - xs.y, hr, hsml[s], mh) < 0.0 ? 0u : 1u;
             }
         }
-        cnt[proc[r]] = fwd;
     }
-    // per-type histogram: wave reduction then one atomic per wave
-    unsigned tv[6] = {t0, t1, t2, t3, t6, t9};
-    const int tid[6] = {0, 1, 2, 3, 6, 9};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        unsigned v = tv[k];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if ((threadIdx.x & 63) == 0 && v) atomicAdd(&split->n_by_type[tid[k]], (unsigned long long)v);
-    }
+    unsigned all = n;
+    for (int off = 8; off > 0; off >>= 1) all += __shfl_down(all, off, 16);
+    if (live && lane == 0) cnt[proc[r]] = all;
+    const int ks = lane % 3;
+    const unsigned v[3] = {ks == 0 ? n : 0u, ks == 1 ? n : 0u, ks == 2 ? n : 0u};
+    block_type_counts(v, sum, types + 3 * (size_t)blockIdx.x);
 }
 
 // Fresh split record: M is the list high-water mark before this search,
@@ -547,17 +550,46 @@ __global__ void k_split_reset(Split *__restrict__ split, int fresh) {
 }
 
 // Locate the processing slot whose discoveries straddle index M (n is the
-// scan total of the per-slot counts, written by the scan).
-__global__ void k_split(const unsigned *__restrict__ cnt, const unsigned *__restrict__ off,
-                        int nslots, Split *__restrict__ split) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nslots) return;
-    unsigned long long M = split->M;
-    unsigned long long o = off[p], c = cnt[p];
-    if (o < M && M < o + c) split->sstar = p;
-    // off + cnt grows with the slot, so the first slot discovering a pair
-    // d >= M is the one slot with off <= M < off + cnt
-    if (o <= M && M < o + c) split->first_rev = p;
+// scan total of the per-slot counts, written by the scan), and add up the
+// pint_type histogram: types holds 3 counts by partner kind of every node
+// tile, stress-point tile and block of dummy receivers (nb in all); the first
+// TYPE_BLOCKS blocks sum a share each.
+constexpr int TYPE_BLOCKS = 16;
+
+__global__ __launch_bounds__(BLOCK) void k_count_split(const unsigned *__restrict__ cnt,
+                                                       const unsigned *__restrict__ off, int nslots,
+                                                       Split *__restrict__ split,
+                                                       const unsigned *__restrict__ types, int ntile_n,
+                                                       int ntile_s, int nb) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < nslots) {
+        const unsigned long long M = split->M;
+        const unsigned long long o = off[p], c = cnt[p];
+        if (o < M && M < o + c) split->sstar = p;
+        // off + cnt grows with the slot, so the first slot discovering a pair
+        // d >= M is the one slot with off <= M < off + cnt
+        if (o <= M && M < o + c) split->first_rev = p;
+    }
+    if (blockIdx.x >= TYPE_BLOCKS) return;
+    const int nblocks = min((int)gridDim.x, TYPE_BLOCKS);
+    unsigned long long v[3][3] = {};   // by receiver kind and partner kind
+    for (int b = p; b < nb; b += nblocks * BLOCK) {
+        const int kr = b < ntile_n ? KIND_NODE : b < ntile_n + ntile_s ? KIND_SP : KIND_DUMMY;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const unsigned t = types[3 * (size_t)b + k];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v[q][k] += q == kr ? t : 0u;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            unsigned long long a = v[q][k];
+            for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+            if ((threadIdx.x & 63) == 0 && a) atomicAdd(&split->n_by_type[pair_type(q, k)], a);
+        }
 }
 
 // First reversed partner of the split slot: its (M - off)-th discovery in
@@ -1316,6 +1348,7 @@ struct PairLists {
     int lg;                         // words per receiver and list; more entries: LIST_NONE
     int ntile_n;                    // node tiles
     const int2 *range;              // per tile: its receivers (k_count_tiles)
+    unsigned *types;                // per tile: pairs its receivers discover, by partner kind
     // each tile's extent and (when it fits) the staging plan of every partner
     // kind, as the search computed them: the stage kernels load them in one
     // round trip instead of deriving them again through dependent loads
@@ -1450,16 +1483,19 @@ __device__ __forceinline__ bool in_list_a(int kr, int ks) {
 template <int KR, bool FILL>
 __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double2 *__restrict__ x,
                                                       const double *__restrict__ hsml,
-                                                      unsigned *__restrict__ cnt, Split *__restrict__ split,
-                                                      PairLists PL, double h_uniform, double skin) {
+                                                      unsigned *__restrict__ cnt, PairLists PL, double h_uniform, double skin) {
     __shared__ StagePlan pl[3];
+    __shared__ unsigned tsum[TWAVES][3];
     constexpr const LdsLayout &LY = LAY_COUNT;
     const WalkCtx C = walk_ctx(V);
     const int tile = tile_index();
     const int ltile = KR == KIND_NODE ? tile : PL.ntile_n + tile;
     const Tile T = make_tile(PL.range[ltile], KR, V, C);
     if (threadIdx.x == 0) PL.tiles[ltile] = T;
-    if (T.first >= T.end) return;
+    if (T.first >= T.end) {
+        if (threadIdx.x < 3) PL.types[3 * (size_t)ltile + threadIdx.x] = 0u;
+        return;
+    }
     const int r = T.first + (int)threadIdx.x;
     // list B: a node's node partners; with XSPH also a stress point's stress-point partners
     const bool list_b = KR == KIND_NODE || PL.wb != nullptr;
@@ -1506,12 +1542,12 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
     if (active) {
         int cx, cy;
         cell_xy(V.cell[r], C.g, cx, cy);
-        const int crm_r = cy * C.g.ndivx + cx;
         const double2 xr = x[r];
         const double hr = hsml[r];
         const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < C.g.ndivx ? cx + 1 : C.g.ndivx - 1;
         const int y0 = cy > 0 ? cy - 1 : 0, y1 = cy + 1 < C.g.ndivy ? cy + 1 : C.g.ndivy - 1;
         const int self = lds ? r - self_base : r;
+        const int crm_r = cy * C.g.ndivx + cx;
         // h_uniform > 0: every particle has this smoothing length
         const AcceptBounds ub = accept_bounds(h_uniform, h_uniform);
         auto walk = [&](const auto &Cs, const auto &A, bool lists, auto slots, auto uni) __attribute__((always_inline)) {
@@ -1594,14 +1630,7 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         }
         cnt[V.proc[r]] = fk[0] + fk[1] + fk[2];
     }
-    // per-type histogram (one pint_type per partner kind of a receiver kind):
-    // wave reduction, then one atomic per wave
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        unsigned v = fk[k];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if ((threadIdx.x & 63) == 0 && v) atomicAdd(&split->n_by_type[pair_type(KR, k)], (unsigned long long)v);
-    }
+    block_type_counts(fk, tsum, PL.types + 3 * (size_t)ltile);
     const int lmax = 4 * PL.lg;
     const bool over = la.n > lmax || lb.n > lmax;
     const bool any_over = lds || FILL ? __syncthreads_or(over) : true;
