@@ -4,8 +4,8 @@
 // One step is the reference's time_integration (code/2_SPH_main_2018.f90
 // :78-184) for the supported flag set:
 //   Check_Out_Domain, grid_find_NEW + Pint_Update  -> k_check_ood .. k_split_partner
-//   RK4 (2_...:653-802)                            -> k_stage_first, 4 x stage, k_rk_final
-//   update_strain, stress_point_update, adapt      -> k_rk_final, k_spu_*
+//   RK4 (2_...:653-802)                            -> k_stage_first, 4 x stage
+//   update_strain, stress_point_update, adapt      -> k_spu_nodes, k_sp_update
 //   position update and displacement               -> k_position
 // The search bins the particles and fixes the order of the pair list; every
 // stage kernel then walks each receiver's cell stencil in that order and
@@ -142,6 +142,7 @@ struct sps_handle {
     // k_sp_update writes here so that k_spu_nodes, reading the first, can
     // run beside it (on stream2; ev_fork / ev_join order the two)
     DBuf<double4> sig2;
+    DBuf<double4> stress_b;  // the stress points' stresses of the odd RK stages (StageStep)
     DBuf<float2> av_nodes;   // the nodes' artificial viscosity of a stage (k_av_nodes)
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -260,14 +261,14 @@ struct sps_handle {
 // ------------------------------------------------------------ profiling
 enum KernelId {
     K_CHECK_OOD, K_BOUNDS, K_CELL_COUNT, K_CELL_SCATTER, K_CELL_SORT, K_PERMUTE, K_PROC,
-    K_COUNT_PAIRS, K_SCAN, K_SPLIT, K_RK_INIT, K_STAGE_BEGIN, K_SPU_NODES,
+    K_COUNT_PAIRS, K_SCAN, K_SPLIT, K_RK_INIT, K_LF_KICK, K_SPU_NODES,
     K_SP_UPDATE, K_DERIV_NODES, K_DUMMY_STRESS, K_RK_FINAL, K_POSITION, K_SURROGATE, K_XSPH, K_SHIFT, K_BCS, K_SURF,
     K_AV_NODES, K_COUNT_DUMMY, K_NKERNELS
 };
 static const char *const kKernelNames[K_NKERNELS] = {
     "k_check_ood", "k_bounds", "k_cell_count", "k_cell_scatter", "k_cell_sort", "k_permute",
     "k_proc_slot", "k_count_lists", "k_scan", "k_split", "k_stage_first",
-    "k_stage_begin", "k_spu_nodes", "k_sp_update", "k_deriv_nodes",
+    "k_lf_kick", "k_spu_nodes", "k_sp_update", "k_deriv_nodes",
     "k_dummy_stress", "k_rk_final", "k_position", "k_surrogate", "k_xsph", "k_shift_sp", "k_bcs", "k_surf",
     "k_av_nodes", "k_count"};
 
@@ -323,6 +324,25 @@ static void prof_collect(sps_handle *h) {
 extern "C" const char *sps_last_error(void) { return g_err; }
 
 static void drop_graphs(sps_handle *h);
+
+// RK stage st of a step of dt (2_...:681-777): its weight, and what its
+// derivative pass leaves.  The stress points' stresses alternate between the
+// state and stress_b, so that the last stage leaves the step's in the state.
+// rhs: the step's end is k_rk_final's.
+static StageStep rk_stage(sps_handle *h, const StateBufs &SB, int st, double dt, bool rhs) {
+    const double f1[4] = {0., 0.5, 0.5, 1.0}, f2[4] = {1., 2., 2., 1.0};
+    StageStep Q;
+    Q.end = st < 3 ? (st ? STAGE_MID : STAGE_FIRST) : rhs ? STAGE_RHS : STAGE_LAST;
+    Q.first = st == 0;
+    Q.f2 = f2[st];
+    Q.c = st < 3 ? f1[st + 1] * dt : dt / 6;
+    Q.sp_in = st & 1 ? h->stress_b.p : SB.stress;
+    Q.sp_out = st & 1 ? SB.stress : h->stress_b.p;
+    return Q;
+}
+
+// A pass on the state's own stresses: the update alone, or the rates.
+static StageStep state_pass(const StateBufs &SB) { return StageStep{STAGE_RHS, 1, 1.0, 0.0, SB.stress, nullptr}; }
 
 #include "sps_surrogate_host.hip"
 extern "C" const char *sps_backend(void) { return "hip-gfx950"; }
@@ -521,7 +541,7 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     rc |= dalloc(h->rk_vel, nn); rc |= dalloc(h->rhs2, nn); rc |= dalloc(h->f_bound, nn);
     rc |= dalloc(h->art_visc, nn); rc |= dalloc(h->stress0, nt); rc |= dalloc(h->rk_stress, nt);
     rc |= dalloc(h->rhs1, nt); rc |= dalloc(h->grad_u, nt); rc |= dalloc(h->rk_dev, nt);
-    rc |= dalloc(h->sig2, nt); rc |= dalloc(h->av_nodes, nn > 0 ? nn : 1);
+    rc |= dalloc(h->sig2, nt); rc |= dalloc(h->stress_b, nt); rc |= dalloc(h->av_nodes, nn > 0 ? nn : 1);
     rc |= dalloc(h->ddev, nt);
     rc |= dalloc(h->grid, 1); rc |= dalloc(h->split, 1); rc |= dalloc(h->err, 1); rc |= dalloc(h->pairs_total, 1);
     h->nbparts = std::min(1024, (int)nblk(nt2));
@@ -842,8 +862,9 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
     const PairLists PL = h->lists();
     const int adapt = h->dp.ncrit == 12;
     const double tanfi = h->dp.tanfi, coh = h->dp.coh;
-    const double f1rk[4] = {0., 0.5, 0.5, 1.0}, f2rk[4] = {1., 2., 2., 1.0};
     const float hu = (float)h->h_uniform;
+    const bool hook = h->mlp || h->log_cap > 0;
+    const double *strain_rate = hook ? nullptr : h->ddev.p;   // update_strain left to the update after the stages
     // prescribed BCs where the reference applies them (as in the FP64 step);
     // a captured step reads the values k_bc_values leaves before each replay
     const bool bcs = h->p.no_bcs > 0 && nn > 0;
@@ -853,15 +874,14 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
         // step's lists (2_...:99-109)
         if (nn > 0)
             LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
-                       tanfi, coh, hu, nn);
+                       tanfi, coh, hu, nn, SB.stress, nullptr, 0.0);
         if (nt > nn)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
-                       h->dp, time_sph, 0.0, 0, adapt, hu, nn, nt, stepv, nullptr);
+                       h->dp, time_sph, state_pass(SB), 0, adapt, hu, nn, nt, stepv, nullptr, nullptr, 0.0, h->err.p);
     }
     LAUNCH(K_RK_INIT, nblk(nt2), BLOCK, k_stage_first, SB, W, adapt, tanfi, coh, nn, nt, nt2);
     for (int st = 0; st < 4; ++st) {
-        const double c1 = f1rk[st] * (dt);
-        if (st > 0) LAUNCH(K_STAGE_BEGIN, nblk(nt), BLOCK, k_stage_begin, SB, W, c1, adapt, tanfi, coh, nn, nt);
+        const StageStep Q = rk_stage(h, SB, st, dt, hook);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
         // the two halves of stress_point_update side by side, as in the FP64
         // step; one stream when kernels are timed or the step is captured
@@ -870,37 +890,41 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
             HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
             HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
             hipStream_t s2 = h->stream2;
-            k_spu_nodes_mix<<<h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, hu, nn);
+            k_spu_nodes_mix<<<h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, hu, nn,
+                                                                               Q.sp_in, nullptr, 0.0);
             if (bcs)
                 k_bcs<<<nblk(nn), BLOCK, 0, s2>>>(SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p,
                                                  h->ifsigman, h->normal.p, nn, nullptr, nullptr);
+            if (st == 3 && nt2 > nt) k_dummy_stress<<<nblk(nt2 - nt), BLOCK, 0, s2>>>(SB, V, nt, nt2);
             // the nodes' artificial viscosity reads only node data, after the
             // node side and the second BC call (k_deriv_nodes_mix takes it)
             if (h->dp.do_av)
-                k_av_nodes_mix<<<h->ntile_n, TILE, LAY_DERIV_NODES_MIX.bytes, s2>>>(SB, V, PL, h->dp, hu,
+                k_av_nodes_mix<<<h->ntile_n, TILE, LAY_AV_NODES_MIX.bytes, s2>>>(SB, V, PL, h->dp, hu,
                                                                                      h->av_nodes.p, nn);
             HIP_TRY(hipEventRecord(h->ev_join, s2));
         } else {
             if (nn > 0)
                 LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
-                           tanfi, coh, hu, nn);
+                           tanfi, coh, hu, nn, Q.sp_in, nullptr, 0.0);
             if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
+            if (st == 3 && nt2 > nt) LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
+            if (h->dp.do_av && nn > 0)
+                LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, LAY_AV_NODES_MIX.bytes, k_av_nodes_mix, SB, V, PL, h->dp, hu,
+                           h->av_nodes.p, nn);
         }
         if (nt > nn)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
-                       h->dp, time_sph, f2rk[st], 1, adapt, hu, nn, nt, stepv, h->sig2.p);
+                       h->dp, time_sph, Q, 1, adapt, hu, nn, nt, stepv, h->sig2.p, nullptr, 0.0, h->err.p);
         if (fork) HIP_TRY(hipStreamWaitEvent(h->stream, h->ev_join, 0));
         if (nn > 0)
             LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, LAY_DERIV_NODES_MIX.bytes, k_deriv_nodes_mix, SB, W, V, PL,
-                       h->dp, gxg, gyg, f2rk[st], h->err.p, hu, nn, stepv, nt > nn ? h->sig2.p : SB.stress,
-                       fork && h->dp.do_av ? h->av_nodes.p : nullptr);
-        if (st == 3 && nt2 > nt)
-            LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
+                       h->dp, gxg, gyg, Q, adapt, h->err.p, hu, nn, stepv, nt > nn ? h->sig2.p : SB.stress,
+                       h->dp.do_av ? h->av_nodes.p : nullptr);
     }
-    const bool hook = h->mlp || h->log_cap > 0;
     if (h->mlp) LAUNCH(K_SURROGATE, 1, 64, k_zero_u32, h->surr_count.p, 1);
-    LAUNCH(K_RK_FINAL, nblk(nt), BLOCK, k_rk_final, SB, W, dt, adapt, tanfi, coh, nn, nt, surrogate_dev(h),
-           hook ? 1 : 0, h->err.p);
+    if (hook)
+        LAUNCH(K_RK_FINAL, nblk(nt), BLOCK, k_rk_final, SB, W, dt, adapt, tanfi, coh, nn, nt, surrogate_dev(h),
+               h->err.p);
     if (h->mlp && adapt) {
         int rc = surrogate_correct(h, SB);
         if (rc) return rc;
@@ -908,10 +932,10 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
     if (nn > 0)
         LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt, tanfi,
-                   coh, hu, nn);
+                   coh, hu, nn, SB.stress, strain_rate, dt);
     if (nt > nn)
         LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL, h->dp,
-                   time_sph, 0.0, 0, adapt, hu, nn, nt, stepv, nullptr);
+                   time_sph, state_pass(SB), 0, adapt, hu, nn, nt, stepv, nullptr, strain_rate, dt, h->err.p);
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
     const bool xsph = h->xsph && h->p.update_x;
     if (xsph && nn > 0)
@@ -1077,17 +1101,17 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
     const PairLists PL = h->lists();
     const int adapt = h->dp.ncrit == 12;
     const double tanfi = h->dp.tanfi, coh = h->dp.coh;
-    const double f1rk[4] = {0., 0.5, 0.5, 1.0}, f2rk[4] = {1., 2., 2., 1.0};
     const bool bcs = h->p.no_bcs > 0 && nn > 0;
     const BcValues &BV = h->bc_vars;
     if (bcs) LAUNCH(K_BCS, 1, 64, k_bc_values, bc_values(h, time_sph), h->bc_vals.p);
     if (h->outside && h->p.sph_shift && itimestep > 1 && (itimestep - 1) % h->p.shift_update == 0) {
         // stress_point_update + adapt_stress2 on the new lists (2_...:99-109)
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn,
+                       SB.stress, nullptr, 0.0);
         if (nt > nn)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp,
-                       time_sph, 0.0, 0, adapt, nn, nt, nullptr);
+                       time_sph, state_pass(SB), 0, adapt, nn, nt, nullptr, nullptr, 0.0, h->err.p);
     }
     const bool lf = h->integrator == SPS_INTEGRATOR_LEAPFROG;
     // bc_int for apply_stress_free: the step's list after its first derivative
@@ -1102,31 +1126,34 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
         const double kdt = h->lf_first ? 0.5 * dt : dt;
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, bci_prev);
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn,
+                       SB.stress, nullptr, 0.0);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, bci_prev);
         if (nt > nn)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph,
-                       0.0, 0, adapt, nn, nt, nullptr);
+                       state_pass(SB), 0, adapt, nn, nt, nullptr, nullptr, 0.0, h->err.p);
         const bool av = h->dp.do_av && nn > 0;
         if (av) LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
         if (nn > 0)
             LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp,
-                       gxg, gyg, 1.0, h->err.p, nn, SB.stress, av ? h->av_nodes.p : nullptr);
-        LAUNCH(K_STAGE_BEGIN, nblk(nn), BLOCK, k_lf_kick, SB, W, kdt, nn);
+                       gxg, gyg, state_pass(SB), adapt, h->err.p, nn, SB.stress, av ? h->av_nodes.p : nullptr);
+        LAUNCH(K_LF_KICK, nblk(nn), BLOCK, k_lf_kick, SB, W, kdt, nn);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
         if (nn > 0)
-            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn,
+                       SB.stress, nullptr, 0.0);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
         if (nt > nn)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
-                       1.0, 1, adapt, nn, nt, nullptr);
+                       state_pass(SB), 1, adapt, nn, nt, nullptr, nullptr, 0.0, h->err.p);
         if (nt2 > nt) LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
         LAUNCH(K_RK_FINAL, nblk(nt), BLOCK, k_lf_final, SB, W, dt, adapt, tanfi, coh, nn, nt, h->err.p);
         h->lf_first = false;
     }
+    const bool hook = h->log_cap > 0;
+    const double *strain_rate = hook || lf ? nullptr : h->ddev.p;   // update_strain left to the update after the stages
     for (int st = 0; st < (lf ? 0 : 4); ++st) {
-        const double c1 = f1rk[st] * (dt);
-        if (st > 0) LAUNCH(K_STAGE_BEGIN, nblk(nt), BLOCK, k_stage_begin, SB, W, c1, adapt, tanfi, coh, nn, nt);
+        const StageStep Q = rk_stage(h, SB, st, dt, hook);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, st ? bci_cur : nullptr, st ? nullptr : bci_prev);
         // stress_point_update's two halves are independent: the node side
         // reads the stress points' stresses before their second return map
@@ -1143,40 +1170,41 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
             HIP_TRY(hipEventRecord(h->ev_fork, s));
             HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
             hipStream_t s2 = h->stream2;
-            k_spu_nodes<<<h->ntile_n, TILE, LAY_SPU_NODES.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, nn);
+            k_spu_nodes<<<h->ntile_n, TILE, LAY_SPU_NODES.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, nn, Q.sp_in,
+                                                                        nullptr, 0.0);
             if (bcs)
                 k_bcs<<<nblk(nn), BLOCK, 0, s2>>>(SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman,
                                                  h->normal.p, nn, st ? bci_cur : nullptr,
                                                  st ? nullptr : bci_prev);
+            if (st == 3 && nt2 > nt) k_dummy_stress<<<nblk(nt2 - nt), BLOCK, 0, s2>>>(SB, V, nt, nt2);
             if (av) k_av_nodes<<<h->ntile_n, TILE, lds_av_nodes(h), s2>>>(SB, V, PL, h->dp, h->av_nodes.p, nn);
             HIP_TRY(hipEventRecord(h->ev_join, s2));
         } else {
             if (nn > 0)
                 LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh,
-                           nn);
+                           nn, Q.sp_in, nullptr, 0.0);
             if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, st ? bci_cur : nullptr, st ? nullptr : bci_prev);
+            if (st == 3 && nt2 > nt) LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
             if (av) LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
         }
         if (nt > nn)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
-                       f2rk[st], 1, adapt, nn, nt, h->sig2.p);
+                       Q, 1, adapt, nn, nt, h->sig2.p, nullptr, 0.0, h->err.p);
         if (fork) HIP_TRY(hipStreamWaitEvent(s, h->ev_join, 0));
         if (nn > 0)
             LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp, gxg,
-                       gyg, f2rk[st], h->err.p, nn, nt > nn ? h->sig2.p : SB.stress, av ? h->av_nodes.p : nullptr);
-        if (st == 3 && nt2 > nt)
-            LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
+                       gyg, Q, adapt, h->err.p, nn, nt > nn ? h->sig2.p : SB.stress, av ? h->av_nodes.p : nullptr);
     }
-    const bool hook = h->log_cap > 0;
-    if (!lf)
+    if (hook && !lf)
         LAUNCH(K_RK_FINAL, nblk(nt), BLOCK, k_rk_final, SB, W, dt, adapt, tanfi, coh, nn, nt, surrogate_dev(h),
-               hook ? 1 : 0, h->err.p);
+               h->err.p);
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
     if (nn > 0)
-        LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn);
+        LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh, nn,
+                   SB.stress, strain_rate, dt);
     if (nt > nn)
-        LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph, 0.0,
-                   0, adapt, nn, nt, nullptr);
+        LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 0), k_sp_update, SB, W, V, PL, h->dp, time_sph,
+                   state_pass(SB), 0, adapt, nn, nt, nullptr, strain_rate, dt, h->err.p);
     if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, bci_cur, nullptr);
     if (h->bcint && nn > 0)   // the next step's first BC calls see this step's list
         LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcint_keep, h->nodeinfo.p, SB.orig, h->bcint_prev.p, nn);
@@ -1535,7 +1563,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     h->S[1].release();
     dfree(h->x0); dfree(h->vel0); dfree(h->rk_vel); dfree(h->rhs2); dfree(h->f_bound);
     dfree(h->art_visc); dfree(h->stress0); dfree(h->rk_stress); dfree(h->rhs1); dfree(h->grad_u);
-    dfree(h->rk_dev); dfree(h->ddev); dfree(h->grid); dfree(h->split); dfree(h->bparts);
+    dfree(h->rk_dev); dfree(h->sig2); dfree(h->stress_b); dfree(h->av_nodes); dfree(h->ddev); dfree(h->grid); dfree(h->split); dfree(h->bparts);
     dfree(h->cellkey); dfree(h->new_cell); dfree(h->cell); dfree(h->kcount); dfree(h->kstart);
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
     dfree(h->cnt); dfree(h->off); dfree(h->scan_tmp); dfree(h->ctot); dfree(h->cstart_rm); dfree(h->err);

@@ -703,6 +703,8 @@ struct GlobalCells {
 // Partner fields from the global state (j is a storage slot).
 struct GlobalFields {
     StateBufs S;
+    const double *dd = nullptr;   // update_strain still to be applied: + dt dd (k_spu_nodes)
+    double dt = 0.0;
     __device__ __forceinline__ double2 xk(int, int j) const { return S.x[j]; }
     __device__ __forceinline__ double hk(int, int j) const { return S.hsml[j]; }
     template <int K> __device__ __forceinline__ double2 x(KindTag<K>, int j) const { return S.x[j]; }
@@ -711,7 +713,9 @@ struct GlobalFields {
     template <int K> __device__ __forceinline__ double rho(KindTag<K>, int j) const { return S.rho[j]; }
     template <int K> __device__ __forceinline__ double2 vel(KindTag<K>, int j) const { return S.vel[j]; }
     template <int K> __device__ __forceinline__ double4 st(KindTag<K>, int j) const { return S.stress[j]; }
-    template <int K> __device__ __forceinline__ double iv(KindTag<K>, int j) const { return S.ivar1[j]; }
+    template <int K> __device__ __forceinline__ double iv(KindTag<K>, int j) const {
+        return dd ? S.ivar1[j] + dt * dd[j] : S.ivar1[j];
+    }
     template <int K> __device__ __forceinline__ double mr(KindTag<K>, int j) const { return S.mass[j] / S.rho[j]; }
     template <int K> __device__ __forceinline__ double3 sr2(KindTag<K>, int j) const {
         const double rs = S.rho[j], rs2 = rs * rs;
@@ -1257,15 +1261,33 @@ struct Work {
     double *rk_dev, *ddev;
 };
 
-// Start of a step and its first RK stage in one pass: vx0, x0 (2_...:114),
-// the RK4 prologue (2_...:681-690: stage-0 state, accumulators and the
-// velocities and stresses zeroed, dummies included) and the stage-0 state
-// with its first adapt_stress2 (2_...:700-701, 715).  The stage-0 update
-// v0 + 0 * rhs of the reference, whose right-hand sides are zero then, is
-// v0 + 0.0 (a zero of either sign becomes +0, as there); node stresses start
-// from the zeroed ones.  The right-hand sides themselves need no clearing:
-// the stage tails write them before any later stage reads them.  vx0 and
-// vel0 are the same velocities: Work.vx0 may alias vel0.
+// What a derivative pass leaves.  The RK stages end with the next stage's
+// state (2_...:700-701 and the return map after it) or, the last one, with
+// the step's (2_...:784-799): the right-hand side then never leaves the
+// registers, and the accumulators are not cleared before the first stage.  As
+// launches of their own the stage updates and the final one moved 0.6 GB of
+// 8.5 GB per step at 1 M + 1 M particles, 210 us of 2530 (STAGE_RHS is left
+// to the steps whose end needs the sums: leapfrog, and the recording of
+// plastic trial states in k_rk_final).  What only the caller reads (grad_u,
+// art_visc) is written by the pass that ends the step.
+enum StageEnd { STAGE_FIRST, STAGE_MID, STAGE_LAST, STAGE_RHS };
+struct StageStep {
+    int end;                        // StageEnd
+    int first;                      // the step's first derivative pass: the wall forces, which depend
+                                    // on positions alone, are computed by it and read by the others
+    double f2;                      // weight of the stage in the sums
+    double c;                       // dt times the next stage's coefficient, or dt / 6
+    const double4 *sp_in;           // the stress points' stresses of the stage
+    double4 *sp_out;                // and of the next one (not sp_in, which the node side reads meanwhile)
+};
+
+// Start of a step and its first RK stage in one pass: vx0 (2_...:114), the
+// RK4 prologue (2_...:681-690: stage-0 state, the velocities and stresses
+// zeroed, dummies included) and the stage-0 state with its first
+// adapt_stress2 (2_...:700-701, 715).  The stage-0 update v0 + 0 * rhs of the
+// reference, whose right-hand sides are zero then, is v0 + 0.0 (a zero of
+// either sign becomes +0, as there); node stresses start from the zeroed
+// ones.  vx0 and vel0 are the same velocities: Work.vx0 may alias vel0.
 __global__ void k_stage_first(StateBufs S, Work W, int adapt, double tanfi, double coh, int nn, int nt,
                               int nt2) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1278,11 +1300,8 @@ __global__ void k_stage_first(StateBufs S, Work W, int adapt, double tanfi, doub
     const double2 v = S.vel[i];
     W.vel0[i] = v;
     if (W.vx0 != W.vel0) W.vx0[i] = v;
-    W.x0[i] = S.x[i];
-    W.rk_dev[i] = 0.0;
     material_tc(S, i, tanfi, coh);
     if (i < nn) {
-        W.rk_vel[i] = make_double2(0, 0);
         S.vel[i] = make_double2(v.x + 0.0, v.y + 0.0);
         double4 s = make_double4(0, 0, 0, 0);
         if (adapt) adapt_stress(s, tanfi, coh);
@@ -1290,32 +1309,8 @@ __global__ void k_stage_first(StateBufs S, Work W, int adapt, double tanfi, doub
     } else {
         const double4 s0 = S.stress[i];
         W.stress0[i] = s0;
-        W.rk_stress[i] = make_double4(0, 0, 0, 0);
         S.vel[i] = make_double2(0, 0);
         double4 s = make_double4(s0.x + 0.0, s0.y + 0.0, s0.z + 0.0, s0.w + 0.0);
-        if (adapt) adapt_stress(s, tanfi, coh);
-        S.stress[i] = s;
-    }
-}
-
-// Stage state of stages 2-4 (2_...:700-701) and the first adapt_stress2 of
-// the stage.
-__global__ void k_stage_begin(StateBufs S, Work W, double c1, int adapt, double tanfi, double coh,
-                              int nn, int nt) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nt) return;
-    material_tc(S, i, tanfi, coh);
-    if (i < nn) {
-        double2 v0 = W.vel0[i], r2 = W.rhs2[i];
-        S.vel[i] = make_double2(v0.x + c1 * r2.x, v0.y + c1 * r2.y);
-        if (adapt) {
-            double4 s = S.stress[i];
-            adapt_stress(s, tanfi, coh);
-            S.stress[i] = s;
-        }
-    } else {
-        double4 s0 = W.stress0[i], r1 = W.rhs1[i];
-        double4 s = make_double4(s0.x + c1 * r1.x, s0.y + c1 * r1.y, s0.z + c1 * r1.z, s0.w + c1 * r1.w);
         if (adapt) adapt_stress(s, tanfi, coh);
         S.stress[i] = s;
     }
@@ -1836,8 +1831,15 @@ __device__ __forceinline__ bool needs_split(const Tile &T, const SearchView &V, 
 
 // stress_point_update (2_...:403-482) for node receivers: CSPM-normalised
 // stress and plastic strain from the stress points, then adapt_stress2.
+// sp_in: the stress points' stresses of the stage.  dd (the update after the
+// RK stages): the step's plastic strain rates, whose update_strain
+// (3_...:1847-1863) the stress points' plastic strain still waits for (it was
+// read by the node side of the last stage beside k_sp_update, which applies
+// it in its own update after this kernel).
 __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, PairLists PL, int adapt,
-                                                    double tanfi, double coh, int nn) {
+                                                    double tanfi, double coh, int nn,
+                                                    const double4 *__restrict__ sp_in,
+                                                    const double *__restrict__ dd, double dt) {
     __shared__ StagePlan pl;
     constexpr const LdsLayout &LY = LAY_SPU_NODES;
     const WalkCtx C = walk_ctx(V);
@@ -1857,7 +1859,9 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, P
             double m, rho, iv;
             double4 st;
         };
-        copy_kind<KIND_SP>(T, V, C, nullptr, pl, [&](int g) { return Item{S.mass[g], S.rho[g], S.ivar1[g], S.stress[g]}; },
+        copy_kind<KIND_SP>(T, V, C, nullptr, pl, [&](int g) {
+                               return Item{S.mass[g], S.rho[g], dd ? S.ivar1[g] + dt * dd[g] : S.ivar1[g], sp_in[g]};
+                           },
                            [&](int i, const Item &v) {
                                lds_at<double>(LY.m[KIND_SP])[i] = v.m;
                                lds_at<double>(LY.rho[KIND_SP])[i] = v.rho;
@@ -1884,16 +1888,19 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, P
         norm = norm + (w * ms) / rs;
     };
     if (inside) {
+        StateBufs S2 = S;   // the stress points' stresses from sp_in (the walks read no node's)
+        S2.stress = const_cast<double4 *>(sp_in);
+        const GlobalFields GF{S2, dd, dt};
         if (lds) {
             lw.run(LdsFields<LY>{}, body);
         } else if (ok == LIST_SLOTS) {
-            lw.run_slots(PL.iah, GlobalFields{S}, body);
+            lw.run_slots(PL.iah, GF, body);
         } else {
             int cx, cy;
             cell_xy(V.cell[r], C.g, cx, cy);
             const bool check = needs_split(T, V, C, r);
             const SplitClass cls{check, check ? V.proc[r] : 0, V.proc, V.cnt, V.off, C.sp};
-            walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy, S.x[r],
+            walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, S.x[r],
                                   S.hsml[r], KIND_NODE, r, C.any_fwd ? check : C.any_rev, C.any_fwd, V.pi, cls,
                                   body);
         }
@@ -1912,12 +1919,14 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, P
 
 // The end of get_derivatives for stress point r (CSPM correction, div1,
 // grad_u; 2_...:596-644) from its velocity-gradient sums and CSPM moments,
-// then plastic_terms, the Jaumann spin, the stress right-hand side and the RK
-// accumulation of the stage (2_...:730-777).  st is its updated stress.
+// then plastic_terms, the Jaumann spin, the stress right-hand side and what
+// the stage leaves (2_...:730-777; StageStep).  st is its updated stress.
 __device__ __forceinline__ void sp_stage_tail(const DevParams &P, const StateBufs &S, const Work &W, int r,
                                               const double4 &st, double g00, double g01, double g10, double g11,
                                               double A0, double A1, double A2, double A3, double time_sph,
-                                              double f2) {
+                                              const StageStep &Q, int adapt, int *__restrict__ err) {
+    const double f2 = Q.f2;
+    const bool last = Q.end >= STAGE_LAST;
     if (P.cspm) {
         double A4 = A0 * A3 - A1 * A2;
         if (fabs(A4) < P.cspm_tol) {
@@ -1936,7 +1945,7 @@ __device__ __forceinline__ void sp_stage_tail(const DevParams &P, const StateBuf
     d1.z = -(P.D33 * g10 + P.D33 * g01);
     d1.w = -(P.D41 * g00 + P.D42 * g11);
     double4 gu = make_double4(g00, g10, g01, g11);
-    W.grad_u[r] = gu;
+    if (last) W.grad_u[r] = gu;
     double4 Gs;
     double der1;
     double fdr = S.fdr[r];
@@ -1955,10 +1964,28 @@ __device__ __forceinline__ void sp_stage_tail(const DevParams &P, const StateBuf
     rh.y = -d1.y + sp.y + Gs.y;
     rh.z = -d1.z + sp.z + Gs.z;
     rh.w = -d1.w + sp.w + Gs.w;
-    W.rhs1[r] = rh;
-    double4 rk = W.rk_stress[r];
-    W.rk_stress[r] = make_double4(rk.x + f2 * rh.x, rk.y + f2 * rh.y, rk.z + f2 * rh.z, rk.w + f2 * rh.w);
-    W.rk_dev[r] = W.rk_dev[r] + der1 * f2;
+    double4 rk = make_double4(0.0, 0.0, 0.0, 0.0);
+    double dev = 0.0;
+    if (!Q.first) {
+        rk = W.rk_stress[r];
+        dev = W.rk_dev[r];
+    }
+    rk = make_double4(rk.x + f2 * rh.x, rk.y + f2 * rh.y, rk.z + f2 * rh.z, rk.w + f2 * rh.w);
+    dev = dev + der1 * f2;
+    if (Q.end == STAGE_RHS) W.rhs1[r] = rh;
+    if (Q.end != STAGE_LAST) {
+        W.rk_stress[r] = rk;
+        W.rk_dev[r] = dev;
+    }
+    if (Q.end == STAGE_RHS) return;
+    const double4 s0 = W.stress0[r], d = Q.end == STAGE_LAST ? rk : rh;
+    double4 s = make_double4(s0.x + Q.c * d.x, s0.y + Q.c * d.y, s0.z + Q.c * d.z, s0.w + Q.c * d.w);
+    if (adapt) adapt_stress(s, P.tanfi, P.coh);
+    Q.sp_out[r] = s;
+    if (Q.end == STAGE_LAST) {
+        if (S.ood[r] == 0 && !finite4(s)) atomicOr(err, ERR_NONFINITE);
+        W.ddev[r] = dev / 6;
+    }
 }
 
 // Stress-point receivers: stress_point_update (CSPM-normalised velocity from
@@ -1972,9 +1999,13 @@ __device__ __forceinline__ void sp_stage_tail(const DevParams &P, const StateBuf
 // sig_out: where the stress after the return map goes (null: the state's
 // stress; the RK stages give a separate buffer, so that the node side of
 // stress_point_update can read the stresses before it at the same time).
+// dd (the update after the RK stages): update_strain's plastic strain rates,
+// applied here.
 __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S, Work W, SearchView V, PairLists PL,
-                                                    DevParams P, double time_sph, double f2, int deriv,
-                                                    int adapt, int nn, int nt, double4 *__restrict__ sig_out) {
+                                                    DevParams P, double time_sph, StageStep Q, int deriv,
+                                                    int adapt, int nn, int nt, double4 *__restrict__ sig_out,
+                                                    const double *__restrict__ dd, double dt,
+                                                    int *__restrict__ err) {
     __shared__ StagePlan pl[2];
     constexpr const LdsLayout &LY = LAY_SP_UPDATE;
     const WalkCtx C = walk_ctx(V);
@@ -2060,14 +2091,17 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
         vr = make_double2(v0 / norm, v1 / norm);
         S.vel[r] = vr;
     }
-    double4 st = S.stress[r];
+    double4 st = Q.sp_in[r];
     const DevParams Pm = material_params(P, S, r);
     if (adapt) adapt_stress(st, Pm.tanfi, Pm.coh);
     if (sig_out)
         sig_out[r] = st;
     else if (adapt)
         S.stress[r] = st;
-    if (!deriv) return;
+    if (!deriv) {
+        if (dd) S.ivar1[r] = S.ivar1[r] + dt * dd[r];   // update_strain (k_spu_nodes)
+        return;
+    }
 
     // get_derivatives
     double g00 = 0, g01 = 0, g10 = 0, g11 = 0;   // grad1_tmp(a,b): d v_a / d x_b
@@ -2127,7 +2161,7 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
             walk_stencil<MASK_NODE | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GlobalFields{S}, C.g, cx, cy,
                                                  xr, hr, KIND_SP, r, rev_g, C.any_fwd, V.pi, cls, grad);
     }
-    sp_stage_tail(Pm, S, W, r, st, g00, g01, g10, g11, A0, A1, A2, A3, time_sph, f2);
+    sp_stage_tail(Pm, S, W, r, st, g00, g01, g10, g11, A0, A1, A2, A3, time_sph, Q, adapt, err);
 }
 
 // boundary_forces for one node: the nonzero terms of its inner-layer dummies
@@ -2192,8 +2226,10 @@ __device__ __forceinline__ void node_stage_tail(const StateBufs &S, const Work &
                                                 double2 xr, double2 vr, double hr, double q00, double q01,
                                                 double q10, double q11, double q20, double q21, double A0,
                                                 double A1, double A2, double A3, int ndum, float ax, float ay,
-                                                double gx_grav, double gy_grav, double f2,
-                                                int *__restrict__ err) {
+                                                double gx_grav, double gy_grav, const StageStep &Q, int adapt,
+                                                double4 sr, int *__restrict__ err) {
+    const bool last = Q.end >= STAGE_LAST;
+    const double f2 = Q.f2;
     if (P.cspm) {
         double A4 = A0 * A3 - A1 * A2;
         if (fabs(A4) < P.cspm_tol) {
@@ -2213,28 +2249,47 @@ __device__ __forceinline__ void node_stage_tail(const StateBufs &S, const Work &
     const double Gy = gy_grav - P.damping * vr.y;
     // boundary_forces
     double2 fb = W.f_bound[r];
-    if (P.do_bforce) {
+    if (P.do_bforce && Q.first) {
         fb = ndum ? wall_force(S, V, C, cx, cy, xr, hr, P, err) : make_double2(0.0, 0.0);
         W.f_bound[r] = fb;
     }
     double2 avf = make_double2(0.0, 0.0);
     if (P.do_av) {
         avf = make_double2(-(double)ax, -(double)ay);
-        W.art_visc[r] = avf;
+        if (last) W.art_visc[r] = avf;
     }
     double2 rh;
     rh.x = -d2x + Gx + avf.x + fb.x + 0.0;
     rh.y = -d2y + Gy + avf.y + fb.y + 0.0;
-    W.rhs2[r] = rh;
-    double2 rk = W.rk_vel[r];
-    W.rk_vel[r] = make_double2(rk.x + f2 * rh.x, rk.y + f2 * rh.y);
+    if (Q.end == STAGE_RHS) W.rhs2[r] = rh;
+    double2 rk = make_double2(0.0, 0.0);
+    if (!Q.first) rk = W.rk_vel[r];
+    rk = make_double2(rk.x + f2 * rh.x, rk.y + f2 * rh.y);
+    if (Q.end != STAGE_LAST) W.rk_vel[r] = rk;
+    if (Q.end == STAGE_RHS) return;
+    const double2 v0 = W.vel0[r], d = Q.end == STAGE_LAST ? rk : rh;
+    const double2 v = make_double2(v0.x + Q.c * d.x, v0.y + Q.c * d.y);
+    S.vel[r] = v;
+    // the return map of the node stresses: only a node without stress-point
+    // partners keeps it, and it mostly changes nothing
+    if (adapt) {
+        const double4 s0 = sr;
+        double tanfi = P.tanfi, coh = P.coh;
+        material_tc(S, r, tanfi, coh);
+        adapt_stress(sr, tanfi, coh);
+        if (sr.x != s0.x || sr.y != s0.y || sr.z != s0.z || sr.w != s0.w) S.stress[r] = sr;
+    }
+    if (Q.end == STAGE_LAST) {
+        if (S.ood[r] == 0 && !(finite4(sr) && finite2(v))) atomicOr(err, ERR_NONFINITE);
+        W.ddev[r] = 0.0;
+    }
 }
 
 // sp_stress: the stress points' stresses after the stage's second return
 // map (k_sp_update's sig_out, or the state's stress).
 __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_deriv_nodes(StateBufs S, Work W, SearchView V, PairLists PL,
-                                                      DevParams P, double gx_grav, double gy_grav, double f2,
-                                                      int *__restrict__ err, int nn,
+                                                      DevParams P, double gx_grav, double gy_grav, StageStep Q,
+                                                      int adapt, int *__restrict__ err, int nn,
                                                       const double4 *__restrict__ sp_stress,
                                                       const float2 *__restrict__ av_in) {
     __shared__ StagePlan pl[2];
@@ -2351,7 +2406,7 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_deriv_nodes(StateBufs 
     }
     const double2 vr = S.vel[r];
     node_stage_tail(S, W, V, C, P, r, cx, cy, xr, vr, hr, q00, q01, q10, q11, q20, q21, A0, A1, A2, A3, ndum,
-                    ax, ay, gx_grav, gy_grav, f2, err);
+                    ax, ay, gx_grav, gy_grav, Q, adapt, sr, err);
 }
 
 // artificial_viscosity (2_...:826-904) for the node receivers: the list-order
@@ -2532,10 +2587,11 @@ __global__ void k_dummy_stress(StateBufs S, SearchView V, int nt, int nt2) {
     if (last >= 0) S.stress[r] = S.stress[last];
 }
 
-// End of RK4 (2_...:784-799) and update_strain (3_...:1847-1863).
-// hook: record the stress points' plastic trial states (SurrogateDev).
+// End of RK4 (2_...:784-799) and update_strain (3_...:1847-1863) of the steps
+// that record the stress points' plastic trial states (SurrogateDev);
+// the others end in the last stage's kernels (StageStep).
 __global__ void k_rk_final(StateBufs S, Work W, double dt, int adapt, double tanfi, double coh,
-                           int nn, int nt, SurrogateDev G, int hook, int *__restrict__ err) {
+                           int nn, int nt, SurrogateDev G, int *__restrict__ err) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nt) return;
     double c = dt / 6;
@@ -2551,17 +2607,15 @@ __global__ void k_rk_final(StateBufs S, Work W, double dt, int adapt, double tan
             S.stress[i] = s;
         }
         if (watched && !(finite4(s) && finite2(v))) atomicOr(err, ERR_NONFINITE);
-        W.ddev[i] = W.rk_dev[i] / 6;
+        W.ddev[i] = 0.0;
     } else {
         double4 s0 = W.stress0[i], rk = W.rk_stress[i];
         double4 s = make_double4(s0.x + c * rk.x, s0.y + c * rk.y, s0.z + c * rk.z, s0.w + c * rk.w);
-        if (adapt && hook) {
+        if (adapt) {
             const double4 tr = s;
             adapt_stress(s, tanfi, coh);
             if (s.x != tr.x || s.y != tr.y || s.z != tr.z || s.w != tr.w)
                 surrogate_record(G, i, s0, tr, s, tanfi, coh);
-        } else if (adapt) {
-            adapt_stress(s, tanfi, coh);
         }
         S.stress[i] = s;
         if (watched && !finite4(s)) atomicOr(err, ERR_NONFINITE);
@@ -2596,7 +2650,7 @@ __global__ void k_lf_final(StateBufs S, Work W, double dt, int adapt, double tan
             S.stress[i] = s;
         }
         if (watched && !(finite4(s) && finite2(S.vel[i]))) atomicOr(err, ERR_NONFINITE);
-        W.ddev[i] = W.rk_dev[i];
+        W.ddev[i] = 0.0;
         return;
     }
     const double4 s0 = W.stress0[i], r = W.rhs1[i];
@@ -2619,9 +2673,10 @@ __global__ void k_position(StateBufs S, Work W, double dt, int update_x, int nn,
     if (i >= nt) return;
     double2 v0 = W.vx0[i], v = S.vel[i];
     double2 xn = make_double2(0.0, 0.0);
+    const double2 x0 = S.x[i];
+    W.x0[i] = x0;   // the positions of the step's pairs (x0, 2_...:114)
     if (drift) {   // leapfrog: the drift with the half-step velocities
         if (update_x) {
-            const double2 x0 = W.x0[i];
             xn = make_double2(x0.x + dt * v.x, x0.y + dt * v.y);
             S.x[i] = xn;
             if (i < nn) {
@@ -2634,7 +2689,7 @@ __global__ void k_position(StateBufs S, Work W, double dt, int update_x, int nn,
         }
     } else if (update_x && xv) {
         const double eps = 0.5;
-        const double2 x0 = W.x0[i], s = xv[i];
+        const double2 s = xv[i];
         xn = make_double2(x0.x + dt * (v.x + eps * s.x), x0.y + dt * (v.y + eps * s.y));
         S.x[i] = xn;
         if (i < nn) {
@@ -2644,7 +2699,6 @@ __global__ void k_position(StateBufs S, Work W, double dt, int update_x, int nn,
     } else if (update_x) {
         float hx = (float)(0.5 * (v0.x + v.x));
         float hy = (float)(0.5 * (v0.y + v.y));
-        double2 x0 = W.x0[i];
         xn = make_double2(x0.x + (double)hx * dt, x0.y + (double)hy * dt);
         S.x[i] = xn;
         if (i < nn) {

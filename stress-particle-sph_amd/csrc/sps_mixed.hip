@@ -68,20 +68,26 @@ constexpr LdsLayout layout_deriv_nodes_mix() {
     L.h[KIND_DUMMY] = o; o += 4 * CAP_D;
     L.m[KIND_DUMMY] = o; o += 4 * CAP_D;
     L.rho[KIND_DUMMY] = o; o += 4 * CAP_D;
-    const int phase1 = o;
-    o = 0;
+    L.bytes = o;
+    return L;
+}
+
+constexpr LdsLayout layout_av_nodes_mix() {
+    LdsLayout L = layout_none();
+    int o = 0;
     L.x[KIND_NODE] = o; o += 8 * CAP;
     L.v[KIND_NODE] = o; o += 8 * CAP;
     L.h[KIND_NODE] = o; o += 4 * CAP;
     L.m[KIND_NODE] = o; o += 4 * CAP;
     L.rho[KIND_NODE] = o; o += 4 * CAP;
-    L.bytes = o > phase1 ? o : phase1;
+    L.bytes = o;
     return L;
 }
 
 constexpr LdsLayout LAY_SPU_NODES_MIX = layout_spu_nodes_mix();
 constexpr LdsLayout LAY_SP_UPDATE_MIX = layout_sp_update_mix();
 constexpr LdsLayout LAY_DERIV_NODES_MIX = layout_deriv_nodes_mix();
+constexpr LdsLayout LAY_AV_NODES_MIX = layout_av_nodes_mix();
 
 // Partner fields of a single-precision window.
 template <const LdsLayout &LY> struct LdsFieldsMix {
@@ -113,6 +119,8 @@ template <const LdsLayout &LY> struct LdsFieldsMix {
 struct GlobalFieldsMix {
     StateBufs S;
     double2 o;
+    const double *dd = nullptr;   // as in GlobalFields
+    double dt = 0.0;
     __device__ __forceinline__ double2 xk(int, int j) const { return S.x[j]; }
     __device__ __forceinline__ double hk(int, int j) const { return S.hsml[j]; }
     template <int K> __device__ __forceinline__ float2 x(KindTag<K>, int j) const { return rel_pos(S.x[j], o); }
@@ -130,7 +138,9 @@ struct GlobalFieldsMix {
         const double4 s = S.stress[j];
         return make_float4((float)s.x, (float)s.y, (float)s.z, (float)s.w);
     }
-    template <int K> __device__ __forceinline__ float iv(KindTag<K>, int j) const { return (float)S.ivar1[j]; }
+    template <int K> __device__ __forceinline__ float iv(KindTag<K>, int j) const {
+        return (float)(dd ? S.ivar1[j] + dt * dd[j] : S.ivar1[j]);
+    }
     template <int K> __device__ __forceinline__ float3 sr2(KindTag<K>, int j) const {
         const double rs = S.rho[j], rs2 = rs * rs;
         const double4 s = S.stress[j];
@@ -169,7 +179,9 @@ __device__ __forceinline__ float2 to_rel(double2 x, double2 o) { return rel_pos(
 // ------------------------------------------------------------------ kernels
 // stress_point_update for node receivers (as k_spu_nodes).
 __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView V, PairLists PL, int adapt,
-                                                        double tanfi, double coh, float hu, int nn) {
+                                                        double tanfi, double coh, float hu, int nn,
+                                                        const double4 *__restrict__ sp_in,
+                                                        const double *__restrict__ dd, double dt) {
     __shared__ StagePlan pl;
     constexpr const LdsLayout &LY = LAY_SPU_NODES_MIX;
     const WalkCtx C = walk_ctx(V);
@@ -194,7 +206,10 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
             double4 st;
         };
         copy_kind<KIND_SP>(T, V, C, nullptr, pl,
-                           [&](int g) { return Item{S.x[g], S.hsml[g], S.mass[g], S.rho[g], S.ivar1[g], S.stress[g]}; },
+                           [&](int g) {
+                               return Item{S.x[g], S.hsml[g], S.mass[g], S.rho[g],
+                                           dd ? S.ivar1[g] + dt * dd[g] : S.ivar1[g], sp_in[g]};
+                           },
                            [&](int i, const Item &v) {
                                lds_at<float2>(LY.x[KIND_SP])[i] = to_rel(v.x, o);
                                lds_at<float>(LY.h[KIND_SP])[i] = (float)v.h;
@@ -227,7 +242,9 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
         } else {
             int cx, cy;
             cell_xy(V.cell[r], C.g, cx, cy);
-            walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GlobalFieldsMix{S, o}, C.g, cx, cy, xr, hr,
+            StateBufs S2 = S;   // the stress points' stresses from sp_in (the walk reads no node's)
+            S2.stress = const_cast<double4 *>(sp_in);
+            walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GlobalFieldsMix{S2, o, dd, dt}, C.g, cx, cy, xr, hr,
                                   KIND_NODE, r, false, true, V.pi, NoClass{}, body);
         }
     }
@@ -249,10 +266,12 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
 // sig_out: where the stress after the return map goes (null: the state's
 // stress), as in k_sp_update.
 __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, SearchView V, PairLists PL,
-                                                        DevParams P, double time_sph, double f2, int deriv,
+                                                        DevParams P, double time_sph, StageStep Q, int deriv,
                                                         int adapt, float hu, int nn, int nt,
                                                         const double *__restrict__ stepv,
-                                                        double4 *__restrict__ sig_out) {
+                                                        double4 *__restrict__ sig_out,
+                                                        const double *__restrict__ dd, double dt,
+                                                        int *__restrict__ err) {
     if (stepv) time_sph = stepv[0];
     __shared__ StagePlan pl[2];
     constexpr const LdsLayout &LY = LAY_SP_UPDATE_MIX;
@@ -337,14 +356,17 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
         vr = make_double2(v0.get() / nd, v1.get() / nd);
         S.vel[r] = vr;
     }
-    double4 st = S.stress[r];
+    double4 st = Q.sp_in[r];
     const DevParams Pm = material_params(P, S, r);
     if (adapt) adapt_stress(st, Pm.tanfi, Pm.coh);
     if (sig_out)
         sig_out[r] = st;
     else if (adapt)
         S.stress[r] = st;
-    if (!deriv) return;
+    if (!deriv) {
+        if (dd) S.ivar1[r] = S.ivar1[r] + dt * dd[r];   // update_strain, as in k_sp_update
+        return;
+    }
 
     // get_derivatives
     const float vrx = (float)vr.x, vry = (float)vr.y;
@@ -401,29 +423,44 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
                                                  r, false, true, V.pi, NoClass{}, grad);
     }
     sp_stage_tail(Pm, S, W, r, st, g00.get(), g01.get(), g10.get(), g11.get(), A0.get(), A1.get(), A2.get(),
-                  A3.get(), time_sph, f2);
+                  A3.get(), time_sph, Q, adapt, err);
 }
 
-// artificial_viscosity (2_...:826-904) of node receiver r in the mixed
-// form: its node partners (list B) with kernel values computed in single
+// artificial_viscosity (2_...:826-904) of the node receivers in the mixed
+// form: node partners (list B) with kernel values computed in single
 // precision from window-relative positions, and compensated sums; rounded
-// to single precision as node_stage_tail takes them.  Every thread of the
-// block calls it (it stages the node window through LDS).
-__device__ __forceinline__ float2 av_mix(const StateBufs &S, const SearchView &V, const PairLists &PL,
-                                         const DevParams &P, const WalkCtx &C, const Tile &T, int tile, int r,
-                                         bool inside, bool tiled, int cx, int cy, double2 xr, double2 vr,
-                                         double hr, double rhor, float2 xrr, double2 o, float hu, StagePlan &pl) {
-    constexpr const LdsLayout &LY = LAY_DERIV_NODES_MIX;
+// to single precision as node_stage_tail takes them, written to av_out for
+// k_deriv_nodes_mix.  It reads only node data that the stress points' update
+// leaves alone, so the RK stages run it beside k_sp_update_mix, and it ends
+// before k_deriv_nodes_mix writes the next stage's velocities.
+__global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V, PairLists PL, DevParams P,
+                                                       float hu, float2 *__restrict__ av_out, int nn) {
+    __shared__ StagePlan pl;
+    constexpr const LdsLayout &LY = LAY_AV_NODES_MIX;
+    const WalkCtx C = walk_ctx(V);
+    const int tile = tile_index();
+    const Tile T = PL.tiles[tile];
+    if (T.first >= T.end) return;
+    const int r = T.first + (int)threadIdx.x;
+    const bool active = r < T.end;
+    const int key_r = active ? V.cell[r] : C.g.ndivt;
+    const bool inside = key_r < C.g.ndivt;
+    const double2 o = S.x[T.first];
+    int cx = 0, cy = 0;
+    if (inside) cell_xy(key_r, C.g, cx, cy);
+    const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
+    const double2 xr = S.x[ra], vr = S.vel[ra];
+    const double rhor = S.rho[ra], hr = S.hsml[ra];
+    const float2 xrr = to_rel(xr, o);
     const LdsFieldsMix<LY> LF{};
     const GlobalFieldsMix GF{S, o};
     KSum ax, ay;
-    if (!P.do_av) return make_float2(0.0f, 0.0f);
     ListWalk<MASK_NODE, false, false> lb;
     lb.start(PL.ib, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_b[r] : 0);
-    bool lds2 = tiled;
+    bool lds2 = PL.ok[tile] == LIST_WINDOW;
     if (lds2) {
         load_plan<KIND_NODE>(PL, tile, 0, pl);
-        __syncthreads();   // also: the phase-1 walks are done with the shared bytes
+        __syncthreads();
         lds2 = pl.total <= CAP;
     }
     if (lds2) {
@@ -463,7 +500,7 @@ __device__ __forceinline__ float2 av_mix(const StateBufs &S, const SearchView &V
             walk_stencil<MASK_NODE>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr, KIND_NODE, r,
                                     false, true, V.pi, NoClass{}, av);
     }
-    return make_float2((float)ax.get(), (float)ay.get());
+    if (active) av_out[r] = make_float2((float)ax.get(), (float)ay.get());
 }
 
 // Node receivers (as k_deriv_nodes).
@@ -471,8 +508,8 @@ __device__ __forceinline__ float2 av_mix(const StateBufs &S, const SearchView &V
 // sp_stress: the stress points' stresses after the stage's return map
 // (k_sp_update_mix's sig_out, or the state's stress).
 __global__ __launch_bounds__(TILE) void k_deriv_nodes_mix(StateBufs S, Work W, SearchView V, PairLists PL,
-                                                          DevParams P, double gx_grav, double gy_grav, double f2,
-                                                          int *__restrict__ err, float hu, int nn,
+                                                          DevParams P, double gx_grav, double gy_grav, StageStep Q,
+                                                          int adapt, int *__restrict__ err, float hu, int nn,
                                                           const double *__restrict__ stepv,
                                                           const double4 *__restrict__ sp_stress,
                                                           const float2 *__restrict__ av_in) {
@@ -593,44 +630,13 @@ __global__ __launch_bounds__(TILE) void k_deriv_nodes_mix(StateBufs S, Work W, S
         }
     }
 
-    // phase 2: artificial viscosity over node partners (type 3), here or,
-    // beside k_sp_update_mix, by k_av_nodes_mix (av_in)
+    // the artificial viscosity over node partners (type 3), summed by k_av_nodes_mix
     float2 avv = make_float2(0.0f, 0.0f);
-    if (av_in) {
-        if (active) avv = av_in[r];
-    } else {
-        avv = av_mix(S, V, PL, P, C, T, tile, r, inside, tiled, cx, cy, xr, vr, hr, rhor, xrr, o, hu, pl[0]);
-    }
+    if (av_in && active) avv = av_in[r];
     if (!active) return;
     node_stage_tail(S, W, V, C, P, r, cx, cy, xr, vr, hr, q00.get(), q01.get(), q10.get(), q11.get(), q20.get(),
-                    q21.get(), A0.get(), A1.get(), A2.get(), A3.get(), ndum, avv.x, avv.y, gx_grav, gy_grav, f2, err);
-}
-
-// artificial_viscosity of the node receivers alone (av_mix), written to
-// av_out for k_deriv_nodes_mix: it reads only node data that the stress
-// points' update leaves alone, so the RK stages run it beside
-// k_sp_update_mix.
-__global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V, PairLists PL, DevParams P,
-                                                       float hu, float2 *__restrict__ av_out, int nn) {
-    __shared__ StagePlan pl[1];
-    const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
-    const Tile T = PL.tiles[tile];
-    if (T.first >= T.end) return;
-    const int r = T.first + (int)threadIdx.x;
-    const bool active = r < T.end;
-    const int key_r = active ? V.cell[r] : C.g.ndivt;
-    const bool inside = key_r < C.g.ndivt;
-    const double2 o = S.x[T.first];
-    const bool tiled = PL.ok[tile] == LIST_WINDOW;
-    int cx = 0, cy = 0;
-    if (inside) cell_xy(key_r, C.g, cx, cy);
-    const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
-    const double2 xr = S.x[ra], vr = S.vel[ra];
-    const double rhor = S.rho[ra], hr = S.hsml[ra];
-    const float2 a = av_mix(S, V, PL, P, C, T, tile, r, inside, tiled, cx, cy, xr, vr, hr, rhor, to_rel(xr, o), o,
-                            hu, pl[0]);
-    if (active) av_out[r] = a;
+                    q21.get(), A0.get(), A1.get(), A2.get(), A3.get(), ndum, avv.x, avv.y, gx_grav, gy_grav, Q, adapt, sr,
+                    err);
 }
 
 // ------------------------------------------------------ captured steps
