@@ -184,13 +184,12 @@ struct sps_handle {
     float curve_f[SPS_MAX_TCURVE * SPS_MAX_CURVES];
     DBuf<int> bc_info, bc_or_not;  // bc_or_not: every particle, by original index
     int ifsigman = 0;
-    // free-surface detection: normals by original index; the pair list in
-    // traversal order and each particle's entries (free_surface)
-    DBuf<double2> normal, surf_nrm0;
-    DBuf<int> surf_pi, surf_pj, surf_pt, surf_sub;
-    DBuf<float> surf_gx, surf_gy;
-    DBuf<unsigned> surf_cnt, surf_start, surf_cur, surf_ent, surf_flag;
-    DBuf<float2> surf_tt, surf_tau;
+    // free-surface detection: normals by original index; each particle's
+    // entries, scan flag and subset (free_surface)
+    DBuf<double2> normal;
+    DBuf<int> surf_n, surf_sub;
+    DBuf<unsigned> surf_ent, surf_flag;
+    DBuf<float2> surf_hf;
     DBuf<double> bc_vals;         // the step's values (k_bc_values)
     BcValues bc_vars{};           // the BC rows' variables (values filled per step)
     DBuf<unsigned short> deg_a, deg_b;
@@ -999,47 +998,23 @@ static int mixed_step_graph(sps_handle *h, double dt, double time_sph, double gx
     return 0;
 }
 
-// get_nodes_on_free_surface (3_...:1116-1411) after the position update:
-// the step's pair list laid out in traversal order by storage slot, each
-// particle's pairs of types 1-3 gathered in that order, then the four steps
-// of the detection; BC_or_not and the normals by original index.
+// get_nodes_on_free_surface (3_...:1116-1411) after the position update, over
+// the step's pairs in list order; BC_or_not and the normals by original index.
 static int free_surface(sps_handle *h, const StateBufs &SB) {
-    int rc0 = sync_search(h);   // the pair count sizes the detection's arrays
-    if (rc0) return rc0;
-    const long long np = (long long)h->n_pairs;
-    const int nn = h->nn, nt = h->nt, nt2 = h->nt2;
+    const int nn = h->nn, nt = h->nt;
+    // entries kept per particle: as many as its two pair lists hold; a body on
+    // its lattice has about 36 with one stress point a cell
+    const int cap = 4 * h->list_words;
+    const size_t ne = (size_t)nblk(nt) * BLOCK * cap;
     int rc = 0;
-    const size_t npa = (size_t)std::max(np, 1LL);
-    rc |= dalloc(h->surf_pi, npa) | dalloc(h->surf_pj, npa) | dalloc(h->surf_pt, npa);
-    rc |= dalloc(h->surf_gx, npa) | dalloc(h->surf_gy, npa) | dalloc(h->surf_ent, 2 * npa);
-    rc |= dalloc(h->surf_cnt, (size_t)nt + 1) | dalloc(h->surf_start, (size_t)nt + 1) | dalloc(h->surf_cur, nt);
-    rc |= dalloc(h->surf_flag, nt) | dalloc(h->surf_sub, nt) | dalloc(h->surf_nrm0, nt);
-    rc |= dalloc(h->surf_tt, nt) | dalloc(h->surf_tau, nt);
+    rc |= dalloc(h->surf_n, nt) | dalloc(h->surf_ent, ne) | dalloc(h->surf_hf, ne);
+    rc |= dalloc(h->surf_flag, nt) | dalloc(h->surf_sub, nt);
     if (rc) return rc;
-    if (np >= (1LL << 31)) return fail(SPS_ECAPACITY, "free surface: %lld pairs", np);
-    hipStream_t s = h->stream;
-    StateSet &S = h->S[h->cur];
-    const SurfBufs B{h->surf_pi.p, h->surf_pj.p, h->surf_pt.p, h->surf_gx.p, h->surf_gy.p, h->surf_start.p,
-                     h->surf_ent.p, h->surf_nrm0.p, h->surf_tt.p, h->surf_tau.p, h->surf_flag.p, h->surf_sub.p};
-    LAUNCH(K_SURF, nblk(nt + 1), BLOCK, k_surf_zero, h->surf_cnt.p, (long long)nt + 1);
-    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_zero, h->surf_cur.p, (long long)nt);
-    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_zero, h->surf_flag.p, (long long)nt);
-    if (np > 0) {
-        LAUNCH(K_SURF, nblk(nt2), BLOCK, k_dump_pairs, S.x.p, h->x0.p, S.hsml.p, h->cell.p, h->kstart.p, S.orig.p,
-               h->off.p, h->proc.p, h->grid.p, h->p.pi, h->surf_pi.p, h->surf_pj.p, h->surf_pt.p, (float *)nullptr,
-               h->surf_gx.p, h->surf_gy.p, nn, nt, nt2, 1, (unsigned long long)np, h->m_prev);
-        LAUNCH(K_SURF, nblk(np), BLOCK, k_surf_count, B, h->surf_cnt.p, np);
-    }
-    rc = scan_u32(h, h->surf_cnt.p, h->surf_start.p, (long long)nt + 1, nullptr);
-    if (rc) return rc;
-    if (np > 0) LAUNCH(K_SURF, nblk(np), BLOCK, k_surf_fill, B, h->surf_cur.p, h->surf_ent.p, np);
-    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_sort, h->surf_start.p, h->surf_ent.p, nt);
-    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_a, SB, B, nt);
-    if (np > 0) LAUNCH(K_SURF, nblk(np), BLOCK, k_surf_hit, SB, B, np);
-    if (h->xsph && np > 0)   // XSPH_update's marks (2_...:224-230) before the detection
-        LAUNCH(K_SURF, nblk(np), BLOCK, k_surf_mark, SB, B, h->bc_or_not.p, np);
+    const SearchView V{h->cell.p, h->kstart.p, h->proc.p, h->cnt.p, h->off.p, h->grid.p, h->split.p, h->p.pi};
+    const SurfBufs B{h->surf_n.p, h->surf_ent.p, h->surf_hf.p, cap, h->surf_flag.p, h->surf_sub.p};
+    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_a, SB, h->x0.p, V, B, h->bc_or_not.p, h->xsph ? 1 : 0, nn, nt);
     LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_sub, SB, B, h->bc_or_not.p, nt);
-    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_b, SB, B, h->normal.p, nt);
+    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_b, SB, h->x0.p, V, B, h->normal.p, nn, nt);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -1407,7 +1382,7 @@ extern "C" int sps_get_pairs(sps_handle *h, int64_t cap, int32_t *pair_i, int32_
     StateSet &S = h->S[h->cur];
     k_dump_pairs<<<nblk(h->nt2), BLOCK, 0, h->stream>>>(S.x.p, h->x0.p, S.hsml.p, h->cell.p, h->kstart.p, S.orig.p,
                                                      h->off.p, h->proc.p, h->grid.p, h->p.pi, di.p, dj.p, dt.p,
-                                                     dw.p, dgx.p, dgy.p, h->nn, h->nt, h->nt2, 0, 0ull, 0ull);
+                                                     dw.p, dgx.p, dgy.p, h->nn, h->nt, h->nt2);
     std::vector<int> hi(np), hj(np), ht(np);
     std::vector<float> hw(np), hgx(np), hgy(np);
     hipError_t e = hipGetLastError();
@@ -1574,10 +1549,8 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->surr_str); dfree(h->surr_feat); dfree(h->surr_stats); dfree(h->plog); dfree(h->surr_mat);
     dfree(h->mtab); dfree(h->mat_orig); dfree(h->pairs_total);
     dfree(h->inv); dfree(h->nodeinfo); dfree(h->x10); dfree(h->disp10); dfree(h->bcint_prev);
-    dfree(h->bc_info); dfree(h->bc_or_not); dfree(h->bc_vals); dfree(h->normal); dfree(h->surf_nrm0);
-    dfree(h->surf_pi); dfree(h->surf_pj); dfree(h->surf_pt); dfree(h->surf_sub); dfree(h->surf_gx);
-    dfree(h->surf_gy); dfree(h->surf_cnt); dfree(h->surf_start); dfree(h->surf_cur); dfree(h->surf_ent);
-    dfree(h->surf_flag); dfree(h->surf_tt); dfree(h->surf_tau);
+    dfree(h->bc_info); dfree(h->bc_or_not); dfree(h->bc_vals); dfree(h->normal); dfree(h->surf_n);
+    dfree(h->surf_ent); dfree(h->surf_hf); dfree(h->surf_flag); dfree(h->surf_sub);
     if (h->pinned) (void)hipHostFree(h->pinned);
     if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
     if (h->ev_join) (void)hipEventDestroy(h->ev_join);
