@@ -573,7 +573,7 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
         // list B: node tiles; with XSPH stress-point tiles too, and its w
         rc |= dalloc(h->list_ib, h->xsph ? wa : wb); rc |= dalloc(h->list_gxb, wb); rc |= dalloc(h->list_gyb, wb);
         if (h->xsph) rc |= dalloc(h->list_wb, wa) | dalloc(h->xsph_v, (size_t)nt);
-        if (!h->mixed) rc |= dalloc(h->list_iah, wa) | dalloc(h->list_ibh, h->xsph ? wa : wb);
+        rc |= dalloc(h->list_iah, wa) | dalloc(h->list_ibh, h->xsph ? wa : wb);
     }
     rc |= dalloc(h->deg_a, nt); rc |= dalloc(h->deg_b, h->xsph ? nt : nn);
     rc |= dalloc(h->tile_ok, h->ntile_n + h->ntile_s + 1);

@@ -1545,7 +1545,7 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         const int crm_r = cy * C.g.ndivx + cx;
         // h_uniform > 0: every particle has this smoothing length
         const AcceptBounds ub = accept_bounds(h_uniform, h_uniform);
-        auto walk = [&](const auto &Cs, const auto &A, bool lists, auto slots, auto uni) __attribute__((always_inline)) {
+        auto walk = [&](const auto &Cs, const auto &A, auto slots, auto uni) __attribute__((always_inline)) {
             constexpr bool SLOTS = decltype(slots)::value;
             for (int y = y0; y <= y1; ++y)
                 for (int xx = x0; xx <= x1; ++xx) {
@@ -1598,7 +1598,6 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
                                     any_dummy = any_dummy || ks == KIND_DUMMY;
                                 }
                             }
-                            if (!lists) continue;
                             const unsigned e = ListEntry<SLOTS>::make(ks, j);
                             if (in_list_a(KR, ks))
                                 la.template put<SLOTS>(PL.lg, ltile, PL.ia, PL.iah, e);
@@ -1612,23 +1611,20 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         using Gen = std::integral_constant<bool, false>;
         if (lds) {
             if (h_uniform > 0)
-                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, true, Gen{}, Uni{});
+                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, Gen{}, Uni{});
             else
-                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, true, Gen{}, Gen{});
+                walk(LdsCells<LY>{T.x0 - 1, T.wy0}, LdsFields<LY>{}, Gen{}, Gen{});
         } else {
-            // the mixed form's stage kernels walk such a tile's cells themselves
-            walk(GlobalCells{V.kstart, C.g, C.L}, XHFields{x, hsml}, FILL, Uni{}, Gen{});
+            walk(GlobalCells{V.kstart, C.g, C.L}, XHFields{x, hsml}, Uni{}, Gen{});
         }
-        if (lds || FILL) {
-            la.finish(PL.lg, ltile, PL.ia, lds ? nullptr : PL.iah);
-            if (list_b) lb.finish(PL.lg, ltile, PL.ib, lds ? nullptr : PL.ibh);
-        }
+        la.finish(PL.lg, ltile, PL.ia, lds ? nullptr : PL.iah);
+        if (list_b) lb.finish(PL.lg, ltile, PL.ib, lds ? nullptr : PL.ibh);
         cnt[V.proc[r]] = fk[0] + fk[1] + fk[2];
     }
     block_type_counts(fk, tsum, PL.types + 3 * (size_t)ltile);
     const int lmax = 4 * PL.lg;
     const bool over = la.n > lmax || lb.n > lmax;
-    const bool any_over = lds || FILL ? __syncthreads_or(over) : true;
+    const bool any_over = __syncthreads_or(over);
     if (threadIdx.x == 0) PL.ok[ltile] = any_over ? LIST_NONE : lds ? LIST_WINDOW : LIST_SLOTS;
     if (FILL && !any_over && active) {
         const double2 xr = x[r];

@@ -17,8 +17,12 @@
 // the return map and the RK update stay in double precision (the shared
 // tails sp_stage_tail / node_stage_tail).  Pairs are summed in forward list
 // order; the double-precision form keeps the reference's linked-list order.
-// A tile whose window does not fit walks the global state (exact kernel
-// values, forward order), as in the double-precision form.
+// A tile whose window does not fit reads the global state (exact kernel
+// values, forward order) through lists of storage slots, as in the
+// double-precision form.  Its tiles are cut every TILE slots, since positions
+// are rounded relative to a tile's first receiver, so on a slope one tile in
+// about twenty-five crosses a strip end; a cell walk tests about a hundred
+// candidates where the list has twenty entries.
 
 namespace sps {
 
@@ -173,6 +177,31 @@ template <typename F> __device__ __forceinline__ OnTheFly<F> on_the_fly(F &f, fl
     return OnTheFly<F>{f, xr, hr, hu};
 }
 
+// A slot list walk's body with the kernel values walk_run computes: exact
+// ones from the state, and its acceptance test (lists kept over steps hold
+// the partners within their skin too).
+template <typename F> struct FromState {
+    F &f;
+    double2 xr;
+    double hr, pi;
+    KernelFactor kf;
+    template <typename KT, typename A>
+    __device__ __forceinline__ void operator()(KT kt, const A &fields, int j, float, float, float) {
+        const double2 xs = fields.xk(0, j);
+        const double dx0 = xr.x - xs.x, dx1 = xr.y - xs.y;
+        double mh;
+        const double rr = pair_distance(dx0, dx1, hr, fields.hk(0, j), mh);
+        if (rr < 0.0) return;
+        float w, gx, gy;
+        cubic_kernel_f(rr, dx0, dx1, mh, kf.get(mh, pi), w, gx, gy);
+        f(kt, fields, j, w, gx, gy);
+    }
+};
+
+template <typename F> __device__ __forceinline__ FromState<F> from_state(F &f, double2 xr, double hr, double pi) {
+    return FromState<F>{f, xr, hr, pi, KernelFactor{}};
+}
+
 // Staging of a position relative to the origin.
 __device__ __forceinline__ float2 to_rel(double2 x, double2 o) { return rel_pos(x, o); }
 
@@ -193,7 +222,8 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
     ListWalk<MASK_SP, false, false> lw;
     lw.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_a[r] : 0);
     const double2 o = S.x[T.first];
-    bool lds = PL.ok[tile] == LIST_WINDOW;
+    const int ok = PL.ok[tile];
+    bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_SP>(PL, tile, 0, pl);
         __syncthreads();
@@ -240,12 +270,17 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
         if (lds) {
             lw.run(LdsFieldsMix<LY>{}, on_the_fly(body, to_rel(xr, o), (float)hr, hu));
         } else {
-            int cx, cy;
-            cell_xy(V.cell[r], C.g, cx, cy);
             StateBufs S2 = S;   // the stress points' stresses from sp_in (the walk reads no node's)
             S2.stress = const_cast<double4 *>(sp_in);
-            walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GlobalFieldsMix{S2, o, dd, dt}, C.g, cx, cy, xr, hr,
-                                  KIND_NODE, r, false, true, V.pi, NoClass{}, body);
+            const GlobalFieldsMix GF{S2, o, dd, dt};
+            if (ok == LIST_SLOTS) {
+                lw.run_slots(PL.iah, GF, from_state(body, xr, hr, V.pi));
+            } else {
+                int cx, cy;
+                cell_xy(V.cell[r], C.g, cx, cy);
+                walk_stencil<MASK_SP>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr, KIND_NODE, r, false,
+                                      true, V.pi, NoClass{}, body);
+            }
         }
     }
     double4 s = S.stress[r];
@@ -286,7 +321,8 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
     ListWalk<MASK_NODE, false, false> lw;
     lw.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, ltile, deg);
     const double2 o = S.x[T.first];
-    bool lds = PL.ok[ltile] == LIST_WINDOW;
+    const int ok = PL.ok[ltile];
+    bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_NODE>(PL, ltile, 0, pl[0]);
         if (deriv) load_plan<KIND_DUMMY>(PL, ltile, 1, pl[1]);
@@ -346,6 +382,8 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
     if (inside) {
         if (lds)
             lw.run(LF, on_the_fly(spu, xrr, (float)hr, hu));
+        else if (ok == LIST_SLOTS)
+            lw.run_slots(PL.iah, GF, from_state(spu, xr, hr, V.pi));
         else
             walk_stencil<MASK_NODE>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr, KIND_SP, r, false,
                                     true, V.pi, NoClass{}, spu);
@@ -414,11 +452,13 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
         }
     };
     if (inside) {
-        if (lds) {
-            ListWalk<MASK_NODE | MASK_DUMMY, false, false> lg;
-            lg.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, ltile, deg);
+        ListWalk<MASK_NODE | MASK_DUMMY, false, false> lg;
+        if (ok != LIST_NONE) lg.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, ltile, deg);
+        if (lds)
             lg.run(LF, on_the_fly(grad, xrr, (float)hr, hu));
-        } else
+        else if (ok == LIST_SLOTS)
+            lg.run_slots(PL.iah, GF, from_state(grad, xr, hr, V.pi));
+        else
             walk_stencil<MASK_NODE | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr, KIND_SP,
                                                  r, false, true, V.pi, NoClass{}, grad);
     }
@@ -457,7 +497,8 @@ __global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V
     KSum ax, ay;
     ListWalk<MASK_NODE, false, false> lb;
     lb.start(PL.ib, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_b[r] : 0);
-    bool lds2 = PL.ok[tile] == LIST_WINDOW;
+    const int ok = PL.ok[tile];
+    bool lds2 = ok == LIST_WINDOW;
     if (lds2) {
         load_plan<KIND_NODE>(PL, tile, 0, pl);
         __syncthreads();
@@ -496,6 +537,8 @@ __global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V
     if (inside) {
         if (lds2)
             lb.run(LF, on_the_fly(av, xrr, hrf, hu));
+        else if (ok == LIST_SLOTS)
+            lb.run_slots(PL.ibh, GF, from_state(av, xr, hr, V.pi));
         else
             walk_stencil<MASK_NODE>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr, KIND_NODE, r,
                                     false, true, V.pi, NoClass{}, av);
@@ -530,7 +573,7 @@ __global__ __launch_bounds__(TILE) void k_deriv_nodes_mix(StateBufs S, Work W, S
     ListWalk<MASK_SP | MASK_DUMMY, false, false> la;
     la.start(PL.ia, nullptr, nullptr, nullptr, PL.lg, tile, inside ? PL.deg_a[r] : 0);
     const double2 o = S.x[T.first];
-    const bool tiled = PL.ok[tile] == LIST_WINDOW;
+    const int ok = PL.ok[tile];
     int cx = 0, cy = 0;
     if (inside) cell_xy(key_r, C.g, cx, cy);
     const int ra = active ? r : T.first;   // a valid slot for the idle lanes' loads
@@ -542,10 +585,9 @@ __global__ __launch_bounds__(TILE) void k_deriv_nodes_mix(StateBufs S, Work W, S
     const float srx = (float)sr.x, sry = (float)sr.y, srz = (float)sr.z;
     const float2 xrr = to_rel(xr, o);
     const LdsFieldsMix<LY> LF{};
-    const GlobalFieldsMix GF{S, o};
 
     // phase 1: stress gradient over stress points (type 1) and dummies (type 6)
-    bool lds = tiled;
+    bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KIND_SP>(PL, tile, 0, pl[0]);
         load_plan<KIND_DUMMY>(PL, tile, 1, pl[1]);
@@ -625,8 +667,12 @@ __global__ __launch_bounds__(TILE) void k_deriv_nodes_mix(StateBufs S, Work W, S
         {
             StateBufs S2 = S;   // stress points' stresses from sp_stress (the walk reads no node's)
             S2.stress = const_cast<double4 *>(sp_stress);
-            walk_stencil<MASK_SP | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GlobalFieldsMix{S2, o}, C.g, cx,
-                                               cy, xr, hr, KIND_NODE, r, false, true, V.pi, NoClass{}, grad);
+            const GlobalFieldsMix GF{S2, o};
+            if (ok == LIST_SLOTS)
+                la.run_slots(PL.iah, GF, from_state(grad, xr, hr, V.pi));
+            else
+                walk_stencil<MASK_SP | MASK_DUMMY>(GlobalCells{V.kstart, C.g, C.L}, GF, C.g, cx, cy, xr, hr,
+                                                   KIND_NODE, r, false, true, V.pi, NoClass{}, grad);
         }
     }
 
@@ -674,7 +720,8 @@ __global__ __launch_bounds__(TILE) void k_xsph_mix(StateBufs S, SearchView V, Pa
     ListWalk<(1 << KR), false, false> lw;
     lw.start(PL.ib, nullptr, nullptr, nullptr, PL.lg, ltile, inside ? PL.deg_b[r] : 0);
     const double2 o = S.x[T.first];
-    bool lds = PL.ok[ltile] == LIST_WINDOW;
+    const int ok = PL.ok[ltile];
+    bool lds = ok == LIST_WINDOW;
     if (lds) {
         load_plan<KR>(PL, ltile, 0, pl);
         __syncthreads();
@@ -710,6 +757,8 @@ __global__ __launch_bounds__(TILE) void k_xsph_mix(StateBufs S, SearchView V, Pa
         const double hr = S.hsml[r];
         if (lds) {
             lw.run(LdsFieldsMix<LY>{}, on_the_fly(body, to_rel(xr, o), (float)hr, hu));
+        } else if (ok == LIST_SLOTS) {
+            lw.run_slots(PL.ibh, GlobalFieldsMix{S, o}, from_state(body, xr, hr, V.pi));
         } else {
             int cx, cy;
             cell_xy(V.cell[r], C.g, cx, cy);

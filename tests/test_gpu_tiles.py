@@ -8,6 +8,7 @@ tile capacity, which falls back to tiles cut every TILE slots) and particles
 outside the domain box are the edges.
 """
 import dataclasses
+import importlib
 
 import numpy as np
 import pytest
@@ -77,3 +78,31 @@ def test_tiles_against_oracle(name):
         gpu.step(1)
         ora.step(1)
         compare(gpu, ora, f"{name} step {step}")
+
+
+# The mixed form cuts its tiles every TILE slots: bodies where few, many and
+# all tiles cross a strip end and read their lists by storage slot.  An
+# elastic deck from rest, so the difference to the double-precision oracle is
+# the rounding of the pair terms: each of about 20 terms of a sum to 2^-24 of
+# itself, compensated; with the smallest sums two orders below their terms,
+# 20 steps stay under 1e-5 of the largest value.
+@pytest.mark.parametrize("skin", [0.0, 0.25])
+@pytest.mark.parametrize("nx,ny,change", [(17, 16, {}), (65, 65, {}), (200, 5, {}), (33, 90, {"xsph": True}),
+                                          (40, 40, {"npoints": 2})])
+def test_mixed_tiles_across_strips(nx, ny, change, skin):
+    sps = load_pkg()
+    acc = importlib.import_module("stress-particle-sph_amd.accuracy")
+    deck = dataclasses.replace(sps.read_deck(deck_dir("t3_elastic")), **change)
+    deck.xs = (0.0, (nx - 0.5) * deck.dx, 0.0, (nx - 0.5) * deck.dx)
+    deck.ys = (0.0, 0.0, (ny - 0.5) * deck.dx, (ny - 0.5) * deck.dx)
+    mix = sps.Simulation.from_deck(deck, mode=sps.MODE_FAST)
+    if skin:
+        mix.set_list_skin(skin * deck.dx)
+    ora = sps.Simulation.from_deck(deck, lib_path=ORACLE_LIB)
+    x0 = ora.get_state(["x"])["x"]
+    print(f"[tiles] mixed {nx} x {ny} {change} skin {skin}", flush=True)
+    mix.step(20)
+    ora.step(20)
+    err = acc.compare_states(mix.get_state(), ora.get_state(), x0)
+    for k in ("disp_rel_max", "vel_rel_max", "stress_rel_max"):
+        assert err[k] <= 1e-5, f"{k} {err[k]:.3e}"
