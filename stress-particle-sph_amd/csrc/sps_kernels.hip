@@ -3136,31 +3136,36 @@ __global__ void k_dump_pairs(const double2 *__restrict__ x, const double2 *__res
         }
 }
 
-// Un-permute state arrays for sps_get_state.
-__global__ void k_gather_out2(const double2 *__restrict__ src, const int *__restrict__ orig,
-                              double2 *__restrict__ dst, int n) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[orig[t]] = src[t];
-}
-__global__ void k_gather_out4(const double4 *__restrict__ src, const int *__restrict__ orig,
-                              double4 *__restrict__ dst, int n) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[orig[t]] = src[t];
-}
-__global__ void k_gather_out1(const double *__restrict__ src, const int *__restrict__ orig,
-                              double *__restrict__ dst, int n) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[orig[t]] = src[t];
-}
-__global__ void k_gather_outi(const int *__restrict__ src, const int *__restrict__ orig,
-                              int *__restrict__ dst, int n) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[orig[t]] = src[t];
-}
-__global__ void k_gather_outf(const float *__restrict__ src, const int *__restrict__ orig,
-                              float *__restrict__ dst, int n) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[orig[t]] = src[t];
+// The fields that sps_get_state takes back, un-permuted into one staging
+// buffer: a launch for all of them (blockIdx.y is the field).  orig: the
+// original index of a slot's particle, or null (the field is by original
+// index already).
+struct ReadField {
+    const void *src;
+    const int *orig;
+    void *dst;      // in the staging buffer, 16-byte aligned
+    int n, words;   // particles, 32-bit words of each (1, 2, 4 or 8)
+};
+constexpr int READ_MAX = 20;
+struct ReadTable {
+    ReadField f[READ_MAX];
+};
+
+__global__ void k_read_back(ReadTable R) {
+    const ReadField &F = R.f[blockIdx.y];
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= F.n) return;
+    const size_t i = (size_t)t, o = F.orig ? (size_t)F.orig[t] : i;
+    if (F.words == 1) {
+        ((int *)F.dst)[o] = ((const int *)F.src)[i];
+    } else if (F.words == 2) {
+        ((double *)F.dst)[o] = ((const double *)F.src)[i];
+    } else if (F.words == 4) {
+        ((double2 *)F.dst)[o] = ((const double2 *)F.src)[i];
+    } else {
+        ((double2 *)F.dst)[2 * o] = ((const double2 *)F.src)[2 * i];
+        ((double2 *)F.dst)[2 * o + 1] = ((const double2 *)F.src)[2 * i + 1];
+    }
 }
 __global__ void k_scatter_in_identity(int *__restrict__ orig, int n) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
