@@ -56,118 +56,313 @@ __device__ __forceinline__ float silu_grad(float z) {
     return s * (1.0f + z * (1.0f - s));
 }
 
-// C = A B for bfloat16 A (M x K) and B (K x N) with element strides, single
-// precision accumulation.  A workgroup of four waves covers 64 x 64 of C,
-// each wave 32 x 32 as 2 x 2 tiles of the 16 x 16 x 16 instruction; blockIdx.z
-// takes K in chunks of kchunk (split K, accumulated with atomics).  M, N, K
-// and kchunk are multiples of 16.  Lane l of a wave holds A[l % 16][4 (l / 16)
-// + q] and B[4 (l / 16) + q][l % 16], q = 0..3, and receives
-// C[4 (l / 16) + q][l % 16].
-struct Gemm {
-    const bf16_t *A;
-    long long sa_i, sa_k;
-    const bf16_t *B;
-    long long sb_k, sb_j;
-    int M, N, K, kchunk;
-    const int *Mdev;         // when set: M = min(M, *Mdev rounded up to 16)
-    const float *bias;       // per column, or null
-    float *Cf;               // single-precision result (or split-K accumulator), or null
-    long long ldc;
-    bf16_t *Cb;              // bfloat16 of act(result), or null
-    long long ldcb;
-    int act;                 // 1: SiLU on the bfloat16 result
-    int accumulate;          // 1: atomicAdd into Cf, no bias / act
+// ---------------------------------------------------------- the network
+// Layout of the matrix instruction (16 x 16 x 16, bfloat16 in, single
+// precision out): lane l holds A[l % 16][4 (l / 16) + q] and
+// B[4 (l / 16) + q][l % 16], q = 0..3, and gets C[4 (l / 16) + q][l % 16].
+// A "tile word" below is a lane's four bfloat16 of a 16 x 16 tile, 8 bytes;
+// tiles are stored as 64 consecutive words, so every load and store of one is
+// a coalesced 512 bytes.
+typedef unsigned long long tword_t;
+
+__device__ __forceinline__ tword_t pack4(const bf16_t (&h)[4]) {
+    return (tword_t)h[0] | (tword_t)h[1] << 16 | (tword_t)h[2] << 32 | (tword_t)h[3] << 48;
+}
+__device__ __forceinline__ v4s unpack4(tword_t u) {
+    v4s r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = (short)(u >> (16 * q));
+    return r;
+}
+
+// Parameter i's bfloat16 value into the two tile orders of the weights: wf as
+// the B operand of H W, wt as that of dZ W^T.  Biases are not packed.
+__device__ __forceinline__ void put_weight(bf16_t *__restrict__ wf, bf16_t *__restrict__ wt, int i, bf16_t v) {
+    const int base = i < PB1 ? PW1 : i < PW2 ? -1 : i < PB2 ? PW2 : i < PW3 ? -1 : i < PB3 ? PW3 : i < PW4 ? -1
+                   : i < PB4 ? PW4 : -1;
+    if (base < 0) return;
+    const int fin = base == PW1 ? MLP_IN : MLP_H, fout = base == PW4 ? MLP_OUT : MLP_H;
+    const int r = (i - base) / fout, c = (i - base) % fout;
+    auto at = [](int k, int j, int nj) { return (((k / 16) * (nj / 16) + j / 16) * 64 + (k % 16) / 4 * 16 + j % 16) * 4 + k % 4; };
+    wf[base + at(r, c, fout)] = v;
+    wt[base + at(c, r, fin)] = v;
+}
+
+// Forward pass of one 64-row block a workgroup, 16 rows a wave, and with GRAD
+// the backward pass down to the gradients at every layer's output.  The rows'
+// activations stay in the wave: a layer's result is laid out for the next
+// product through 4 KiB of LDS of the wave's own, the pre-activations keep
+// their registers for the way back, and only what k_gemm_bf16_dw contracts
+// over the rows is stored, as tile words (four consecutive rows of a column
+// are what a lane holds of a result and what it needs as an operand there).
+// The weights of a layer (32 KiB, in operand order) are fetched into registers
+// while the layer before multiplies.  A launch per product with its operands
+// gathered two bytes at a time took 530 us for 58 k rows, with 46 us for the
+// activation's derivative and 390 us for the bias gradients; this takes 83 us,
+// k_gemm_bf16_dw 23 us.  What is left here is mostly the activation: two
+// exponentials and two correctly rounded divisions a value.
+// Rows past nb (or *nbdev) count as zero inputs and have zero gradients.
+struct NetPass {
+    const float *feat, *targ;        // n x 10 and n x 4
+    const unsigned *idx;             // row r of the batch is row idx[r] of the set (null: r)
+    int nb;
+    const int *nbdev;                // when set: nb = min(nb, *nbdev)
+    const bf16_t *wf, *wt;
+    const float *w;                  // single-precision parameters (the biases)
+    float *Y;                        // rows x 16
+    tword_t *X, *H[3], *dZ[3], *dY;  // GRAD: tiles of 16 rows
 };
 
-__global__ __launch_bounds__(256) void k_gemm_bf16(Gemm g) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int M = g.M;
-    if (g.Mdev) {
-        const int m = (*g.Mdev + 15) / 16 * 16;
-        M = m < M ? m : M;
-    }
-    const int r0 = blockIdx.x * 64 + 32 * (wave >> 1), c0 = blockIdx.y * 64 + 32 * (wave & 1);
-    if (r0 >= M || c0 >= g.N) return;     // the whole wave: no barrier in this kernel
-    const bool rv1 = r0 + 16 < M, cv1 = c0 + 16 < g.N;
-    const int kb = blockIdx.z * g.kchunk;
-    const int ke = kb + g.kchunk < g.K ? kb + g.kchunk : g.K;
-    const int li = lane & 15, lk = 4 * (lane >> 4);
-    v4f acc00 = {0.f, 0.f, 0.f, 0.f}, acc01 = acc00, acc10 = acc00, acc11 = acc00;
-    for (int k = kb; k < ke; k += 16) {
-        v4s a0, a1, b0, b1;
+constexpr int NET_ROWS = 64;         // rows of a workgroup
+constexpr int NET_TS = MLP_H + 8;    // LDS row of a wave's transposition (16-byte steps, banks apart)
+
+template <bool GRAD> __global__ __launch_bounds__(256, 2) void k_gemm_bf16_chain(NetPass g) {
+    __shared__ __align__(16) tword_t sW[64 * 64];
+    __shared__ __align__(16) bf16_t sT[4][16 * NET_TS];
+    int nb = g.nb;
+    if (g.nbdev) nb = min(nb, *g.nbdev);
+    if ((int)blockIdx.x * NET_ROWS >= nb) return;   // the whole workgroup
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, lg = lane >> 4;
+    const int rb = blockIdx.x * (NET_ROWS / 16) + wave, r0 = 16 * rb;
+    bf16_t *const mine = sT[wave];
+    auto source = [&](int row) { return row < nb ? (g.idx ? (long long)g.idx[row] : (long long)row) : -1ll; };
+
+    // weights on their way, 16 bytes (two tile words) at a time
+    double2 pre[8];
+    auto fetch = [&](const bf16_t *src, auto nw) {
+        constexpr int N = decltype(nw)::value / 512;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const long long kk = k + lk + q;
-            a0[q] = (short)g.A[(r0 + li) * g.sa_i + kk * g.sa_k];
-            a1[q] = rv1 ? (short)g.A[(r0 + 16 + li) * g.sa_i + kk * g.sa_k] : (short)0;
-            b0[q] = (short)g.B[kk * g.sb_k + (c0 + li) * g.sb_j];
-            b1[q] = cv1 ? (short)g.B[kk * g.sb_k + (c0 + 16 + li) * g.sb_j] : (short)0;
-        }
-        acc00 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, b0, acc00, 0, 0, 0);
-        acc01 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, b1, acc01, 0, 0, 0);
-        acc10 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b0, acc10, 0, 0, 0);
-        acc11 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b1, acc11, 0, 0, 0);
-    }
-    auto put = [&](const v4f &acc, int ti, int tj) {
-        if ((ti && !rv1) || (tj && !cv1)) return;
-        const int col = c0 + 16 * tj + li;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int row = r0 + 16 * ti + lk + q;
-            if (g.accumulate) {
-                atomicAdd(&g.Cf[row * g.ldc + col], acc[q]);
-                continue;
-            }
-            const float v = acc[q] + (g.bias ? g.bias[col] : 0.0f);
-            if (g.Cf) g.Cf[row * g.ldc + col] = v;
-            if (g.Cb) g.Cb[row * g.ldcb + col] = f2bf(g.act ? silu(v) : v);
-        }
+        for (int k = 0; k < N; ++k) pre[k] = reinterpret_cast<const double2 *>(src)[t + 256 * k];
     };
-    put(acc00, 0, 0);
-    put(acc01, 0, 1);
-    put(acc10, 1, 0);
-    put(acc11, 1, 1);
-}
+    auto commit = [&](auto nw) {
+        constexpr int N = decltype(nw)::value / 512;
+#pragma unroll
+        for (int k = 0; k < N; ++k) reinterpret_cast<double2 *>(sW)[t + 256 * k] = pre[k];
+    };
+    using Small = std::integral_constant<int, 8 * 64>;
+    using Large = std::integral_constant<int, 64 * 64>;
+    // acc = (the wave's 16 rows in LDS) x (the layer in sW)
+    v4f acc[8];
+    auto multiply = [&](auto kt_, auto nt_) {
+        constexpr int KT = decltype(kt_)::value, NT = decltype(nt_)::value;
+        v4s a[KT];
+#pragma unroll
+        for (int k = 0; k < KT; ++k)
+            a[k] = unpack4(*reinterpret_cast<const tword_t *>(mine + li * NET_TS + 16 * k + 4 * lg));
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KT; ++k)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                acc[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[k], unpack4(sW[(k * NT + n) * 64 + lane]), acc[n],
+                                                                   0, 0, 0);
+    };
+    using T1 = std::integral_constant<int, 1>;
+    using T8 = std::integral_constant<int, 8>;
+    auto put = [&](int n, const bf16_t (&h)[4]) {   // a result tile's words to the wave's rows
+#pragma unroll
+        for (int q = 0; q < 4; ++q) mine[(4 * lg + q) * NET_TS + 16 * n + li] = h[q];
+    };
 
-// Rows idx[r] (or r) of the n x 10 single-precision features (and n x 4
-// targets) into the padded bfloat16 batch X (rows >= nb: zero).
-// With nbdev, nb is at most *nbdev and only rows below nb rounded up to 64
-// are written (the rows a launch of k_gemm_bf16 with Mdev reads).
-__global__ void k_mlp_batch(const float *__restrict__ feat, const float *__restrict__ targ,
-                            const unsigned *__restrict__ idx, int nb, int rows, bf16_t *__restrict__ X,
-                            float *__restrict__ T, const unsigned *__restrict__ nbdev) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (nbdev) {
-        nb = min(nb, (int)*nbdev);
-        rows = min(rows, (nb + 63) / 64 * 64);
+    // inputs
+    fetch(g.wf + PW1, Small{});
+    {
+        const long long src = source(r0 + li);
+        bf16_t h[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int c = 4 * lg + q;
+            h[q] = f2bf(src >= 0 && c < MLP_NIN ? g.feat[src * MLP_NIN + c] : 0.0f);
+        }
+        *reinterpret_cast<tword_t *>(mine + li * NET_TS + 4 * lg) = pack4(h);
     }
-    if (r >= rows) return;
-    const long long src = r < nb ? (idx ? (long long)idx[r] : (long long)r) : -1;
+    if (GRAD) {
+        bf16_t h[4];
 #pragma unroll
-    for (int c = 0; c < MLP_IN; ++c)
-        X[(long long)r * MLP_IN + c] = f2bf(src >= 0 && c < MLP_NIN ? feat[src * MLP_NIN + c] : 0.0f);
-    if (T)
+        for (int q = 0; q < 4; ++q) {
+            const long long src = source(r0 + 4 * lg + q);
+            h[q] = f2bf(src >= 0 && li < MLP_NIN ? g.feat[src * MLP_NIN + li] : 0.0f);
+        }
+        g.X[(size_t)rb * 64 + lane] = pack4(h);
+    }
+    commit(Small{});
+    __syncthreads();
+    fetch(g.wf + PW2, Large{});
+    multiply(T1{}, T8{});
+
+    // hidden layers
+    v4f Z[3][8];
 #pragma unroll
-        for (int c = 0; c < MLP_NOUT; ++c) T[(long long)r * MLP_NOUT + c] = src >= 0 ? targ[src * MLP_NOUT + c] : 0.0f;
+    for (int l = 0; l < 3; ++l) {
+        const float *bias = g.w + (l == 0 ? PB1 : l == 1 ? PB2 : PB3);
+        __syncthreads();   // every wave has read the weights and its rows
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            const float bc = bias[16 * n + li];
+            bf16_t h[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float z = acc[n][q] + bc;
+                if (GRAD) Z[l][n][q] = z;
+                h[q] = f2bf(silu(z));
+            }
+            put(n, h);
+            if (GRAD) g.H[l][((size_t)rb * 8 + n) * 64 + lane] = pack4(h);
+        }
+        if (l < 2) commit(Large{});
+        else commit(Small{});
+        __syncthreads();
+        if (l == 0) fetch(g.wf + PW3, Large{});
+        if (l == 1) fetch(g.wf + PW4, Small{});
+        if (l == 2 && GRAD) fetch(g.wt + PW4, Small{});
+        if (l < 2) multiply(T8{}, T8{});
+        else multiply(T8{}, T1{});
+    }
+
+    // output, and the gradient of the mean squared error at it
+    const float inv = 1.0f / (float)(nb * MLP_NOUT);
+    const float b4 = g.w[PB4 + li];
+    __syncthreads();
+    {
+        bf16_t h[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int row = r0 + 4 * lg + q;
+            const float y = acc[0][q] + b4;
+            g.Y[(size_t)row * MLP_OUT + li] = y;
+            if (GRAD) {
+                const long long src = source(row);
+                const float d = src >= 0 && li < MLP_NOUT ? y - g.targ[src * MLP_NOUT + li] : 0.0f;
+                h[q] = f2bf(2.0f * d * inv);
+            }
+        }
+        if (!GRAD) return;
+        put(0, h);
+        g.dY[(size_t)rb * 64 + lane] = pack4(h);
+    }
+    commit(Small{});
+    __syncthreads();
+    fetch(g.wt + PW3, Large{});
+    multiply(T1{}, T8{});
+#pragma unroll
+    for (int l = 2; l >= 0; --l) {   // dZ = dH * SiLU'(Z), then dH of the layer below
+        if (l > 0) __syncthreads();
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            bf16_t h[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) h[q] = f2bf((acc[n][q] + 0.0f) * silu_grad(Z[l][n][q]));
+            if (l > 0) put(n, h);
+            g.dZ[l][((size_t)rb * 8 + n) * 64 + lane] = pack4(h);
+        }
+        if (l == 0) break;
+        commit(Large{});
+        __syncthreads();
+        if (l == 2) fetch(g.wt + PW2, Large{});
+        multiply(T8{}, T8{});
+    }
 }
 
-// Squared-error loss of the nb rows and dL/dY as bfloat16 (mean over rows
-// and the 4 outputs; padding columns and rows get 0).
-__global__ void k_mlp_loss(const float *__restrict__ Y, const float *__restrict__ T, int nb, int rows,
-                           bf16_t *__restrict__ dY, float *__restrict__ loss) {
-    __shared__ float s[256];
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.0f;
-    if (r < rows) {
-        const float inv = 1.0f / (float)(nb * MLP_NOUT);
+// Weight gradients: dW = H^T dZ of the layers and the bias gradients (a row
+// of ones in the place of H^T), over a chunk of 16-row tiles a workgroup;
+// blockIdx.y: 0 the second layer, 1 the third, 2 the first and the last.
+// Its sums are part[chunk], which k_mlp_reduce adds up: with atomics on the
+// 37 k gradients every chunk had to be long to keep their number down.
+// A wave takes two rows of 16 x 16 tiles of dW (64 registers of sums).
+__global__ __launch_bounds__(256) void k_gemm_bf16_dw(NetPass g, int nrb, int chunk, float *__restrict__ part) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+    const int lo = blockIdx.x * chunk, hi = min(lo + chunk, nrb);
+    float *const out = part + (size_t)blockIdx.x * MLP_NPARAM;
+    const v4s ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    auto mm = [](const v4s &a, const v4s &b, const v4f &c) {
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+    };
+    auto store = [&](const v4f &c, int pw, int fout, int it, int jt) {
 #pragma unroll
-        for (int c = 0; c < MLP_OUT; ++c) {
-            float d = 0.0f;
-            if (r < nb && c < MLP_NOUT) {
-                d = Y[(long long)r * MLP_OUT + c] - T[(long long)r * MLP_NOUT + c];
-                l += d * d * inv;
+        for (int q = 0; q < 4; ++q) out[pw + (16 * it + 4 * lg + q) * fout + 16 * jt + li] = c[q];
+    };
+    auto store_bias = [&](const v4f &c, int pb, int jt) {   // every row holds the sum
+        if (lg == 0) out[pb + 16 * jt + li] = c[0];
+    };
+    if (blockIdx.y < 2) {
+        const tword_t *__restrict__ A = g.H[blockIdx.y], *__restrict__ B = g.dZ[blockIdx.y + 1];
+        v4f acc[2][8], bias[2] = {zero, zero};
+#pragma unroll
+        for (int n = 0; n < 8; ++n) acc[0][n] = acc[1][n] = zero;
+        for (int rb = lo; rb < hi; ++rb) {
+            const size_t at = (size_t)rb * 8 * 64 + lane;
+            const v4s a0 = unpack4(A[at + 128 * wave]), a1 = unpack4(A[at + 128 * wave + 64]);
+            const v4s c0 = unpack4(B[at + 128 * wave]), c1 = unpack4(B[at + 128 * wave + 64]);
+            v4s b[8];
+#pragma unroll
+            for (int n = 0; n < 8; ++n) b[n] = unpack4(B[at + 64 * n]);
+#pragma unroll
+            for (int n = 0; n < 8; ++n) {
+                acc[0][n] = mm(a0, b[n], acc[0][n]);
+                acc[1][n] = mm(a1, b[n], acc[1][n]);
             }
-            dY[(long long)r * MLP_OUT + c] = f2bf(2.0f * d * inv);
+            bias[0] = mm(ones, c0, bias[0]);
+            bias[1] = mm(ones, c1, bias[1]);
+        }
+        const int pw = blockIdx.y ? PW3 : PW2, pb = blockIdx.y ? PB3 : PB2;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            store(acc[0][n], pw, MLP_H, 2 * wave, n);
+            store(acc[1][n], pw, MLP_H, 2 * wave + 1, n);
+        }
+        store_bias(bias[0], pb, 2 * wave);
+        store_bias(bias[1], pb, 2 * wave + 1);
+    } else {
+        v4f w1[2] = {zero, zero}, b1[2] = {zero, zero}, w4[2] = {zero, zero}, b4 = zero;
+        for (int rb = lo; rb < hi; ++rb) {
+            const size_t at = (size_t)rb * 8 * 64 + lane, at1 = (size_t)rb * 64 + lane;
+            const v4s x = unpack4(g.X[at1]), dy = unpack4(g.dY[at1]);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const v4s d = unpack4(g.dZ[0][at + 64 * (2 * wave + k)]), h = unpack4(g.H[2][at + 64 * (2 * wave + k)]);
+                w1[k] = mm(x, d, w1[k]);
+                b1[k] = mm(ones, d, b1[k]);
+                w4[k] = mm(h, dy, w4[k]);
+            }
+            b4 = mm(ones, dy, b4);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            store(w1[k], PW1, MLP_H, 0, 2 * wave + k);
+            store_bias(b1[k], PB1, 2 * wave + k);
+            store(w4[k], PW4, MLP_OUT, 2 * wave + k, 0);
+        }
+        if (wave == 0) store_bias(b4, PB4, 0);
+    }
+}
+
+// The first blocks: g = the chunks' gradients added up (a parameter a
+// thread).  The rest: the squared-error loss (mean over rows and the 4
+// outputs), 256 rows a block, added to *loss.
+constexpr int REDUCE_BLOCKS = (MLP_NPARAM + 255) / 256;
+__global__ void k_mlp_loss_reduce(NetPass g, const float *__restrict__ part, int nchunk, float *__restrict__ grad,
+                                  float *__restrict__ loss) {
+    if ((int)blockIdx.x < REDUCE_BLOCKS) {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (i >= MLP_NPARAM) return;
+        float s = 0.0f;
+#pragma unroll 8
+        for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * MLP_NPARAM + i];
+        grad[i] = s;
+        return;
+    }
+    __shared__ float s[256];
+    const int r = ((int)blockIdx.x - REDUCE_BLOCKS) * 256 + threadIdx.x;
+    float l = 0.0f;
+    if (r < g.nb) {
+        const long long src = g.idx ? (long long)g.idx[r] : (long long)r;
+        const float inv = 1.0f / (float)(g.nb * MLP_NOUT);
+#pragma unroll
+        for (int c = 0; c < MLP_NOUT; ++c) {
+            const float d = g.Y[(size_t)r * MLP_OUT + c] - g.targ[src * MLP_NOUT + c];
+            l += d * d * inv;
         }
     }
     s[threadIdx.x] = l;
@@ -176,35 +371,14 @@ __global__ void k_mlp_loss(const float *__restrict__ Y, const float *__restrict_
         if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0 && loss) atomicAdd(loss, s[0]);
+    if (threadIdx.x == 0) atomicAdd(loss, s[0]);
 }
 
-// dZ = dH * SiLU'(Z) as bfloat16 (rows x 128).
-__global__ void k_mlp_silu_back(const float *__restrict__ dH, const float *__restrict__ Z, long long n,
-                                bf16_t *__restrict__ dZ) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dZ[i] = f2bf(dH[i] * silu_grad(Z[i]));
-}
-
-// Column sums of a rows x ncol bfloat16 matrix added to out (bias gradients).
-__global__ void k_mlp_colsum(const bf16_t *__restrict__ D, int rows, int ncol, float *__restrict__ out) {
-    const int c = blockIdx.x;   // one block per column
-    float s = 0.0f;
-    for (int r = threadIdx.x; r < rows; r += blockDim.x) s += bf2f(D[(long long)r * ncol + c]);
-    __shared__ float red[256];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] += red[0];
-}
-
-// Adam (Kingma & Ba 2015) on the single-precision masters, then their
-// bfloat16 copies.
+// Adam (Kingma & Ba 2015) on the single-precision masters, then the weights'
+// bfloat16 copies in operand order.
 __global__ void k_mlp_adam(float *__restrict__ w, float *__restrict__ m, float *__restrict__ v,
-                           const float *__restrict__ g, bf16_t *__restrict__ wb, int n, float lr, float b1,
+                           const float *__restrict__ g, bf16_t *__restrict__ wf, bf16_t *__restrict__ wt,
+                           int n, float lr, float b1,
                            float b2, float eps, float c1, float c2) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -215,12 +389,12 @@ __global__ void k_mlp_adam(float *__restrict__ w, float *__restrict__ m, float *
     v[i] = vi;
     const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     w[i] = wi;
-    wb[i] = f2bf(wi);
+    put_weight(wf, wt, i, f2bf(wi));
 }
 
-__global__ void k_mlp_to_bf16(const float *__restrict__ w, bf16_t *__restrict__ wb, int n) {
+__global__ void k_mlp_to_bf16(const float *__restrict__ w, bf16_t *__restrict__ wf, bf16_t *__restrict__ wt, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) wb[i] = f2bf(w[i]);
+    if (i < n) put_weight(wf, wt, i, f2bf(w[i]));
 }
 
 // ------------------------------------------------------- use in the step

@@ -7,37 +7,31 @@ struct sps_mlp {
     int device = 0;
     hipStream_t stream = nullptr;
     DBuf<float> w, m, v, g;            // master weights, Adam moments, gradient (MLP_NPARAM)
-    DBuf<bf16_t> wb;                   // bfloat16 weights, same offsets
+    DBuf<bf16_t> wf, wt;               // bfloat16 weights in operand order, same offsets (put_weight)
     int rows = 0;                      // batch rows the buffers hold (multiple of 64)
-    DBuf<bf16_t> X, H1, H2, H3, dY, dZ;
-    DBuf<float> Z1, Z2, Z3, Y, dH, T, loss;
+    DBuf<tword_t> X, H[3], dZ[3], dY;  // what the weight gradients contract (NetPass)
+    DBuf<float> Y, part, loss;
     DBuf<float> feat, targ;            // a training set on the device
     DBuf<unsigned> perm;
     long long adam_t = 0;
 };
+
+// Row chunks of k_gemm_bf16_dw, at most: with its three kinds of workgroup
+// 384 of them, enough for the 256 CUs, while the partial sums stay 19 MB.
+constexpr int DW_CHUNKS = 128;
 
 static int mlp_reserve(sps_mlp *ml, int rows) {
     rows = (rows + 63) / 64 * 64;
     if (rows <= ml->rows) return 0;
     const size_t r = (size_t)rows;
     int rc = 0;
-    rc |= dalloc(ml->X, r * MLP_IN); rc |= dalloc(ml->H1, r * MLP_H); rc |= dalloc(ml->H2, r * MLP_H);
-    rc |= dalloc(ml->H3, r * MLP_H); rc |= dalloc(ml->dY, r * MLP_OUT); rc |= dalloc(ml->dZ, r * MLP_H);
-    rc |= dalloc(ml->Z1, r * MLP_H); rc |= dalloc(ml->Z2, r * MLP_H); rc |= dalloc(ml->Z3, r * MLP_H);
-    rc |= dalloc(ml->Y, r * MLP_OUT); rc |= dalloc(ml->dH, r * MLP_H); rc |= dalloc(ml->T, r * MLP_NOUT);
+    rc |= dalloc(ml->Y, r * MLP_OUT); rc |= dalloc(ml->X, r * MLP_IN / 4); rc |= dalloc(ml->dY, r * MLP_OUT / 4);
+    for (int l = 0; l < 3; ++l) rc |= dalloc(ml->H[l], r * MLP_H / 4) | dalloc(ml->dZ[l], r * MLP_H / 4);
+    rc |= dalloc(ml->part, (size_t)std::min(DW_CHUNKS, rows / NET_ROWS) * MLP_NPARAM);
     rc |= dalloc(ml->loss, 1);
     if (rc) return rc;
     ml->rows = rows;
     return 0;
-}
-
-static Gemm gemm_of(const bf16_t *A, long long sa_i, long long sa_k, const bf16_t *B, long long sb_k,
-                    long long sb_j, int M, int N, int K) {
-    Gemm g{};
-    g.A = A; g.sa_i = sa_i; g.sa_k = sa_k;
-    g.B = B; g.sb_k = sb_k; g.sb_j = sb_j;
-    g.M = M; g.N = N; g.K = K; g.kchunk = K;
-    return g;
 }
 
 // Launches on `st`; through the handle's timed launches when h is given.
@@ -49,65 +43,38 @@ static Gemm gemm_of(const bf16_t *A, long long sa_i, long long sa_k, const bf16_
             KERN<<<(GRID), (BLK), 0, st>>>(__VA_ARGS__);               \
     } while (0)
 
-static void mlp_gemm(hipStream_t st, sps_handle *h, const Gemm &g, int zsplit) {
-    const dim3 grid((unsigned)((g.M + 63) / 64), (unsigned)((g.N + 63) / 64), (unsigned)zsplit);
-    MLAUNCH(grid, 256, k_gemm_bf16, g);
-}
-
-// Y = network(X) over `rows` rows (or the first *Mdev of them); Z kept for
-// a backward pass when keepZ.
-static void mlp_forward(sps_mlp *ml, hipStream_t st, sps_handle *h, int rows, const int *Mdev, bool keepZ) {
-    Gemm g = gemm_of(ml->X.p, MLP_IN, 1, ml->wb.p + PW1, MLP_H, 1, rows, MLP_H, MLP_IN);
-    g.Mdev = Mdev; g.bias = ml->w.p + PB1; g.Cf = keepZ ? ml->Z1.p : nullptr; g.ldc = MLP_H;
-    g.Cb = ml->H1.p; g.ldcb = MLP_H; g.act = 1;
-    mlp_gemm(st, h, g, 1);
-    g = gemm_of(ml->H1.p, MLP_H, 1, ml->wb.p + PW2, MLP_H, 1, rows, MLP_H, MLP_H);
-    g.Mdev = Mdev; g.bias = ml->w.p + PB2; g.Cf = keepZ ? ml->Z2.p : nullptr; g.ldc = MLP_H;
-    g.Cb = ml->H2.p; g.ldcb = MLP_H; g.act = 1;
-    mlp_gemm(st, h, g, 1);
-    g = gemm_of(ml->H2.p, MLP_H, 1, ml->wb.p + PW3, MLP_H, 1, rows, MLP_H, MLP_H);
-    g.Mdev = Mdev; g.bias = ml->w.p + PB3; g.Cf = keepZ ? ml->Z3.p : nullptr; g.ldc = MLP_H;
-    g.Cb = ml->H3.p; g.ldcb = MLP_H; g.act = 1;
-    mlp_gemm(st, h, g, 1);
-    g = gemm_of(ml->H3.p, MLP_H, 1, ml->wb.p + PW4, MLP_OUT, 1, rows, MLP_OUT, MLP_H);
-    g.Mdev = Mdev; g.bias = ml->w.p + PB4; g.Cf = ml->Y.p; g.ldc = MLP_OUT;
-    mlp_gemm(st, h, g, 1);
-}
-
-// Gradient of the mean squared error of the first nb rows (of `rows`) with
-// respect to every parameter, into ml->g (cleared first); the loss is added
-// to ml->loss.
-static int mlp_backward(sps_mlp *ml, hipStream_t st, int nb, int rows) {
-    sps_handle *h = nullptr;
-    HIP_TRY(hipMemsetAsync(ml->g.p, 0, MLP_NPARAM * sizeof(float), st));
-    MLAUNCH((unsigned)((rows + 255) / 256), 256, k_mlp_loss, ml->Y.p, ml->T.p, nb, rows, ml->dY.p, ml->loss.p);
-    const int kchunk = 256, zs = (rows + kchunk - 1) / kchunk;
-    struct Layer {
-        const bf16_t *Hin;   // layer input (rows x fin)
-        int fin, fout, pw, pb;
-        const float *Zin;    // pre-activation of the input (null for the first layer)
-    };
-    const Layer L[4] = {{ml->X.p, MLP_IN, MLP_H, PW1, PB1, nullptr},
-                        {ml->H1.p, MLP_H, MLP_H, PW2, PB2, ml->Z1.p},
-                        {ml->H2.p, MLP_H, MLP_H, PW3, PB3, ml->Z2.p},
-                        {ml->H3.p, MLP_H, MLP_OUT, PW4, PB4, ml->Z3.p}};
-    const bf16_t *dOut = ml->dY.p;   // gradient at the layer's output (rows x fout), bfloat16
-    for (int l = 3; l >= 0; --l) {
-        const Layer &Ly = L[l];
-        // dW += Hin^T dOut (split over the rows)
-        Gemm g = gemm_of(Ly.Hin, 1, Ly.fin, dOut, Ly.fout, 1, Ly.fin, Ly.fout, rows);
-        g.kchunk = kchunk; g.Cf = ml->g.p + Ly.pw; g.ldc = Ly.fout; g.accumulate = 1;
-        mlp_gemm(st, h, g, zs);
-        MLAUNCH((unsigned)Ly.fout, 256, k_mlp_colsum, dOut, rows, Ly.fout, ml->g.p + Ly.pb);
-        if (l == 0) break;
-        // dHin = dOut W^T, then through the activation
-        g = gemm_of(dOut, Ly.fout, 1, ml->wb.p + Ly.pw, 1, Ly.fout, rows, Ly.fin, Ly.fout);
-        g.Cf = ml->dH.p; g.ldc = Ly.fin;
-        mlp_gemm(st, h, g, 1);
-        const long long n = (long long)rows * Ly.fin;
-        MLAUNCH((unsigned)((n + 255) / 256), 256, k_mlp_silu_back, ml->dH.p, Ly.Zin, n, ml->dZ.p);
-        dOut = ml->dZ.p;
+static NetPass net_pass(sps_mlp *ml, const float *feat, const float *targ, const unsigned *idx, int nb) {
+    NetPass g{};
+    g.feat = feat; g.targ = targ; g.idx = idx; g.nb = nb;
+    g.wf = ml->wf.p; g.wt = ml->wt.p; g.w = ml->w.p; g.Y = ml->Y.p;
+    g.X = ml->X.p; g.dY = ml->dY.p;
+    for (int l = 0; l < 3; ++l) {
+        g.H[l] = ml->H[l].p;
+        g.dZ[l] = ml->dZ[l].p;
     }
+    return g;
+}
+
+// Y = network of the nb rows of feat (or the first *nbdev of them).
+static void mlp_forward(sps_mlp *ml, hipStream_t st, sps_handle *h, const float *feat, int nb, const int *nbdev) {
+    NetPass g = net_pass(ml, feat, nullptr, nullptr, nb);
+    g.nbdev = nbdev;
+    MLAUNCH((unsigned)((nb + NET_ROWS - 1) / NET_ROWS), 256, k_gemm_bf16_chain<false>, g);
+}
+
+// Gradient of the mean squared error of nb rows (idx, or the first) of the
+// set with respect to every parameter, into ml->g; the loss is added to
+// ml->loss.
+static int mlp_gradient(sps_mlp *ml, hipStream_t st, const unsigned *idx, const float *feat, const float *targ, int nb) {
+    sps_handle *h = nullptr;
+    const NetPass g = net_pass(ml, feat, targ, idx, nb);
+    const int blocks = (nb + NET_ROWS - 1) / NET_ROWS, nrb = blocks * (NET_ROWS / 16);
+    // a chunk is at least one workgroup's rows, so that a small batch's partial sums stay few
+    const int chunk = std::max(NET_ROWS / 16, (nrb + DW_CHUNKS - 1) / DW_CHUNKS), nchunk = (nrb + chunk - 1) / chunk;
+    MLAUNCH((unsigned)blocks, 256, k_gemm_bf16_chain<true>, g);
+    MLAUNCH(dim3((unsigned)nchunk, 3), 256, k_gemm_bf16_dw, g, nrb, chunk, ml->part.p);
+    MLAUNCH((unsigned)(REDUCE_BLOCKS + (nb + 255) / 256), 256, k_mlp_loss_reduce, g, ml->part.p, nchunk, ml->g.p,
+            ml->loss.p);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -117,8 +84,8 @@ static int mlp_adam(sps_mlp *ml, hipStream_t st, float lr) {
     ++ml->adam_t;
     const float c1 = 1.0f - powf(b1, (float)ml->adam_t), c2 = 1.0f - powf(b2, (float)ml->adam_t);
     sps_handle *h = nullptr;
-    MLAUNCH((unsigned)((MLP_NPARAM + 255) / 256), 256, k_mlp_adam, ml->w.p, ml->m.p, ml->v.p, ml->g.p, ml->wb.p,
-            MLP_NPARAM, lr, b1, b2, eps, c1, c2);
+    MLAUNCH((unsigned)((MLP_NPARAM + 255) / 256), 256, k_mlp_adam, ml->w.p, ml->m.p, ml->v.p, ml->g.p, ml->wf.p,
+            ml->wt.p, MLP_NPARAM, lr, b1, b2, eps, c1, c2);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -129,7 +96,7 @@ static int mlp_upload_params(sps_mlp *ml, const float *w) {
     HIP_TRY(hipMemcpyAsync(ml->w.p, w, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemsetAsync(ml->m.p, 0, MLP_NPARAM * sizeof(float), st));
     HIP_TRY(hipMemsetAsync(ml->v.p, 0, MLP_NPARAM * sizeof(float), st));
-    MLAUNCH((unsigned)((MLP_NPARAM + 255) / 256), 256, k_mlp_to_bf16, ml->w.p, ml->wb.p, MLP_NPARAM);
+    MLAUNCH((unsigned)((MLP_NPARAM + 255) / 256), 256, k_mlp_to_bf16, ml->w.p, ml->wf.p, ml->wt.p, MLP_NPARAM);
     HIP_TRY(hipStreamSynchronize(st));
     ml->adam_t = 0;
     return 0;
@@ -160,7 +127,7 @@ extern "C" int sps_mlp_create(int32_t batch_rows, uint64_t seed, sps_mlp **out) 
     if (hipStreamCreateWithFlags(&ml->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(SPS_EDEVICE, "hipStreamCreate failed"));
     int rc = dalloc(ml->w, MLP_NPARAM) | dalloc(ml->m, MLP_NPARAM) | dalloc(ml->v, MLP_NPARAM) |
-             dalloc(ml->g, MLP_NPARAM) | dalloc(ml->wb, MLP_NPARAM);
+             dalloc(ml->g, MLP_NPARAM) | dalloc(ml->wf, MLP_NPARAM) | dalloc(ml->wt, MLP_NPARAM);
     if (rc || (rc = mlp_reserve(ml, batch_rows))) return bail(rc);
     // Glorot-uniform weights over the real (unpadded) fan-in / fan-out, zero biases
     std::vector<float> w(MLP_NPARAM, 0.0f);
@@ -184,9 +151,12 @@ extern "C" void sps_mlp_destroy(sps_mlp *ml) {
     if (!ml) return;
     (void)hipSetDevice(ml->device);
     if (ml->stream) (void)hipStreamSynchronize(ml->stream);
-    dfree(ml->w); dfree(ml->m); dfree(ml->v); dfree(ml->g); dfree(ml->wb);
-    dfree(ml->X); dfree(ml->H1); dfree(ml->H2); dfree(ml->H3); dfree(ml->dY); dfree(ml->dZ);
-    dfree(ml->Z1); dfree(ml->Z2); dfree(ml->Z3); dfree(ml->Y); dfree(ml->dH); dfree(ml->T); dfree(ml->loss);
+    dfree(ml->w); dfree(ml->m); dfree(ml->v); dfree(ml->g); dfree(ml->wf); dfree(ml->wt);
+    for (int l = 0; l < 3; ++l) {
+        dfree(ml->H[l]);
+        dfree(ml->dZ[l]);
+    }
+    dfree(ml->X); dfree(ml->dY); dfree(ml->Y); dfree(ml->part); dfree(ml->loss);
     dfree(ml->feat); dfree(ml->targ); dfree(ml->perm);
     if (ml->stream) (void)hipStreamDestroy(ml->stream);
     delete ml;
@@ -222,16 +192,12 @@ extern "C" int sps_mlp_forward(sps_mlp *ml, int64_t n, const float *x, float *y)
     if (!ml || !x || !y || n < 0) return fail(SPS_EINVAL, "bad argument");
     HIP_TRY(hipSetDevice(ml->device));
     hipStream_t st = ml->stream;
-    sps_handle *h = nullptr;
     int rc = mlp_upload_set(ml, n, x, nullptr);
     if (rc) return rc;
     std::vector<float> yb;
     for (int64_t off = 0; off < n; off += ml->rows) {
         const int nb = (int)std::min<int64_t>(ml->rows, n - off);
-        const int rows = (nb + 63) / 64 * 64;
-        MLAUNCH((unsigned)((rows + 255) / 256), 256, k_mlp_batch, ml->feat.p + off * MLP_NIN, nullptr, nullptr, nb,
-                rows, ml->X.p, nullptr, nullptr);
-        mlp_forward(ml, st, nullptr, rows, nullptr, false);
+        mlp_forward(ml, st, nullptr, ml->feat.p + off * MLP_NIN, nb, nullptr);
         yb.resize((size_t)nb * MLP_OUT);
         HIP_TRY(hipMemcpyAsync(yb.data(), ml->Y.p, yb.size() * sizeof(float), hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
@@ -246,15 +212,10 @@ extern "C" int sps_mlp_gradient(sps_mlp *ml, int64_t n, const float *x, const fl
         return fail(SPS_EINVAL, "sps_mlp_gradient: bad argument (n must be 1..batch rows)");
     HIP_TRY(hipSetDevice(ml->device));
     hipStream_t st = ml->stream;
-    sps_handle *h = nullptr;
     int rc = mlp_upload_set(ml, n, x, t);
     if (rc) return rc;
-    const int rows = (int)((n + 63) / 64 * 64);
-    MLAUNCH((unsigned)((rows + 255) / 256), 256, k_mlp_batch, ml->feat.p, ml->targ.p, nullptr, (int)n, rows,
-            ml->X.p, ml->T.p, nullptr);
-    mlp_forward(ml, st, nullptr, rows, nullptr, true);
     HIP_TRY(hipMemsetAsync(ml->loss.p, 0, sizeof(float), st));
-    if ((rc = mlp_backward(ml, st, (int)n, rows))) return rc;
+    if ((rc = mlp_gradient(ml, st, nullptr, ml->feat.p, ml->targ.p, (int)n))) return rc;
     HIP_TRY(hipMemcpyAsync(grad, ml->g.p, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(loss, ml->loss.p, sizeof(float), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
@@ -282,11 +243,7 @@ extern "C" int sps_mlp_train(sps_mlp *ml, int64_t n, const float *x, const float
         int nbatch = 0;
         for (int64_t off = 0; off < n; off += batch, ++nbatch) {
             const int nb = (int)std::min<int64_t>(batch, n - off);
-            const int rows = (nb + 63) / 64 * 64;
-            MLAUNCH((unsigned)((rows + 255) / 256), 256, k_mlp_batch, ml->feat.p, ml->targ.p, ml->perm.p + off, nb,
-                    rows, ml->X.p, ml->T.p, nullptr);
-            mlp_forward(ml, st, nullptr, rows, nullptr, true);
-            if ((rc = mlp_backward(ml, st, nb, rows))) return rc;
+            if ((rc = mlp_gradient(ml, st, ml->perm.p + off, ml->feat.p, ml->targ.p, nb))) return rc;
             if ((rc = mlp_adam(ml, st, lr))) return rc;
         }
         float l = 0.0f;
@@ -416,11 +373,9 @@ static SurrogateDev surrogate_dev(sps_handle *h) {
 static int surrogate_correct(sps_handle *h, const StateBufs &SB) {
     sps_mlp *ml = h->mlp;
     hipStream_t st = h->stream;
-    const int cap = h->surr_cap, rows = (cap + 63) / 64 * 64;
+    const int cap = h->surr_cap;
     const SurrogateDev G = surrogate_dev(h);
-    MLAUNCH((unsigned)((rows + 255) / 256), 256, k_mlp_batch, h->surr_feat.p, nullptr, nullptr, cap, rows, ml->X.p,
-            nullptr, h->surr_count.p);
-    mlp_forward(ml, st, h, rows, (const int *)h->surr_count.p, false);
+    mlp_forward(ml, st, h, h->surr_feat.p, cap, (const int *)h->surr_count.p);
     MLAUNCH((unsigned)((cap + 255) / 256), 256, k_surrogate_apply, G, ml->Y.p, SB.stress, h->surr_tol);
     HIP_TRY(hipGetLastError());
     return 0;
