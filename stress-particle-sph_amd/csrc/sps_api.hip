@@ -3,7 +3,7 @@
 //
 // One step is the reference's time_integration (code/2_SPH_main_2018.f90
 // :78-184) for the supported flag set:
-//   Check_Out_Domain, grid_find_NEW + Pint_Update  -> k_check_ood .. k_split_partner
+//   Check_Out_Domain, grid_find_NEW + Pint_Update  -> k_bounds_partial .. k_split_partner
 //   RK4 (2_...:653-802)                            -> k_stage_first, 4 x stage
 //   update_strain, stress_point_update, adapt      -> k_spu_nodes, k_sp_update
 //   position update and displacement               -> k_position
@@ -157,7 +157,10 @@ struct sps_handle {
     int nbparts = 0;
     DBuf<int> cellkey, new_cell, cell, kcount, kstart, kfill, tmp_orig, tmp_src, proc, proc_to_slot;
     DBuf<unsigned char> moved;    // per block of slots: the permutation moves a particle of it
-    DBuf<unsigned> cnt, off, scan_tmp, ctot, cstart_rm;
+    DBuf<unsigned> cnt, off, cstart_rm;
+    DBuf<unsigned long long> scan_state;   // k_scan_sums: a word per tile, the launch's number, the ticket counter
+    unsigned scan_epoch = 0;
+    DBuf<unsigned> scan_ticket;
     // per-step pair lists of the tiled stage kernels
     DBuf<unsigned long long> list_ia, list_ib, list_iah, list_ibh;
     int list_words = 12;          // words of four entries per receiver and list
@@ -266,14 +269,13 @@ struct sps_handle {
 
 // ------------------------------------------------------------ profiling
 enum KernelId {
-    K_CHECK_OOD, K_BOUNDS, K_CELL_COUNT, K_CELL_SCATTER, K_CELL_SORT, K_PERMUTE, K_PROC,
+    K_BOUNDS, K_CELL_COUNT, K_CELL_SCATTER, K_CELL_SORT, K_PERMUTE,
     K_COUNT_PAIRS, K_SCAN, K_SPLIT, K_RK_INIT, K_LF_KICK, K_SPU_NODES,
     K_SP_UPDATE, K_DERIV_NODES, K_DUMMY_STRESS, K_RK_FINAL, K_POSITION, K_SURROGATE, K_XSPH, K_SHIFT, K_BCS, K_SURF,
     K_AV_NODES, K_COUNT_DUMMY, K_NKERNELS
 };
 static const char *const kKernelNames[K_NKERNELS] = {
-    "k_check_ood", "k_bounds", "k_cell_count", "k_cell_scatter", "k_cell_sort", "k_permute",
-    "k_proc_slot", "k_count_lists", "k_scan", "k_split", "k_stage_first",
+    "k_bounds", "k_cell_count", "k_cell_scatter", "k_cell_sort", "k_permute", "k_count_lists", "k_scan", "k_split", "k_stage_first",
     "k_lf_kick", "k_spu_nodes", "k_sp_update", "k_deriv_nodes",
     "k_dummy_stress", "k_rk_final", "k_position", "k_surrogate", "k_xsph", "k_shift_sp", "k_bcs", "k_surf",
     "k_av_nodes", "k_count"};
@@ -361,17 +363,19 @@ static size_t lds_count(const sps_handle *h) {
 
 // ------------------------------------------------------------------ scans
 // Exclusive scan of n unsigned values; optional device total.  With a
-// device count (sc.g set) n is only the launch bound: the kernels scan the
-// first sc.get(n) values, as many as the current grid has.
-static int scan_u32(sps_handle *h, const unsigned *in, unsigned *out, long long n,
-                    unsigned long long *dtotal, ScanCount sc = ScanCount{nullptr, 0, 0}) {
-    long long nb = (n + BLOCK * 4 - 1) / (BLOCK * 4);
-    if (nb == 0) nb = 1;
-    int rc = dalloc(h->scan_tmp, (size_t)nb);
-    if (rc) return rc;
-    LAUNCH(K_SCAN, (unsigned)nb, BLOCK, k_scan_local, in, out, h->scan_tmp.p, n, sc);
-    LAUNCH(K_SCAN, 1, BLOCK, k_scan_sums, h->scan_tmp.p, (int)nb, dtotal, n, sc);
-    LAUNCH(K_SCAN, (unsigned)nb, BLOCK, k_scan_add, out, h->scan_tmp.p, n, sc);
+// device count (sc.g set) n is only the bound: the kernel scans the first
+// sc.get(n) values, as many as the current grid has.
+template <typename In>
+static int scan_u32(sps_handle *h, In in, unsigned *out, long long n, unsigned long long *dtotal,
+                    ScanCount sc = ScanCount{nullptr, 0, 0}) {
+    const long long nb = std::max(1ll, (n + SCAN_TILE - 1) / SCAN_TILE);
+    if ((size_t)nb > h->scan_state.n) return fail(SPS_ECAPACITY, "scan of %lld values", n);
+    if (++h->scan_epoch >= SCAN_EPOCHS) {   // the numbers of earlier launches come again
+        HIP_TRY(hipMemsetAsync(h->scan_state.p, 0, h->scan_state.n * sizeof(unsigned long long), h->stream));
+        h->scan_epoch = 1;
+    }
+    LAUNCH(K_SCAN, (unsigned)std::min<long long>(nb, SCAN_BLOCKS), BLOCK, k_scan_sums<In>, in, out, h->scan_state.p,
+           h->scan_ticket.p, (unsigned long long)h->scan_epoch, dtotal, n, sc);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -635,10 +639,16 @@ static int size_cells(sps_handle *h, const double *hsml) {
     int rc = 0;
     size_t L = 3 * ((size_t)cap + 1) + 1;
     rc |= dalloc(h->kcount, L); rc |= dalloc(h->kstart, L); rc |= dalloc(h->kfill, L);
-    rc |= dalloc(h->ctot, (size_t)cap + 2); rc |= dalloc(h->cstart_rm, (size_t)cap + 2);
-    // block sums of the largest scan of a step (the bucket counts or the slots)
-    rc |= dalloc(h->scan_tmp, std::max(L, (size_t)h->nt2 + 1) / (BLOCK * 4) + 2);
+    rc |= dalloc(h->cstart_rm, (size_t)cap + 2);
+    // tiles of the largest scan of a step (the bucket counts or the slots)
+    rc |= dalloc(h->scan_state, std::max(L, (size_t)h->nt2 + 1) / SCAN_TILE + 2) | dalloc(h->scan_ticket, 1);
     if (rc) return rc;
+    // a search clears the counters it has used for the next one
+    HIP_TRY(hipMemsetAsync(h->kcount.p, 0, h->kcount.n * sizeof(int), h->stream));
+    HIP_TRY(hipMemsetAsync(h->kfill.p, 0, h->kfill.n * sizeof(int), h->stream));
+    HIP_TRY(hipMemsetAsync(h->scan_state.p, 0, h->scan_state.n * sizeof(unsigned long long), h->stream));
+    HIP_TRY(hipMemsetAsync(h->scan_ticket.p, 0, sizeof(unsigned), h->stream));
+    h->scan_epoch = 0;
     h->cell_cap = cap;
     return 0;
 }
@@ -730,40 +740,34 @@ static int search(sps_handle *h, bool fresh_list) {
     StateSet &A = h->S[h->cur];
     StateSet &B = h->S[1 - h->cur];
     // domain check and grid
-    LAUNCH(K_CHECK_OOD, nblk(nt2), BLOCK, k_check_ood, A.x.p, A.ood.p, nt2, h->p.xmin_domain[0], h->p.xmin_domain[1],
-                                           h->p.xmax_domain[0], h->p.xmax_domain[1]);
-    LAUNCH(K_BOUNDS, h->nbparts, BLOCK, k_bounds_partial, A.x.p, A.hsml.p, A.ood.p, nt2, h->bparts.p);
-    LAUNCH(K_BOUNDS, 1, BLOCK, k_bounds_final, h->bparts.p, h->nbparts, h->grid.p, h->cell_cap, h->skin, h->err.p);
+    LAUNCH(K_BOUNDS, h->nbparts, BLOCK, k_bounds_partial, A.x.p, A.hsml.p, A.ood.p, nt2, h->p.xmin_domain[0],
+           h->p.xmin_domain[1], h->p.xmax_domain[0], h->p.xmax_domain[1], h->bparts.p);
+    LAUNCH(K_BOUNDS, 1, BLOCK, k_bounds_final, h->bparts.p, h->nbparts, h->grid.p, h->cell_cap, h->skin, h->split.p,
+           fresh_list ? 1 : 0, h->err.p);
     // bucket arrays: 3 (ndivt + 1) + 1 entries of the current grid, at most
     // those of the capacity
     const long long L3max = 3LL * (h->cell_cap + 1);
-    LAUNCH(K_CELL_COUNT, nstride(L3max + 1), BLOCK, k_zero_cells, h->kcount.p, h->kfill.p, h->grid.p);
     LAUNCH(K_CELL_COUNT, nblk(nt2), BLOCK, k_cell_count, A.x.p, A.ood.p, h->grid.p, h->cellkey.p, h->kcount.p, nn, nt, nt2);
-    int rc = scan_u32(h, (const unsigned *)h->kcount.p, (unsigned *)h->kstart.p, L3max + 1, nullptr,
+    int rc = scan_u32(h, ScanArray{(const unsigned *)h->kcount.p}, (unsigned *)h->kstart.p, L3max + 1, nullptr,
                       ScanCount{h->grid.p, 3, 4});
     if (rc) return rc;
     LAUNCH(K_CELL_SCATTER, nblk(nt2), BLOCK, k_cell_scatter, h->cellkey.p, A.orig.p, h->kstart.p, h->kfill.p, h->grid.p,
                                               h->tmp_orig.p, h->tmp_src.p, h->cell.p, nn, nt, nt2);
-    LAUNCH(K_CELL_SORT, nstride(L3max), BLOCK, k_cell_sort, h->kstart.p, h->tmp_orig.p, h->tmp_src.p, h->grid.p,
-           h->err.p);
+    LAUNCH(K_CELL_SORT, TILES_BLOCKS + nstride(L3max), BLOCK, k_count_tiles_sort, h->kstart.p, h->grid.p,
+           h->tile_start.p, h->tile_range.p, h->ntile_n, h->ntile_s, nn, nt, h->mixed ? 0 : 1, h->tmp_orig.p,
+           h->tmp_src.p, h->err.p);
     // permute the state into (kind, cell, original index) order: the blocks
     // whose particles moved go through the scratch set and back
     LAUNCH(K_PERMUTE, nblk(nt2), BLOCK, k_permute, B.view(), A.view(), h->tmp_src.p, nn, nt, nt2, h->moved.p);
-    LAUNCH(K_PERMUTE, nblk(nt2), BLOCK, k_permute_commit, A.view(), B.view(), h->moved.p, nn, nt, nt2);
+    rc = scan_u32(h, ScanCells{h->kstart.p, h->grid.p}, h->cstart_rm.p, (long long)h->cell_cap + 1, nullptr,
+                  ScanCount{h->grid.p, 1, 1});
+    if (rc) return rc;
+    LAUNCH(K_PERMUTE, nblk(nt2), BLOCK, k_permute_commit, A.view(), B.view(), h->moved.p, h->cell.p, h->kstart.p,
+           h->cstart_rm.p, h->grid.p, h->proc.p, h->proc_to_slot.p, h->cnt.p, h->outside ? h->inv.p : nullptr,
+           h->kcount.p, h->kfill.p, nn, nt, nt2);
     HIP_TRY(hipGetLastError());
     StateSet &C = A;
-    if (h->outside) LAUNCH(K_PERMUTE, nblk(nt2), BLOCK, k_inv_slots, C.orig.p, h->inv.p, nt2);
-    LAUNCH(K_PROC, nstride((long long)h->cell_cap + 1), BLOCK, k_cell_totals, h->kstart.p, h->grid.p, h->ctot.p);
-    rc = scan_u32(h, h->ctot.p, h->cstart_rm.p, (long long)h->cell_cap + 1, nullptr, ScanCount{h->grid.p, 1, 1});
-    if (rc) return rc;
-    LAUNCH(K_PROC, nblk(nt2), BLOCK, k_proc_slot, h->cell.p, h->kstart.p, h->cstart_rm.p, h->grid.p, h->proc.p,
-           nn, nt, nt2);
-    LAUNCH(K_PROC, nblk(nt2), BLOCK, k_proc_to_slot, h->proc.p, h->proc_to_slot.p, nt2);
-    LAUNCH(K_PROC, 2, TILES_BLOCK, k_count_tiles, h->kstart.p, h->grid.p, h->tile_start.p, h->tile_range.p, h->ntile_n,
-           h->ntile_s, nn, nt, h->mixed ? 0 : 1);
     // counts, offsets, split
-    LAUNCH(K_SPLIT, nblk(nt2), BLOCK, k_surf_zero, h->cnt.p, (long long)nt2);
-    LAUNCH(K_SPLIT, 1, 64, k_split_reset, h->split.p, fresh_list ? 1 : 0);
     {
         const SearchView V{h->cell.p, h->kstart.p, h->proc.p, h->cnt.p, h->off.p, h->grid.p, h->split.p, h->p.pi};
         const PairLists PL = h->lists();
@@ -803,7 +807,7 @@ static int search(sps_handle *h, bool fresh_list) {
     }
     HIP_TRY(hipGetLastError());
     // discovery offsets over all slots (slots past the in-domain count hold 0)
-    rc = scan_u32(h, h->cnt.p, h->off.p, nt2, &h->split.p->n);
+    rc = scan_u32(h, ScanArray{h->cnt.p}, h->off.p, nt2, &h->split.p->n);
     if (rc) return rc;
     LAUNCH(K_SPLIT, nblk(nt2), BLOCK, k_count_split, h->cnt.p, h->off.p, nt2, h->split.p, h->type_counts.p, h->ntile_n,
            h->ntile_s, h->ntile_n + h->ntile_s + (int)count_blocks(nt2 - nt));
@@ -1640,7 +1644,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->rk_dev); dfree(h->sig2); dfree(h->stress_b); dfree(h->av_nodes); dfree(h->ddev); dfree(h->grid); dfree(h->split); dfree(h->bparts);
     dfree(h->cellkey); dfree(h->new_cell); dfree(h->cell); dfree(h->kcount); dfree(h->kstart);
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
-    dfree(h->cnt); dfree(h->off); dfree(h->scan_tmp); dfree(h->ctot); dfree(h->cstart_rm); dfree(h->err);
+    dfree(h->cnt); dfree(h->off); dfree(h->scan_state); dfree(h->scan_ticket); dfree(h->cstart_rm); dfree(h->err);
     dfree(h->list_ia); dfree(h->list_iah); dfree(h->list_ibh); dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya); dfree(h->list_ib);
     dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->type_counts); dfree(h->tiles); dfree(h->plans);
     dfree(h->list_wb); dfree(h->xsph_v);

@@ -106,3 +106,27 @@ def test_mixed_tiles_across_strips(nx, ny, change, skin):
     err = acc.compare_states(mix.get_state(), ora.get_state(), x0)
     for k in ("disp_rel_max", "vel_rel_max", "stress_rel_max"):
         assert err[k] <= 1e-5, f"{k} {err[k]:.3e}"
+
+
+# The search's prefix sums run over 3 (cells + 1) + 1 buckets and over the
+# cells, 2048 elements a tile: one particle far from the body stretches the
+# grid to a few cells under and over a tile, over the 64 tiles that one look
+# back takes and over the 1024 blocks of a launch.
+@pytest.mark.parametrize("cells", [100, 681, 682, 683, 2047, 2048, 45000, 800000])
+def test_search_on_stretched_grids(cells):
+    sps = load_pkg()
+    deck = sps.read_deck(deck_dir("t1_tiny"))
+    reach = 2 * 1.2 * deck.dx
+    side = max(1.0, np.sqrt(cells))
+    deck.xmax_domain = np.array([side + 40.0, cells / side + 40.0]) * reach
+    gpu = sps.Simulation.from_deck(deck)
+    ora = sps.Simulation.from_deck(deck, lib_path=ORACLE_LIB)
+    st = sps.initial_state(gpu.parts, gpu.niv)
+    st["x"][gpu.nn - 1] = np.array([side - 0.5, cells / side - 0.5]) * reach
+    for sim in (gpu, ora):
+        sim.set_state(st)
+    print(f"[search] about {cells} cells", flush=True)
+    for step in range(1, 4):
+        gpu.step(1)
+        ora.step(1)
+        compare(gpu, ora, f"{cells} cells, step {step}")
