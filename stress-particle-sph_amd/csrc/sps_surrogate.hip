@@ -128,16 +128,16 @@ template <bool GRAD> __global__ __launch_bounds__(256, 2) void k_gemm_bf16_chain
     auto source = [&](int row) { return row < nb ? (g.idx ? (long long)g.idx[row] : (long long)row) : -1ll; };
 
     // weights on their way, 16 bytes (two tile words) at a time
-    double2 pre[8];
+    v4f pre[8];
     auto fetch = [&](const bf16_t *src, auto nw) {
         constexpr int N = decltype(nw)::value / 512;
 #pragma unroll
-        for (int k = 0; k < N; ++k) pre[k] = reinterpret_cast<const double2 *>(src)[t + 256 * k];
+        for (int k = 0; k < N; ++k) pre[k] = reinterpret_cast<const v4f *>(src)[t + 256 * k];
     };
     auto commit = [&](auto nw) {
         constexpr int N = decltype(nw)::value / 512;
 #pragma unroll
-        for (int k = 0; k < N; ++k) reinterpret_cast<double2 *>(sW)[t + 256 * k] = pre[k];
+        for (int k = 0; k < N; ++k) reinterpret_cast<v4f *>(sW)[t + 256 * k] = pre[k];
     };
     using Small = std::integral_constant<int, 8 * 64>;
     using Large = std::integral_constant<int, 64 * 64>;
