@@ -59,8 +59,10 @@ static inline int ntiles(long long n, double strips) {
 }
 
 
-// blocks of k_count for n dummy receivers, sixteen lanes each
-static inline unsigned count_blocks(long long n) { return (unsigned)((n * 16 + BLOCK - 1) / BLOCK); }
+// workgroups of TILE lanes for n items
+static inline unsigned tblk(long long n) { return (unsigned)((n + TILE - 1) / TILE); }
+// and for the count of n dummy receivers, sixteen lanes each
+static inline unsigned count_blocks(long long n) { return tblk(n * 16); }
 
 template <typename T>
 struct DBuf {
@@ -141,13 +143,11 @@ struct sps_handle {
     DBuf<double2> x0, vel0, rk_vel, rhs2, f_bound, art_visc;   // vel0 is also the step's vx0
     DBuf<double4> stress0, rk_stress, rhs1, grad_u;
     // the stress points' stresses after a stage's second return map, which
-    // k_sp_update writes here so that k_spu_nodes, reading the first, can
-    // run beside it (on stream2; ev_fork / ev_join order the two)
+    // k_sp_update writes here so that the nodes' half, reading the first, can
+    // run beside it (k_sp_update_beside)
     DBuf<double4> sig2;
     DBuf<double4> stress_b;  // the stress points' stresses of the odd RK stages (StageStep)
     DBuf<float2> av_nodes;   // the nodes' artificial viscosity of a stage (k_av_nodes)
-    hipStream_t stream2 = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     DBuf<double> rk_dev, ddev;
     // search
     int cell_cap = 0;
@@ -272,13 +272,13 @@ enum KernelId {
     K_BOUNDS, K_CELL_COUNT, K_CELL_SCATTER, K_CELL_SORT, K_PERMUTE,
     K_COUNT_PAIRS, K_SCAN, K_SPLIT, K_RK_INIT, K_LF_KICK, K_SPU_NODES,
     K_SP_UPDATE, K_DERIV_NODES, K_DUMMY_STRESS, K_RK_FINAL, K_POSITION, K_SURROGATE, K_XSPH, K_SHIFT, K_BCS, K_SURF,
-    K_AV_NODES, K_COUNT_DUMMY, K_NKERNELS
+    K_AV_NODES, K_NKERNELS
 };
 static const char *const kKernelNames[K_NKERNELS] = {
     "k_bounds", "k_cell_count", "k_cell_scatter", "k_cell_sort", "k_permute", "k_count_lists", "k_scan", "k_split", "k_stage_first",
     "k_lf_kick", "k_spu_nodes", "k_sp_update", "k_deriv_nodes",
     "k_dummy_stress", "k_rk_final", "k_position", "k_surrogate", "k_xsph", "k_shift_sp", "k_bcs", "k_surf",
-    "k_av_nodes", "k_count"};
+    "k_av_nodes"};
 
 static hipEvent_t prof_begin(sps_handle *h) {
     if (!h->prof) return nullptr;
@@ -537,12 +537,8 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
         sps_destroy(h);
         return code;
     };
-    if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking) != hipSuccess)
+    if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(SPS_EDEVICE, "hipStreamCreate failed"));
-    if (hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming) != hipSuccess)
-        return bail(fail(SPS_EDEVICE, "hipEventCreate failed"));
     int nt2 = h->nt2, nt = h->nt, nn = h->nn;
     rc = 0;
     rc |= h->S[0].alloc(nn, nt, nt2);
@@ -771,39 +767,14 @@ static int search(sps_handle *h, bool fresh_list) {
     {
         const SearchView V{h->cell.p, h->kstart.p, h->proc.p, h->cnt.p, h->off.p, h->grid.p, h->split.p, h->p.pi};
         const PairLists PL = h->lists();
-        // the stress-point receivers' lists (their tiles, counts and list
-        // words are their own; the type histogram is summed with atomics)
-        // are built beside the nodes' on the second stream, unless kernel
-        // timing (one stream) is on
-        const bool fork = !h->prof && nn > 0 && nt > nn;
-        if (fork) {
-            HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
-            HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
-            if (!h->mixed)
-                k_count_lists<KIND_SP, true><<<h->ntile_s, TILE, lds_count(h), h->stream2>>>(
-                    V, C.x.p, C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
-            else
-                k_count_lists<KIND_SP, false><<<h->ntile_s, TILE, lds_count(h), h->stream2>>>(
-                    V, C.x.p, C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
-            HIP_TRY(hipEventRecord(h->ev_join, h->stream2));
-        }
+        const unsigned blocks = (unsigned)(h->ntile_n + h->ntile_s) + (nt2 > nt ? count_blocks(nt2 - nt) : 0u);
         // the mixed-precision stage kernels compute the kernel values themselves
-        if (nn > 0 && !h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_n, TILE, lds_count(h), (k_count_lists<KIND_NODE, true>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
-        if (nn > 0 && h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_n, TILE, lds_count(h), (k_count_lists<KIND_NODE, false>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
-        if (!fork && nt > nn && !h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_s, TILE, lds_count(h), (k_count_lists<KIND_SP, true>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
-        if (!fork && nt > nn && h->mixed)
-            LAUNCH_LDS(K_COUNT_PAIRS, h->ntile_s, TILE, lds_count(h), (k_count_lists<KIND_SP, false>), V, C.x.p,
-                       C.hsml.p, h->cnt.p, PL, h->h_uniform, h->skin);
-        if (nt2 > nt)
-            LAUNCH(K_COUNT_DUMMY, count_blocks(nt2 - nt), BLOCK, k_count, C.x.p, C.hsml.p, h->cell.p, h->kstart.p,
-                   h->proc.p, h->grid.p, h->cnt.p, h->type_counts.p + 3 * ((size_t)h->ntile_n + h->ntile_s), nt, nt2);
-        if (fork) HIP_TRY(hipStreamWaitEvent(h->stream, h->ev_join, 0));
+        if (h->mixed)
+            LAUNCH_LDS(K_COUNT_PAIRS, blocks, TILE, lds_count(h), k_count_lists<false>, V, C.x.p, C.hsml.p, h->cnt.p,
+                       PL, h->h_uniform, h->skin, h->ntile_s, nt, nt2);
+        else
+            LAUNCH_LDS(K_COUNT_PAIRS, blocks, TILE, lds_count(h), k_count_lists<true>, V, C.x.p, C.hsml.p, h->cnt.p,
+                       PL, h->h_uniform, h->skin, h->ntile_s, nt, nt2);
     }
     HIP_TRY(hipGetLastError());
     // discovery offsets over all slots (slots past the in-domain count hold 0)
@@ -893,39 +864,30 @@ static int mixed_step_kernels(sps_handle *h, double dt, double time_sph, double 
     for (int st = 0; st < 4; ++st) {
         const StageStep Q = rk_stage(h, SB, st, dt, hook);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
-        // the two halves of stress_point_update side by side, as in the FP64
-        // step; one stream when kernels are timed or the step is captured
-        const bool fork = !h->prof && !stepv && nn > 0 && nt > nn;
-        if (fork) {
-            HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
-            HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
-            hipStream_t s2 = h->stream2;
-            k_spu_nodes_mix<<<h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, hu, nn,
-                                                                               Q.sp_in, nullptr, 0.0);
-            if (bcs)
-                k_bcs<<<nblk(nn), BLOCK, 0, s2>>>(SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p,
-                                                 h->ifsigman, h->normal.p, nn, nullptr, nullptr);
-            if (st == 3 && nt2 > nt) k_dummy_stress<<<nblk(nt2 - nt), BLOCK, 0, s2>>>(SB, V, nt, nt2);
-            // the nodes' artificial viscosity reads only node data, after the
-            // node side and the second BC call (k_deriv_nodes_mix takes it)
-            if (h->dp.do_av)
-                k_av_nodes_mix<<<h->ntile_n, TILE, LAY_AV_NODES_MIX.bytes, s2>>>(SB, V, PL, h->dp, hu,
-                                                                                     h->av_nodes.p, nn);
-            HIP_TRY(hipEventRecord(h->ev_join, s2));
+        // as in the FP64 step
+        const bool both = !h->prof && nn > 0 && nt > nn, av = h->dp.do_av && nn > 0;
+        const unsigned nodes = (unsigned)(h->ntile_s + h->ntile_n), dum = st == 3 && nt2 > nt ? tblk(nt2 - nt) : 0u;
+        if (both && !av)
+            LAUNCH_LDS(K_SP_UPDATE, nodes, TILE, std::max(LAY_SP_UPDATE_MIX.bytes, LAY_SPU_NODES_MIX.bytes),
+                       k_sp_update_beside_mix<true>, SB, W, V, PL, h->dp, time_sph, Q, adapt, hu, h->ntile_s, stepv,
+                       h->sig2.p, nullptr, nt, nt2, h->err.p);
+        else if (nn > 0)
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
+                       tanfi, coh, hu, nn, Q.sp_in, nullptr, 0.0);
+        if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
+        if (both && av) {
+            LAUNCH_LDS(K_SP_UPDATE, nodes + dum, TILE, std::max(LAY_SP_UPDATE_MIX.bytes, LAY_AV_NODES_MIX.bytes),
+                       k_sp_update_beside_mix<false>, SB, W, V, PL, h->dp, time_sph, Q, adapt, hu, h->ntile_s, stepv,
+                       h->sig2.p, h->av_nodes.p, nt, nt2, h->err.p);
         } else {
-            if (nn > 0)
-                LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES_MIX.bytes, k_spu_nodes_mix, SB, V, PL, adapt,
-                           tanfi, coh, hu, nn, Q.sp_in, nullptr, 0.0);
-            if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, h->bc_vars, h->bc_vals.p, h->ifsigman, h->normal.p, nn, nullptr, nullptr);
-            if (st == 3 && nt2 > nt) LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
-            if (h->dp.do_av && nn > 0)
+            if (dum) LAUNCH(K_DUMMY_STRESS, dum, TILE, k_dummy_stress, SB, V, nt, nt2);
+            if (av)
                 LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, LAY_AV_NODES_MIX.bytes, k_av_nodes_mix, SB, V, PL, h->dp, hu,
                            h->av_nodes.p, nn);
         }
-        if (nt > nn)
+        if (nt > nn && !both)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, LAY_SP_UPDATE_MIX.bytes, k_sp_update_mix, SB, W, V, PL,
                        h->dp, time_sph, Q, 1, adapt, hu, nn, nt, stepv, h->sig2.p, nullptr, 0.0, h->err.p);
-        if (fork) HIP_TRY(hipStreamWaitEvent(h->stream, h->ev_join, 0));
         if (nn > 0)
             LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, LAY_DERIV_NODES_MIX.bytes, k_deriv_nodes_mix, SB, W, V, PL,
                        h->dp, gxg, gyg, Q, adapt, h->err.p, hu, nn, stepv, nt > nn ? h->sig2.p : SB.stress,
@@ -1141,42 +1103,31 @@ static int one_step(sps_handle *h, int itimestep, double time_sph, double dt) {
     for (int st = 0; st < (lf ? 0 : 4); ++st) {
         const StageStep Q = rk_stage(h, SB, st, dt, hook);
         if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, st ? bci_cur : nullptr, st ? nullptr : bci_prev);
-        // stress_point_update's two halves are independent: the node side
-        // reads the stress points' stresses before their second return map
-        // (k_sp_update leaves that in sig2) and changes node velocities only
-        // where no stress point reads them (nodes without stress-point
-        // partners); the second BC call sets the node velocities the first
-        // set.  So they run side by side, unless kernel timing (one stream)
-        // is on.
-        // The artificial viscosity (k_av_nodes) reads only node data, after
-        // the node side and the second BC call, and goes with them.
-        const bool fork = !h->prof && nn > 0 && nt > nn;
-        const bool av = h->dp.do_av && nn > 0;
-        if (fork) {
-            HIP_TRY(hipEventRecord(h->ev_fork, s));
-            HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
-            hipStream_t s2 = h->stream2;
-            k_spu_nodes<<<h->ntile_n, TILE, LAY_SPU_NODES.bytes, s2>>>(SB, V, PL, adapt, tanfi, coh, nn, Q.sp_in,
-                                                                        nullptr, 0.0);
-            if (bcs)
-                k_bcs<<<nblk(nn), BLOCK, 0, s2>>>(SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman,
-                                                 h->normal.p, nn, st ? bci_cur : nullptr,
-                                                 st ? nullptr : bci_prev);
-            if (st == 3 && nt2 > nt) k_dummy_stress<<<nblk(nt2 - nt), BLOCK, 0, s2>>>(SB, V, nt, nt2);
-            if (av) k_av_nodes<<<h->ntile_n, TILE, lds_av_nodes(h), s2>>>(SB, V, PL, h->dp, h->av_nodes.p, nn);
-            HIP_TRY(hipEventRecord(h->ev_join, s2));
+        // k_sp_update_beside runs what is independent of the stress points'
+        // update in its launch, unless kernels are timed; BC calls have to
+        // follow the node half and precede the viscosity, so with viscosity
+        // that goes beside and the node half before
+        const bool both = !h->prof && nn > 0 && nt > nn, av = h->dp.do_av && nn > 0;
+        const unsigned nodes = (unsigned)(h->ntile_s + h->ntile_n), dum = st == 3 && nt2 > nt ? tblk(nt2 - nt) : 0u;
+        if (both && !av)
+            LAUNCH_LDS(K_SP_UPDATE, nodes, TILE, std::max(lds_sp_update(h, 1), (size_t)LAY_SPU_NODES.bytes),
+                       k_sp_update_beside<true>, SB, W, V, PL, h->dp, time_sph, Q, adapt, h->ntile_s, h->sig2.p,
+                       nullptr, nt, nt2, h->err.p);
+        else if (nn > 0)
+            LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh,
+                       nn, Q.sp_in, nullptr, 0.0);
+        if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, st ? bci_cur : nullptr, st ? nullptr : bci_prev);
+        if (both && av) {
+            LAUNCH_LDS(K_SP_UPDATE, nodes + dum, TILE, std::max(lds_sp_update(h, 1), lds_av_nodes(h)),
+                       k_sp_update_beside<false>, SB, W, V, PL, h->dp, time_sph, Q, adapt, h->ntile_s, h->sig2.p,
+                       h->av_nodes.p, nt, nt2, h->err.p);
         } else {
-            if (nn > 0)
-                LAUNCH_LDS(K_SPU_NODES, h->ntile_n, TILE, LAY_SPU_NODES.bytes, k_spu_nodes, SB, V, PL, adapt, tanfi, coh,
-                           nn, Q.sp_in, nullptr, 0.0);
-            if (bcs) LAUNCH(K_BCS, nblk(nn), BLOCK, k_bcs, SB, h->bc_info.p, h->bc_or_not.p, BV, h->bc_vals.p, h->ifsigman, h->normal.p, nn, st ? bci_cur : nullptr, st ? nullptr : bci_prev);
-            if (st == 3 && nt2 > nt) LAUNCH(K_DUMMY_STRESS, nblk(nt2 - nt), BLOCK, k_dummy_stress, SB, V, nt, nt2);
+            if (dum) LAUNCH(K_DUMMY_STRESS, dum, TILE, k_dummy_stress, SB, V, nt, nt2);
             if (av) LAUNCH_LDS(K_AV_NODES, h->ntile_n, TILE, lds_av_nodes(h), k_av_nodes, SB, V, PL, h->dp, h->av_nodes.p, nn);
         }
-        if (nt > nn)
+        if (nt > nn && !both)
             LAUNCH_LDS(K_SP_UPDATE, h->ntile_s, TILE, lds_sp_update(h, 1), k_sp_update, SB, W, V, PL, h->dp, time_sph,
                        Q, 1, adapt, nn, nt, h->sig2.p, nullptr, 0.0, h->err.p);
-        if (fork) HIP_TRY(hipStreamWaitEvent(s, h->ev_join, 0));
         if (nn > 0)
             LAUNCH_LDS(K_DERIV_NODES, h->ntile_n, TILE, lds_deriv_nodes(h), k_deriv_nodes, SB, W, V, PL, h->dp, gxg,
                        gyg, Q, adapt, h->err.p, nn, nt > nn ? h->sig2.p : SB.stress, av ? h->av_nodes.p : nullptr);
@@ -1659,9 +1610,6 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->read_dev);
     for (hipEvent_t e : h->read_ev)
         if (e) (void)hipEventDestroy(e);
-    if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
-    if (h->ev_join) (void)hipEventDestroy(h->ev_join);
-    if (h->stream2) (void)hipStreamDestroy(h->stream2);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }

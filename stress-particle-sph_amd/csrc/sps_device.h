@@ -209,17 +209,20 @@ constexpr int NUM_XCD = 8;
 // consecutive workgroups to the XCDs in turn; each XCD gets runs of TILE_RUN
 // consecutive tiles, the runs dealt out round-robin, so that neighbouring
 // tiles (which share window data) mostly share an L2 while every XCD gets
-// tiles from the whole domain (tiles differ in cost by region).  A bijection
-// of [0, gridDim.x) when gridDim.x is a multiple of NUM_XCD: the blocks
-// beyond the last whole run of each XCD take the remaining tiles in order.
+// tiles from the whole domain (tiles differ in cost by region).  b is the
+// workgroup among the n that share these tiles, the launch's first ones or
+// after a multiple of NUM_XCD others.  A bijection of [0, n) when n is a
+// multiple of NUM_XCD: the blocks beyond the last whole run of each XCD take
+// the remaining tiles in order.
 constexpr int TILE_RUN = 16;
-__device__ __forceinline__ int tile_index() {
-    const int xcd = blockIdx.x % NUM_XCD, k = blockIdx.x / NUM_XCD;
-    const int per = gridDim.x / NUM_XCD;
+__device__ __forceinline__ int tile_index(int b, int n) {
+    const int xcd = b % NUM_XCD, k = b / NUM_XCD;
+    const int per = n / NUM_XCD;
     const int full = per / TILE_RUN * TILE_RUN;
     if (k < full) return ((k / TILE_RUN) * NUM_XCD + xcd) * TILE_RUN + (k % TILE_RUN);
     return full * NUM_XCD + xcd * (per - full) + (k - full);
 }
+__device__ __forceinline__ int tile_index() { return tile_index(blockIdx.x, gridDim.x); }
 
 // adapt_stress2 for one particle (code/3_SPH_material_2018.f90:2066-2140).
 __device__ __forceinline__ void adapt_stress(double4 &s, double tanfi, double coh) {

@@ -515,49 +515,6 @@ __device__ __forceinline__ void block_type_counts(const unsigned (&v)[3], unsign
     }
 }
 
-// For every dummy receiver (slots [r0, r1)): pairs it discovers (partners
-// later in processing order; the reference counts n_pairs with these), by
-// partner kind.  The node and stress-point receivers are counted by the tiled
-// k_count_lists below.  Sixteen lanes per receiver, lane 3 c + k taking the
-// partners of kind k in the c-th of the five cells that can hold later ones
-// (its own and the four visited after it).
-__global__ __launch_bounds__(BLOCK) void k_count(const double2 *__restrict__ x, const double *__restrict__ hsml,
-                                                 const int *__restrict__ cell, const int *__restrict__ kstart,
-                                                 const int *__restrict__ proc, const Grid *__restrict__ g,
-                                                 unsigned *__restrict__ cnt, unsigned *__restrict__ types, int r0,
-                                                 int r1) {
-    __shared__ unsigned sum[BLOCK / 64][3];
-    const int lane = threadIdx.x & 15;
-    const int r = r0 + (int)(blockIdx.x * (BLOCK / 16) + (threadIdx.x >> 4));
-    const Grid gg = *g;
-    const int key_r = r < r1 ? cell[r] : gg.ndivt;
-    const bool live = key_r < gg.ndivt;
-    unsigned n = 0;
-    if (live && lane < 15) {
-        const int c = lane / 3, ks = lane - 3 * c;
-        int cx, cy;
-        cell_xy(key_r, gg, cx, cy);
-        const int gx = cx + (c == 0 || c == 3 ? 0 : c == 2 ? -1 : 1), gy = cy + (c > 1 ? 1 : 0);
-        if (gx >= 0 && gx < gg.ndivx && gy < gg.ndivy && (c > 0 || ks == KIND_DUMMY)) {
-            const int *__restrict__ k0 = kstart + ks * (gg.ndivt + 1) + cell_key(gx, gy, gg);
-            const int lo = c == 0 ? r + 1 : k0[0], hi = k0[1];
-            const double2 xr = x[r];
-            const double hr = hsml[r];
-            for (int s = lo; s < hi; ++s) {
-                const double2 xs = x[s];
-                double mh;
-                n += pair_distance(xr.x - xs.x, xr.y - xs.y, hr, hsml[s], mh) < 0.0 ? 0u : 1u;
-            }
-        }
-    }
-    unsigned all = n;
-    for (int off = 8; off > 0; off >>= 1) all += __shfl_down(all, off, 16);
-    if (live && lane == 0) cnt[proc[r]] = all;
-    const int ks = lane % 3;
-    const unsigned v[3] = {ks == 0 ? n : 0u, ks == 1 ? n : 0u, ks == 2 ? n : 0u};
-    block_type_counts(v, sum, types + 3 * (size_t)blockIdx.x);
-}
-
 // Locate the processing slot whose discoveries straddle index M (n is the
 // scan total of the per-slot counts, written by the scan), and add up the
 // pint_type histogram: types holds 3 counts by partner kind of every node
@@ -1482,19 +1439,59 @@ __device__ __forceinline__ bool in_list_a(int kr, int ks) {
     return kr == KIND_NODE ? ks != KIND_NODE : ks != KIND_SP;
 }
 
-// Counting of k_count for the node (KR = 0) or stress-point (KR = 1)
-// receivers [base, base + count), tiled as the stage kernels are, and the
-// tile's pair lists; with FILL, also the lists' kernel values (the
+// For every dummy receiver (slots [r0, r1)): pairs it discovers (partners
+// later in processing order; the reference counts n_pairs with these), by
+// partner kind.  The node and stress-point receivers are counted by the tiled
+// list build.  Sixteen lanes per receiver, lane 3 c + k taking the
+// partners of kind k in the c-th of the five cells that can hold later ones
+// (its own and the four visited after it).
+__device__ __forceinline__ void count_dummies(int block, const double2 *__restrict__ x,
+                                              const double *__restrict__ hsml, const SearchView &V,
+                                              unsigned *__restrict__ cnt, unsigned *__restrict__ types, int r0, int r1) {
+    __shared__ unsigned sum[TWAVES][3];
+    const int *__restrict__ cell = V.cell, *__restrict__ kstart = V.kstart, *__restrict__ proc = V.proc;
+    const int lane = threadIdx.x & 15;
+    const int r = r0 + block * (TILE / 16) + (int)(threadIdx.x >> 4);
+    const Grid gg = *V.g;
+    const int key_r = r < r1 ? cell[r] : gg.ndivt;
+    const bool live = key_r < gg.ndivt;
+    unsigned n = 0;
+    if (live && lane < 15) {
+        const int c = lane / 3, ks = lane - 3 * c;
+        int cx, cy;
+        cell_xy(key_r, gg, cx, cy);
+        const int gx = cx + (c == 0 || c == 3 ? 0 : c == 2 ? -1 : 1), gy = cy + (c > 1 ? 1 : 0);
+        if (gx >= 0 && gx < gg.ndivx && gy < gg.ndivy && (c > 0 || ks == KIND_DUMMY)) {
+            const int *__restrict__ k0 = kstart + ks * (gg.ndivt + 1) + cell_key(gx, gy, gg);
+            const int lo = c == 0 ? r + 1 : k0[0], hi = k0[1];
+            const double2 xr = x[r];
+            const double hr = hsml[r];
+            for (int s = lo; s < hi; ++s) {
+                const double2 xs = x[s];
+                double mh;
+                n += pair_distance(xr.x - xs.x, xr.y - xs.y, hr, hsml[s], mh) < 0.0 ? 0u : 1u;
+            }
+        }
+    }
+    unsigned all = n;
+    for (int off = 8; off > 0; off >>= 1) all += __shfl_down(all, off, 16);
+    if (live && lane == 0) cnt[proc[r]] = all;
+    const int ks = lane % 3;
+    const unsigned v[3] = {ks == 0 ? n : 0u, ks == 1 ? n : 0u, ks == 2 ? n : 0u};
+    block_type_counts(v, sum, types);
+}
+
+// The same count for a tile of node (KR = 0) or stress-point (KR = 1)
+// receivers, cut as the stage kernels' are, and the tile's pair lists; with FILL, also the lists' kernel values (the
 // mixed-precision stage kernels compute them as they go).
 template <int KR, bool FILL>
-__global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double2 *__restrict__ x,
-                                                      const double *__restrict__ hsml,
-                                                      unsigned *__restrict__ cnt, PairLists PL, double h_uniform, double skin) {
+__device__ __forceinline__ void list_tile(int tile, const SearchView &V, const double2 *__restrict__ x,
+                                          const double *__restrict__ hsml, unsigned *__restrict__ cnt,
+                                          const PairLists &PL, double h_uniform, double skin) {
     __shared__ StagePlan pl[3];
     __shared__ unsigned tsum[TWAVES][3];
     constexpr const LdsLayout &LY = LAY_COUNT;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const int ltile = KR == KIND_NODE ? tile : PL.ntile_n + tile;
     const Tile T = make_tile(PL.range[ltile], KR, V, C);
     if (threadIdx.x == 0) PL.tiles[ltile] = T;
@@ -1663,6 +1660,24 @@ __global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double
         if (list_b) PL.deg_b[r] = (unsigned short)(lb.n < lmax ? lb.n : lmax);
         if (KR == KIND_NODE && PL.nodeinfo) PL.nodeinfo[r] = (int)(2u * n_node + (any_dummy ? 1u : 0u));
     }
+}
+
+// The node tiles, the stress points' and the dummies' blocks (count_blocks)
+// of a launch, longest first.  One launch: on a second stream the stress
+// points' tiles started 10 to 20 us after the event they waited for, and the
+// dummies' count came after both.
+template <bool FILL>
+__global__ __launch_bounds__(TILE) void k_count_lists(SearchView V, const double2 *__restrict__ x,
+                                                      const double *__restrict__ hsml, unsigned *__restrict__ cnt,
+                                                      PairLists PL, double h_uniform, double skin, int ntile_s, int nt,
+                                                      int nt2) {
+    const int b = blockIdx.x, bs = b - PL.ntile_n, bd = bs - ntile_s;
+    if (bs < 0)
+        list_tile<KIND_NODE, FILL>(tile_index(b, PL.ntile_n), V, x, hsml, cnt, PL, h_uniform, skin);
+    else if (bd < 0)
+        list_tile<KIND_SP, FILL>(tile_index(bs, ntile_s), V, x, hsml, cnt, PL, h_uniform, skin);
+    else
+        count_dummies(bd, x, hsml, V, cnt, PL.types + 3 * ((size_t)PL.ntile_n + ntile_s + bd), nt, nt2);
 }
 
 // The lists into the order in which the reference's linked list holds the
@@ -1843,14 +1858,12 @@ __device__ __forceinline__ bool needs_split(const Tile &T, const SearchView &V, 
 // (3_...:1847-1863) the stress points' plastic strain still waits for (it was
 // read by the node side of the last stage beside k_sp_update, which applies
 // it in its own update after this kernel).
-__global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, PairLists PL, int adapt,
-                                                    double tanfi, double coh, int nn,
-                                                    const double4 *__restrict__ sp_in,
-                                                    const double *__restrict__ dd, double dt) {
+__device__ __forceinline__ void spu_nodes_tile(int tile, const StateBufs &S, const SearchView &V, const PairLists &PL,
+                                               int adapt, double tanfi, double coh, const double4 *__restrict__ sp_in,
+                                               const double *__restrict__ dd, double dt) {
     __shared__ StagePlan pl;
     constexpr const LdsLayout &LY = LAY_SPU_NODES;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const Tile T = PL.tiles[tile];
     if (T.first >= T.end) return;
     const int r = T.first + (int)threadIdx.x;
@@ -1922,6 +1935,13 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, P
     material_tc(S, r, tanfi, coh);
     if (adapt) adapt_stress(s, tanfi, coh);
     S.stress[r] = s;
+}
+
+__global__ __launch_bounds__(TILE) void k_spu_nodes(StateBufs S, SearchView V, PairLists PL, int adapt,
+                                                    double tanfi, double coh, int nn,
+                                                    const double4 *__restrict__ sp_in,
+                                                    const double *__restrict__ dd, double dt) {
+    spu_nodes_tile(tile_index(), S, V, PL, adapt, tanfi, coh, sp_in, dd, dt);
 }
 
 // The end of get_derivatives for stress point r (CSPM correction, div1,
@@ -2008,15 +2028,13 @@ __device__ __forceinline__ void sp_stage_tail(const DevParams &P, const StateBuf
 // stress_point_update can read the stresses before it at the same time).
 // dd (the update after the RK stages): update_strain's plastic strain rates,
 // applied here.
-__global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S, Work W, SearchView V, PairLists PL,
-                                                    DevParams P, double time_sph, StageStep Q, int deriv,
-                                                    int adapt, int nn, int nt, double4 *__restrict__ sig_out,
-                                                    const double *__restrict__ dd, double dt,
-                                                    int *__restrict__ err) {
+__device__ __forceinline__ void sp_update_tile(int tile, const StateBufs &S, const Work &W, const SearchView &V,
+                                               const PairLists &PL, const DevParams &P, double time_sph,
+                                               const StageStep &Q, int deriv, int adapt, double4 *__restrict__ sig_out,
+                                               const double *__restrict__ dd, double dt, int *__restrict__ err) {
     __shared__ StagePlan pl[2];
     constexpr const LdsLayout &LY = LAY_SP_UPDATE;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const int ltile = PL.ntile_n + tile;
     const Tile T = PL.tiles[ltile];
     if (T.first >= T.end) return;
@@ -2169,6 +2187,14 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S,
                                                  xr, hr, KIND_SP, r, rev_g, C.any_fwd, V.pi, cls, grad);
     }
     sp_stage_tail(Pm, S, W, r, st, g00, g01, g10, g11, A0, A1, A2, A3, time_sph, Q, adapt, err);
+}
+
+__global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update(StateBufs S, Work W, SearchView V, PairLists PL,
+                                                    DevParams P, double time_sph, StageStep Q, int deriv,
+                                                    int adapt, int nn, int nt, double4 *__restrict__ sig_out,
+                                                    const double *__restrict__ dd, double dt,
+                                                    int *__restrict__ err) {
+    sp_update_tile(tile_index(), S, W, V, PL, P, time_sph, Q, deriv, adapt, sig_out, dd, dt, err);
 }
 
 // boundary_forces for one node: the nonzero terms of its inner-layer dummies
@@ -2421,12 +2447,11 @@ __global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_deriv_nodes(StateBufs 
 // accumulates them, written to av_out for k_deriv_nodes.  It reads only node
 // data that the stress points' update leaves alone, so the RK stages run it
 // beside k_sp_update.
-__global__ __launch_bounds__(TILE) void k_av_nodes(StateBufs S, SearchView V, PairLists PL, DevParams P,
-                                                   float2 *__restrict__ av_out, int nn) {
+__device__ __forceinline__ void av_nodes_tile(int tile, const StateBufs &S, const SearchView &V, const PairLists &PL,
+                                              const DevParams &P, float2 *__restrict__ av_out) {
     __shared__ StagePlan pl[2];
     constexpr const LdsLayout &LY = LAY_AV_NODES;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const Tile T = PL.tiles[tile];
     if (T.first >= T.end) return;
     const int r = T.first + (int)threadIdx.x;
@@ -2500,6 +2525,11 @@ __global__ __launch_bounds__(TILE) void k_av_nodes(StateBufs S, SearchView V, Pa
         }
     }
     if (active) av_out[r] = make_float2(ax, ay);
+}
+
+__global__ __launch_bounds__(TILE) void k_av_nodes(StateBufs S, SearchView V, PairLists PL, DevParams P,
+                                                   float2 *__restrict__ av_out, int nn) {
+    av_nodes_tile(tile_index(), S, V, PL, P, av_out);
 }
 
 // XSPH_update (2_...:189-239) for the receivers of kind KR: the list-order
@@ -2577,8 +2607,7 @@ __global__ __launch_bounds__(TILE) void k_xsph(StateBufs S, SearchView V, PairLi
 
 // The type-6 loop of get_derivatives overwrites each dummy's stress with
 // that of its node partners in list order (2_...:580); the last one stays.
-__global__ void k_dummy_stress(StateBufs S, SearchView V, int nt, int nt2) {
-    int r = nt + blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void dummy_stress(int r, const StateBufs &S, const SearchView &V, int nt2) {
     if (r >= nt2) return;
     const WalkCtx C = walk_ctx(V);
     const int key_r = V.cell[r];
@@ -2592,6 +2621,38 @@ __global__ void k_dummy_stress(StateBufs S, SearchView V, int nt, int nt2) {
                             KIND_DUMMY, r, C.any_fwd ? check : C.any_rev, C.any_fwd, V.pi, cls,
                             [&](auto, const auto &, int j, float, float, float) { last = j; });
     if (last >= 0) S.stress[r] = S.stress[last];
+}
+
+__global__ void k_dummy_stress(StateBufs S, SearchView V, int nt, int nt2) {
+    dummy_stress(nt + (int)(blockIdx.x * blockDim.x + threadIdx.x), S, V, nt2);
+}
+
+// A stage's independent passes in one launch, the longest first: the stress
+// points' update and derivative beside the nodes' half of stress_point_update
+// (SPU), or beside the nodes' artificial viscosity and, in the last stage, the
+// wall particles' stresses (nt2 > nt).  What makes them independent: the node
+// half reads the stress points' stresses of the stage, of which sp_update
+// writes the next in another buffer, and changes node velocities only where no
+// stress point reads them; the viscosity reads node data alone.
+// On two streams ordered by events each stage lost about 20 us to the events
+// on a small body, as much as it won by running them side by side (10 k
+// collapse 419 us per step with two streams, 415 with every pass on one, 315
+// with this and the list build's one launch; 2 M slope 2.30 -> 2.20 ms).
+template <bool SPU>
+__global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update_beside(StateBufs S, Work W, SearchView V,
+                                                    PairLists PL, DevParams P, double time_sph, StageStep Q, int adapt,
+                                                    int ntile_s, double4 *__restrict__ sig_out,
+                                                    float2 *__restrict__ av_out, int nt, int nt2,
+                                                    int *__restrict__ err) {
+    const int b = blockIdx.x, bn = b - ntile_s, bd = bn - PL.ntile_n;
+    if (bn < 0)
+        sp_update_tile(tile_index(b, ntile_s), S, W, V, PL, P, time_sph, Q, 1, adapt, sig_out, nullptr, 0.0, err);
+    else if (SPU)
+        spu_nodes_tile(tile_index(bn, PL.ntile_n), S, V, PL, adapt, P.tanfi, P.coh, Q.sp_in, nullptr, 0.0);
+    else if (bd < 0)
+        av_nodes_tile(tile_index(bn, PL.ntile_n), S, V, PL, P, av_out);
+    else
+        dummy_stress(nt + bd * TILE + (int)threadIdx.x, S, V, nt2);
 }
 
 // End of RK4 (2_...:784-799) and update_strain (3_...:1847-1863) of the steps

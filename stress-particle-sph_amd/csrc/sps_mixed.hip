@@ -207,14 +207,13 @@ __device__ __forceinline__ float2 to_rel(double2 x, double2 o) { return rel_pos(
 
 // ------------------------------------------------------------------ kernels
 // stress_point_update for node receivers (as k_spu_nodes).
-__global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView V, PairLists PL, int adapt,
-                                                        double tanfi, double coh, float hu, int nn,
-                                                        const double4 *__restrict__ sp_in,
-                                                        const double *__restrict__ dd, double dt) {
+__device__ __forceinline__ void spu_nodes_tile_mix(int tile, const StateBufs &S, const SearchView &V,
+                                                   const PairLists &PL, int adapt, double tanfi, double coh, float hu,
+                                                   const double4 *__restrict__ sp_in, const double *__restrict__ dd,
+                                                   double dt) {
     __shared__ StagePlan pl;
     constexpr const LdsLayout &LY = LAY_SPU_NODES_MIX;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const Tile T = PL.tiles[tile];
     if (T.first >= T.end) return;
     const int r = T.first + (int)threadIdx.x;
@@ -296,22 +295,26 @@ __global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView 
     S.stress[r] = s;
 }
 
+__global__ __launch_bounds__(TILE) void k_spu_nodes_mix(StateBufs S, SearchView V, PairLists PL, int adapt,
+                                                        double tanfi, double coh, float hu, int nn,
+                                                        const double4 *__restrict__ sp_in,
+                                                        const double *__restrict__ dd, double dt) {
+    spu_nodes_tile_mix(tile_index(), S, V, PL, adapt, tanfi, coh, hu, sp_in, dd, dt);
+}
+
 // Stress-point receivers (as k_sp_update).
-// stepv (a captured step): time_sph from stepv[0] instead of the argument.
+// stepv (a captured step) in the kernels: time_sph from stepv[0] instead of
+// the argument.
 // sig_out: where the stress after the return map goes (null: the state's
 // stress), as in k_sp_update.
-__global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, SearchView V, PairLists PL,
-                                                        DevParams P, double time_sph, StageStep Q, int deriv,
-                                                        int adapt, float hu, int nn, int nt,
-                                                        const double *__restrict__ stepv,
-                                                        double4 *__restrict__ sig_out,
-                                                        const double *__restrict__ dd, double dt,
-                                                        int *__restrict__ err) {
-    if (stepv) time_sph = stepv[0];
+__device__ __forceinline__ void sp_update_tile_mix(int tile, const StateBufs &S, const Work &W, const SearchView &V,
+                                                   const PairLists &PL, const DevParams &P, double time_sph,
+                                                   const StageStep &Q, int deriv, int adapt, float hu,
+                                                   double4 *__restrict__ sig_out, const double *__restrict__ dd,
+                                                   double dt, int *__restrict__ err) {
     __shared__ StagePlan pl[2];
     constexpr const LdsLayout &LY = LAY_SP_UPDATE_MIX;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const int ltile = PL.ntile_n + tile;
     const Tile T = PL.tiles[ltile];
     if (T.first >= T.end) return;
@@ -466,6 +469,17 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
                   A3.get(), time_sph, Q, adapt, err);
 }
 
+__global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, SearchView V, PairLists PL,
+                                                        DevParams P, double time_sph, StageStep Q, int deriv,
+                                                        int adapt, float hu, int nn, int nt,
+                                                        const double *__restrict__ stepv,
+                                                        double4 *__restrict__ sig_out,
+                                                        const double *__restrict__ dd, double dt,
+                                                        int *__restrict__ err) {
+    if (stepv) time_sph = stepv[0];
+    sp_update_tile_mix(tile_index(), S, W, V, PL, P, time_sph, Q, deriv, adapt, hu, sig_out, dd, dt, err);
+}
+
 // artificial_viscosity (2_...:826-904) of the node receivers in the mixed
 // form: node partners (list B) with kernel values computed in single
 // precision from window-relative positions, and compensated sums; rounded
@@ -473,12 +487,12 @@ __global__ __launch_bounds__(TILE) void k_sp_update_mix(StateBufs S, Work W, Sea
 // k_deriv_nodes_mix.  It reads only node data that the stress points' update
 // leaves alone, so the RK stages run it beside k_sp_update_mix, and it ends
 // before k_deriv_nodes_mix writes the next stage's velocities.
-__global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V, PairLists PL, DevParams P,
-                                                       float hu, float2 *__restrict__ av_out, int nn) {
+__device__ __forceinline__ void av_nodes_tile_mix(int tile, const StateBufs &S, const SearchView &V,
+                                                  const PairLists &PL, const DevParams &P, float hu,
+                                                  float2 *__restrict__ av_out) {
     __shared__ StagePlan pl;
     constexpr const LdsLayout &LY = LAY_AV_NODES_MIX;
     const WalkCtx C = walk_ctx(V);
-    const int tile = tile_index();
     const Tile T = PL.tiles[tile];
     if (T.first >= T.end) return;
     const int r = T.first + (int)threadIdx.x;
@@ -544,6 +558,32 @@ __global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V
                                     false, true, V.pi, NoClass{}, av);
     }
     if (active) av_out[r] = make_float2((float)ax.get(), (float)ay.get());
+}
+
+__global__ __launch_bounds__(TILE) void k_av_nodes_mix(StateBufs S, SearchView V, PairLists PL, DevParams P,
+                                                       float hu, float2 *__restrict__ av_out, int nn) {
+    av_nodes_tile_mix(tile_index(), S, V, PL, P, hu, av_out);
+}
+
+// A stage's independent passes in one launch (as k_sp_update_beside).
+template <bool SPU>
+__global__ __launch_bounds__(TILE) STAGE_OCCUPANCY void k_sp_update_beside_mix(StateBufs S, Work W, SearchView V, PairLists PL,
+                                                               DevParams P, double time_sph, StageStep Q, int adapt,
+                                                               float hu, int ntile_s, const double *__restrict__ stepv,
+                                                               double4 *__restrict__ sig_out,
+                                                               float2 *__restrict__ av_out, int nt, int nt2,
+                                                               int *__restrict__ err) {
+    if (stepv) time_sph = stepv[0];
+    const int b = blockIdx.x, bn = b - ntile_s, bd = bn - PL.ntile_n;
+    if (bn < 0)
+        sp_update_tile_mix(tile_index(b, ntile_s), S, W, V, PL, P, time_sph, Q, 1, adapt, hu, sig_out, nullptr, 0.0,
+                           err);
+    else if (SPU)
+        spu_nodes_tile_mix(tile_index(bn, PL.ntile_n), S, V, PL, adapt, P.tanfi, P.coh, hu, Q.sp_in, nullptr, 0.0);
+    else if (bd < 0)
+        av_nodes_tile_mix(tile_index(bn, PL.ntile_n), S, V, PL, P, hu, av_out);
+    else
+        dummy_stress(nt + bd * TILE + (int)threadIdx.x, S, V, nt2);
 }
 
 // Node receivers (as k_deriv_nodes).
