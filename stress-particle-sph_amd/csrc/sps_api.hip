@@ -978,14 +978,14 @@ static int free_surface(sps_handle *h, const StateBufs &SB) {
     // entries kept per particle: as many as its two pair lists hold; a body on
     // its lattice has about 36 with one stress point a cell
     const int cap = 4 * h->list_words;
-    const size_t ne = (size_t)nblk(nt) * BLOCK * cap;
+    const size_t ne = (size_t)nt * cap;
     int rc = 0;
     rc |= dalloc(h->surf_n, nt) | dalloc(h->surf_ent, ne) | dalloc(h->surf_hf, ne);
     rc |= dalloc(h->surf_flag, nt) | dalloc(h->surf_sub, nt);
     if (rc) return rc;
     const SearchView V{h->cell.p, h->kstart.p, h->proc.p, h->cnt.p, h->off.p, h->grid.p, h->split.p, h->p.pi};
     const SurfBufs B{h->surf_n.p, h->surf_ent.p, h->surf_hf.p, cap, h->surf_flag.p, h->surf_sub.p};
-    LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_a, SB, h->x0.p, V, B, h->bc_or_not.p, h->xsph ? 1 : 0, nn, nt);
+    LAUNCH(K_SURF, nblk((long long)nt * SURF_LANES), BLOCK, k_count_surface, SB, h->x0.p, V, B, h->bc_or_not.p, h->xsph ? 1 : 0, nn, nt);
     LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_sub, SB, B, h->bc_or_not.p, nt);
     LAUNCH(K_SURF, nblk(nt), BLOCK, k_surf_b, SB, h->x0.p, V, B, h->normal.p, nn, nt);
     HIP_TRY(hipGetLastError());

@@ -2869,7 +2869,7 @@ __global__ void k_bcint_keep(const int *__restrict__ nodeinfo, const int *__rest
 // took 1.1 ms of a 1.6 ms step on the 100 k localisation test.
 struct SurfBufs {
     int *n;          // per particle: its pairs of types 1-3
-    unsigned *ent;   // [block][cap][BLOCK]: partner slot, bit 31: the particle is pair_j
+    unsigned *ent;   // [particle][cap], in list order: partner slot, bit 31: the particle is pair_j
     float2 *hf;      // m_p / rho_p dW of the entry, the reference's hf1 / hf2 of that end
     int cap;         // entries kept per particle (step 4 walks again where there are more)
     unsigned *flag;  // step 3: a partner in the scan region (f_int = -1)
@@ -2930,43 +2930,196 @@ __device__ __forceinline__ bool surf_hit(double2 xr, double hr, double2 n, float
 // a free-surface node among its node partners becomes 3, so the detection
 // resets even a prescribed node to 0 (concurrent marks cannot change any
 // test's outcome: they only turn a value other than 2 into 3).
-__global__ __launch_bounds__(BLOCK) void k_surf_a(StateBufs S, const double2 *__restrict__ x0, SearchView V,
-                                                  SurfBufs B, int *__restrict__ bc_or_not, int mark, int nn, int nt) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nt) return;
+//
+// SURF_LANES lanes a particle: lane c finds the pairs of the c-th row of three
+// cells, whose number gives each lane its partners' places in the list order;
+// the entries, with their kernel values and two divisions each, are then dealt
+// out evenly; the renormalisation's sums, whose terms have to be added in that
+// order, are spread over the lanes, and so is the test.  One lane walking all
+// nine cells tested about a hundred candidates one after the other, 286 us on
+// 60 k particles and 230 us on 100 k; a lane a cell, or a row, making the
+// entries it found took 176 to 223 us, most of it arithmetic of lanes waiting
+// for the longest cell; this 103 and 118 us.
+constexpr int SURF_LANES = 4;
+constexpr int SURF_LDS = 96;   // partners of a particle held in LDS; with more its sums walk the cells
+__global__ __launch_bounds__(BLOCK) void k_count_surface(StateBufs S, const double2 *__restrict__ x0, SearchView V,
+                                                         SurfBufs B, int *__restrict__ bc_or_not, int mark, int nn,
+                                                         int nt) {
+    __shared__ int sj[BLOCK / SURF_LANES][SURF_LDS];
+    int *const lj = sj[threadIdx.x / SURF_LANES];
+    const int lane = threadIdx.x & (SURF_LANES - 1);
+    const int r = blockIdx.x * (BLOCK / SURF_LANES) + (int)(threadIdx.x / SURF_LANES);
+    const bool live = r < nt;
+    const int rl = live ? r : 0;   // a valid slot for the idle lanes' loads
     const WalkCtx C = walk_ctx(V);
     const SearchFields A{x0, S.x, S.hsml, nt};
-    const int kr = kind_of(r, nn, nt);
-    const double2 xr = S.x[r];
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, f0 = 0.f, f1 = 0.f;
-    int n = 0;
-    bool by_surface = false;
-    const size_t at = (size_t)blockIdx.x * B.cap * BLOCK + threadIdx.x;
-    surf_walk<MASK_NODE | MASK_SP>(V, C, A, r, kr, [&](int p, float gx, float gy) {
-        unsigned e;
-        float2 h;
-        const int kp = kind_of(p, nn, nt);
-        surf_entry(S, V, r, kr, p, kp, gx, gy, e, h);
-        if (n < B.cap) {
-            B.ent[at + (size_t)n * BLOCK] = e;
-            B.hf[at + (size_t)n * BLOCK] = h;
+    const int kr = kind_of(rl, nn, nt);
+    const double2 xs = A.xk(kr, rl), xr = S.x[rl];
+    const double hr = S.hsml[rl];
+    const int key = live ? V.cell[r] : C.g.ndivt;
+    const bool inside = key < C.g.ndivt;
+    const bool check = inside && C.mixed && V.proc[rl] >= C.sp.first_rev;
+    const SplitClass cls{check, check ? V.proc[rl] : 0, V.proc, V.cnt, V.off, C.sp};
+    const bool do_rev = C.any_fwd ? check : C.any_rev, do_fwd = C.any_fwd;
+    // the slots of this lane's cells, by kind
+    int lo[3][3], cnt[3][3];
+    {
+        int cx = 0, cy = 0;
+        if (inside) cell_xy(key, C.g, cx, cy);
+        cy += lane - 1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int gx = cx + c - 1;
+            const bool in = inside && lane < 3 && gx >= 0 && gx < C.g.ndivx && cy >= 0 && cy < C.g.ndivy;
+            const int ckey = in ? cell_key(gx, cy, C.g) : 0;
+#pragma unroll
+            for (int K = 0; K < 3; ++K) {
+                lo[c][K] = in ? V.kstart[K * C.L + ckey] : 0;
+                cnt[c][K] = in ? V.kstart[K * C.L + ckey + 1] - lo[c][K] : 0;
+            }
         }
-        ++n;
-        if (mark && kr == KIND_NODE && kp == KIND_NODE) by_surface = by_surface || bc_or_not[S.orig[p]] == 2;
-        const double2 xp = S.x[p];
-        const double d0 = xp.x - xr.x, d1 = xp.y - xr.y;
-        a0 = (float)((double)a0 + d0 * (double)h.x);
-        f0 = f0 + h.x;
-        a1 = (float)((double)a1 + d1 * (double)h.x);
-        a2 = (float)((double)a2 + d0 * (double)h.y);
-        a3 = (float)((double)a3 + d1 * (double)h.y);
-        f1 = f1 + h.y;
-    });
-    B.n[r] = n;
+    }
+    // the particle's pairs with the partners of a kind in a cell, slots
+    // ascending, four positions in flight: f(slot, place in the cell)
+    auto pairs = [&](int K, int first, int n, auto &&f) __attribute__((always_inline)) {
+        for (int q0 = 0; q0 < n; q0 += 4) {
+            double2 xp[4];
+            double hp[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int j = first + min(q0 + i, n - 1);
+                xp[i] = A.xk(K, j);
+                hp[i] = A.hk(K, j);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (q0 + i < n && first + q0 + i != r &&
+                    accepted_by(xs.x - xp[i].x, xs.y - xp[i].y, accept_bounds(hr, hp[i])))
+                    f(first + q0 + i, q0 + i);
+        }
+    };
+    // which of the cells' nodes and stress points are partners, by place, of
+    // the reversed pairs and the others (a cell of more than 32 of a kind: the
+    // whole particle is left to the serial walk)
+    unsigned rev[3][2], fwd[3][2];
+    int n_rev = 0, n_fwd = 0, over = 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int K = KIND_NODE; K <= KIND_SP; ++K) {
+            unsigned b = 0, f = 0;
+            if (cnt[c][K] > 32) over = 1;
+            else
+                pairs(K, lo[c][K], cnt[c][K], [&](int j, int q) {
+                    if (do_rev && cls(j, true)) b |= 1u << q;
+                    if (do_fwd && cls(j, false)) f |= 1u << q;
+                });
+            rev[c][K] = b;
+            fwd[c][K] = f;
+            n_rev += __popcll(b);
+            n_fwd += __popcll(f);
+        }
+    // first the reversed pairs, cells descending, then the others
+    int up_fwd = n_fwd, up_rev = n_rev;
+    for (int o = 1; o < SURF_LANES; o <<= 1) {
+        const int f = __shfl_up(up_fwd, o, SURF_LANES), b = __shfl_up(up_rev, o, SURF_LANES),
+                  v = __shfl_up(over, o, SURF_LANES);
+        if (lane >= o) {
+            up_fwd += f;
+            up_rev += b;
+            over |= v;
+        }
+    }
+    const int all_rev = __shfl(up_rev, SURF_LANES - 1, SURF_LANES);
+    int n = all_rev + __shfl(up_fwd, SURF_LANES - 1, SURF_LANES);
+    const bool kept = !__shfl(over, SURF_LANES - 1, SURF_LANES) && n <= min(B.cap, SURF_LDS);
+    bool by_surface = false;
+    const size_t at = (size_t)rl * B.cap;
+    if (kept) {
+        int place = all_rev - up_rev;
+        if (do_rev)
+#pragma unroll
+            for (int c = 2; c >= 0; --c)
+#pragma unroll
+                for (int K = KIND_SP; K >= KIND_NODE; --K)
+                    for (unsigned long long m = rev[c][K]; m;) {
+                        const int q = 63 - __clzll((long long)m);
+                        m &= ~(1ull << q);
+                        lj[place++] = lo[c][K] + q;
+                    }
+        place = all_rev + up_fwd - n_fwd;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int K = KIND_NODE; K <= KIND_SP; ++K)
+                for (unsigned long long m = fwd[c][K]; m; m &= m - 1) lj[place++] = lo[c][K] + __ffsll(m) - 1;
+    }
+    __syncthreads();
+    if (kept) {
+        KernelFactor kf;
+        for (int k = lane; k < n; k += SURF_LANES) {
+            const int j = lj[k], kp = kind_of(j, nn, nt);
+            if (mark && kr == KIND_NODE && kp == KIND_NODE) by_surface = by_surface || bc_or_not[S.orig[j]] == 2;
+            const double2 xp = A.xk(kp, j);
+            const double dx0 = xs.x - xp.x, dx1 = xs.y - xp.y;
+            double mh;
+            const double rr = pair_distance(dx0, dx1, hr, A.hk(kp, j), mh);
+            float w, gx, gy;
+            cubic_kernel_f(rr, dx0, dx1, mh, kf.get(mh, V.pi), w, gx, gy);
+            unsigned e;
+            float2 h;
+            surf_entry(S, V, r, kr, j, kp, gx, gy, e, h);
+            B.ent[at + k] = e;
+            B.hf[at + k] = h;
+        }
+    }
+    __syncthreads();
+    // lane 2 i + k: the sums of d_k hf_i and of hf_i
+    float a = 0.f, f = 0.f;
+    auto term = [&](double2 xp, float2 h) {
+        const float hv = lane & 2 ? h.y : h.x;
+        a = (float)((double)a + (lane & 1 ? xp.y - xr.y : xp.x - xr.x) * (double)hv);
+        f = f + hv;
+    };
+    if (kept) {
+        for (int k0 = 0; k0 < n; k0 += 8) {   // eight entries in flight
+            double2 xp[8];
+            float2 h[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int k = min(k0 + i, n - 1);
+                xp[i] = S.x[lj[k]];
+                h[i] = B.hf[at + k];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (k0 + i < n) term(xp[i], h[i]);
+        }
+    } else {   // each lane walks the cells itself; the first keeps what fits
+        n = 0;
+        surf_walk<MASK_NODE | MASK_SP>(V, C, A, rl, kr, [&](int p, float gx, float gy) {
+            unsigned e;
+            float2 h;
+            const int kp = kind_of(p, nn, nt);
+            surf_entry(S, V, rl, kr, p, kp, gx, gy, e, h);
+            if (lane == 0) {
+                if (mark && kr == KIND_NODE && kp == KIND_NODE) by_surface = by_surface || bc_or_not[S.orig[p]] == 2;
+                if (n < B.cap) {
+                    B.ent[at + n] = e;
+                    B.hf[at + n] = h;
+                }
+            }
+            term(S.x[p], h);
+            ++n;
+        });
+    }
     if (by_surface) {
         const int o = S.orig[r];
         if (bc_or_not[o] != 2) bc_or_not[o] = 3;
     }
+    float a0 = __shfl(a, 0, SURF_LANES), a1 = __shfl(a, 1, SURF_LANES), a2 = __shfl(a, 2, SURF_LANES),
+          a3 = __shfl(a, 3, SURF_LANES);
+    const float f0 = __shfl(f, 0, SURF_LANES), f1 = __shfl(f, 2, SURF_LANES);
     if (fabsf(a0) <= 1.e-8f) a0 = 0.f;
     if (fabsf(a1) <= 1.e-8f) a1 = 0.f;
     if (fabsf(a2) <= 1.e-8f) a2 = 0.f;
@@ -2974,26 +3127,30 @@ __global__ __launch_bounds__(BLOCK) void k_surf_a(StateBufs S, const double2 *__
     const float v1 = -(a0 * f0 + a1 * f1), v2 = -(a2 * f0 + a3 * f1);
     const float v3 = sqrtf(v1 * v1 + v2 * v2);
     const double n0 = (double)(v1 / v3), n1 = (double)(v2 / v3);
-    const double hr = S.hsml[r];
     const double2 nrm = make_double2(n0, n1);
     const float2 tt = make_float2((float)(xr.x + hr * n0), (float)(xr.y + hr * n1));
     const float2 tau = make_float2((float)(-n1), (float)n0);
     // node pairs and stress-point pairs test both ends, dummy pairs their
     // non-dummy end; the outcome does not depend on the order
     bool hit = false;
-    auto test = [&](int p) { hit = hit || surf_hit(xr, hr, nrm, tt, tau, S.x[p]); };
-    if (n <= B.cap) {
-        for (int k = 0; k < n && !hit; ++k) {
-            const int p = (int)(B.ent[at + (size_t)k * BLOCK] & 0x7fffffffu);
-            if (kind_of(p, nn, nt) == kr) test(p);
-        }
+    auto test = [&](int j, int) { hit = hit || surf_hit(xr, hr, nrm, tt, tau, S.x[j]); };
+    if (kept) {
+        for (int k = lane; k < n && !hit; k += SURF_LANES)
+            if (kind_of(lj[k], nn, nt) == kr) test(lj[k], 0);
     } else {
-        surf_walk<MASK_NODE | MASK_SP>(V, C, A, r, kr, [&](int p, float, float) {
-            if (kind_of(p, nn, nt) == kr) test(p);
-        });
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int K = KIND_NODE; K <= KIND_SP; ++K)
+                if (K == kr) pairs(K, lo[c][K], cnt[c][K], test);
     }
-    if (!hit) surf_walk<MASK_DUMMY>(V, C, A, r, kr, [&](int p, float, float) { test(p); });
-    B.flag[r] = hit ? 1u : 0u;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) pairs(KIND_DUMMY, lo[c][KIND_DUMMY], cnt[c][KIND_DUMMY], test);
+    for (int o = SURF_LANES / 2; o > 0; o >>= 1) hit = __shfl_down((int)hit, o, SURF_LANES) || hit;
+    if (live && lane == 0) {
+        B.n[r] = n;
+        B.flag[r] = hit ? 1u : 0u;
+    }
 }
 
 // 3_...:1321-1349: subsets and BC_or_not (2 on the surface, 0 inside, 1 kept)
@@ -3040,8 +3197,9 @@ __global__ __launch_bounds__(BLOCK) void k_surf_b(StateBufs S, const double2 *__
         };
         const int n = B.n[r];
         if (n <= B.cap) {
-            const size_t at = (size_t)blockIdx.x * B.cap * BLOCK + threadIdx.x;
-            for (int k = 0; k < n; ++k) add(B.ent[at + (size_t)k * BLOCK], B.hf[at + (size_t)k * BLOCK]);
+            const size_t at = (size_t)r * B.cap;
+#pragma unroll 4
+            for (int k = 0; k < n; ++k) add(B.ent[at + k], B.hf[at + k]);
         } else {
             const WalkCtx C = walk_ctx(V);
             const int kr = kind_of(r, nn, nt);

@@ -130,3 +130,30 @@ def test_search_on_stretched_grids(cells):
         gpu.step(1)
         ora.step(1)
         compare(gpu, ora, f"{cells} cells, step {step}")
+
+
+# The free surface: four lanes share a particle's pairs in list order.  Few and
+# many partners (over the 96 held in LDS, over 32 of a kind in a cell: then a
+# lane walks them all), particles on both sides of the list's high-water mark,
+# a body of fewer particles than a block.
+@pytest.mark.parametrize("deck_name,nx,ny,change", [
+    ("c1_collapse", 5, 3, {}), ("c1_collapse", 65, 33, {}), ("c1_collapse", 40, 40, {"sml": 2.4}),
+    ("c1_collapse", 40, 30, {"sml": 3.4}), ("t5_sp4", 30, 30, {}), ("t4_xsph", 33, 47, {"npoints": 2})])
+def test_surface_against_oracle(deck_name, nx, ny, change):
+    sps = load_pkg()
+    deck = dataclasses.replace(sps.read_deck(deck_dir(deck_name)), **change)
+    deck.xs = (0.0, (nx - 0.5) * deck.dx, 0.0, (nx - 0.5) * deck.dx)
+    deck.ys = (0.0, 0.0, (ny - 0.5) * deck.dx, (ny - 0.5) * deck.dx)
+    deck.dy = deck.dx
+    gpu = sps.Simulation.from_deck(deck)
+    ora = sps.Simulation.from_deck(deck, lib_path=ORACLE_LIB)
+    st = sps.initial_state(gpu.parts, gpu.niv)
+    st["vel"][:gpu.n] = 2.0 * np.random.default_rng(3).standard_normal((gpu.n, 2))
+    for sim in (gpu, ora):
+        sim.set_state(st)
+    print(f"[surface] {deck_name} {nx} x {ny} {change}", flush=True)
+    for step in range(1, 5):
+        gpu.step(1)
+        ora.step(1)
+        for what, a, b in zip(("bc_or_not", "normal"), ora.get_surface(), gpu.get_surface()):
+            assert bits_equal(a, b), f"step {step}: {what}"
