@@ -368,7 +368,8 @@ static size_t lds_count(const sps_handle *h) {
 template <typename In>
 static int scan_u32(sps_handle *h, In in, unsigned *out, long long n, unsigned long long *dtotal,
                     ScanCount sc = ScanCount{nullptr, 0, 0}) {
-    const long long nb = std::max(1ll, (n + SCAN_TILE - 1) / SCAN_TILE);
+    constexpr int TILE_ITEMS = BLOCK * In::ITEMS;
+    const long long nb = std::max(1ll, (n + TILE_ITEMS - 1) / TILE_ITEMS);
     if ((size_t)nb > h->scan_state.n) return fail(SPS_ECAPACITY, "scan of %lld values", n);
     if (++h->scan_epoch >= SCAN_EPOCHS) {   // the numbers of earlier launches come again
         HIP_TRY(hipMemsetAsync(h->scan_state.p, 0, h->scan_state.n * sizeof(unsigned long long), h->stream));
@@ -637,7 +638,9 @@ static int size_cells(sps_handle *h, const double *hsml) {
     rc |= dalloc(h->kcount, L); rc |= dalloc(h->kstart, L); rc |= dalloc(h->kfill, L);
     rc |= dalloc(h->cstart_rm, (size_t)cap + 2);
     // tiles of the largest scan of a step (the bucket counts or the slots)
-    rc |= dalloc(h->scan_state, std::max(L, (size_t)h->nt2 + 1) / SCAN_TILE + 2) | dalloc(h->scan_ticket, 1);
+    const size_t st = std::max(std::max(L, (size_t)h->nt2 + 1) / (BLOCK * ScanArray::ITEMS),
+                               ((size_t)cap + 1) / (BLOCK * ScanCells::ITEMS)) + 2;
+    rc |= dalloc(h->scan_state, st) | dalloc(h->scan_ticket, 1);
     if (rc) return rc;
     // a search clears the counters it has used for the next one
     HIP_TRY(hipMemsetAsync(h->kcount.p, 0, h->kcount.n * sizeof(int), h->stream));

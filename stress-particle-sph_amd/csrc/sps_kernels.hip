@@ -317,12 +317,15 @@ __device__ __forceinline__ void cell_sort(const int *__restrict__ kstart, int *_
 }
 
 // What a scan adds up: an array, or the particles per cell in the
-// reference's row-major visiting order.
+// reference's row-major visiting order (fewer values a lane: each takes two
+// divisions and six loads).
 struct ScanArray {
+    static constexpr int ITEMS = 16;
     const unsigned *in;
     __device__ __forceinline__ unsigned operator()(long long i) const { return in[i]; }
 };
 struct ScanCells {
+    static constexpr int ITEMS = 4;
     const int *kstart;
     const Grid *g;
     __device__ __forceinline__ unsigned operator()(long long i) const {
@@ -3437,9 +3440,13 @@ struct ScanCount {
 // back to the first published prefix; each waits only for tiles taken before
 // its own, whose blocks are running.  A tile's word holds the launch's number
 // (epoch), whether the value is the tile's sum (1) or its prefix (2), and the
-// value, so that the words need no clearing between launches.  The last block
-// to find no tile left takes the counter back to zero.
-constexpr int SCAN_ITEMS = 8, SCAN_TILE = BLOCK * SCAN_ITEMS, SCAN_BLOCKS = 1024;
+// value, so that the words need no clearing between launches.  The block with
+// the last number takes the counter back to zero.  The numbers are what a
+// scan of many tiles costs (one at a time, some 15 ns each): at most 256
+// blocks, a second number only where a block may have a second tile, tiles of
+// 4096 array elements (2048 for up to 1024 blocks: 31 us a scan at 2 M
+// particles, so 24 us).
+constexpr int SCAN_BLOCKS = 256;
 constexpr unsigned SCAN_EPOCHS = 1u << 30;
 
 template <typename In>
@@ -3448,18 +3455,19 @@ __global__ __launch_bounds__(BLOCK) void k_scan_sums(In in, unsigned *__restrict
                                                      unsigned *__restrict__ ticket, unsigned long long epoch,
                                                      unsigned long long *__restrict__ total, long long n_max,
                                                      ScanCount sc) {
+    constexpr int SCAN_ITEMS = In::ITEMS, SCAN_TILE = BLOCK * SCAN_ITEMS;
     __shared__ unsigned sh_id, sh_prefix;
     const int t = threadIdx.x, lane = t & 63;
     const long long n = sc.get(n_max);
     const unsigned nb = n > 0 ? (unsigned)((n + SCAN_TILE - 1) / SCAN_TILE) : 1u;
+    const bool once = gridDim.x >= nb;
+    const unsigned tickets = once ? gridDim.x : nb + gridDim.x;
     for (;;) {
         if (t == 0) sh_id = atomicAdd(ticket, 1u);
         __syncthreads();
         const unsigned id = sh_id;
-        if (id >= nb) {
-            if (t == 0 && id == nb + gridDim.x - 1) atomicAdd(ticket, 0u - (nb + gridDim.x));
-            return;
-        }
+        if (t == 0 && id == tickets - 1) atomicAdd(ticket, 0u - tickets);
+        if (id >= nb) return;
         const long long base = (long long)id * SCAN_TILE + (long long)t * SCAN_ITEMS;
         unsigned v[SCAN_ITEMS], s = 0;
 #pragma unroll
@@ -3500,6 +3508,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_sums(In in, unsigned *__restrict
             if (base + k < n) out[base + k] = ex;
             ex += v[k];
         }
+        if (once) return;
     }
 }
 
