@@ -50,7 +50,7 @@ static int fail(int code, const char *fmt, ...) {
 
 static inline unsigned nblk(long long n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
 // Tiles held for n receivers, a multiple of the XCD count: n / TILE rounded
-// up, and with `strips` > 0 (tiles that end at strip ends, k_count_tiles) one more
+// up, and with `strips` > 0 (tiles that end at strip ends, k_count_tiles_sort) one more
 // per strip of the domain box, at most twice as many in all.
 static inline int ntiles(long long n, double strips) {
     const long long plain = (n + TILE - 1) / TILE;
@@ -202,7 +202,7 @@ struct sps_handle {
     DBuf<Tile> tiles;
     DBuf<StagePlan> plans;
     int ntile_n = 0, ntile_s = 0;
-    DBuf<int> tile_start;         // k_count_tiles: first tile of each strip (scratch)
+    DBuf<int> tile_start;         // k_count_tiles_sort: first tile of each strip (scratch)
     DBuf<int2> tile_range;        // per tile: its receivers
     DBuf<unsigned> type_counts;   // pairs by partner kind: per tile, then per block of dummy receivers
     double h_uniform = 0.0;   // the smoothing length of every particle, or 0 when they differ
@@ -558,7 +558,7 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     rc |= dalloc(h->moved, nblk(nt2));
     rc |= dalloc(h->proc_to_slot, nt2); rc |= dalloc(h->cnt, nt2); rc |= dalloc(h->off, nt2);
     // strips of 8 cells 2h wide with h = 0.8 dx, as small as the decks have it
-    // (with smaller h and a body across the whole box k_count_tiles may not find
+    // (with smaller h and a body across the whole box k_count_tiles_sort may not find
     // room for tiles that end at strip ends and falls back)
     const double strips = h->mixed || !(params->dx > 0) ? 0.0
         : (params->xmax_domain[0] - params->xmin_domain[0]) / (STRIP * 1.6 * params->dx) + 2;

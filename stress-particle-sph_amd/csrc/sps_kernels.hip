@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(BLOCK) k_bounds_final(const double *__restrict
 // strips of STRIP cells, cells run row by row inside a strip.  Walking the
 // storage (and so the receivers) up a strip keeps the partner data of three
 // consecutive rows in one L2.  The reference's own visiting order (row-major
-// cells, 2_...:1322-1324) is kept separately for the list order (k_proc_slot).
+// cells, 2_...:1322-1324) is kept separately for the list order (proc_slot).
 constexpr int STRIP = 8;
 
 __device__ __forceinline__ int cell_key(int cx, int cy, const Grid &g) {
@@ -1313,7 +1313,7 @@ struct PairLists {
     unsigned char *ok;              // per tile (node tiles, then SP tiles): LIST_*
     int lg;                         // words per receiver and list; more entries: LIST_NONE
     int ntile_n;                    // node tiles
-    const int2 *range;              // per tile: its receivers (k_count_tiles)
+    const int2 *range;              // per tile: its receivers (k_count_tiles_sort)
     unsigned *types;                // per tile: pairs its receivers discover, by partner kind
     // each tile's extent and (when it fits) the staging plan of every partner
     // kind, as the search computed them: the stage kernels load them in one
