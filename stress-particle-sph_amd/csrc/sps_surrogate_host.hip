@@ -423,6 +423,8 @@ extern "C" int sps_set_plastic_log(sps_handle *h, int64_t cap) {
     if (!h || cap < 0 || cap > (1ll << 30)) return fail(SPS_EINVAL, "bad argument");
     if (cap > 0 && h->integrator == SPS_INTEGRATOR_LEAPFROG) return fail(SPS_EINVAL, "the log records RK4 steps");
     HIP_TRY(hipSetDevice(h->device));
+    drop_graphs(h);   // a captured step records into the log it was captured with
+    h->log_cap = 0;   // and no step into a log that could not be allocated
     int rc = dalloc(h->surr_count, 2) | dalloc(h->plog, (size_t)(cap ? cap : 1) * SPS_PLOG_ROW);
     if (rc) return rc;
     h->log_cap = (int)cap;

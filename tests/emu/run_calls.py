@@ -1,0 +1,68 @@
+"""Sequences of calls on the CPU build of the HIP kernels (run under
+AddressSanitizer by tests/test_emu_calls.py): `run_calls.py EMU_LIB NAME`.
+Prints one line; exit status 0 when the sequence gives what it should."""
+import importlib
+import os
+import sys
+
+import numpy as np
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(os.path.dirname(HERE))
+sys.path.insert(0, ROOT)
+sps = importlib.import_module("stress-particle-sph_amd")
+surrogate = importlib.import_module("stress-particle-sph_amd.surrogate")
+
+
+def deck_of(name):
+    return sps.read_deck(os.path.join(ROOT, "stress-particle-sph_amd", "decks", name))
+
+
+def equal(a, b):
+    return a.shape == b.shape and a.tobytes() == b.tobytes()
+
+
+def same_state(a, b):
+    a, b = a.get_state(), b.get_state()
+    return [k for k in a if not equal(a[k], b[k])]
+
+
+def direct_and_captured(lib, deck, parts=None):
+    """The mixed form with kept lists, launched step by step and replayed."""
+    sims = []
+    for graph in (False, True):
+        sim = sps.Simulation.from_deck(deck, lib_path=lib, mode=sps.MODE_FAST, parts=parts)
+        sim.set_list_skin(0.25 * sim.params.dx)
+        sim.set_graph(graph)
+        sims.append(sim)
+    return sims
+
+
+def plastic_log_after_capture(lib):
+    """A log set before and after a step was captured, made longer (another
+    buffer) and taken away."""
+    bad = []
+    for caps in ((None, 16, 4096, 0), (16, 4096, 0)):
+        sims = direct_and_captured(lib, deck_of("t2_cspm"))
+        for k, cap in enumerate(caps):
+            logs = []
+            for sim in sims:
+                if cap is not None:
+                    surrogate.log_plastic(sim, cap)
+                sim.step(4 if k else 12)     # the deck yields from its tenth step on
+                logs.append(surrogate.plastic_log(sim, cap or 1))
+            rows = [len(g[0]) for g in logs]
+            if rows[0] != rows[1] or any(not equal(np.sort(a, axis=0), np.sort(b, axis=0)) for a, b in zip(*logs)):
+                bad.append(f"log of {cap}: {rows[0]} rows, captured {rows[1]}")
+            if cap and not rows[0]:
+                bad.append(f"log of {cap} is empty")
+        bad += same_state(*sims)
+    return bad
+
+
+CASES = {f.__name__: f for f in (plastic_log_after_capture,)}
+
+if __name__ == "__main__":
+    bad = CASES[sys.argv[2]](sys.argv[1])
+    print(f"{sys.argv[2]}: " + ("ok" if not bad else "; ".join(bad)))
+    sys.exit(1 if bad else 0)
