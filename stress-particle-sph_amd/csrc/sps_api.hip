@@ -1207,6 +1207,7 @@ extern "C" int sps_set_bcs(sps_handle *h, const sps_bcs *b) {
             if (b->bc_info[8 * i + k] < 0 || b->bc_info[8 * i + k] > b->no_bcs)
                 return fail(SPS_EINVAL, "node %d: BC number %d of %d", i + 1, b->bc_info[8 * i + k], b->no_bcs);
     HIP_TRY(hipSetDevice(h->device));
+    drop_graphs(h);   // a captured step holds the variables it was captured with (bc_vars)
     h->nbc = b->no_bcs;
     h->ncurves = b->ncurves;
     h->bcint = b->ifsigman == 1 && h->nt2 > h->nt;

@@ -1,6 +1,7 @@
 """Sequences of calls on the CPU build of the HIP kernels (run under
 AddressSanitizer by tests/test_emu_calls.py): `run_calls.py EMU_LIB NAME`.
 Prints one line; exit status 0 when the sequence gives what it should."""
+import dataclasses
 import importlib
 import os
 import sys
@@ -60,7 +61,25 @@ def plastic_log_after_capture(lib):
     return bad
 
 
-CASES = {f.__name__: f for f in (plastic_log_after_capture,)}
+def prescribed_values_after_capture(lib):
+    """Other prescribed variables (the components exchanged) after a step was captured."""
+    deck = deck_of("l1_localisation")
+    sims = direct_and_captured(lib, deck)
+    for sim in sims:
+        sim.step(3)
+    before = sims[0].get_state(["vel"])["vel"]
+    other = dataclasses.replace(deck, bc_list=np.array(deck.bc_list))
+    var = other.bc_list[:, 1]
+    other.bc_list[:, 1] = np.select([var == 5, var == 6], [6, 5], var)
+    if equal(other.bc_list, np.array(deck.bc_list)):
+        return ["the deck prescribes no velocities"]
+    for sim in sims:
+        sim.set_bcs(other, sim.parts)
+        sim.step(3)
+    return same_state(*sims) + (["nothing moved"] if equal(before, sims[0].get_state(["vel"])["vel"]) else [])
+
+
+CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])
