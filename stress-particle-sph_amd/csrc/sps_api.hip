@@ -230,6 +230,7 @@ struct sps_handle {
     bool use_graph = false;
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     double graph_dt[2] = {0.0, 0.0};
+    int graph_rows[2] = {0, 0};   // rows that the network's buffers held at the capture
     long long graph_steps = 0;
     DBuf<double> stepv;
     DBuf<float> surr_feat;
@@ -940,11 +941,13 @@ static void drop_graphs(sps_handle *h) {
 }
 
 // The mixed form's step as a replayed graph (one per state set, captured on
-// first use and whenever dt changes).
+// first use, whenever dt changes and when the network's buffers were laid out
+// anew since, for a larger simulation that uses it too).
 static int mixed_step_graph(sps_handle *h, double dt, double time_sph, double gxg, double gyg) {
     hipStream_t s = h->stream;
     const int c = h->cur;
-    if (h->gexec[c] && h->graph_dt[c] != dt) {
+    const int rows = h->mlp ? h->mlp->rows : 0;
+    if (h->gexec[c] && (h->graph_dt[c] != dt || h->graph_rows[c] != rows)) {
         (void)hipGraphExecDestroy(h->gexec[c]);
         h->gexec[c] = nullptr;
     }
@@ -965,6 +968,7 @@ static int mixed_step_graph(sps_handle *h, double dt, double time_sph, double gx
             return fail(SPS_EDEVICE, "step graph instantiation failed: %s", hipGetErrorString(e));
         }
         h->graph_dt[c] = dt;
+        h->graph_rows[c] = rows;
     }
     k_set_step<<<1, 64, 0, s>>>(h->stepv.p, time_sph, gxg, gyg);
     if (h->p.no_bcs > 0 && h->nn > 0) k_bc_values<<<1, 64, 0, s>>>(bc_values(h, time_sph), h->bc_vals.p);

@@ -1,6 +1,7 @@
 """Sequences of calls on the CPU build of the HIP kernels (run under
 AddressSanitizer by tests/test_emu_calls.py): `run_calls.py EMU_LIB NAME`.
 Prints one line; exit status 0 when the sequence gives what it should."""
+import ctypes
 import dataclasses
 import importlib
 import os
@@ -79,7 +80,25 @@ def prescribed_values_after_capture(lib):
     return same_state(*sims) + (["nothing moved"] if equal(before, sims[0].get_state(["vel"])["vel"]) else [])
 
 
-CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture)}
+def network_attached_again_after_capture(lib):
+    """A network whose work buffers grow, when a larger simulation takes it
+    too, after a step with it was captured."""
+    net = surrogate.Network(ctypes.CDLL(lib), seed=3, batch_rows=64)
+    sims = direct_and_captured(lib, deck_of("t2_cspm"))
+    for sim in sims:
+        surrogate.attach(sim, net, 1e4, 1e4)
+        sim.step(12)     # the deck yields from its tenth step on
+    if not surrogate.stats(sims[0])[0]:
+        return ["the network was not used"]
+    larger = sps.Simulation.from_deck(deck_of("v3_vslope_sp3"), lib_path=lib, mode=sps.MODE_FAST)
+    surrogate.attach(larger, net, 1e4, 1e4)
+    for sim in sims:
+        sim.step(2)
+    return same_state(*sims)
+
+
+CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
+                                 network_attached_again_after_capture)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])

@@ -13,7 +13,8 @@ from test_emu import _asan_runtime
 sys.path.insert(0, os.path.join(ROOT, "tests", "emu"))
 import build_emu  # noqa: E402
 
-CASES = ["plastic_log_after_capture", "prescribed_values_after_capture"]
+CASES = ["plastic_log_after_capture", "prescribed_values_after_capture",
+         "network_attached_again_after_capture"]
 
 
 @pytest.fixture(scope="module")
