@@ -754,8 +754,8 @@ static int search(sps_handle *h, bool fresh_list) {
     LAUNCH(K_CELL_SCATTER, nblk(nt2), BLOCK, k_cell_scatter, h->cellkey.p, A.orig.p, h->kstart.p, h->kfill.p, h->grid.p,
                                               h->tmp_orig.p, h->tmp_src.p, h->cell.p, nn, nt, nt2);
     LAUNCH(K_CELL_SORT, TILES_BLOCKS + nstride(L3max), BLOCK, k_count_tiles_sort, h->kstart.p, h->grid.p,
-           h->tile_start.p, h->tile_range.p, h->ntile_n, h->ntile_s, nn, nt, h->mixed ? 0 : 1, h->tmp_orig.p,
-           h->tmp_src.p, h->err.p);
+           h->tile_start.p, h->tile_range.p, h->ntile_n, h->ntile_s, nn, nt, h->mixed ? 0 : 1, h->kcount.p,
+           h->kfill.p, h->tmp_orig.p, h->tmp_src.p, h->err.p);
     // permute the state into (kind, cell, original index) order: the blocks
     // whose particles moved go through the scratch set and back
     LAUNCH(K_PERMUTE, nblk(nt2), BLOCK, k_permute, B.view(), A.view(), h->tmp_src.p, nn, nt, nt2, h->moved.p);
@@ -763,8 +763,8 @@ static int search(sps_handle *h, bool fresh_list) {
                   ScanCount{h->grid.p, 1, 1});
     if (rc) return rc;
     LAUNCH(K_PERMUTE, nblk(nt2), BLOCK, k_permute_commit, A.view(), B.view(), h->moved.p, h->cell.p, h->kstart.p,
-           h->cstart_rm.p, h->grid.p, h->proc.p, h->proc_to_slot.p, h->cnt.p, h->outside ? h->inv.p : nullptr,
-           h->kcount.p, h->kfill.p, nn, nt, nt2);
+           h->cstart_rm.p, h->grid.p, h->proc.p, h->proc_to_slot.p, h->cnt.p, h->outside ? h->inv.p : nullptr, nn,
+           nt, nt2);
     HIP_TRY(hipGetLastError());
     StateSet &C = A;
     // counts, offsets, split
