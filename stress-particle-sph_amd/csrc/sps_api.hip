@@ -158,7 +158,7 @@ struct sps_handle {
     DBuf<int> cellkey, new_cell, cell, kcount, kstart, kfill, tmp_orig, tmp_src, proc, proc_to_slot;
     DBuf<unsigned char> moved;    // per block of slots: the permutation moves a particle of it
     DBuf<unsigned> cnt, off, cstart_rm;
-    DBuf<unsigned long long> scan_state;   // k_scan_sums: a word per tile, the launch's number, the ticket counter
+    DBuf<unsigned long long> scan_state;   // k_scan_sums: a word per run, the launch's number, the ticket counter
     unsigned scan_epoch = 0;
     DBuf<unsigned> scan_ticket;
     // per-step pair lists of the tiled stage kernels
@@ -369,14 +369,14 @@ static size_t lds_count(const sps_handle *h) {
 template <typename In>
 static int scan_u32(sps_handle *h, In in, unsigned *out, long long n, unsigned long long *dtotal,
                     ScanCount sc = ScanCount{nullptr, 0, 0}) {
-    constexpr int TILE_ITEMS = BLOCK * In::ITEMS;
-    const long long nb = std::max(1ll, (n + TILE_ITEMS - 1) / TILE_ITEMS);
+    constexpr int TILE_ITEMS = BLOCK * 4 * In::GROUPS;
+    const long long nb = std::min<long long>(SCAN_BLOCKS, std::max(1ll, (n + TILE_ITEMS - 1) / TILE_ITEMS));
     if ((size_t)nb > h->scan_state.n) return fail(SPS_ECAPACITY, "scan of %lld values", n);
     if (++h->scan_epoch >= SCAN_EPOCHS) {   // the numbers of earlier launches come again
         HIP_TRY(hipMemsetAsync(h->scan_state.p, 0, h->scan_state.n * sizeof(unsigned long long), h->stream));
         h->scan_epoch = 1;
     }
-    LAUNCH(K_SCAN, (unsigned)std::min<long long>(nb, SCAN_BLOCKS), BLOCK, k_scan_sums<In>, in, out, h->scan_state.p,
+    LAUNCH(K_SCAN, (unsigned)nb, BLOCK, k_scan_sums<In>, in, out, h->scan_state.p,
            h->scan_ticket.p, (unsigned long long)h->scan_epoch, dtotal, n, sc);
     HIP_TRY(hipGetLastError());
     return 0;
@@ -638,10 +638,7 @@ static int size_cells(sps_handle *h, const double *hsml) {
     size_t L = 3 * ((size_t)cap + 1) + 1;
     rc |= dalloc(h->kcount, L); rc |= dalloc(h->kstart, L); rc |= dalloc(h->kfill, L);
     rc |= dalloc(h->cstart_rm, (size_t)cap + 2);
-    // tiles of the largest scan of a step (the bucket counts or the slots)
-    const size_t st = std::max(std::max(L, (size_t)h->nt2 + 1) / (BLOCK * ScanArray::ITEMS),
-                               ((size_t)cap + 1) / (BLOCK * ScanCells::ITEMS)) + 2;
-    rc |= dalloc(h->scan_state, st) | dalloc(h->scan_ticket, 1);
+    rc |= dalloc(h->scan_state, SCAN_BLOCKS) | dalloc(h->scan_ticket, 1);
     if (rc) return rc;
     // a search clears the counters it has used for the next one
     HIP_TRY(hipMemsetAsync(h->kcount.p, 0, h->kcount.n * sizeof(int), h->stream));

@@ -323,23 +323,45 @@ __device__ __forceinline__ void cell_sort(const int *__restrict__ kstart, int *_
 }
 
 // What a scan adds up: an array, or the particles per cell in the
-// reference's row-major visiting order (fewer values a lane: each takes two
-// divisions and six loads).
+// reference's row-major visiting order.  four() gives elements [i, i + 4),
+// zero from n on; GROUPS: a lane's groups of four in a tile; KEEP: dear to
+// read, so a run of several tiles keeps them in the output between its passes.
 struct ScanArray {
-    static constexpr int ITEMS = 16;
+    static constexpr int GROUPS = 4;
+    static constexpr bool KEEP = false;
     const unsigned *in;
-    __device__ __forceinline__ unsigned operator()(long long i) const { return in[i]; }
+    __device__ __forceinline__ void four(long long i, long long n, unsigned (&v)[4]) const {
+        if (i + 4 <= n) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = in[i + k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = i + k < n ? in[i + k] : 0u;
+        }
+    }
 };
 struct ScanCells {
-    static constexpr int ITEMS = 4;
+    static constexpr int GROUPS = 1;
+    static constexpr bool KEEP = true;
     const int *kstart;
     const Grid *g;
-    __device__ __forceinline__ unsigned operator()(long long i) const {
-        const int c = (int)i, ndivt = g->ndivt, L = ndivt + 1;
-        if (c >= ndivt) return 0u;
-        const int key = cell_key(c % g->ndivx, c / g->ndivx, *g);
-        return (unsigned)((kstart[key + 1] - kstart[key]) + (kstart[L + key + 1] - kstart[L + key]) +
-                          (kstart[2 * L + key + 1] - kstart[2 * L + key]));
+    __device__ __forceinline__ void four(long long i, long long n, unsigned (&v)[4]) const {
+        const Grid gg = *g;
+        const int L = gg.ndivt + 1;
+        int cy = i < gg.ndivt ? (int)i / gg.ndivx : 0, cx = i < gg.ndivt ? (int)i - cy * gg.ndivx : 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = 0u;
+            if (i + k < gg.ndivt && i + k < n) {
+                const int key = cell_key(cx, cy, gg);
+                v[k] = (unsigned)((kstart[key + 1] - kstart[key]) + (kstart[L + key + 1] - kstart[L + key]) +
+                                  (kstart[2 * L + key + 1] - kstart[2 * L + key]));
+            }
+            if (++cx == gg.ndivx) {
+                cx = 0;
+                ++cy;
+            }
+        }
     }
 };
 
@@ -3398,30 +3420,32 @@ __global__ void k_scatter_in_identity(int *__restrict__ orig, int n) {
 }
 
 // ------------------------------------------------------------------- scans
-// Sums of unsigned values over a wave and a block.
-__device__ __forceinline__ unsigned wave_incl_scan(unsigned v) {
-    int lane = threadIdx.x & 63;
-    for (int off = 1; off < 64; off <<= 1) {
-        unsigned t = __shfl_up(v, off, 64);
-        if (lane >= off) v += t;
+// Exclusive prefix sums ex of a block's values s in the order of the groups
+// and, inside one, of the lanes; their total.
+template <int G>
+__device__ __forceinline__ void block_excl_scan(const unsigned (&s)[G], unsigned (&ex)[G], unsigned *total) {
+    __shared__ unsigned wsum[G][BLOCK / 64];
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+        unsigned v = s[j];
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned u = __shfl_up(v, off, 64);
+            if (lane >= off) v += u;
+        }
+        if (lane == 63) wsum[j][wid] = v;
+        ex[j] = v - s[j];
     }
-    return v;
-}
-
-__device__ __forceinline__ unsigned block_excl_scan(unsigned v, unsigned *total) {
-    __shared__ unsigned wsum[BLOCK / 64];
-    unsigned incl = wave_incl_scan(v);
-    int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 63) wsum[wid] = incl;
     __syncthreads();
-    unsigned base = 0, tot = 0;
-    for (int k = 0; k < BLOCK / 64; ++k) {
-        if (k < wid) base += wsum[k];
-        tot += wsum[k];
-    }
+    unsigned tot = 0;
+#pragma unroll
+    for (int j = 0; j < G; ++j)
+        for (int k = 0; k < BLOCK / 64; ++k) {
+            if (k == wid) ex[j] += tot;
+            tot += wsum[j][k];
+        }
     __syncthreads();
     *total = tot;
-    return base + incl - v;
 }
 
 // Element count of a scan: the host's n, or (with g) a * ndivt + b of the
@@ -3436,21 +3460,28 @@ struct ScanCount {
     }
 };
 
-// Exclusive scan in one launch (three, with the block sums between them, cost
-// three times the 4 us between dependent launches, and with a grid for the
-// cell capacity of the whole domain box 49 and 21 us for empty blocks on a
-// 100 k-particle sample).  Blocks take SCAN_TILE elements at a time in the
-// order of a counter, publish their sum, and add up the sums before theirs
-// back to the first published prefix; each waits only for tiles taken before
-// its own, whose blocks are running.  A tile's word holds the launch's number
-// (epoch), whether the value is the tile's sum (1) or its prefix (2), and the
-// value, so that the words need no clearing between launches.  The block with
-// the last number takes the counter back to zero.  The numbers are what a
-// scan of many tiles costs (one at a time, some 15 ns each): at most 256
-// blocks, a second number only where a block may have a second tile, tiles of
-// 4096 array elements (2048 for up to 1024 blocks: 31 us a scan at 2 M
-// particles, so 24 us).
-constexpr int SCAN_BLOCKS = 256;
+// Exclusive scan in one launch, by the published decoupled look-back (Merrill
+// and Garland, Single-pass Parallel Prefix Scan with Decoupled Look-back,
+// 2016); three launches, with the block sums between them, cost three times the
+// 4 us between dependent launches.  Each block takes a run of tiles in the order
+// of a counter, publishes its sum, and adds up the sums before its own back to
+// the first published prefix; it waits only for runs taken before its own, whose
+// blocks are running.  A run's word holds the launch's number (epoch), whether
+// the value is the run's sum (1) or its prefix (2), and the value, so that the
+// words need no clearing between launches.  The block with the last number
+// takes the counter back to zero.
+//
+// A lane takes four elements in a row, the next lane the next four, so that the
+// accesses of a wave are whole lines.  The numbers go out one at a time, some
+// 15 ns each, so there are at most SCAN_BLOCKS runs: one tile each up to 4 M array
+// elements or 1 M cells, and beyond that as many as it takes, whose elements
+// are read twice.  On 8 M cells (24 M buckets) the buckets' scan takes 56 us, with
+// sixteen elements in a row a lane and 256 blocks 203 us, in three launches 160;
+// the cells' totals 163 us (their loads lie a strip apart), without keeping them
+// 254, as before 214, as a launch of their own and three of a scan 135; on 800 k
+// cells 18 and 28 us (before 29 and 29).  The grid is sized for the cell
+// capacity; a block with no run leaves without a number.
+constexpr int SCAN_BLOCKS = 1024;
 constexpr unsigned SCAN_EPOCHS = 1u << 30;
 
 template <typename In>
@@ -3459,60 +3490,91 @@ __global__ __launch_bounds__(BLOCK) void k_scan_sums(In in, unsigned *__restrict
                                                      unsigned *__restrict__ ticket, unsigned long long epoch,
                                                      unsigned long long *__restrict__ total, long long n_max,
                                                      ScanCount sc) {
-    constexpr int SCAN_ITEMS = In::ITEMS, SCAN_TILE = BLOCK * SCAN_ITEMS;
+    constexpr int G = In::GROUPS, SCAN_TILE = BLOCK * 4 * G;
     __shared__ unsigned sh_id, sh_prefix;
     const int t = threadIdx.x, lane = t & 63;
     const long long n = sc.get(n_max);
-    const unsigned nb = n > 0 ? (unsigned)((n + SCAN_TILE - 1) / SCAN_TILE) : 1u;
-    const bool once = gridDim.x >= nb;
-    const unsigned tickets = once ? gridDim.x : nb + gridDim.x;
-    for (;;) {
-        if (t == 0) sh_id = atomicAdd(ticket, 1u);
-        __syncthreads();
-        const unsigned id = sh_id;
-        if (t == 0 && id == tickets - 1) atomicAdd(ticket, 0u - tickets);
-        if (id >= nb) return;
-        const long long base = (long long)id * SCAN_TILE + (long long)t * SCAN_ITEMS;
-        unsigned v[SCAN_ITEMS], s = 0;
+    const long long tiles = n > 0 ? (n + SCAN_TILE - 1) / SCAN_TILE : 1;
+    const long long run = (tiles + gridDim.x - 1) / gridDim.x;   // tiles of a run
+    const unsigned nb = (unsigned)((tiles + run - 1) / run);
+    if (blockIdx.x >= nb) return;
+    if (t == 0) sh_id = atomicAdd(ticket, 1u);
+    __syncthreads();
+    const unsigned id = sh_id;
+    if (t == 0 && id == nb - 1) atomicAdd(ticket, 0u - nb);
+    const long long base = (long long)id * run * SCAN_TILE + 4 * t;
+    unsigned v[G][4], s[G], ex[G], tot;
+    auto load = [&](const auto &from, long long r) {   // this lane's elements of the run's tile r
 #pragma unroll
-        for (int k = 0; k < SCAN_ITEMS; ++k) {
-            v[k] = base + k < n ? in(base + k) : 0u;
-            s += v[k];
+        for (int j = 0; j < G; ++j) {
+            from.four(base + r * SCAN_TILE + j * (BLOCK * 4), n, v[j]);
+            s[j] = v[j][0] + v[j][1] + v[j][2] + v[j][3];
         }
-        unsigned tot;
-        unsigned ex = block_excl_scan(s, &tot);
-        if (t < 64) {
-            unsigned prefix = 0;
-            if (id > 0) {
-                if (lane == 0) atomicMax(&state[id], epoch << 34 | 1ull << 32 | tot);
-                for (int p = (int)id - 1;; p -= 64) {   // lane l: tile p - l
-                    unsigned long long w = 2ull << 32;
-                    if (p - lane >= 0)
-                        do {
-                            w = __hip_atomic_load(&state[p - lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        } while (w >> 34 != epoch);
-                    const unsigned long long done = __ballot(((w >> 32) & 3) == 2);
-                    const int first = done ? __ffsll(done) - 1 : 63;
-                    unsigned a = lane <= first ? (unsigned)w : 0u;
-                    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-                    prefix += __shfl(a, 0, 64);
-                    if (done) break;
-                }
-            }
-            if (lane == 0) {
-                atomicMax(&state[id], epoch << 34 | 2ull << 32 | (prefix + tot));
-                sh_prefix = prefix;
-                if (total && id == nb - 1) *total = prefix + tot;
-            }
-        }
-        __syncthreads();
-        ex += sh_prefix;
+    };
+    auto store = [&](long long at, const unsigned (&o)[4]) {
+        if (at + 4 <= n) {
 #pragma unroll
-        for (int k = 0; k < SCAN_ITEMS; ++k) {
-            if (base + k < n) out[base + k] = ex;
-            ex += v[k];
+            for (int k = 0; k < 4; ++k) out[at + k] = o[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (at + k < n) out[at + k] = o[k];
         }
-        if (once) return;
+    };
+    load(in, run - 1);
+    if (run > 1) {   // the run's sum, its first tile last
+        unsigned all[1] = {0}, none[1];
+        for (long long r = run - 1;; load(in, --r)) {
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+                all[0] += s[j];
+                if (In::KEEP) store(base + r * SCAN_TILE + j * (BLOCK * 4), v[j]);
+            }
+            if (r == 0) break;
+        }
+        block_excl_scan(all, none, &tot);
+    } else {
+        block_excl_scan(s, ex, &tot);
+    }
+    if (t < 64) {
+        unsigned prefix = 0;
+        if (id > 0) {
+            if (lane == 0) atomicMax(&state[id], epoch << 34 | 1ull << 32 | tot);
+            for (int p = (int)id - 1;; p -= 64) {   // lane l: run p - l
+                unsigned long long w = 2ull << 32;
+                if (p - lane >= 0)
+                    do {
+                        w = __hip_atomic_load(&state[p - lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    } while (w >> 34 != epoch);
+                const unsigned long long done = __ballot(((w >> 32) & 3) == 2);
+                const int first = done ? __ffsll(done) - 1 : 63;
+                unsigned a = lane <= first ? (unsigned)w : 0u;
+                for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+                prefix += __shfl(a, 0, 64);
+                if (done) break;
+            }
+        }
+        if (lane == 0) {
+            atomicMax(&state[id], epoch << 34 | 2ull << 32 | (prefix + tot));
+            sh_prefix = prefix;
+            if (total && id == nb - 1) *total = prefix + tot;
+        }
+    }
+    __syncthreads();
+    unsigned before = sh_prefix;
+    for (long long r = 0;;) {
+        if (run > 1) block_excl_scan(s, ex, &tot);   // of the tile that v holds
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+            const long long at = base + r * SCAN_TILE + j * (BLOCK * 4);
+            unsigned e = ex[j] + before;
+            const unsigned o[4] = {e, e + v[j][0], e + v[j][0] + v[j][1], e + v[j][0] + v[j][1] + v[j][2]};
+            store(at, o);
+        }
+        before += tot;
+        if (++r == run) break;
+        if constexpr (In::KEEP) load(ScanArray{out}, r);
+        else load(in, r);
     }
 }
 
