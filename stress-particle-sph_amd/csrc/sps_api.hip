@@ -37,6 +37,8 @@ static int fail(int code, const char *fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(g_err, sizeof g_err, fmt, ap);
     va_end(ap);
+    // reported here: not again by the next launch's check
+    if (code == SPS_EDEVICE || code == SPS_ENOMEM) (void)hipGetLastError();
     return code;
 }
 
@@ -1320,9 +1322,9 @@ static int read_back(sps_handle *h, ReadBack &R) {
         h->read_slots = 0;
         if (hipHostMalloc((void **)&h->read_pin, slots * READ_CHUNK, hipHostMallocDefault) != hipSuccess)
             return fail(SPS_ENOMEM, "pinned read-back buffer of %zu bytes", slots * READ_CHUNK);
-        h->read_slots = slots;
         for (int k = 0; k < slots; ++k)
             if (!h->read_ev[k]) HIP_TRY(hipEventCreateWithFlags(&h->read_ev[k], hipEventDisableTiming));
+        h->read_slots = slots;   // every slot has its event
     }
     for (int k = 0; k < R.n; ++k) R.table.f[k].dst = h->read_dev.p + R.off[k];
     k_read_back<<<dim3(nblk(R.nmax), (unsigned)R.n), BLOCK, 0, h->stream>>>(R.table);

@@ -31,6 +31,8 @@ bool needs_sync(const char *name) {
 unsigned char *lds_base = nullptr;
 size_t lds_bytes = 0;
 
+int events_left = -1;
+
 bool capturing = false;
 struct Launch {
     dim3 grid;
@@ -217,3 +219,5 @@ void launch(dim3 grid, unsigned block, size_t lds, const std::function<void()> &
 }
 
 }  // namespace emu
+
+extern "C" void emu_set_events_left(int n) { emu::events_left = n; }

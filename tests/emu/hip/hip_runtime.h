@@ -72,6 +72,9 @@ struct Graph;
 Graph *end_capture();
 void replay(const Graph *g);
 void drop(Graph *g);
+// events that can still be created (-1: any number); a test sets it through
+// emu_set_events_left
+extern int events_left;
 extern unsigned char *lds_base;   // the launch's dynamic LDS
 extern size_t lds_bytes;
 }  // namespace emu
@@ -235,11 +238,17 @@ inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = null
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 inline hipError_t hipEventCreate(hipEvent_t *e) { *e = (void *)1; return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+// as on the device, an event that was not created is refused
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { return e ? hipSuccess : hipErrorUnknown; }
 // launches run in order here, so a stream waiting for an event has nothing to wait for
 inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 #define hipEventDisableTiming 2
-inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = (void *)1; return hipSuccess; }
-inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    if (emu::events_left == 0) return hipErrorUnknown;
+    if (emu::events_left > 0) --emu::events_left;
+    *e = (void *)1;
+    return hipSuccess;
+}
+inline hipError_t hipEventSynchronize(hipEvent_t e) { return e ? hipSuccess : hipErrorUnknown; }
 inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return "emulated"; }

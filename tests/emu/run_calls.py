@@ -97,8 +97,30 @@ def network_attached_again_after_capture(lib):
     return same_state(*sims)
 
 
+def state_after_failed_event(lib):
+    """The state taken back when an event of the read-back could not be
+    created: an error, and the state from the next call."""
+    deck = dataclasses.replace(deck_of("t3_elastic"))
+    deck.xs = (0.0, 249.5 * deck.dx, 0.0, 249.5 * deck.dx)     # a field takes more than one chunk
+    deck.ys = (0.0, 0.0, 249.5 * deck.dx, 249.5 * deck.dx)
+    deck.xmax_domain = np.array([2.0, 2.0]) + 250 * deck.dx
+    sim = sps.Simulation.from_deck(deck, lib_path=lib)
+    want = sps.initial_state(sim.parts, sim.niv)
+    emu = ctypes.CDLL(lib)
+    emu.emu_set_events_left(1)
+    bad = []
+    try:
+        sim.get_state(["x", "vel"])
+        bad.append("no error")
+    except sps.SpsError:
+        pass
+    emu.emu_set_events_left(-1)
+    got = sim.get_state(["x", "vel"])
+    return bad + [k for k in got if not equal(got[k], want[k])]
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
-                                 network_attached_again_after_capture)}
+                                 network_attached_again_after_capture, state_after_failed_event)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])
