@@ -11,6 +11,8 @@
 
 #include <csetjmp>
 #include <cstring>
+#include <mutex>
+#include <unordered_map>
 
 dim3e threadIdx, blockIdx, blockDim, gridDim;
 
@@ -32,6 +34,39 @@ unsigned char *lds_base = nullptr;
 size_t lds_bytes = 0;
 
 int events_left = -1;
+
+namespace {
+std::mutex mem_mu;
+std::unordered_map<void *, size_t> mem_sizes;
+size_t mem_used = 0, mem_total = (size_t)1 << 40;
+}  // namespace
+
+void *device_alloc(size_t n) {
+    std::lock_guard<std::mutex> lock(mem_mu);
+    if (n > mem_total - std::min(mem_used, mem_total)) return nullptr;
+    void *p = malloc(n);
+    if (p) {
+        mem_sizes[p] = n;
+        mem_used += n;
+    }
+    return p;
+}
+
+void device_free(void *p) {
+    std::lock_guard<std::mutex> lock(mem_mu);
+    const auto it = mem_sizes.find(p);
+    if (it != mem_sizes.end()) {
+        mem_used -= it->second;
+        mem_sizes.erase(it);
+    }
+    free(p);
+}
+
+void device_memory(size_t *free_bytes, size_t *total) {
+    std::lock_guard<std::mutex> lock(mem_mu);
+    *free_bytes = mem_total - std::min(mem_used, mem_total);
+    *total = mem_total;
+}
 
 bool capturing = false;
 struct Launch {
@@ -221,3 +256,8 @@ void launch(dim3 grid, unsigned block, size_t lds, const std::function<void()> &
 }  // namespace emu
 
 extern "C" void emu_set_events_left(int n) { emu::events_left = n; }
+// n bytes beyond those in use (negative: as good as any number)
+extern "C" void emu_set_memory(long long n) {
+    std::lock_guard<std::mutex> lock(emu::mem_mu);
+    emu::mem_total = n < 0 ? (size_t)1 << 40 : emu::mem_used + (size_t)n;
+}

@@ -75,6 +75,10 @@ void drop(Graph *g);
 // events that can still be created (-1: any number); a test sets it through
 // emu_set_events_left
 extern int events_left;
+// device memory: what is allocated, and what there is (emu_set_memory)
+void *device_alloc(size_t n);
+void device_free(void *p);
+void device_memory(size_t *free_bytes, size_t *total);
 extern unsigned char *lds_base;   // the launch's dynamic LDS
 extern size_t lds_bytes;
 }  // namespace emu
@@ -175,8 +179,9 @@ typedef void *hipStream_t;
 typedef void *hipEvent_t;
 #define hipStreamNonBlocking 1
 #define hipHostMallocDefault 0
-inline hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n ? n : 1); return *p ? hipSuccess : hipErrorUnknown; }
-inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+inline hipError_t hipMalloc(void **p, size_t n) { *p = emu::device_alloc(n ? n : 1); return *p ? hipSuccess : hipErrorUnknown; }
+inline hipError_t hipFree(void *p) { emu::device_free(p); return hipSuccess; }
+inline hipError_t hipMemGetInfo(size_t *f, size_t *t) { emu::device_memory(f, t); return hipSuccess; }
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = malloc(n); return hipSuccess; }
 inline hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {

@@ -97,14 +97,19 @@ def network_attached_again_after_capture(lib):
     return same_state(*sims)
 
 
+def block(nx):
+    """An elastic block of nx x nx nodes."""
+    deck = dataclasses.replace(deck_of("t3_elastic"))
+    deck.xs = (0.0, (nx - 0.5) * deck.dx, 0.0, (nx - 0.5) * deck.dx)
+    deck.ys = (0.0, 0.0, (nx - 0.5) * deck.dx, (nx - 0.5) * deck.dx)
+    deck.xmax_domain = np.array([2.0, 2.0]) + nx * deck.dx
+    return deck
+
+
 def state_after_failed_event(lib):
     """The state taken back when an event of the read-back could not be
     created: an error, and the state from the next call."""
-    deck = dataclasses.replace(deck_of("t3_elastic"))
-    deck.xs = (0.0, 249.5 * deck.dx, 0.0, 249.5 * deck.dx)     # a field takes more than one chunk
-    deck.ys = (0.0, 0.0, 249.5 * deck.dx, 249.5 * deck.dx)
-    deck.xmax_domain = np.array([2.0, 2.0]) + 250 * deck.dx
-    sim = sps.Simulation.from_deck(deck, lib_path=lib)
+    sim = sps.Simulation.from_deck(block(250), lib_path=lib)   # a field takes more than one chunk
     want = sps.initial_state(sim.parts, sim.niv)
     emu = ctypes.CDLL(lib)
     emu.emu_set_events_left(1)
@@ -119,8 +124,19 @@ def state_after_failed_event(lib):
     return bad + [k for k in got if not equal(got[k], want[k])]
 
 
+def state_short_of_memory(lib):
+    """The state taken back where the device has room for its largest field
+    and no more."""
+    sim = sps.Simulation.from_deck(block(120), lib_path=lib)
+    want = sps.initial_state(sim.parts, sim.niv)
+    ctypes.CDLL(lib).emu_set_memory(32 * sim.n2 + 256)
+    got = sim.get_state()
+    return [k for k in ("x", "vel", "stress", "mass", "internal_vars", "x00") if not equal(got[k], want[k])]
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
-                                 network_attached_again_after_capture, state_after_failed_event)}
+                                 network_attached_again_after_capture, state_after_failed_event,
+                                 state_short_of_memory)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])

@@ -14,7 +14,8 @@ sys.path.insert(0, os.path.join(ROOT, "tests", "emu"))
 import build_emu  # noqa: E402
 
 CASES = ["plastic_log_after_capture", "prescribed_values_after_capture",
-         "network_attached_again_after_capture", "state_after_failed_event"]
+         "network_attached_again_after_capture", "state_after_failed_event",
+         "state_short_of_memory"]
 
 
 @pytest.fixture(scope="module")
