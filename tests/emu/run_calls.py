@@ -134,9 +134,18 @@ def state_short_of_memory(lib):
     return [k for k in ("x", "vel", "stress", "mass", "internal_vars", "x00") if not equal(got[k], want[k])]
 
 
+def small_state_without_events(lib):
+    """What fits one chunk is taken back with a copy and a wait, no event."""
+    sim = sps.Simulation.from_deck(deck_of("t3_elastic"), lib_path=lib)
+    want = sps.initial_state(sim.parts, sim.niv)
+    ctypes.CDLL(lib).emu_set_events_left(0)
+    got = sim.get_state()
+    return [k for k in ("x", "vel", "stress", "mass", "internal_vars", "x00") if not equal(got[k], want[k])]
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
                                  network_attached_again_after_capture, state_after_failed_event,
-                                 state_short_of_memory)}
+                                 state_short_of_memory, small_state_without_events)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])
