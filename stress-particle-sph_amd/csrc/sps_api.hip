@@ -22,6 +22,7 @@
 #include <atomic>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 
 #include "../../include/sps.h"
 #include "sps_kernels.hip"
@@ -148,7 +149,6 @@ struct sps_handle {
     // k_sp_update writes here so that the nodes' half, reading the first, can
     // run beside it (k_sp_update_beside)
     DBuf<double4> sig2;
-    DBuf<double4> stress_b;  // the stress points' stresses of the odd RK stages (StageStep)
     DBuf<float2> av_nodes;   // the nodes' artificial viscosity of a stage (k_av_nodes)
     DBuf<double> rk_dev, ddev;
     // search
@@ -157,16 +157,18 @@ struct sps_handle {
     DBuf<Split> split;
     DBuf<double> bparts;
     int nbparts = 0;
-    DBuf<int> cellkey, new_cell, cell, kcount, kstart, kfill, tmp_orig, tmp_src, proc, proc_to_slot;
+    DBuf<int> cellkey, cell, kcount, kstart, kfill, tmp_orig, tmp_src, proc, proc_to_slot;
     DBuf<unsigned char> moved;    // per block of slots: the permutation moves a particle of it
     DBuf<unsigned> cnt, off, cstart_rm;
     DBuf<unsigned long long> scan_state;   // k_scan_sums: a word per run, the launch's number, the ticket counter
     unsigned scan_epoch = 0;
     DBuf<unsigned> scan_ticket;
-    // per-step pair lists of the tiled stage kernels
-    DBuf<unsigned long long> list_ia, list_ib, list_iah, list_ibh;
-    int list_words = 12;          // words of four entries per receiver and list
-    DBuf<float4> list_wa, list_gxa, list_gya, list_gxb, list_gyb, list_wb;
+    // per-step pair lists of the tiled stage kernels, in list_mem (lay_lists)
+    DBuf<char> list_mem;
+    unsigned long long *list_ia = nullptr, *list_ib = nullptr, *list_iah = nullptr, *list_ibh = nullptr;
+    float4 *list_wa = nullptr, *list_gxa = nullptr, *list_gya = nullptr;
+    float4 *list_gxb = nullptr, *list_gyb = nullptr, *list_wb = nullptr;
+    int list_words = LIST_WORDS;  // words of four entries per receiver and list
     bool xsph = false;            // XSPH position update (list B also for stress points, with w)
     DBuf<double2> xsph_v;
     // the outside approach: each node's stress points follow it
@@ -264,9 +266,10 @@ struct sps_handle {
     long long prof_n[32] = {0};
 
     PairLists lists() {
-        return PairLists{list_ia.p,  list_ib.p,  list_iah.p, list_ibh.p, list_wa.p, list_gxa.p, list_gya.p,
-                         list_gxb.p, list_gyb.p, xsph ? list_wb.p : nullptr, deg_a.p, deg_b.p,
-                         tile_ok.p,  list_words, ntile_n,    tile_range.p, type_counts.p, tiles.p,   plans.p, (outside || bcint) ? nodeinfo.p : nullptr};
+        return PairLists{list_ia,  list_ib,   list_iah, list_ibh, list_wa, list_gxa,   list_gya,
+                         list_gxb, list_gyb,  list_wb,  deg_a.p,  deg_b.p, tile_ok.p,  list_words,
+                         xsph,     ntile_n,   tile_range.p, type_counts.p, tiles.p, plans.p,
+                         (outside || bcint) ? nodeinfo.p : nullptr};
     }
 };
 
@@ -338,7 +341,8 @@ static void drop_graphs(sps_handle *h);
 
 // RK stage st of a step of dt (2_...:681-777): its weight, and what its
 // derivative pass leaves.  The stress points' stresses alternate between the
-// state and stress_b, so that the last stage leaves the step's in the state.
+// state and the other state set's, which only the search uses (as scratch), so
+// that the last stage leaves the step's in the state.
 // rhs: the step's end is k_rk_final's.
 static StageStep rk_stage(sps_handle *h, const StateBufs &SB, int st, double dt, bool rhs) {
     const double f1[4] = {0., 0.5, 0.5, 1.0}, f2[4] = {1., 2., 2., 1.0};
@@ -347,8 +351,9 @@ static StageStep rk_stage(sps_handle *h, const StateBufs &SB, int st, double dt,
     Q.first = st == 0;
     Q.f2 = f2[st];
     Q.c = st < 3 ? f1[st + 1] * dt : dt / 6;
-    Q.sp_in = st & 1 ? h->stress_b.p : SB.stress;
-    Q.sp_out = st & 1 ? SB.stress : h->stress_b.p;
+    double4 *const other = h->S[1 - h->cur].stress.p;
+    Q.sp_in = st & 1 ? other : SB.stress;
+    Q.sp_out = st & 1 ? SB.stress : other;
     return Q;
 }
 
@@ -494,6 +499,60 @@ static double gravity_factor(const sps_params *P, double time_sph) {
     return factg * P->ft_grav;
 }
 
+// The arrays of the pair lists with `words` words of four entries a list, laid
+// one after the other from base (null: no pointers, only the bytes); slots:
+// with the upper halves that lists of storage slots need.  One allocation for
+// all of them: each of 2 MiB or more takes up to 0.3 ms to make and to free.
+static size_t lay_lists(sps_handle *h, int words, bool slots, char *base) {
+    size_t at = 0;
+    auto take = [&](auto *&p, size_t n) {
+        p = base ? reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at) : nullptr;
+        at += (n * sizeof(*p) + 255) & ~(size_t)255;
+    };
+    const size_t wt = (size_t)words * TILE;
+    const size_t a = (size_t)(h->ntile_n + h->ntile_s) * wt, nodes = (size_t)h->ntile_n * wt;
+    const size_t b = h->xsph ? a : nodes;   // list B: node tiles; with XSPH stress-point tiles too, and its w
+    take(h->list_ia, a);
+    take(h->list_ib, b);
+    if (slots) {
+        take(h->list_iah, a);
+        take(h->list_ibh, b);
+    }
+    if (!h->mixed) {   // the mixed form computes the kernel values as it goes
+        take(h->list_wa, a);
+        take(h->list_gxa, a);
+        take(h->list_gya, a);
+        take(h->list_gxb, nodes);
+        take(h->list_gyb, nodes);
+        if (h->xsph) take(h->list_wb, a);
+    }
+    return at;
+}
+
+// 48 entries a list, and 24 more per further stress point a node or cell (about
+// 18 partners within 2h = 2.4 dx each; the mixed form keeps 48), and lists of
+// storage slots for tiles without a window.  Both only save time: a tile that
+// has no lists walks its cells in every stage, with the same results.  So they
+// are left out where they would take more than half of the memory that the
+// lists leave: a body fits where it fits without them.
+static int alloc_lists(sps_handle *h) {
+    int words = LIST_WORDS;
+    if (!h->mixed) words += 6 * (std::max(1, std::min(4, (h->ns + h->nn - 1) / h->nn)) - 1);
+    size_t mem_free = 0, mem_total = 0;
+    HIP_TRY(hipMemGetInfo(&mem_free, &mem_total));
+    const size_t least = lay_lists(h, LIST_WORDS, false, nullptr), full = lay_lists(h, words, true, nullptr);
+    bool slots = mem_free > least && full - least <= (mem_free - least) / 2;
+    if (slots && dalloc(h->list_mem, full)) slots = false;
+    if (!slots) {
+        words = LIST_WORDS;
+        const int rc = dalloc(h->list_mem, least);
+        if (rc) return rc;
+    }
+    h->list_words = words;
+    lay_lists(h, words, slots, h->list_mem.p);
+    return 0;
+}
+
 extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     if (!params || !out) return fail(SPS_EINVAL, "null argument");
     int rc = check_params(params);
@@ -551,12 +610,12 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     rc |= dalloc(h->rk_vel, nn); rc |= dalloc(h->rhs2, nn); rc |= dalloc(h->f_bound, nn);
     rc |= dalloc(h->art_visc, nn); rc |= dalloc(h->stress0, nt); rc |= dalloc(h->rk_stress, nt);
     rc |= dalloc(h->rhs1, nt); rc |= dalloc(h->grad_u, nt); rc |= dalloc(h->rk_dev, nt);
-    rc |= dalloc(h->sig2, nt); rc |= dalloc(h->stress_b, nt); rc |= dalloc(h->av_nodes, nn > 0 ? nn : 1);
+    rc |= dalloc(h->sig2, nt); rc |= dalloc(h->av_nodes, nn > 0 ? nn : 1);
     rc |= dalloc(h->ddev, nt);
     rc |= dalloc(h->grid, 1); rc |= dalloc(h->split, 1); rc |= dalloc(h->err, 1); rc |= dalloc(h->pairs_total, 1);
     h->nbparts = std::min(1024, (int)nblk(nt2));
     rc |= dalloc(h->bparts, 5 * (size_t)h->nbparts);
-    rc |= dalloc(h->cellkey, nt2); rc |= dalloc(h->new_cell, nt2); rc |= dalloc(h->cell, nt2);
+    rc |= dalloc(h->cellkey, nt2); rc |= dalloc(h->cell, nt2);
     rc |= dalloc(h->tmp_orig, nt2); rc |= dalloc(h->tmp_src, nt2); rc |= dalloc(h->proc, nt2);
     rc |= dalloc(h->moved, nblk(nt2));
     rc |= dalloc(h->proc_to_slot, nt2); rc |= dalloc(h->cnt, nt2); rc |= dalloc(h->off, nt2);
@@ -570,22 +629,6 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     rc |= dalloc(h->tile_start, 2 * (size_t)TSTART_MAX);
     rc |= dalloc(h->tile_range, (size_t)h->ntile_n + h->ntile_s);
     rc |= dalloc(h->type_counts, 3 * ((size_t)h->ntile_n + h->ntile_s + count_blocks(nt2 - nt)));
-    {
-        // 48 entries a list, and 24 more per further stress point a node or
-        // cell (about 18 partners within 2h = 2.4 dx each); a receiver with
-        // more leaves its tile without lists.  (The mixed form keeps 48: which
-        // tiles it walks in double precision is part of its result.)
-        if (!h->mixed) h->list_words = 12 + 6 * (std::min(4, (h->ns + nn - 1) / nn) - 1);
-        if (h->list_words < 12) h->list_words = 12;
-        const size_t wt = (size_t)h->list_words * TILE;
-        const size_t wa = (size_t)(h->ntile_n + h->ntile_s) * wt, wb = (size_t)h->ntile_n * wt;
-        rc |= dalloc(h->list_ia, wa); rc |= dalloc(h->list_wa, wa); rc |= dalloc(h->list_gxa, wa);
-        rc |= dalloc(h->list_gya, wa);
-        // list B: node tiles; with XSPH stress-point tiles too, and its w
-        rc |= dalloc(h->list_ib, h->xsph ? wa : wb); rc |= dalloc(h->list_gxb, wb); rc |= dalloc(h->list_gyb, wb);
-        if (h->xsph) rc |= dalloc(h->list_wb, wa) | dalloc(h->xsph_v, (size_t)nt);
-        rc |= dalloc(h->list_iah, wa) | dalloc(h->list_ibh, h->xsph ? wa : wb);
-    }
     rc |= dalloc(h->deg_a, nt); rc |= dalloc(h->deg_b, h->xsph ? nt : nn);
     rc |= dalloc(h->tile_ok, h->ntile_n + h->ntile_s + 1);
     rc |= dalloc(h->tiles, h->ntile_n + h->ntile_s + 1);
@@ -603,6 +646,8 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     // bc_int for apply_stress_free (sps_set_bcs with ifsigman = 1 and wall
     // dummies): zero before the first derivative pass (cleared below)
     if (params->no_bcs > 0 && nt2 > nt) rc |= dalloc(h->nodeinfo, nn) | dalloc(h->bcint_prev, nn);
+    if (h->xsph) rc |= dalloc(h->xsph_v, (size_t)nt);
+    if (!rc) rc = alloc_lists(h);
     if (rc) return bail(rc);
     if (hipHostMalloc((void **)&h->pinned, 64 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
         return bail(fail(SPS_ENOMEM, "pinned staging allocation"));
@@ -1631,13 +1676,12 @@ extern "C" void sps_destroy(sps_handle *h) {
     h->S[1].release();
     dfree(h->x0); dfree(h->vel0); dfree(h->rk_vel); dfree(h->rhs2); dfree(h->f_bound);
     dfree(h->art_visc); dfree(h->stress0); dfree(h->rk_stress); dfree(h->rhs1); dfree(h->grad_u);
-    dfree(h->rk_dev); dfree(h->sig2); dfree(h->stress_b); dfree(h->av_nodes); dfree(h->ddev); dfree(h->grid); dfree(h->split); dfree(h->bparts);
-    dfree(h->cellkey); dfree(h->new_cell); dfree(h->cell); dfree(h->kcount); dfree(h->kstart);
+    dfree(h->rk_dev); dfree(h->sig2); dfree(h->av_nodes); dfree(h->ddev); dfree(h->grid); dfree(h->split); dfree(h->bparts);
+    dfree(h->cellkey); dfree(h->cell); dfree(h->kcount); dfree(h->kstart);
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
     dfree(h->cnt); dfree(h->off); dfree(h->scan_state); dfree(h->scan_ticket); dfree(h->cstart_rm); dfree(h->err);
-    dfree(h->list_ia); dfree(h->list_iah); dfree(h->list_ibh); dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya); dfree(h->list_ib);
-    dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->type_counts); dfree(h->tiles); dfree(h->plans);
-    dfree(h->list_wb); dfree(h->xsph_v);
+    dfree(h->list_mem); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->type_counts); dfree(h->tiles); dfree(h->plans);
+    dfree(h->xsph_v);
     dfree(h->x_build); dfree(h->dmax); dfree(h->surr_count); dfree(h->surr_slot); dfree(h->surr_sn);
     dfree(h->surr_str); dfree(h->surr_feat); dfree(h->surr_stats); dfree(h->plog); dfree(h->surr_mat);
     dfree(h->mtab); dfree(h->mat_orig); dfree(h->pairs_total);

@@ -1330,14 +1330,15 @@ __global__ void k_stage_first(StateBufs S, Work W, int adapt, double tanfi, doub
 // of a second array; its walks read the partners' fields from the state.
 struct PairLists {
     unsigned long long *ia, *ib;    // [tile][lg][TILE]: four entries per word
-    unsigned long long *iah, *ibh;  // the same, upper halves of the entries by slot
+    unsigned long long *iah, *ibh;  // the same, upper halves of the entries by slot (null: no
+                                    // lists for tiles without a window)
     float4 *wa, *gxa, *gya;         // list A: w, dW/dx_r, dW/dy_r of those entries
     float4 *gxb, *gyb;              // list B (nodes): dW/dx_r, dW/dy_r
-    float4 *wb;                     // list B: w (XSPH only; null otherwise, and then stress
-                                    // points have no list B)
+    float4 *wb;                     // list B: w (XSPH)
     unsigned short *deg_a, *deg_b;  // per slot: nodes and stress points / nodes
     unsigned char *ok;              // per tile (node tiles, then SP tiles): LIST_*
     int lg;                         // words per receiver and list; more entries: LIST_NONE
+    bool sp_b;                      // stress points have a list B too (XSPH)
     int ntile_n;                    // node tiles
     const int2 *range;              // per tile: its receivers (k_count_tiles_sort)
     unsigned *types;                // per tile: pairs its receivers discover, by partner kind
@@ -1351,6 +1352,9 @@ struct PairLists {
     // the reference (2_...:579, 870-871), counted within 2h at the search
     int *nodeinfo;
 };
+
+// Words of a list where memory allows no more (alloc_lists).
+constexpr int LIST_WORDS = 12;
 
 // What a tile's lists hold: nothing (a receiver has more partners than they
 // take), window indices, or storage slots.
@@ -1530,7 +1534,7 @@ __device__ __forceinline__ void list_tile(int tile, const SearchView &V, const d
     }
     const int r = T.first + (int)threadIdx.x;
     // list B: a node's node partners; with XSPH also a stress point's stress-point partners
-    const bool list_b = KR == KIND_NODE || PL.wb != nullptr;
+    const bool list_b = KR == KIND_NODE || PL.sp_b;
     int self_base = 0;
     bool lds = T.fits;
     if (lds) {
@@ -1570,6 +1574,8 @@ __device__ __forceinline__ void list_tile(int tile, const SearchView &V, const d
     unsigned n_node = 0;          // node receivers: node partners (all, not only discovered)
     bool any_dummy = false;       // node receivers: a wall-dummy partner
     IdxWriter la, lb;
+    const bool keep = lds || PL.iah != nullptr;
+    const int lg = keep ? PL.lg : 0;   // 0: the entries are only counted
     const bool active = r < T.end && V.cell[r] < C.g.ndivt;
     if (active) {
         int cx, cy;
@@ -1637,9 +1643,9 @@ __device__ __forceinline__ void list_tile(int tile, const SearchView &V, const d
                             }
                             const unsigned e = ListEntry<SLOTS>::make(ks, j);
                             if (in_list_a(KR, ks))
-                                la.template put<SLOTS>(PL.lg, ltile, PL.ia, PL.iah, e);
+                                la.template put<SLOTS>(lg, ltile, PL.ia, PL.iah, e);
                             else if (ks == KR && list_b)
-                                lb.template put<SLOTS>(PL.lg, ltile, PL.ib, PL.ibh, e);
+                                lb.template put<SLOTS>(lg, ltile, PL.ib, PL.ibh, e);
                         }
                     }
                 }
@@ -1654,13 +1660,13 @@ __device__ __forceinline__ void list_tile(int tile, const SearchView &V, const d
         } else {
             walk(GlobalCells{V.kstart, C.g, C.L}, XHFields{x, hsml}, Uni{}, Gen{});
         }
-        la.finish(PL.lg, ltile, PL.ia, lds ? nullptr : PL.iah);
-        if (list_b) lb.finish(PL.lg, ltile, PL.ib, lds ? nullptr : PL.ibh);
+        la.finish(lg, ltile, PL.ia, lds ? nullptr : PL.iah);
+        if (list_b) lb.finish(lg, ltile, PL.ib, lds ? nullptr : PL.ibh);
         cnt[V.proc[r]] = fk[0] + fk[1] + fk[2];
     }
     block_type_counts(fk, tsum, PL.types + 3 * (size_t)ltile);
     const int lmax = 4 * PL.lg;
-    const bool over = la.n > lmax || lb.n > lmax;
+    const bool over = !keep || la.n > lmax || lb.n > lmax;
     const bool any_over = __syncthreads_or(over);
     if (threadIdx.x == 0) PL.ok[ltile] = any_over ? LIST_NONE : lds ? LIST_WINDOW : LIST_SLOTS;
     if (FILL && !any_over && active) {
@@ -1754,7 +1760,7 @@ __global__ __launch_bounds__(TILE) void k_list_order(SearchView V, PairLists PL)
     const int pr = C.any_fwd ? V.proc[r] : 0;
     const bool node = tile < PL.ntile_n;
     for (int l = 0; l < 2; ++l) {
-        if (l && !node && !PL.wb) continue;
+        if (l && !node && !PL.sp_b) continue;
         const int n = l ? PL.deg_b[r] : PL.deg_a[r];
         unsigned long long *ip = l ? PL.ib : PL.ia, *hp = ok == LIST_SLOTS ? (l ? PL.ibh : PL.iah) : nullptr;
         int fwd = C.any_fwd ? n : 0;   // entries with d < M

@@ -261,3 +261,7 @@ extern "C" void emu_set_memory(long long n) {
     std::lock_guard<std::mutex> lock(emu::mem_mu);
     emu::mem_total = n < 0 ? (size_t)1 << 40 : emu::mem_used + (size_t)n;
 }
+extern "C" long long emu_memory_used() {
+    std::lock_guard<std::mutex> lock(emu::mem_mu);
+    return (long long)emu::mem_used;
+}

@@ -143,9 +143,39 @@ def small_state_without_events(lib):
     return [k for k in ("x", "vel", "stress", "mass", "internal_vars", "x00") if not equal(got[k], want[k])]
 
 
+def lists_short_of_memory(lib):
+    """Bodies whose lists of storage slots, and longer lists for several stress
+    points a cell, do not fit beside the rest: the same steps without them."""
+    emu = ctypes.CDLL(lib)
+    emu.emu_memory_used.restype = ctypes.c_longlong
+    bad = []
+    for name, mode, least in (("t5_sp4", sps.MODE_ORDERED, 0.5), ("t4_xsph", sps.MODE_ORDERED, 0.9),
+                              ("t3_elastic", sps.MODE_FAST, 0.9)):
+        sims, used = [], []
+        for limit in (None, least):
+            before = emu.emu_memory_used()
+            if limit:
+                emu.emu_set_memory(int(limit * used[0]))
+            deck = deck_of(name)
+            parts = sps.build_particles(deck)
+            sim = sps.Simulation(sps.make_params(deck, parts, mode=mode), lib)
+            used.append(emu.emu_memory_used() - before)
+            emu.emu_set_memory(-1)
+            sim.set_state(sps.initial_state(parts, sim.niv))
+            sim.deck, sim.parts = deck, parts
+            sim.step(4)
+            sims.append(sim)
+        print(f"{name}: {used[0]} and {used[1]} bytes")
+        bad += [f"{name}: {k}" for k in same_state(*sims)]
+        for sim in sims:
+            sim.close()
+    return bad
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
                                  network_attached_again_after_capture, state_after_failed_event,
-                                 state_short_of_memory, small_state_without_events)}
+                                 state_short_of_memory, small_state_without_events,
+                                 lists_short_of_memory)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])
