@@ -10,7 +10,7 @@ order and results.  These are compile-time constants of the LDS layouts
 
   python stress-particle-sph_amd/tune_tiles.py build        # any machine with hipcc
   python stress-particle-sph_amd/tune_tiles.py measure      # on the GPU
-  python stress-particle-sph_amd/tune_tiles.py write T.json
+  python stress-particle-sph_amd/tune_tiles.py write T.json [NAME]
 
 `build` compiles the library once per candidate into _build/tiles/<name>/.
 `measure` runs each candidate in a process of its own on the workloads --
@@ -20,7 +20,9 @@ reuse) -- over `--steps` steps after a warm-up, checks that each
 candidate's state after the FP64 steps is bitwise the first candidate's
 (the results may not depend on the tile), and prints a JSON table.
 `write` puts the candidate with the smallest geometric mean of times
-relative to the first candidate into csrc/sps_tiles.h.
+relative to the first candidate into csrc/sps_tiles.h, or NAME (the candidate
+in use, say, where the fastest is ahead by less than two runs of one differ: the
+mixed form's results depend on which tiles have a window).
 """
 from __future__ import annotations
 
@@ -45,12 +47,14 @@ BUILD = os.path.join(ROOT, "_build", "tiles")
 # 37.3 KiB at t256, 33.6 at t256s, 22.9 at t128, 19.1 at t128s; the stage
 # kernels at most 35 KiB at t256.  With one smoothing length the list build
 # leaves h out of its window: 27.9 KiB with its plans at t256, five
-# workgroups per CU; 26.9 KiB at t256m (608), six.  The stage kernels k_sp_update and
-# k_deriv_nodes are held to 3 waves per SIMD by their registers unless
-# compiled for 4 (STAGE_WAVES), which spills a few of them.
+# workgroups per CU; 26.9 KiB at t256m (608), six.  The stage kernels k_sp_update,
+# k_deriv_nodes and the launches of k_sp_update beside the nodes' passes (both
+# forms) are held to 3 waves per SIMD by their registers unless compiled for
+# 4 (STAGE_WAVES), which spills a few of them.
 CANDIDATES = {
     "t256": (256, 24, 640, 192, 0),
     "t256m": (256, 24, 608, 192, 0),
+    "t256mw4": (256, 24, 608, 192, 4),
     "t256w4": (256, 24, 640, 192, 4),
     "t256s": (256, 24, 576, 160, 0),
     "t256sw4": (256, 24, 576, 160, 4),
@@ -134,23 +138,23 @@ def measure(names, steps, warmup, instances, timeout):
     return table
 
 
-def write(table_path):
+def write(table_path, name=None):
     table = json.load(open(table_path))
-    best = next(r for r in table["candidates"] if r["name"] == table["best"])
+    best = next(r for r in table["candidates"] if r["name"] == (name or table["best"]))
     t, r, c, d, w = best["tile"]
     lines = ["// Tile width and window capacities of the tiled pair kernels.",
-             "// tune_tiles.py rewrites this file with the fastest candidate it measured;",
+             f"// tune_tiles.py rewrites this file with a candidate it measured, here {best['name']};",
              "// a compiler definition (-DSPS_TILE=... and the others) overrides it.",
              "// Measured (ms per step: FP64 on the 1 M slope; batched ensemble, mixed):"]
     for row in table["candidates"]:
-        lines.append(f"//   {row['name']:6s} {tuple(row['tile'])}: {row['fp64_1m_ms_per_step']}"
+        lines.append(f"//   {row['name']:7s} {tuple(row['tile'])}: {row['fp64_1m_ms_per_step']}"
                      + (f", {row['batched_ms_per_step']}" if "batched_ms_per_step" in row else "")
                      + f" (relative {row['relative_time']})")
     lines += ["#pragma once"]
     for macro, val, what in (("SPS_TILE", t, "receivers per workgroup"), ("SPS_TROWS", r, "most window rows staged"),
                              ("SPS_CAP", c, "staged partners of a main kind per window"),
                              ("SPS_CAP_D", d, "staged dummies per window"),
-                             ("SPS_STAGE_WAVES", w, "waves per SIMD of the FP64 stage kernels (0: the compiler's choice)")):
+                             ("SPS_STAGE_WAVES", w, "waves per SIMD of the stage kernels with STAGE_OCCUPANCY (0: the compiler's choice)")):
         lines += [f"#ifndef {macro}", f"#define {macro} {val}  // {what}", "#endif"]
     open(os.path.join(CSRC, "sps_tiles.h"), "w").write("\n".join(lines) + "\n")
     print(f"[tune_tiles] wrote {best['name']} {tuple(best['tile'])} into csrc/sps_tiles.h")
@@ -172,7 +176,7 @@ def main():
     elif a.what == "measure":
         measure(names, a.steps, a.warmup, a.instances, a.timeout)
     elif a.what == "write":
-        write(a.rest[0])
+        write(*a.rest[:2])
     else:
         measure_one(a.rest[0], int(a.rest[1]), int(a.rest[2]), int(a.rest[3]))
 
