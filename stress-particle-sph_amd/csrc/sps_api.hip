@@ -7,9 +7,9 @@
 //   RK4 (2_...:653-802)                            -> k_stage_first, 4 x stage
 //   update_strain, stress_point_update, adapt      -> k_spu_nodes, k_sp_update
 //   position update and displacement               -> k_position
-// The search bins the particles and fixes the order of the pair list; every
-// stage kernel then walks each receiver's cell stencil in that order and
-// recomputes w and grad w, so no pair list is stored.
+// The search bins the particles, finds every receiver's pairs once and keeps
+// them in the order of the reference's list (PairLists); the stage kernels sum
+// over those lists.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -54,7 +54,7 @@ static int fail(int code, const char *fmt, ...) {
 static inline unsigned nblk(long long n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
 // Tiles held for n receivers, a multiple of the XCD count: n / TILE rounded
 // up, and with `strips` > 0 (tiles that end at strip ends, k_count_tiles_sort) one more
-// per strip of the domain box, at most twice as many in all.
+// per strip of the domain box, at most as many again and 16.
 static inline int ntiles(long long n, double strips) {
     const long long plain = (n + TILE - 1) / TILE;
     const long long extra = strips > 0 ? (long long)std::min(strips, (double)plain + 16) : 0;
@@ -1026,8 +1026,10 @@ static int mixed_step_graph(sps_handle *h, double dt, double time_sph, double gx
 // the step's pairs in list order; BC_or_not and the normals by original index.
 static int free_surface(sps_handle *h, const StateBufs &SB) {
     const int nn = h->nn, nt = h->nt;
-    // entries kept per particle: as many as its two pair lists hold; a body on
-    // its lattice has about 36 with one stress point a cell
+    // entries kept per particle: as many as one of its lists holds, 48 with one
+    // stress point a cell, where a body on its lattice has about 36.  (The four
+    // lanes of a particle share up to SURF_LDS of them; with more than either
+    // number they walk its cells.)
     const int cap = 4 * h->list_words;
     const size_t ne = (size_t)nt * cap;
     int rc = 0;

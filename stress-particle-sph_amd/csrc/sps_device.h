@@ -122,37 +122,6 @@ __device__ __forceinline__ void cubic_kernel_f(double r, double dx0, double dx1,
     gy = (float)g1;
 }
 
-// The w of cubic_kernel alone, with the same operations.
-__device__ __forceinline__ float cubic_w_f(double r, double hs, double factor) {
-    double q = r / hs;
-    double wd;
-    if (q >= 0.0 && q <= 1.0) {
-        wd = factor * ((double)(2.0f / 3.0f) - q * q + (q * (q * q)) / 2.0);
-    } else if (q > 1.0 && q <= 2.0) {
-        double t = 2.0 - q;
-        wd = factor * 1.0 / 6.0 * (t * (t * t));
-    } else {
-        wd = 0.0;
-    }
-    return (float)wd;
-}
-
-// The w of cubic_kernel alone, with the same operations.
-__device__ __forceinline__ float cubic_w(double r, double hs, double pi) {
-    double q = r / hs;
-    double factor = 15.0 / (7.0 * pi * hs * hs);
-    double wd;
-    if (q >= 0.0 && q <= 1.0) {
-        wd = factor * ((double)(2.0f / 3.0f) - q * q + (q * (q * q)) / 2.0);
-    } else if (q > 1.0 && q <= 2.0) {
-        double t = 2.0 - q;
-        wd = factor * 1.0 / 6.0 * (t * (t * t));
-    } else {
-        wd = 0.0;
-    }
-    return (float)wd;
-}
-
 // The acceptance decision of pair_distance alone, for a pair whose limit
 // 2*mhsml and squared-distance bounds are precomputed (per pair, or once
 // per receiver when every h is the same: (h + h)/2 is then h exactly).

@@ -19,12 +19,12 @@
 // the order of its partners in (cell, kind, original index) -- the forward
 // stencil walk -- so a receiver's partners are visited with a reverse walk
 // (pairs d >= M) followed by a forward walk (pairs d < M) and added one by
-// one in that order.  The search (k_count_lists) does that walk once per
-// step and stores each receiver's accepted partners in forward walk order
-// with the pair's single-precision w and grad w (PairLists); the stage
-// kernels read the lists forwards, and backwards for the pairs d >= M, from
-// windows of the partners staged in LDS: one lane per receiver, no atomics,
-// results bitwise equal to the reference.
+// one in that order.  The search does that walk once per step (k_count_lists),
+// stores each receiver's accepted partners with the pair's single-precision w
+// and grad w (PairLists) and, where pairs lie past M, turns the lists into that
+// order (k_list_order); the stage kernels read them forwards, from windows of
+// the partners staged in LDS or, by storage slot, from the state: one lane per
+// receiver, no atomics, results bitwise equal to the reference.
 #include <type_traits>
 
 #include "sps_device.h"
@@ -74,7 +74,7 @@ struct Split {
 //
 // The search is a chain of small passes: on bodies of up to 100 k particles
 // each costs the 4 us between two dependent launches whatever it does, so
-// passes that read the same fields share a launch (fifteen launches for
+// passes that read the same fields share a launch (fourteen launches for
 // thirty-one; 10 k collapse 449 -> 419 us per step).
 __global__ void k_bounds_partial(const double2 *__restrict__ x, const double *__restrict__ hsml,
                                  int *__restrict__ ood, int nt2, double xmin0, double xmin1, double xmax0,
@@ -723,10 +723,10 @@ struct GlobalFields {
 // the strip part of the window is ONE contiguous storage run (rows follow
 // each other inside a strip) and each halo cell a short run, so staging is
 // a coalesced copy.  A table gives every window cell its LDS run.  A tile
-// whose receivers span two strips or too many rows, whose window overflows
-// the LDS capacity, or that holds a receiver with pairs on both sides of M
-// walks the global storage instead; both paths visit the same pairs in the
-// same order.
+// whose receivers span two strips or too many rows, or whose window overflows
+// the LDS capacity, reads its partners from the global storage through lists
+// of slots, and one that has no lists walks its cells there; all visit the
+// same pairs in the same order.
 //
 // The tile width and the window capacities are build parameters
 // (sps_tiles.h, written by tune_tiles.py from timings of the candidates;
@@ -752,9 +752,11 @@ constexpr int TWAVES = TILE / 64;      // waves of a tile
 static_assert(CAP > 0 && CAP < (1 << 14) && CAP_D > 0 && CAP_D < (1 << 14),
               "list entries carry a 14-bit window index");
 static_assert(CAP % 8 == 0 && CAP_D % 8 == 0, "every staged field starts 16-byte aligned");
-// waves per SIMD the FP64 stage kernels k_sp_update and k_deriv_nodes are
-// compiled for (their registers otherwise allow 3): 0 leaves it to the
-// compiler; more waves may cost register spills
+// waves per SIMD that k_sp_update, k_deriv_nodes and the launches of the stress
+// points' update beside the nodes' passes (both forms) are compiled for (their
+// registers otherwise allow 3): 0 leaves it to the compiler; more waves may
+// cost register spills (the mixed form's beside launches spill 6 and 12 of 127
+// and still gain: 8.0 -> 7.3 ms per step of the batched ensemble)
 #if SPS_STAGE_WAVES > 0
 #define STAGE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(SPS_STAGE_WAVES)))
 #else
@@ -1050,14 +1052,14 @@ __device__ __forceinline__ Tile make_tile(int2 range, int kr, const SearchView &
 
 // Receivers [x, y) of every tile (empty past the last one): block 0 the node
 // tiles, block 1 the stress points'.  A tile that crosses from one strip into
-// the next has no window and walks the global storage, 86 us against 15 us
+// the next has no window.  Walking the global storage it took 86 us against 15 us
 // for a tile in its strip on the 10 k-particle collapse, where one tile in
 // four crossed and every stage kernel took as long as its crossing tiles; so
 // each strip starts a tile of its own (the last tile of a strip is partly
 // idle: half a tile per strip of about 75 at 1 M nodes).  The out-of-domain
 // particles' bucket counts as one more strip.  When the strips would need
-// more tiles than the capacity cap holds (bodies much taller than wide in
-// many strips), or with aligned = 0, the receivers are cut every TILE slots.
+// more tiles than the capacity cap holds (low, wide bodies in many strips), or
+// with aligned = 0, the receivers are cut every TILE slots.
 // aligned is 0 for the mixed form: its positions are rounded relative to the
 // tile's first receiver, so its tiles are part of its result.  tstart holds
 // TSTART_MAX entries per block.  The launch's other blocks sort the buckets.
@@ -1319,8 +1321,7 @@ __global__ void k_stage_first(StateBufs S, Work W, int adapt, double tanfi, doub
 // forward walk order as 16-bit entries kind << 14 | window index (the window
 // laid out exactly as the stage kernels stage it), with w and grad w rounded
 // to single precision as the reference's pair list stores them
-// (2_...:1376-1378).  The reverse walk order is the forward list read
-// backwards.  List A: a node's stress-point and dummy partners, a stress
+// (2_...:1376-1378).  List A: a node's stress-point and dummy partners, a stress
 // point's node and dummy partners; list B: a node's node partners.  Entries
 // come four to a word, words of a tile lane-interleaved, so a wave reads its
 // lanes' next four entries with one coalesced load per array.

@@ -92,7 +92,7 @@ __device__ __forceinline__ void put_weight(bf16_t *__restrict__ wf, bf16_t *__re
 // the backward pass down to the gradients at every layer's output.  The rows'
 // activations stay in the wave: a layer's result is laid out for the next
 // product through 4 KiB of LDS of the wave's own, the pre-activations keep
-// their registers for the way back, and only what k_gemm_bf16_dw contracts
+// their registers for the way back (256 registers, 12 of them in scratch), and only what k_gemm_bf16_dw contracts
 // over the rows is stored, as tile words (four consecutive rows of a column
 // are what a lane holds of a result and what it needs as an operand there).
 // The weights of a layer (32 KiB, in operand order) are fetched into registers
@@ -267,7 +267,7 @@ template <bool GRAD> __global__ __launch_bounds__(256, 2) void k_gemm_bf16_chain
 // Weight gradients: dW = H^T dZ of the layers and the bias gradients (a row
 // of ones in the place of H^T), over a chunk of 16-row tiles a workgroup;
 // blockIdx.y: 0 the second layer, 1 the third, 2 the first and the last.
-// Its sums are part[chunk], which k_mlp_reduce adds up: with atomics on the
+// Its sums are part[chunk], which k_mlp_loss_reduce adds up: with atomics on the
 // 37 k gradients every chunk had to be long to keep their number down.
 // A wave takes two rows of 16 x 16 tiles of dW (64 registers of sums).
 __global__ __launch_bounds__(256) void k_gemm_bf16_dw(NetPass g, int nrb, int chunk, float *__restrict__ part) {
