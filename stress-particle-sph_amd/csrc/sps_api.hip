@@ -682,6 +682,10 @@ static int size_cells(sps_handle *h, const double *hsml) {
         return fail(SPS_EINVAL, "domain box too large for the cell grid (%.3g cells)", cells);
     int cap = (int)cells + 16;
     int rc = 0;
+    // from here on the old state has no search buffers to step with, and a
+    // captured step none to replay
+    h->have_state = false;
+    drop_graphs(h);
     size_t L = 3 * ((size_t)cap + 1) + 1;
     rc |= dalloc(h->kcount, L); rc |= dalloc(h->kstart, L); rc |= dalloc(h->kfill, L);
     rc |= dalloc(h->cstart_rm, (size_t)cap + 2);
@@ -710,20 +714,21 @@ extern "C" int sps_set_state(sps_handle *h, const sps_state *st) {
             return fail(SPS_EINVAL, "itype(%d) = %d; the hot path needs 2 for nodes, 1 for stress points, 25 for dummies",
                         i + 1, st->itype[i]);
     }
+    if (h->dp.do_bforce) {
+        double hmin = 1e300;
+        for (int i = 0; i < h->nt2; ++i) hmin = std::min(hmin, st->hsml[i]);
+        if (hmin > 0 && !(0.75 * h->p.dx < 2 * hmin))
+            return fail(SPS_EINVAL, "wall force reach 0.75*dx must lie inside the kernel support");
+    }
+    HIP_TRY(hipSetDevice(h->device));
     int rc = size_cells(h, st->hsml);
+    if (rc) return rc;
     // smoothing lengths do not change on the path: one value for all lets
     // the search precompute its acceptance bounds
     h->h_uniform = st->hsml[0] > 0 ? st->hsml[0] : 0.0;
     for (int i = 1; i < h->nt2 && h->h_uniform > 0; ++i)
         if (!(st->hsml[i] == h->h_uniform)) h->h_uniform = 0.0;
     h->dp.h_uni = h->h_uniform > 0;
-    if (rc) return rc;
-    if (h->dp.do_bforce) {
-        double hmin = 1e300;
-        for (int i = 0; i < h->nt2; ++i) hmin = std::min(hmin, st->hsml[i]);
-        if (!(0.75 * h->p.dx < 2 * hmin))
-            return fail(SPS_EINVAL, "wall force reach 0.75*dx must lie inside the kernel support");
-    }
     const int nt2 = h->nt2, nt = h->nt, nn = h->nn;
     StateSet &S = h->S[h->cur];
     std::vector<double> tmp((size_t)nt2 * 4);

@@ -172,10 +172,45 @@ def lists_short_of_memory(lib):
     return bad
 
 
+def state_refused(lib):
+    """A state that is refused leaves the one before, and its captured step;
+    one that finds no memory leaves none to step on."""
+    deck = deck_of("c1_collapse")
+    deck.xs, deck.ys = (0.0, 5.5 * deck.dx, 0.0, 5.5 * deck.dx), (0.0, 0.0, 5.5 * deck.dx, 5.5 * deck.dx)
+    sims = direct_and_captured(lib, deck)
+    small = sps.initial_state(sims[0].parts, sims[0].niv)
+    small["hsml"] = 0.3 * small["hsml"]       # less than the wall force's reach, and a larger grid
+    bad = []
+
+    def refused(what, call, code):
+        try:
+            call()
+            bad.append(f"{what}: no error")
+        except sps.SpsError as e:
+            if e.code != code:
+                bad.append(f"{what}: {e}")
+
+    for sim in sims:
+        sim.step(2)
+    refused("small h", lambda: sims[1].set_state(small), -1)
+    for sim in sims:
+        sim.step(2)
+    bad += same_state(*sims)
+    small["hsml"] = 1.5 * small["hsml"]
+    emu = ctypes.CDLL(lib)
+    emu.emu_set_memory(0)
+    refused("no memory", lambda: sims[1].set_state(small), -2)
+    emu.emu_set_memory(-1)
+    refused("step", lambda: sims[1].step(1), -5)
+    sims[1].set_state(small)
+    sims[1].step(1)
+    return bad
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
                                  network_attached_again_after_capture, state_after_failed_event,
                                  state_short_of_memory, small_state_without_events,
-                                 lists_short_of_memory)}
+                                 lists_short_of_memory, state_refused)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])
