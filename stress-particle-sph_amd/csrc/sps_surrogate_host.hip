@@ -24,6 +24,7 @@ static int mlp_reserve(sps_mlp *ml, int rows) {
     rows = (rows + 63) / 64 * 64;
     if (rows <= ml->rows) return 0;
     const size_t r = (size_t)rows;
+    ml->rows = 0;   // until every buffer is there
     int rc = 0;
     rc |= dalloc(ml->Y, r * MLP_OUT); rc |= dalloc(ml->X, r * MLP_IN / 4); rc |= dalloc(ml->dY, r * MLP_OUT / 4);
     for (int l = 0; l < 3; ++l) rc |= dalloc(ml->H[l], r * MLP_H / 4) | dalloc(ml->dZ[l], r * MLP_H / 4);
@@ -192,6 +193,7 @@ extern "C" int sps_mlp_forward(sps_mlp *ml, int64_t n, const float *x, float *y)
     if (!ml || !x || !y || n < 0) return fail(SPS_EINVAL, "bad argument");
     HIP_TRY(hipSetDevice(ml->device));
     hipStream_t st = ml->stream;
+    if (!ml->rows) return fail(SPS_ENOMEM, "the network has no work buffers: an earlier call found no memory");
     int rc = mlp_upload_set(ml, n, x, nullptr);
     if (rc) return rc;
     std::vector<float> yb;
@@ -374,6 +376,7 @@ static int surrogate_correct(sps_handle *h, const StateBufs &SB) {
     sps_mlp *ml = h->mlp;
     hipStream_t st = h->stream;
     const int cap = h->surr_cap;
+    if (ml->rows < cap) return fail(SPS_ENOMEM, "the network has no work buffers: an earlier call found no memory");
     const SurrogateDev G = surrogate_dev(h);
     mlp_forward(ml, st, h, h->surr_feat.p, cap, (const int *)h->surr_count.p);
     MLAUNCH((unsigned)((cap + 255) / 256), 256, k_surrogate_apply, G, ml->Y.p, SB.stress, h->surr_tol);
@@ -388,7 +391,7 @@ extern "C" int sps_set_surrogate(sps_handle *h, sps_mlp *ml, double stress_scale
         return fail(SPS_EINVAL, "scales must be > 0 and the tolerance >= 0");
     if (ml && ml->device != h->device) return fail(SPS_EINVAL, "network and handle on different devices");
     HIP_TRY(hipSetDevice(h->device));
-    h->mlp = ml;
+    h->mlp = nullptr;   // until all that a step with it needs is there
     drop_graphs(h);
     if (!ml) return 0;
     const int cap = h->ns > 0 ? h->ns : 1;
@@ -404,6 +407,7 @@ extern "C" int sps_set_surrogate(sps_handle *h, sps_mlp *ml, double stress_scale
     HIP_TRY(hipMemsetAsync(h->surr_count.p, 0, 2 * sizeof(unsigned), h->stream));
     HIP_TRY(hipMemsetAsync(h->surr_stats.p, 0, 2 * sizeof(unsigned long long), h->stream));
     HIP_TRY(hipStreamSynchronize(ml->stream));   // the network's own uploads are done
+    h->mlp = ml;
     return 0;
 }
 

@@ -207,10 +207,43 @@ def state_refused(lib):
     return bad
 
 
+def network_without_memory(lib):
+    """A network that finds no memory to grow for a larger simulation: an
+    error there, and in the next step of the one that used it; both work once
+    it has grown."""
+    net = surrogate.Network(sps.load_library(lib), seed=3, batch_rows=64)
+    first = direct_and_captured(lib, deck_of("t2_cspm"))[1]
+    surrogate.attach(first, net, 1e4, 1e4)
+    first.step(12)
+    larger = sps.Simulation.from_deck(deck_of("v3_vslope_sp3"), lib_path=lib, mode=sps.MODE_FAST)
+    emu, bad = ctypes.CDLL(lib), []
+
+    def refused(what, call):
+        try:
+            call()
+            bad.append(f"{what}: no error")
+        except sps.SpsError as e:
+            if e.code != -2:
+                bad.append(f"{what}: {e}")
+
+    emu.emu_set_memory(1 << 20)
+    refused("attach", lambda: surrogate.attach(larger, net, 1e4, 1e4))
+    emu.emu_set_memory(-1)
+    refused("step", lambda: first.step(1))
+    refused("forward", lambda: net.forward(np.zeros((3, 10), dtype=np.float32)))
+    larger.step(1)                               # without the network
+    surrogate.attach(larger, net, 1e4, 1e4)
+    larger.step(1)
+    first.set_state(sps.initial_state(first.parts, first.niv))
+    first.step(12)
+    return bad
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
                                  network_attached_again_after_capture, state_after_failed_event,
                                  state_short_of_memory, small_state_without_events,
-                                 lists_short_of_memory, state_refused)}
+                                 lists_short_of_memory, state_refused,
+                                 network_without_memory)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])

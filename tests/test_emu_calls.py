@@ -16,7 +16,8 @@ import build_emu  # noqa: E402
 CASES = ["plastic_log_after_capture", "prescribed_values_after_capture",
          "network_attached_again_after_capture", "state_after_failed_event",
          "state_short_of_memory", "small_state_without_events",
-         "lists_short_of_memory", "state_refused"]
+         "lists_short_of_memory", "state_refused",
+         "network_without_memory"]
 
 
 @pytest.fixture(scope="module")
