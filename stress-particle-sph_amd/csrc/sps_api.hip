@@ -1590,8 +1590,17 @@ extern "C" int sps_set_materials(sps_handle *h, int32_t nmat, const double *tabl
         const double *t = table + 10 * k;
         tab[k] = Material{t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9]};
     }
-    int rc = dalloc(h->mtab, (size_t)nmat) | dalloc(h->mat_orig, (size_t)h->nt2) | h->S[0].mat_alloc(h->nt2) |
-             h->S[1].mat_alloc(h->nt2);
+    // the table last, and beside the one in use: without memory that stays
+    int rc = dalloc(h->mat_orig, (size_t)h->nt2) | h->S[0].mat_alloc(h->nt2) | h->S[1].mat_alloc(h->nt2);
+    if (!rc && h->mtab.n < (size_t)nmat) {
+        DBuf<Material> larger;
+        rc = dalloc(larger, (size_t)nmat);
+        if (!rc) {
+            drop_graphs(h);
+            dfree(h->mtab);
+            h->mtab = larger;
+        }
+    }
     if (rc) return rc;
     HIP_TRY(hipMemcpy(h->mtab.p, tab.data(), (size_t)nmat * sizeof(Material), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(h->mat_orig.p, mat, (size_t)h->nt2 * sizeof(int), hipMemcpyHostToDevice));

@@ -239,11 +239,35 @@ def network_without_memory(lib):
     return bad
 
 
+def materials_without_memory(lib):
+    """A larger table of materials that finds no memory leaves the one before."""
+    sims = direct_and_captured(lib, deck_of("t3_elastic"))
+    p = sims[0].params
+    row = [p.props[12], p.props[13], p.props[2], p.props[3], p.D11, p.D22, p.D12, p.D33, p.D41, p.D42]
+    mat = np.zeros(sims[0].n2, dtype=np.int32)
+    for sim in sims:
+        sim.set_materials(np.array([row]), mat)
+        sim.step(2)
+    bad = []
+    emu = ctypes.CDLL(lib)
+    emu.emu_set_memory(0)
+    try:
+        sims[1].set_materials(np.array([row] * 50), mat)
+        bad.append("no error")
+    except sps.SpsError as e:
+        if e.code != -2:
+            bad.append(str(e))
+    emu.emu_set_memory(-1)
+    for sim in sims:
+        sim.step(2)
+    return bad + same_state(*sims)
+
+
 CASES = {f.__name__: f for f in (plastic_log_after_capture, prescribed_values_after_capture,
                                  network_attached_again_after_capture, state_after_failed_event,
                                  state_short_of_memory, small_state_without_events,
                                  lists_short_of_memory, state_refused,
-                                 network_without_memory)}
+                                 network_without_memory, materials_without_memory)}
 
 if __name__ == "__main__":
     bad = CASES[sys.argv[2]](sys.argv[1])

@@ -17,7 +17,7 @@ CASES = ["plastic_log_after_capture", "prescribed_values_after_capture",
          "network_attached_again_after_capture", "state_after_failed_event",
          "state_short_of_memory", "small_state_without_events",
          "lists_short_of_memory", "state_refused",
-         "network_without_memory"]
+         "network_without_memory", "materials_without_memory"]
 
 
 @pytest.fixture(scope="module")
