@@ -185,7 +185,8 @@ int sps_create(const sps_params *params, sps_handle **out);
 /* Copy the state in (host -> library).  Replaces the implicit sharing of the
  * module globals listed in sps_state.  The pair-list high-water mark is not
  * touched: like the reference (2_...:1290-1294) it restarts at zero on the
- * step whose itimestep_sph is 1. */
+ * step whose itimestep_sph is 1.  A refused state (SPS_EINVAL) leaves the one
+ * before; after SPS_ENOMEM the handle has none until one is set. */
 int sps_set_state(sps_handle *h, const sps_state *st);
 
 /* Advance nsteps steps of dt.  One step is one `call time_integration`
