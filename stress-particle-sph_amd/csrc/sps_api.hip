@@ -22,7 +22,6 @@
 #include <atomic>
 #include <mutex>
 #include <thread>
-#include <type_traits>
 
 #include "../../include/sps.h"
 #include "sps_kernels.hip"
@@ -71,14 +70,16 @@ template <typename T>
 struct DBuf {
     T *p = nullptr;
     size_t n = 0;
+    bool own = true;   // an allocation of its own (Carver)
 };
 
 template <typename T>
 static int dalloc(DBuf<T> &b, size_t n) {
     if (b.n >= n && b.p) return 0;
-    if (b.p) (void)hipFree(b.p);
+    if (b.p && b.own) (void)hipFree(b.p);
     b.p = nullptr;
     b.n = 0;
+    b.own = true;
     size_t cnt = n ? n : 1;
     hipError_t e = hipMalloc((void **)&b.p, cnt * sizeof(T));
     if (e != hipSuccess) return fail(SPS_ENOMEM, "hipMalloc of %zu bytes: %s", cnt * sizeof(T), hipGetErrorString(e));
@@ -88,9 +89,55 @@ static int dalloc(DBuf<T> &b, size_t n) {
 
 template <typename T>
 static void dfree(DBuf<T> &b) {
-    if (b.p) (void)hipFree(b.p);
+    if (b.p && b.own) (void)hipFree(b.p);
     b.p = nullptr;
     b.n = 0;
+    b.own = true;
+}
+
+// Buffers laid one after the other in one device allocation: each allocation of
+// 2 MiB or more takes up to 0.3 ms to make and 0.7 to free, whatever its size
+// (opening and closing a simulation of 42 k / 128 k / 507 k particles with one per
+// buffer 2.0 / 7.6 / 15.6 ms, so 0.8 / 1.1 / 1.9).  Used through lay_out.
+// SPS_SEPARATE_BUFFERS gives each an allocation of its own all the same, for builds
+// that check accesses.
+struct Carver {
+    char *base = nullptr;   // null: only the bytes are counted
+    size_t at = 0;
+    int rc = 0;
+    template <typename T> void operator()(DBuf<T> &b, size_t n) {
+        const size_t cnt = n ? n : 1;
+        if (base && !b.p) {
+#ifdef SPS_SEPARATE_BUFFERS
+            rc |= dalloc(b, cnt);
+#else
+            b.p = reinterpret_cast<T *>(base + at);
+            b.n = cnt;
+            b.own = false;
+#endif
+        }
+        at += (cnt * sizeof(T) + 255) & ~(size_t)255;
+    }
+};
+
+template <typename F> static size_t laid_out_bytes(F &&buffers) {
+    Carver c;
+    buffers(c);
+    return c.at;
+}
+
+// buffers(carver) names them and their lengths, the same in both calls.
+template <typename F> static int lay_out(DBuf<char> &mem, F &&buffers) {
+    Carver c;
+#ifdef SPS_SEPARATE_BUFFERS
+    const int rc = dalloc(mem, 1);
+#else
+    const int rc = dalloc(mem, laid_out_bytes(buffers));
+#endif
+    if (rc) return rc;
+    c.base = mem.p;
+    buffers(c);
+    return c.rc;
 }
 
 struct StateSet {
@@ -111,14 +158,12 @@ struct StateSet {
         s.mtab = mtab;
         return s;
     }
-    int alloc(int nn, int nt, int nt2) {
-        int rc = 0;
-        rc |= dalloc(x, nt2); rc |= dalloc(vel, nt2); rc |= dalloc(x00, nt2); rc |= dalloc(displ, nn);
-        rc |= dalloc(stress, nt2); rc |= dalloc(mass, nt2); rc |= dalloc(rho, nt2);
-        rc |= dalloc(hsml, nt2); rc |= dalloc(ivar1, nt); rc |= dalloc(fdr, nt);
-        rc |= dalloc(orig, nt2); rc |= dalloc(ood, nt2); rc |= dalloc(wallpos, nt2);
-        rc |= dalloc(horiz, nt2);
-        return rc;
+    void lay_out(Carver &take, int nn, int nt, int nt2) {
+        take(x, nt2); take(vel, nt2); take(x00, nt2); take(displ, nn);
+        take(stress, nt2); take(mass, nt2); take(rho, nt2);
+        take(hsml, nt2); take(ivar1, nt); take(fdr, nt);
+        take(orig, nt2); take(ood, nt2); take(wallpos, nt2);
+        take(horiz, nt2);
     }
     int mat_alloc(int nt2) { return dalloc(mat, nt2); }
     void release() {
@@ -163,11 +208,11 @@ struct sps_handle {
     DBuf<unsigned long long> scan_state;   // k_scan_sums: a word per run, the launch's number, the ticket counter
     unsigned scan_epoch = 0;
     DBuf<unsigned> scan_ticket;
+    DBuf<char> mem;               // the buffers that sps_create lays out
     // per-step pair lists of the tiled stage kernels, in list_mem (lay_lists)
     DBuf<char> list_mem;
-    unsigned long long *list_ia = nullptr, *list_ib = nullptr, *list_iah = nullptr, *list_ibh = nullptr;
-    float4 *list_wa = nullptr, *list_gxa = nullptr, *list_gya = nullptr;
-    float4 *list_gxb = nullptr, *list_gyb = nullptr, *list_wb = nullptr;
+    DBuf<unsigned long long> list_ia, list_ib, list_iah, list_ibh;
+    DBuf<float4> list_wa, list_gxa, list_gya, list_gxb, list_gyb, list_wb;
     int list_words = LIST_WORDS;  // words of four entries per receiver and list
     bool xsph = false;            // XSPH position update (list B also for stress points, with w)
     DBuf<double2> xsph_v;
@@ -266,9 +311,9 @@ struct sps_handle {
     long long prof_n[32] = {0};
 
     PairLists lists() {
-        return PairLists{list_ia,  list_ib,   list_iah, list_ibh, list_wa, list_gxa,   list_gya,
-                         list_gxb, list_gyb,  list_wb,  deg_a.p,  deg_b.p, tile_ok.p,  list_words,
-                         xsph,     ntile_n,   tile_range.p, type_counts.p, tiles.p, plans.p,
+        return PairLists{list_ia.p,  list_ib.p,  list_iah.p, list_ibh.p, list_wa.p, list_gxa.p, list_gya.p,
+                         list_gxb.p, list_gyb.p, list_wb.p,  deg_a.p,    deg_b.p,   tile_ok.p,  list_words,
+                         xsph,       ntile_n,    tile_range.p, type_counts.p, tiles.p, plans.p,
                          (outside || bcint) ? nodeinfo.p : nullptr};
     }
 };
@@ -499,16 +544,9 @@ static double gravity_factor(const sps_params *P, double time_sph) {
     return factg * P->ft_grav;
 }
 
-// The arrays of the pair lists with `words` words of four entries a list, laid
-// one after the other from base (null: no pointers, only the bytes); slots:
-// with the upper halves that lists of storage slots need.  One allocation for
-// all of them: each of 2 MiB or more takes up to 0.3 ms to make and to free.
-static size_t lay_lists(sps_handle *h, int words, bool slots, char *base) {
-    size_t at = 0;
-    auto take = [&](auto *&p, size_t n) {
-        p = base ? reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at) : nullptr;
-        at += (n * sizeof(*p) + 255) & ~(size_t)255;
-    };
+// The arrays of the pair lists with `words` words of four entries a list; slots:
+// with the upper halves that lists of storage slots need.
+static void lay_lists(sps_handle *h, int words, bool slots, Carver &take) {
     const size_t wt = (size_t)words * TILE;
     const size_t a = (size_t)(h->ntile_n + h->ntile_s) * wt, nodes = (size_t)h->ntile_n * wt;
     const size_t b = h->xsph ? a : nodes;   // list B: node tiles; with XSPH stress-point tiles too, and its w
@@ -526,7 +564,13 @@ static size_t lay_lists(sps_handle *h, int words, bool slots, char *base) {
         take(h->list_gyb, nodes);
         if (h->xsph) take(h->list_wb, a);
     }
-    return at;
+}
+
+static void free_lists(sps_handle *h) {
+    dfree(h->list_ia); dfree(h->list_ib); dfree(h->list_iah); dfree(h->list_ibh);
+    dfree(h->list_wa); dfree(h->list_gxa); dfree(h->list_gya);
+    dfree(h->list_gxb); dfree(h->list_gyb); dfree(h->list_wb);
+    dfree(h->list_mem);
 }
 
 // 48 entries a list, and 24 more per further stress point a node or cell (about
@@ -540,17 +584,16 @@ static int alloc_lists(sps_handle *h) {
     if (!h->mixed) words += 6 * (std::max(1, std::min(4, (h->ns + h->nn - 1) / h->nn)) - 1);
     size_t mem_free = 0, mem_total = 0;
     HIP_TRY(hipMemGetInfo(&mem_free, &mem_total));
-    const size_t least = lay_lists(h, LIST_WORDS, false, nullptr), full = lay_lists(h, words, true, nullptr);
-    bool slots = mem_free > least && full - least <= (mem_free - least) / 2;
-    if (slots && dalloc(h->list_mem, full)) slots = false;
-    if (!slots) {
-        words = LIST_WORDS;
-        const int rc = dalloc(h->list_mem, least);
-        if (rc) return rc;
+    auto longest = [&](Carver &take) { lay_lists(h, words, true, take); };
+    auto least = [&](Carver &take) { lay_lists(h, LIST_WORDS, false, take); };
+    const size_t need = laid_out_bytes(least), more = laid_out_bytes(longest) - need;
+    if (mem_free > need && more <= (mem_free - need) / 2 && !lay_out(h->list_mem, longest)) {
+        h->list_words = words;
+        return 0;
     }
-    h->list_words = words;
-    lay_lists(h, words, slots, h->list_mem.p);
-    return 0;
+    free_lists(h);
+    h->list_words = LIST_WORDS;
+    return lay_out(h->list_mem, least);
 }
 
 extern "C" int sps_create(const sps_params *params, sps_handle **out) {
@@ -603,22 +646,7 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(SPS_EDEVICE, "hipStreamCreate failed"));
     int nt2 = h->nt2, nt = h->nt, nn = h->nn;
-    rc = 0;
-    rc |= h->S[0].alloc(nn, nt, nt2);
-    rc |= h->S[1].alloc(nn, nt, nt2);
-    rc |= dalloc(h->x0, nt); rc |= dalloc(h->vel0, nt);
-    rc |= dalloc(h->rk_vel, nn); rc |= dalloc(h->rhs2, nn); rc |= dalloc(h->f_bound, nn);
-    rc |= dalloc(h->art_visc, nn); rc |= dalloc(h->stress0, nt); rc |= dalloc(h->rk_stress, nt);
-    rc |= dalloc(h->rhs1, nt); rc |= dalloc(h->grad_u, nt); rc |= dalloc(h->rk_dev, nt);
-    rc |= dalloc(h->sig2, nt); rc |= dalloc(h->av_nodes, nn > 0 ? nn : 1);
-    rc |= dalloc(h->ddev, nt);
-    rc |= dalloc(h->grid, 1); rc |= dalloc(h->split, 1); rc |= dalloc(h->err, 1); rc |= dalloc(h->pairs_total, 1);
     h->nbparts = std::min(1024, (int)nblk(nt2));
-    rc |= dalloc(h->bparts, 5 * (size_t)h->nbparts);
-    rc |= dalloc(h->cellkey, nt2); rc |= dalloc(h->cell, nt2);
-    rc |= dalloc(h->tmp_orig, nt2); rc |= dalloc(h->tmp_src, nt2); rc |= dalloc(h->proc, nt2);
-    rc |= dalloc(h->moved, nblk(nt2));
-    rc |= dalloc(h->proc_to_slot, nt2); rc |= dalloc(h->cnt, nt2); rc |= dalloc(h->off, nt2);
     // strips of 8 cells 2h wide with h = 0.8 dx, as small as the decks have it
     // (with smaller h and a body across the whole box k_count_tiles_sort may not find
     // room for tiles that end at strip ends and falls back)
@@ -626,27 +654,48 @@ extern "C" int sps_create(const sps_params *params, sps_handle **out) {
         : (params->xmax_domain[0] - params->xmin_domain[0]) / (STRIP * 1.6 * params->dx) + 2;
     h->ntile_n = ntiles(nn, strips);
     h->ntile_s = ntiles(nt - nn, strips);
-    rc |= dalloc(h->tile_start, 2 * (size_t)TSTART_MAX);
-    rc |= dalloc(h->tile_range, (size_t)h->ntile_n + h->ntile_s);
-    rc |= dalloc(h->type_counts, 3 * ((size_t)h->ntile_n + h->ntile_s + count_blocks(nt2 - nt)));
-    rc |= dalloc(h->deg_a, nt); rc |= dalloc(h->deg_b, h->xsph ? nt : nn);
-    rc |= dalloc(h->tile_ok, h->ntile_n + h->ntile_s + 1);
-    rc |= dalloc(h->tiles, h->ntile_n + h->ntile_s + 1);
-    rc |= dalloc(h->plans, 3 * (size_t)(h->ntile_n + h->ntile_s + 1));
-    rc |= dalloc(h->x_build, nt); rc |= dalloc(h->dmax, 1); rc |= dalloc(h->stepv, 4);
-    if (params->no_bcs > 0)
-        rc |= dalloc(h->bc_info, 8 * (size_t)nn) | dalloc(h->bc_vals, SPS_MAX_BCS);
-    // BC_or_not and the surface normals exist with BCs and with the position
-    // update, which runs the free-surface detection (3_...:1045-1047, 918)
-    if (params->no_bcs > 0 || params->update_x) rc |= dalloc(h->bc_or_not, nt) | dalloc(h->normal, nt);
-    if (h->outside) {
-        rc |= dalloc(h->inv, nt2); rc |= dalloc(h->nodeinfo, nn);
-        rc |= dalloc(h->x10, nn); rc |= dalloc(h->disp10, nn);
-    }
-    // bc_int for apply_stress_free (sps_set_bcs with ifsigman = 1 and wall
-    // dummies): zero before the first derivative pass (cleared below)
-    if (params->no_bcs > 0 && nt2 > nt) rc |= dalloc(h->nodeinfo, nn) | dalloc(h->bcint_prev, nn);
-    if (h->xsph) rc |= dalloc(h->xsph_v, (size_t)nt);
+    rc = lay_out(h->mem, [&](Carver &take) {
+        h->S[0].lay_out(take, nn, nt, nt2);
+        h->S[1].lay_out(take, nn, nt, nt2);
+        take(h->x0, nt); take(h->vel0, nt);
+        take(h->rk_vel, nn); take(h->rhs2, nn); take(h->f_bound, nn);
+        take(h->art_visc, nn); take(h->stress0, nt); take(h->rk_stress, nt);
+        take(h->rhs1, nt); take(h->grad_u, nt); take(h->rk_dev, nt);
+        take(h->sig2, nt); take(h->av_nodes, nn > 0 ? nn : 1);
+        take(h->ddev, nt);
+        take(h->grid, 1); take(h->split, 1); take(h->err, 1); take(h->pairs_total, 1);
+        take(h->bparts, 5 * (size_t)h->nbparts);
+        take(h->cellkey, nt2); take(h->cell, nt2);
+        take(h->tmp_orig, nt2); take(h->tmp_src, nt2); take(h->proc, nt2);
+        take(h->moved, nblk(nt2));
+        take(h->proc_to_slot, nt2); take(h->cnt, nt2); take(h->off, nt2);
+        take(h->tile_start, 2 * (size_t)TSTART_MAX);
+        take(h->tile_range, (size_t)h->ntile_n + h->ntile_s);
+        take(h->type_counts, 3 * ((size_t)h->ntile_n + h->ntile_s + count_blocks(nt2 - nt)));
+        take(h->deg_a, nt); take(h->deg_b, h->xsph ? nt : nn);
+        take(h->tile_ok, h->ntile_n + h->ntile_s + 1);
+        take(h->tiles, h->ntile_n + h->ntile_s + 1);
+        take(h->plans, 3 * (size_t)(h->ntile_n + h->ntile_s + 1));
+        take(h->x_build, nt); take(h->dmax, 1); take(h->stepv, 4);
+        if (params->no_bcs > 0) {
+            take(h->bc_info, 8 * (size_t)nn); take(h->bc_vals, SPS_MAX_BCS);
+        }
+        // BC_or_not and the surface normals exist with BCs and with the position
+        // update, which runs the free-surface detection (3_...:1045-1047, 918)
+        if (params->no_bcs > 0 || params->update_x) {
+            take(h->bc_or_not, nt); take(h->normal, nt);
+        }
+        if (h->outside) {
+            take(h->inv, nt2); take(h->nodeinfo, nn);
+            take(h->x10, nn); take(h->disp10, nn);
+        }
+        // bc_int for apply_stress_free (sps_set_bcs with ifsigman = 1 and wall
+        // dummies): zero before the first derivative pass (cleared below)
+        if (params->no_bcs > 0 && nt2 > nt) {
+            take(h->nodeinfo, nn); take(h->bcint_prev, nn);
+        }
+        if (h->xsph) take(h->xsph_v, (size_t)nt);
+    });
     if (!rc) rc = alloc_lists(h);
     if (rc) return bail(rc);
     if (hipHostMalloc((void **)&h->pinned, 64 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
@@ -1687,6 +1736,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     for (auto e : h->ev_pool) (void)hipEventDestroy(e);
     if (h->ev_disp) (void)hipEventDestroy(h->ev_disp);
     drop_graphs(h);
+    free_lists(h);
     dfree(h->stepv);
     h->S[0].release();
     h->S[1].release();
@@ -1696,7 +1746,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     dfree(h->cellkey); dfree(h->cell); dfree(h->kcount); dfree(h->kstart);
     dfree(h->kfill); dfree(h->tmp_orig); dfree(h->tmp_src); dfree(h->proc); dfree(h->proc_to_slot); dfree(h->moved);
     dfree(h->cnt); dfree(h->off); dfree(h->scan_state); dfree(h->scan_ticket); dfree(h->cstart_rm); dfree(h->err);
-    dfree(h->list_mem); dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->type_counts); dfree(h->tiles); dfree(h->plans);
+    dfree(h->deg_a); dfree(h->deg_b); dfree(h->tile_ok); dfree(h->tile_start); dfree(h->tile_range); dfree(h->type_counts); dfree(h->tiles); dfree(h->plans);
     dfree(h->xsph_v);
     dfree(h->x_build); dfree(h->dmax); dfree(h->surr_count); dfree(h->surr_slot); dfree(h->surr_sn);
     dfree(h->surr_str); dfree(h->surr_feat); dfree(h->surr_stats); dfree(h->plog); dfree(h->surr_mat);
@@ -1707,6 +1757,7 @@ extern "C" void sps_destroy(sps_handle *h) {
     if (h->pinned) (void)hipHostFree(h->pinned);
     if (h->read_pin) (void)hipHostFree(h->read_pin);
     dfree(h->read_dev);
+    dfree(h->mem);
     for (hipEvent_t e : h->read_ev)
         if (e) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamDestroy(h->stream);

@@ -115,7 +115,7 @@ def build(out=None, asan=True, defines=()):
     generate(gen)
     out = out or os.path.join(BUILD, f"libsps_emu{'_' + tag if tag else ''}.so")
     flags = ["-std=c++17", "-O1", "-g", "-fPIC", "-shared", "-ffp-contract=off", "-fno-fast-math",
-             "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0", "-Wno-unknown-pragmas", "-Wno-unused-result",
+             "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0", "-DSPS_SEPARATE_BUFFERS", "-Wno-unknown-pragmas", "-Wno-unused-result",
              "-I" + HERE, "-I" + os.path.join(ROOT, "include"), "-I" + gen]
     if asan:
         flags += ["-fsanitize=address", "-fno-omit-frame-pointer"]
