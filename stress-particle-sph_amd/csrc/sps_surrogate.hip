@@ -98,8 +98,8 @@ __device__ __forceinline__ void put_weight(bf16_t *__restrict__ wf, bf16_t *__re
 // The weights of a layer (32 KiB, in operand order) are fetched into registers
 // while the layer before multiplies.  A launch per product with its operands
 // gathered two bytes at a time took 530 us for 58 k rows, with 46 us for the
-// activation's derivative and 390 us for the bias gradients; this takes 83 us,
-// k_gemm_bf16_dw 23 us.  What is left here is mostly the activation: two
+// activation's derivative and 390 us for the bias gradients; this takes 62 us,
+// k_gemm_bf16_dw 22 us.  What is left here is mostly the activation: two
 // exponentials and two correctly rounded divisions a value.
 // Rows past nb (or *nbdev) count as zero inputs and have zero gradients.
 struct NetPass {
